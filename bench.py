@@ -71,11 +71,26 @@ def kernel_bytes(sim, electric):
     return s * (2 * n_own + n_other) + 4 * s * n_cpml + 2 * s * n_upml
 
 
+def sweep_bytes(sim):
+    """Algorithmic HBM bytes of a one-sweep step: every field word read and
+    written once, and the absorber words of both field types as in
+    kernel_bytes."""
+    from gmes_amd import constant as const
+    from gmes_amd._abi import NUMPY_DTYPE
+    s = NUMPY_DTYPE[sim.dtype_code]().itemsize
+    n = sum(sim._arrays[c].size for c in const.COMPONENTS if c in sim._active)
+    # kernel_bytes counts 2 own + 1 other per launch: the second reading of
+    # each type falls away
+    return kernel_bytes(sim, True) + kernel_bytes(sim, False) - s * n
+
+
 def measured_traffic(n, fam):
     """HBM bytes per launch of the dominant kernel from the committed
     rocprofv3 FETCH_SIZE/WRITE_SIZE summary (copy-kernel scaled), for the
-    256^3 FP32 workload only; None otherwise."""
-    path = os.path.join(ROOT, "profiles", "k_main3d_spheres256_fp32.md")
+    256^3 FP32 workload only; None otherwise.  fam: "step" (one-sweep step)
+    or "E", "H" (two-kernel step)."""
+    path = os.path.join(ROOT, "profiles", "k_step3d_spheres256_fp32.md" if fam == "step"
+                        else "k_main3d_spheres256_fp32.md")
     if n != 256 or not os.path.exists(path):
         return None
     key = "traffic_bytes_per_launch_%s:" % fam
@@ -565,20 +580,22 @@ def main():
     lib.profile(sim._sim, 0)
     fam = 0 if ms[0] >= ms[1] else 1
     avg_ms = ms[fam] / max(1, launches[fam])
-    nbytes = kernel_bytes(sim, electric=(fam == 0))
+    sweep = launches[1] == 0  # E and H in one kernel
+    nbytes = sweep_bytes(sim) if sweep else kernel_bytes(sim, electric=(fam == 0))
     achieved = nbytes / (avg_ms * 1e-3) / 1e9
     other = 1 - fam
     other_avg = ms[other] / max(1, launches[other])
-    other_gbps = kernel_bytes(sim, electric=(other == 0)) / (other_avg * 1e-3) / 1e9
+    other_gbps = None if sweep else round(kernel_bytes(sim, electric=(other == 0)) / (other_avg * 1e-3) / 1e9, 1)
     log("kernel ms/launch: E %.4f H %.4f ghost %.4f src %.4f" % (
         ms[0] / max(1, launches[0]), ms[1] / max(1, launches[1]),
         ms[4] / max(1, launches[4]), ms[3] / max(1, launches[3])))
     roofline = dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK_GBPS, unit="GB/s",
                     frac=round(achieved / HBM_PEAK_GBPS, 4),
-                    traffic=measured_traffic(n, "E" if fam == 0 else "H"),
-                    kernel="k_main3d<%s, float, 1, false, true, true, false>" % ("true" if fam == 0 else "false"),
+                    traffic=measured_traffic(n, "step" if sweep else "E" if fam == 0 else "H"),
+                    kernel="k_step3d<float, 1, false>" if sweep else
+                    "k_main3d<%s, float, 1, false, true, true, false>" % ("true" if fam == 0 else "false"),
                     bytes_per_launch=int(nbytes), avg_launch_ms=round(avg_ms, 5),
-                    other_kernel_gbps=round(other_gbps, 1))
+                    other_kernel_gbps=other_gbps)
     cg = copy_gbps()
     roofline["copy_gbps"] = round(cg, 1)
     if roofline["traffic"]:

@@ -7,11 +7,13 @@ order; packed-FP32 instructions are disabled for the device code.
 import os
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "lib", "libgmes_engine.so")
-SOURCES = ["engine.hip", "kernels.hip"]
+# (file, extra flags): kernels.hip is compiled once per storage type
+SOURCES = [("engine.hip", [])] + [("kernels.hip", ["-DGMES_TYPE=%d" % t]) for t in range(4)] + [("step3d.hip", [])]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("GMES_OFFLOAD_ARCH", "gfx950")
 
@@ -22,12 +24,24 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared", "--offload-arch=" + ARCH,
 
 
 def build(verbose=True):
+    """Compile the sources side by side, then link them."""
     os.makedirs(os.path.dirname(LIB), exist_ok=True)
     tmp = LIB + ".tmp"
-    cmd = [HIPCC] + FLAGS + ["-o", tmp] + [os.path.join(HERE, s) for s in SOURCES]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.run(cmd, check=True)
+    with tempfile.TemporaryDirectory() as d:
+        jobs = []
+        for n, (src, extra) in enumerate(SOURCES):
+            obj = os.path.join(d, "%d.o" % n)
+            cmd = [HIPCC] + [f for f in FLAGS if f != "-shared"] + extra + ["-c", "-o", obj, os.path.join(HERE, src)]
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            jobs.append((cmd, obj, subprocess.Popen(cmd)))
+        for cmd, _, p in jobs:
+            if p.wait() != 0:
+                raise subprocess.CalledProcessError(p.returncode, cmd)
+        cmd = [HIPCC, "-shared", "-fPIC", "--offload-arch=" + ARCH, "-o", tmp] + [o for _, o, _ in jobs]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        subprocess.run(cmd, check=True)
     os.replace(tmp, LIB)
     return LIB
 

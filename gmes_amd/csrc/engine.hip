@@ -18,6 +18,10 @@
 #include <numeric>
 #include <shared_mutex>
 #include <string>
+#include <unordered_set>
+#include <system_error>
+#include <thread>
+#include <atomic>
 #include <vector>
 
 #include "engine_kernels.h"
@@ -80,6 +84,30 @@ struct CaptureGuard {
     if (held) g_capture_mu.lock_shared();
   }
 };
+
+// f(0) .. f(n - 1) on a few threads (passes over all cells of a sim while it
+// is being set up); f writes only what is its own.
+template <class F>
+void host_parallel(int n, F f) {
+  const int nt = std::min<int>(n, std::min(8u, std::max(1u, std::thread::hardware_concurrency())));
+  std::atomic<int> next{0};
+  std::atomic<bool> failed{false};
+  auto work = [&] {
+    try {
+      for (int q = next++; q < n; q = next++) f(q);
+    } catch (const std::bad_alloc&) {
+      failed = true;
+    }
+  };
+  std::vector<std::thread> t;
+  try {
+    for (int q = 1; q < nt; ++q) t.emplace_back(work);
+  } catch (const std::system_error&) {  // no more threads: the ones there do it
+  }
+  work();
+  for (auto& x : t) x.join();
+  if (failed) throw std::bad_alloc();
+}
 
 hipError_t dev_release(void* p) { return hipFree(p); }
 hipError_t device_drain() { return hipDeviceSynchronize(); }
@@ -176,16 +204,10 @@ int upload_byte_ids(gmes_sim* s) {
       int rc = dev_alloc(s, (void**)&s->ids8[c], (size_t)s->dsize[c]);
       if (rc) return rc;
     }
-    const std::vector<uint16_t>& ids = s->host_ids[c];
-    std::vector<uint8_t> dev((size_t)s->dsize[c], 0);
-    const int64_t rows = s->shape[c][0] * s->shape[c][1], n2 = s->shape[c][2];
-    for (int64_t r = 0; r < rows; ++r) {
-      uint8_t* d = dev.data() + kPad - s->koff[c] + r * s->pitch[c];
-      const uint16_t* h = ids.data() + r * n2;
-      for (int64_t k = 0; k < n2; ++k) d[k] = (uint8_t)h[k];
-    }
-    HIP_TRY(hipMemcpy(s->ids8[c], dev.data(), dev.size(), hipMemcpyHostToDevice));
+    launch_narrow_ids(s->ids[c], s->ids8[c], s->dsize[c], s->stream);  // pads included
+    HIP_TRY(hipGetLastError());
   }
+  HIP_TRY(hipStreamSynchronize(s->stream));
   return GMES_OK;
 }
 
@@ -712,16 +734,24 @@ void dft_jobs(const gmes_sim* s, std::vector<DftJob<T>>& out, int64_t& block0) {
   }
 }
 
+// The device table holds the jobs on the buffers of either parity
+// (gmes_sim::par), half after half.
 template <class T>
 int upload_dft_jobs_t(gmes_sim* s) {
   std::vector<DftJob<T>> jobs;
-  int64_t nb = 0;
-  dft_jobs<T>(s, jobs, nb);
-  s->dft_blocks = nb;
+  for (int p = 0; p < 2; ++p) {
+    int64_t nb = 0;
+    std::vector<DftJob<T>> half;
+    dft_jobs<T>(s, half, nb);
+    if (p != s->par && s->f_alt[0])
+      for (auto& J : half) J.f = static_cast<T*>(s->f_alt[J.comp]);
+    s->dft_blocks = nb;
+    jobs.insert(jobs.end(), half.begin(), half.end());
+  }
   if (jobs.empty()) return GMES_OK;
-  // capacity for 16 monitors: adding monitors rarely reallocates (a free
+  // capacity for 16 monitors on two buffer sets: adding monitors rarely reallocates (a free
   // would wait for every kernel on the device)
-  const int64_t need = std::max<int64_t>(16, (int64_t)jobs.size());
+  const int64_t need = std::max<int64_t>(32, (int64_t)jobs.size());
   if (need > s->dft_jobs_cap) {
     if (s->d_dft_jobs) HIP_TRY(dev_release(s->d_dft_jobs));
     s->d_dft_jobs = nullptr;
@@ -744,7 +774,8 @@ int upload_dft_jobs(gmes_sim* s) {
 template <class T>
 void enqueue_dft(gmes_sim* s, hipStream_t st) {
   if (s->dfts.empty()) return;
-  launch_dft_batch<T>(static_cast<const DftJob<T>*>(s->d_dft_jobs), (int)s->dfts.size(), s->dft_blocks, st);
+  launch_dft_batch<T>(static_cast<const DftJob<T>*>(s->d_dft_jobs) + s->par * s->dfts.size(), (int)s->dfts.size(),
+                      s->dft_blocks, st);
 }
 
 void enqueue_step(gmes_sim* s, hipStream_t st);
@@ -760,8 +791,567 @@ void enqueue_aux_steps(gmes_sim* s, hipStream_t st) {
   }
 }
 
+bool on_ghost_copy_plane(const gmes_sim* s, int c, int64_t x, bool source, bool ghost);
+hipError_t sync_exec(gmes_sim* s);
+
+// ---- one-sweep steps (step3d.hip)
+//
+// A real FP32 or FP64, or complex FP32, 3-D sim takes them when
+//   * it holds only Dummy, Const and Dielectric cells and, in real FP32, one
+//     kind of absorber with one profile set, whose two rows per axis agree (a
+//     single Shell).  (With 8-byte words the absorber kernels need more than
+//     128 registers: FP64 171 x 150 x 139 CPML 230 us per step, 188 us with
+//     two kernels.)
+//   * three whole (j, k) rows fit a block (nz <= 341), so that at most half of
+//     the E work is done twice,
+//   * its distinct triples of records fit a block's LDS,
+//   * every source is a single point operation per cell, on few cells, off
+//     the ghost planes, and no E probe sits on a ghost plane (it reads the
+//     plane before the copy),
+//   * a component's CPML state is under 4 GiB (32-bit byte offsets), and
+//   * the caller asked for no tile and did not turn ghost fusion off.
+// Other sims keep the two-kernel step.
+constexpr int kSweepMinRows = 3;
+constexpr int64_t kSweepMaxTab = 24 * 1024;  // bytes of entries in LDS
+constexpr int kSweepMaxSrc = 16;
+constexpr int kSweepFloor = 20;        // waves whose plane takes as long as the latency of one
+constexpr int64_t kSweepLds = 160 * 1024;
+
+// The two rows read along each axis by one field type agree; CPML: inside
+// the run without live state every row is (b, 0, 1).
+bool sweep_rows_agree(const gmes_sim* s, int width) {
+  for (int e = 0; e < 2; ++e) {
+    const int32_t* run = e ? s->sweep_run_h : s->sweep_run_e;
+    const int c0 = e ? 3 : 0;
+    const int pairs[3][2] = {{c0 + 1, c0 + 2}, {c0, c0 + 2}, {c0, c0 + 1}};
+    for (int a = 0; a < 3; ++a) {
+      const std::vector<double>& r0 = s->prof_host[0][pairs[a][0]][a];
+      const std::vector<double>& r1 = s->prof_host[0][pairs[a][1]][a];
+      if (s->prof_w[0][pairs[a][0]][a] != width || r0.empty() || r0 != r1 || s->prof_w[0][pairs[a][1]][a] != width)
+        return false;
+      if (width == 6 && (s->prof_w[0][c0 + a][a] != 6 || s->prof_host[0][c0 + a][a].empty())) return false;
+      if (width == 3)
+        for (int q = run[a] & 0xFFFF; q < (run[a] >> 16) && 3 * (size_t)q + 2 < r0.size(); ++q)
+          if (r0[3 * (size_t)q + 1] != 0.0 || r0[3 * (size_t)q + 2] != 1.0) return false;
+    }
+  }
+  return true;
+}
+
+// A box of storage coordinates (per axis lo | hi << 16) holding no UPML cell
+// of any component, from the runs of non-UPML cells through the centres;
+// empty runs when the box is not free.
+void upml_free_box(const gmes_sim* s, int32_t box[3]) {
+  for (int a = 0; a < 3; ++a) box[a] = 0;
+  int64_t lo[3] = {0, 0, 0}, hi[3] = {0x7FFF, 0x7FFF, 0x7FFF};
+  for (int c = 0; c < 6; ++c) {
+    const int64_t* n = s->shape[c];
+    const std::vector<uint16_t>& ids = s->host_ids[c];
+    for (int a = 0; a < 3; ++a) {
+      int64_t ix[3] = {n[0] / 2, n[1] / 2, n[2] / 2};
+      auto upml_at = [&](int64_t v) {
+        ix[a] = v;
+        return s->recs[ids[(ix[0] * n[1] + ix[1]) * n[2] + ix[2]]].cls == GMES_CLS_UPML;
+      };
+      const int64_t mid = n[a] / 2;
+      if (upml_at(mid)) return;
+      int64_t l = mid, h = mid + 1;
+      while (l > 0 && !upml_at(l - 1)) --l;
+      while (h < n[a] && !upml_at(h)) ++h;
+      lo[a] = std::max(lo[a], l);
+      hi[a] = std::min(hi[a], h);
+    }
+  }
+  for (int a = 0; a < 3; ++a)
+    if (lo[a] >= hi[a]) return;
+  for (int c = 0; c < 6; ++c) {
+    const int64_t* n = s->shape[c];
+    const std::vector<uint16_t>& ids = s->host_ids[c];
+    std::vector<char> upml(s->recs.size());
+    for (size_t r = 0; r < upml.size(); ++r) upml[r] = s->recs[r].cls == GMES_CLS_UPML;
+    for (int64_t i = lo[0]; i < std::min(hi[0], n[0]); ++i)
+      for (int64_t j = lo[1]; j < std::min(hi[1], n[1]); ++j)
+        for (int64_t k = lo[2]; k < std::min(hi[2], n[2]); ++k)
+          if (upml[ids[(i * n[1] + j) * n[2] + k]]) return;
+  }
+  for (int a = 0; a < 3; ++a) box[a] = (int32_t)(lo[a] | (hi[a] << 16));
+}
+
+// The coordinates lo | hi << 16 along an axis where the CPML rows that E (or
+// H) components read there have no live state: c = 0 on the longest run.
+// (The H rows of the two components are read at storage index i + 1, up to
+// the last one.)
+int32_t sweep_dead_run(const gmes_sim* s, bool electric, int axis) {
+  const int c = (electric ? 0 : 3) + (axis == 0 ? 1 : 0);  // a component with that curl axis
+  const std::vector<double>& v = s->prof_host[0][c][axis];
+  if (s->prof_w[0][c][axis] != 3 || v.empty()) return 0;
+  const int len = (int)(v.size() / 3);
+  int lo = 0, hi = 0;
+  for (int q = 0; q < len;) {
+    if (v[3 * (size_t)q + 1] != 0.0) { ++q; continue; }
+    int e = q;
+    while (e < len && v[3 * (size_t)e + 1] == 0.0) ++e;
+    if (e - q > hi - lo) { lo = q; hi = e; }
+    q = e;
+  }
+  return hi > 0x7FFF ? 0 : lo | (hi << 16);
+}
+
+// Whether every cell with live CPML state is a CPML cell (or a flagged one):
+// the sweep takes the update from the coordinate.
+bool sweep_live_cells_cpml(const gmes_sim* s) {
+  std::vector<char> ok(s->recs.size());
+  for (size_t r = 0; r < ok.size(); ++r) {
+    const int cls = s->recs[r].cls;
+    ok[r] = cls == GMES_CLS_CPML || cls == GMES_CLS_DUMMY || cls == GMES_CLS_CONST;
+  }
+  std::atomic<bool> all{true};
+  host_parallel(12, [&](int q) {
+    const int c = q / 2, a = q % 2 ? kAx2[c] : kAx1[c];
+    const int64_t* n = s->shape[c];
+    const int run = c < 3 ? s->sweep_run_e[a] : s->sweep_run_h[a], lo = run & 0xFFFF, hi = run >> 16;
+    int64_t ix[3];
+    for (ix[0] = 0; ix[0] < n[0] && all; ++ix[0]) {
+      if (a == 0 && ix[0] >= lo && ix[0] < hi) continue;
+      for (ix[1] = 0; ix[1] < n[1]; ++ix[1]) {
+        if (a == 1 && ix[1] >= lo && ix[1] < hi) continue;
+        const uint16_t* row = s->host_ids[c].data() + (ix[0] * n[1] + ix[1]) * n[2];
+        for (int64_t k = 0; k < n[2]; ++k) {
+          if (a == 2 && k >= lo && k < hi) { k = hi - 1; continue; }
+          if (!ok[row[k]]) all = false;
+        }
+      }
+    }
+  });
+  return all;
+}
+
+// The distinct triples of records of the cells one thread owns, of one field
+// type; entries[id] are the record ids of a triple's three components.
+// False when there are more than `most`.
+bool sweep_triples(const gmes_sim* s, bool electric, size_t most, std::vector<std::array<uint16_t, 3>>& entries) {
+  const int c0 = electric ? 0 : 3;
+  const int64_t nx = s->g.nx, ny = s->g.ny, nz = s->g.nz;
+  constexpr int kParts = 16;
+  std::vector<uint64_t> found[kParts];  // in the order of the cells
+  host_parallel(kParts, [&](int part) {
+    std::unordered_set<uint64_t> seen;
+    uint64_t last = ~0ull;
+    const uint16_t* src[3];
+    for (int64_t i = nx * part / kParts; i < nx * (part + 1) / kParts; ++i)
+      for (int64_t j = 0; j < ny; ++j) {
+        for (int t = 0; t < 3; ++t) {
+          const int64_t* n = s->shape[c0 + t];
+          // H cells sit one up along the axes across their own
+          const int64_t ii = i + (!electric && t != 0), jj = j + (!electric && t != 1), kk = !electric && t != 2;
+          src[t] = s->host_ids[c0 + t].data() + (ii * n[1] + jj) * n[2] + kk;
+        }
+        for (int64_t k = 0; k < nz; ++k) {
+          const uint64_t key = step_key(src[0][k], src[1][k], src[2][k]);
+          if (key == last) continue;
+          last = key;
+          if (seen.size() <= most && seen.insert(key).second) found[part].push_back(key);
+        }
+      }
+  });
+  std::unordered_set<uint64_t> seen;
+  for (const auto& part : found)
+    for (const uint64_t key : part) {
+      if (!seen.insert(key).second) continue;
+      if (entries.size() >= most) return false;
+      entries.push_back({(uint16_t)key, (uint16_t)(key >> 16), (uint16_t)(key >> 32)});
+    }
+  return true;
+}
+
+// Writes the entry ids of every cell on the device, from the material ids
+// there and hash tables of the triples (building them on the host and
+// copying them took 40 ms at 256^3).
+int sweep_ids(gmes_sim* s) {
+  std::vector<StepKey> tab[2];
+  for (int h = 0; h < 2; ++h) {
+    const auto& ent = h ? s->step_h : s->step_e;
+    size_t cap = 64;
+    while (cap < 4 * ent.size()) cap *= 2;
+    tab[h].assign(cap, StepKey{~0ull, 0});
+    for (size_t e = 0; e < ent.size(); ++e) {
+      const uint64_t key = step_key(ent[e][0], ent[e][1], ent[e][2]);
+      uint32_t at = step_hash(key, (uint32_t)cap - 1);
+      while (tab[h][at].key != ~0ull) at = (at + 1) & ((uint32_t)cap - 1);
+      tab[h][at] = StepKey{key, (uint64_t)e};
+    }
+  }
+  StepIdArgs a{};
+  const size_t b0 = tab[0].size() * sizeof(StepKey), b1 = tab[1].size() * sizeof(StepKey);
+  char* d = nullptr;
+  HIP_TRY(hipMalloc((void**)&d, b0 + b1));
+  hipError_t e = hipMemcpy(d, tab[0].data(), b0, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(d + b0, tab[1].data(), b1, hipMemcpyHostToDevice);
+  for (int h = 0; h < 2; ++h) {
+    a.tab[h] = reinterpret_cast<const StepKey*>(d + (h ? b0 : 0));
+    a.mask[h] = (uint32_t)tab[h].size() - 1;
+  }
+  for (int c = 0; c < 6; ++c) {
+    a.ids[c] = s->ids[c];
+    a.first[c] = dev_index(s, c, c >= 3 && c != 3, c >= 3 && c != 4, c >= 3 && c != 5);
+    a.plane[c] = s->shape[c][1] * s->pitch[c];
+    a.row[c] = s->pitch[c];
+  }
+  a.n[0] = s->g.nx; a.n[1] = s->g.ny; a.n[2] = s->g.nz;
+  a.pitch = s->pitch[0];
+  a.out = s->d_step_ids;
+  if (e == hipSuccess) {
+    launch_step_ids(a, s->stream);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
+  (void)dev_release(d);
+  HIP_TRY(e);
+  return GMES_OK;
+}
+
+template <class R>
+void sweep_entry(const gmes_sim* s, const std::array<uint16_t, 3>& rec, StepEnt<R>& e, StepRare rare[3]) {
+  e = StepEnt<R>{};
+  for (int t = 0; t < 3; ++t) {
+    const gmes_mat_rec& r = s->recs[rec[t]];
+    const bool upml = r.cls == GMES_CLS_UPML;
+    rare[t] = StepRare{r.cls == GMES_CLS_DUMMY ? 1 : r.cls == GMES_CLS_CONST ? 2 : 0, -1, GMES_SRC_SET, 0,
+                       r.value[0], r.value[1]};
+    if (rare[t].keep) e.meta |= kStepRareCell;
+    else e.c[t] = upml ? (s->fp64 ? (R)r.eps_mu : (R)(1.0 / r.eps_mu)) : (R)(s->g.dt / r.eps_mu);
+    if (upml) e.meta |= 2u << t;
+  }
+}
+
+// Rows per block and planes per block.  A block's march costs its planes and
+// two more (the rim plane, the prologue); blocks run in rounds over the 256
+// CUs, a last incomplete round costing about half of one; a CU with few
+// waves still pays the latency of a plane (kSweepFloor).  256^3 CPML, rows
+// of 256, blocks of 3 rows: 64 planes (one full round) 285 us, 32 planes 303,
+// 16 planes 312; 181 x 203 x 225 UPML: 3 rows 190 us, 4 rows (one block per
+// CU) 204.
+template <class T>
+void sweep_shape_t(gmes_sim* s, int nent) {
+  const int nx = s->g.nx, ny = s->g.ny, nz = s->g.nz;
+  double best = 1e300;
+  for (int rows = 2; rows <= ny + 1; ++rows) {
+    const int threads = (rows * nz + 63) / 64 * 64;
+    if (threads > kStepMaxThreads) break;
+    if (rows < kSweepMinRows && kSweepMinRows * nz <= kStepMaxThreads && ny + 1 >= kSweepMinRows) continue;
+    const int64_t lds = (int64_t)step3_lds<T>(threads, nent, rows, nz, s->sweep_absorber);
+    if (lds > kSweepLds) break;
+    const int waves = threads / 64, held = s->sweep_absorber ? 24 : sizeof(T) == 4 ? 32 : 20;
+    const int per_cu = std::max<int>(1, (int)std::min<int64_t>(held / waves, kSweepLds / lds));
+    const int nj = (ny + rows - 2) / (rows - 1);
+    const double plane = std::max(per_cu * waves, kSweepFloor);
+    for (int nch = 1; nch <= nx; ++nch) {
+      const int ch = (nx + nch - 1) / nch;
+      const double x = (double)nj * ((nx + ch - 1) / ch) / (256.0 * per_cu);
+      const double rounds = x <= 1 ? 1 : x + (std::ceil(x) > x ? 0.5 : 0);
+      const double cost = rounds * (ch + 2.0) * plane;
+      if (cost < best * 0.999) {
+        best = cost;
+        s->sweep_rows = rows;
+        s->sweep_threads = threads;
+        s->sweep_ch = ch;
+      }
+    }
+  }
+}
+
+void sweep_shape(gmes_sim* s) {
+  const int nent = (int)(s->step_e.size() + s->step_h.size()) + 2 * kSweepMaxSrc;
+  s->sweep_rows = 0;
+  switch (s->g.dtype) {
+    case GMES_F32: sweep_shape_t<float>(s, nent); break;
+    case GMES_F64: sweep_shape_t<double>(s, nent); break;
+    default: sweep_shape_t<cplx<float>>(s, nent); break;
+  }
+}
+
+void sweep_release(gmes_sim* s) {
+  void** bufs[] = {&s->f_alt[0], &s->f_alt[1], &s->f_alt[2], &s->f_alt[3], &s->f_alt[4], &s->f_alt[5],
+                   &s->pml_alt[0], &s->pml_alt[1], &s->pml_alt[2], (void**)&s->d_step_ids, &s->d_step_tab, (void**)&s->d_rare};
+  for (void** b : bufs)
+    if (*b) {
+      (void)dev_release(*b);
+      *b = nullptr;
+    }
+  s->bytes -= s->sweep_bytes;
+  s->sweep_bytes = 0;
+  s->sweep_ok = false;
+  s->step_tab_cap = 0;
+}
+
+int sweep_alloc(gmes_sim* s, void** p, size_t bytes) {
+  const int rc = dev_alloc(s, p, bytes);
+  if (!rc) s->sweep_bytes += (int64_t)std::max<size_t>(16, bytes);
+  return rc;
+}
+
+// Uploads the entry tables, those of source cells (after the step_net /
+// step_nht plain ones) included.
+template <class R>
+int sweep_upload_tab(gmes_sim* s, const std::vector<std::array<int, 3>>& se, const std::vector<std::array<int, 3>>& sh) {
+  // se, sh: (base entry, component 0..2, op index) of each source cell
+  const int net = (int)(s->step_e.size() + se.size()), nht = (int)(s->step_h.size() + sh.size());
+  std::vector<StepEnt<R>> tab((size_t)(net + nht));
+  std::vector<StepRare> rare((size_t)(net + nht) * 3);
+  for (size_t e = 0; e < s->step_e.size(); ++e) sweep_entry<R>(s, s->step_e[e], tab[e], &rare[3 * e]);
+  for (size_t e = 0; e < s->step_h.size(); ++e) sweep_entry<R>(s, s->step_h[e], tab[net + e], &rare[3 * (net + e)]);
+  for (int h = 0; h < 2; ++h) {
+    const auto& src = h ? sh : se;
+    const size_t base = h ? (size_t)net : 0, first = h ? (size_t)net + s->step_h.size() : s->step_e.size();
+    for (size_t q = 0; q < src.size(); ++q) {
+      const gmes_src_op& o = s->ops[src[q][2]];
+      const size_t d = first + q, b = base + src[q][0];
+      tab[d] = tab[b];
+      for (int t = 0; t < 3; ++t) rare[3 * d + t] = rare[3 * b + t];
+      tab[d].meta |= kStepRareCell;
+      rare[3 * d + src[q][1]].wave = o.wave;
+      rare[3 * d + src[q][1]].kind = o.kind;
+    }
+  }
+  HIP_TRY(hipMemcpy(s->d_step_tab, tab.data(), tab.size() * sizeof(StepEnt<R>), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(s->d_rare, rare.data(), rare.size() * sizeof(StepRare), hipMemcpyHostToDevice));
+  s->step_net = net;
+  s->step_nht = nht;
+  return GMES_OK;
+}
+
+// Marks the cells of the sim's source operations in the sweep's ids, when
+// all of them can be applied there (sweep_src_ok).
+int sweep_sources(gmes_sim* s) {
+  if (!s->sweep_ok) return GMES_OK;
+  HIP_TRY(sync_exec(s));
+  for (const auto& x : s->src_ids)
+    HIP_TRY(hipMemcpy(s->d_step_ids + x.first, &x.second, sizeof(uint32_t), hipMemcpyHostToDevice));
+  s->src_ids.clear();
+  s->sweep_src_ok = (int)s->ops.size() <= kSweepMaxSrc;
+  s->has_waves = false;
+  std::vector<std::array<int, 3>> src[2];
+  std::vector<int64_t> cell(s->ops.size());
+  const int64_t n[3] = {s->g.nx, s->g.ny, s->g.nz};
+  for (size_t q = 0; s->sweep_src_ok && q < s->ops.size(); ++q) {
+    const gmes_src_op& o = s->ops[q];
+    const int c = o.comp, h = c >= 3;
+    const int64_t sy = s->shape[c][1], sz = s->shape[c][2];
+    int64_t ix[3] = {o.cell / (sy * sz), (o.cell / sz) % sy, o.cell % sz};
+    bool ok = o.kind == GMES_SRC_SET || o.kind == GMES_SRC_SUB;
+    for (int a = 0; a < 3; ++a) {
+      if (h && a != c % 3) --ix[a];
+      if (ix[a] < 0 || ix[a] >= n[a]) ok = false;  // a ghost cell
+    }
+    cell[q] = (ix[0] * n[1] + ix[1]) * s->pitch[0] + ix[2];
+    for (size_t p = 0; p < q; ++p)
+      if (cell[p] == cell[q]) ok = false;  // two operations on one thread's cells
+    if (!ok) s->sweep_src_ok = false;
+  }
+  if (!s->sweep_src_ok) return GMES_OK;
+  for (size_t q = 0; q < s->ops.size(); ++q) {
+    const int h = s->ops[q].comp >= 3;
+    uint32_t w = 0;
+    HIP_TRY(hipMemcpy(&w, s->d_step_ids + cell[q], sizeof w, hipMemcpyDeviceToHost));
+    s->src_ids.push_back({cell[q], w});
+    const uint32_t id = (uint32_t)((h ? s->step_h.size() : s->step_e.size()) + src[h].size());
+    src[h].push_back({(int)(h ? w >> 16 : w & 0xFFFFu), s->ops[q].comp % 3, (int)q});
+    w = h ? (w & 0xFFFFu) | id << 16 : (w & 0xFFFF0000u) | id;
+    HIP_TRY(hipMemcpy(s->d_step_ids + cell[q], &w, sizeof w, hipMemcpyHostToDevice));
+  }
+  s->has_waves = !s->ops.empty();
+  return s->fp64 ? sweep_upload_tab<double>(s, src[0], src[1]) : sweep_upload_tab<float>(s, src[0], src[1]);
+}
+
+// Builds what one-sweep steps need (at commit); leaves sweep_ok false when
+// the sim does not qualify.
+int sweep_build(gmes_sim* s) {
+  sweep_release(s);
+  if (!is3d(s) || s->g.dtype == GMES_C128) return GMES_OK;
+  const int nz = s->g.nz;
+  if (kSweepMinRows * nz > kStepMaxThreads || s->g.ny < 2) return GMES_OK;
+  for (int c = 0; c < 6; ++c)  // 32-bit byte offsets, both state words included
+    if (2 * s->dsize[c] * s->esize >= (int64_t)0xFFFFFF00) return GMES_OK;
+  bool cpml = false, upml = false;
+  for (int c = 0; c < 6; ++c) {
+    cpml |= s->has_cls[c][GMES_CLS_CPML];
+    upml |= s->has_cls[c][GMES_CLS_UPML];
+    for (int k = GMES_CLS_DRUDE; k < GMES_NCLS; ++k)
+      if (s->has_cls[c][k]) return GMES_OK;
+  }
+  if ((cpml && upml) || ((cpml || upml) && s->nprof != 1)) return GMES_OK;
+  // the kernels keep every component's absorber state
+  if (cpml || upml) {
+    if (s->esize > 4) return GMES_OK;
+    for (int c = 0; c < 6; ++c)
+      if (!s->pml_state[c]) return GMES_OK;
+  }
+  s->sweep_absorber = cpml ? 1 : upml ? 2 : 0;
+  if (cpml)
+    for (int a = 0; a < 3; ++a) {
+      s->sweep_run_e[a] = sweep_dead_run(s, true, a);
+      s->sweep_run_h[a] = sweep_dead_run(s, false, a);
+    }
+  if (upml) {
+    upml_free_box(s, s->sweep_run_e);
+    for (int a = 0; a < 3; ++a) s->sweep_run_h[a] = s->sweep_run_e[a];
+  }
+  if (s->sweep_absorber && !sweep_rows_agree(s, cpml ? 3 : 6)) return GMES_OK;
+  if (cpml && !sweep_live_cells_cpml(s)) return GMES_OK;
+  // FP64: divisions by powers of two are exact multiplications
+  auto pow2 = [](double v) { int e; return std::frexp(v, &e) == 0.5; };
+  bool exact = pow2(s->g.dx) && pow2(s->g.dy) && pow2(s->g.dz);
+  for (int c = 0; c < 6 && cpml; ++c)
+    for (int a = 0; a < 3; ++a)
+      for (size_t q = 2; q < s->prof_host[0][c][a].size(); q += 3) exact = exact && s->prof_host[0][c][a][q] == 1.0;
+  s->sweep_exact = exact;
+  s->step_e.clear();
+  s->step_h.clear();
+  const size_t ent = s->fp64 ? sizeof(StepEnt<double>) : sizeof(StepEnt<float>);
+  const size_t most = (size_t)kSweepMaxTab / ent - 2 * kSweepMaxSrc;
+  if (!sweep_triples(s, true, most, s->step_e) || !sweep_triples(s, false, most, s->step_h) ||
+      s->step_e.size() + s->step_h.size() > most)
+    return GMES_OK;
+  sweep_shape(s);
+  if (!s->sweep_rows) return GMES_OK;
+  int rc = GMES_OK;
+  for (int c = 0; c < 6 && !rc; ++c) rc = sweep_alloc(s, &s->f_alt[c], (size_t)s->dsize[c] * s->esize);
+  for (int c = 0; c < 3 && !rc; ++c) {
+    if (!s->pml_state[c]) continue;
+    const size_t b = (size_t)(cpml ? 2 : 1) * s->dsize[c] * s->esize;
+    rc = sweep_alloc(s, &s->pml_alt[c], b);
+    if (!rc) HIP_TRY(hipMemset(s->pml_alt[c], 0, b));
+  }
+  if (!rc) rc = sweep_alloc(s, (void**)&s->d_step_ids, (size_t)s->g.nx * s->g.ny * s->pitch[0] * sizeof(uint32_t));
+  s->step_tab_cap = (int64_t)(s->step_e.size() + s->step_h.size()) + 2 * kSweepMaxSrc;
+  if (!rc) rc = sweep_alloc(s, &s->d_step_tab, (size_t)s->step_tab_cap * ent);
+  if (!rc) rc = sweep_alloc(s, (void**)&s->d_rare, (size_t)s->step_tab_cap * 3 * sizeof(StepRare));
+  if (rc) {  // no room for a second set of buffers: the two-kernel step needs none
+    (void)hipGetLastError();
+    sweep_release(s);
+    return GMES_OK;
+  }
+  if ((rc = sweep_ids(s))) return rc;
+  s->src_ids.clear();
+  s->sweep_ok = true;
+  return GMES_OK;
+}
+
+// Whether the next step of s is a one-sweep step.
+bool sweeps(const gmes_sim* s) {
+  if (!s->sweep_ok || !s->sweep_src_ok || !s->allow_fuse || s->naux || s->parent) return false;
+  if (s->tile_bx > 0 && !s->tile_tuned) return false;
+  for (const auto& p : s->probes)
+    if (p.comp < 3 && on_ghost_copy_plane(s, p.comp, p.cell, false, true)) return false;
+  return true;
+}
+
+// Whether something reads ghost planes between the steps of one call (else
+// only its last step writes them).
+bool sweep_ghosts(const gmes_sim* s) {
+  auto on_ghost = [&](int c, int a, int64_t lo, int64_t hi) {
+    return a != c % 3 && (c < 3 ? hi > s->shape[c][a] - 1 : lo < 1);
+  };
+  for (const auto& p : s->probes) {
+    const int64_t sy = s->shape[p.comp][1], sz = s->shape[p.comp][2];
+    const int64_t ix[3] = {p.cell / (sy * sz), (p.cell / sz) % sy, p.cell % sz};
+    for (int a = 0; a < 3; ++a)
+      if (on_ghost(p.comp, a, ix[a], ix[a] + 1)) return true;
+  }
+  for (const auto& d : s->dfts)
+    for (int a = 0; a < 3; ++a)
+      if (on_ghost(d.comp, a, d.lo[a], d.lo[a] + d.n[a])) return true;
+  return false;
+}
+
+template <class T>
+Step3Args<T> step3_args(const gmes_sim* s) {
+  using R = typename real_of<T>::type;
+  Step3Args<T> m{};
+  auto rsrc = [](const void* p, int64_t bytes) {
+    const uint64_t a = (uint64_t)(uintptr_t)p;
+    // raw buffer: stride 0, 32-bit data format
+    return i4_t{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)(uint32_t)bytes, 0x00020000};
+  };
+  for (int c = 0; c < 6; ++c) {
+    const int64_t o = (int64_t)(kPad - s->koff[c]) * s->esize, b = s->dsize[c] * s->esize - o;
+    const int64_t sb = b + (s->sweep_absorber == 1 ? s->dsize[c] * s->esize : 0);
+    auto at = [&](const void* p, int64_t n) { return p ? rsrc(static_cast<const char*>(p) + o, n) : i4_t{0, 0, 0, 0}; };
+    (c < 3 ? m.ei[c] : m.hi[c - 3]) = at(s->f[c], b);
+    (c < 3 ? m.eo[c] : m.ho[c - 3]) = at(s->f_alt[c], b);
+    if (c < 3) {
+      m.si[c] = at(s->pml_state[c], sb);
+      m.so[c] = at(s->pml_alt[c], sb);
+    } else {
+      m.sh[c - 3] = at(s->pml_state[c], sb);
+    }
+    m.ds[c] = (unsigned)(s->dsize[c] * s->esize);
+    for (int a = 0; a < 3; ++a) {
+      const cplx<R> ph{(R)s->g.phase[c][a][0], (R)s->g.phase[c][a][1]};
+      if (c < 3) m.pe[c][a] = ph;
+      else m.ph[c - 3][a] = ph;
+    }
+  }
+  m.W0 = s->pitch[0];
+  m.W2 = s->pitch[2];
+  m.n[0] = s->g.nx; m.n[1] = s->g.ny; m.n[2] = s->g.nz;
+  m.ids = rsrc(s->d_step_ids, (int64_t)s->g.nx * s->g.ny * s->pitch[0] * 4);
+  m.exact = s->sweep_exact;
+  m.ghosts = s->sweep_ghosts;
+  m.tab = s->d_step_tab;
+  m.rare = s->d_rare;
+  m.net = s->step_net;
+  m.nht = s->step_nht;
+  m.d[0] = (R)s->g.dx; m.d[1] = (R)s->g.dy; m.d[2] = (R)s->g.dz;
+  m.inv_d[0] = (R)(1.0 / s->g.dx); m.inv_d[1] = (R)(1.0 / s->g.dy); m.inv_d[2] = (R)(1.0 / s->g.dz);
+  const R* prof = static_cast<const R*>(s->d_prof);
+  // rows two components share: x of the 2nd, y and z of the 1st; own rows
+  const int sc[3] = {1, 0, 0};
+  for (int a = 0; a < 3; ++a) {
+    m.re[a] = prof + s->prof_off0[sc[a]][a];
+    m.rh[a] = prof + s->prof_off0[3 + sc[a]][a];
+    m.oe[a] = prof + s->prof_off0[a][a];
+    m.oh[a] = prof + s->prof_off0[3 + a][a];
+    m.run_e[a] = s->sweep_run_e[a];
+    m.run_h[a] = s->sweep_run_h[a];
+  }
+  m.rows = s->sweep_rows;
+  m.ch = s->sweep_ch;
+  m.nj = (s->g.ny + m.rows - 2) / (m.rows - 1);
+  m.nblk = m.nj * ((s->g.nx + m.ch - 1) / m.ch);
+  m.waves = s->has_waves ? s->d_waves : nullptr;
+  m.ctl = reinterpret_cast<Ctl*>(s->d_clock);
+  m.par = s->par;
+  return m;
+}
+
+// The current buffers become the other set.
+void sweep_swap(gmes_sim* s) {
+  for (int c = 0; c < 6; ++c) std::swap(s->f[c], s->f_alt[c]);
+  for (int c = 0; c < 3; ++c)
+    if (s->pml_alt[c]) std::swap(s->pml_state[c], s->pml_alt[c]);
+  s->par ^= 1;
+}
+
+template <class T>
+void enqueue_sweep(gmes_sim* s, hipStream_t st) {
+  if constexpr (!std::is_same<T, cplx<double>>::value) {
+    time_begin(s, 0, st);
+    launch_step3d<T>(step3_args<T>(s), s->sweep_absorber, s->sweep_threads, st);
+    time_end(s, st);
+    sweep_swap(s);
+  }
+}
+
 template <class T>
 void enqueue_step_t(gmes_sim* s, hipStream_t st) {
+  if (sweeps(s)) {
+    enqueue_sweep<T>(s, st);
+    enqueue_probe<T>(s, true, st);
+    enqueue_probe<T>(s, false, st);
+    enqueue_dft<T>(s, st);
+    return;
+  }
   enqueue_ghost<T>(s, false, 1, st);
   enqueue_main<T>(s, true, st);
   enqueue_ade<T>(s, st);
@@ -872,7 +1462,11 @@ int build_graph(gmes_sim* s) {
   {
     CaptureGuard capture;
     HIP_TRY(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_step(s, s->stream);
+    // one-sweep steps swap the buffers: a graph of two returns them
+    s->graph_par = s->par;
+    s->graph_steps = sweeps(s) ? 2 : 1;
+    s->sweep_ghosts = sweep_ghosts(s);
+    for (int t = 0; t < s->graph_steps; ++t) enqueue_step(s, s->stream);
     HIP_TRY(hipStreamEndCapture(s->stream, &graph));
   }
   hipError_t e = hipGraphInstantiate(&s->graph_exec, graph, nullptr, nullptr, 0);
@@ -908,14 +1502,34 @@ int do_step(gmes_sim* s, int64_t n) {
   if (rc) return rc;
   if ((rc = ensure_probe_capacity(s, n))) return rc;
   HIP_TRY(hipSetDevice(s->device));
+  const bool sweep = sweeps(s);
+  if (!sweep) {
+    s->clk_stale = true;
+  } else if (s->clk_stale && n > 0) {
+    launch_clock_copy(reinterpret_cast<Ctl*>(s->d_clock), s->stream);
+    s->clk_stale = false;
+  }
+  const int par = s->par;
   if (s->use_graph && !any_graph_blocker(s)) {
-    if (s->graph_dirty || !s->graph_exec)
+    if (s->graph_dirty || !s->graph_exec || s->graph_steps != (sweep ? 2 : 1))
       if ((rc = build_graph(s))) return rc;
-    for (int64_t t = 0; t < n; ++t) HIP_TRY(hipGraphLaunch(s->graph_exec, s->stream));
+    int64_t t = 0;
+    const int64_t last = sweep ? 1 : 0;  // the step that writes the ghost planes
+    if (s->par != s->graph_par && t + last < n) { enqueue_step(s, s->stream); ++t; }
+    for (; t + s->graph_steps + last <= n; t += s->graph_steps) HIP_TRY(hipGraphLaunch(s->graph_exec, s->stream));
+    for (; t < n; ++t) {
+      s->sweep_ghosts = sweep_ghosts(s) || t == n - 1;
+      enqueue_step(s, s->stream);
+    }
+    HIP_TRY(hipGetLastError());
   } else {
-    for (int64_t t = 0; t < n; ++t) enqueue_step(s, s->stream);
+    for (int64_t t = 0; t < n; ++t) {
+      s->sweep_ghosts = sweep_ghosts(s) || t == n - 1;
+      enqueue_step(s, s->stream);
+    }
     HIP_TRY(hipGetLastError());
   }
+  if (s->par != par) ++s->gen;  // a batch's graph may hold the other set's pointers
   advance_host_clock(s, n);
   s->probe_n = s->step - s->probe_base;
   if (s->timing.on && s->timing.pending.size() > 4096) return collect_timing(s);
@@ -1244,6 +1858,7 @@ int gmes_sim_destroy(gmes_sim* s) {
     if (s->pml_state[c]) (void)dev_release(s->pml_state[c]);
   }
   free_ade(s);
+  sweep_release(s);
   for (auto& d : s->dfts)
     if (d.acc) (void)dev_release(d.acc);
   void* bufs[] = {s->d_recs, s->d_coef, s->d_prof, s->d_prof_off, s->d_ops, s->d_groups, s->d_waves,
@@ -1350,6 +1965,18 @@ int gmes_sim_commit(gmes_sim* s) {
   HIP_TRY(sync_exec(s));
   free_ade(s);
   s->ade_on_ghost_source = false;
+  std::vector<int64_t> counts[6];  // cells per record; empty: an id is out of range
+  host_parallel(6, [&](int c) {
+    if (!active(s, c)) return;
+    counts[c].assign(s->recs.size(), 0);
+    for (const uint16_t id : s->host_ids[c]) {
+      if (id >= counts[c].size()) {
+        counts[c].clear();
+        return;
+      }
+      ++counts[c][id];
+    }
+  });
   for (int c = 0; c < 6; ++c) {
     for (int k = 0; k < GMES_NCLS; ++k) s->has_cls[c][k] = false;
     if (!active(s, c)) continue;
@@ -1360,12 +1987,8 @@ int gmes_sim_commit(gmes_sim* s) {
     std::vector<std::vector<uint16_t>> recs(GMES_NCLS);
     std::vector<int> words(GMES_NCLS, 0);
     // records in use
-    std::vector<int64_t> count(s->recs.size(), 0);
-    for (int64_t x = 0; x < s->ncell[c]; ++x) {
-      const uint16_t id = ids[x];
-      if (id >= s->recs.size()) return set_error(GMES_ERANGE, "material id out of range");
-      ++count[id];
-    }
+    const std::vector<int64_t>& count = counts[c];
+    if (count.empty()) return set_error(GMES_ERANGE, "material id out of range");
     bool any_ade = false;
     for (size_t id = 0; id < s->recs.size(); ++id) {
       if (!count[id]) continue;
@@ -1458,10 +2081,12 @@ int gmes_sim_commit(gmes_sim* s) {
   profile_prefetch(s);
   upml_box(s);
   upml_rows(s);
+  if ((rc = sweep_build(s))) return rc;
+  if ((rc = sweep_sources(s))) return rc;
   s->committed = true;
   destroy_graph(s);
   decide_fusion(s);
-  return GMES_OK;
+  return s->dfts.empty() ? GMES_OK : upload_dft_jobs(s);  // the jobs hold the buffers' addresses
 }
 
 int gmes_sim_set_sources(gmes_sim* s, const gmes_src_op* ops, int64_t nops, int32_t nwaves) {
@@ -1492,6 +2117,7 @@ int gmes_sim_set_sources(gmes_sim* s, const gmes_src_op* ops, int64_t nops, int3
   s->ops.assign(ops, ops + nops);
   s->nwaves = nwaves;
   int rc = s->fp64 ? upload_sources<double>(s) : upload_sources<float>(s);
+  if (!rc) rc = sweep_sources(s);
   destroy_graph(s);
   decide_fusion(s);
   return rc;
@@ -1798,6 +2424,7 @@ static int blob_copy(gmes_sim* s, char* p, bool save, int64_t& done) {
     Ctl c;
     HIP_TRY(hipMemcpy(&c, s->d_clock, sizeof c, hipMemcpyDeviceToHost));
     c.clock = s->step;
+    s->clk_stale = true;
     c.probe_base = s->probe_base;
     c.err = 0;
     HIP_TRY(hipMemcpy(s->d_clock, &c, sizeof c, hipMemcpyHostToDevice));
@@ -1917,6 +2544,7 @@ int gmes_sim_set_ghost_fusion(gmes_sim* s, int32_t enable, int32_t* fused) {
   HIP_TRY(hipSetDevice(s->device));
   HIP_TRY(sync_exec(s));
   s->allow_fuse = enable != 0;
+  destroy_graph(s);  // one-sweep steps end or begin with it
   decide_fusion(s);
   if (fused) *fused = (s->fuse_e || s->fuse_hz) ? 1 : 0;
   return GMES_OK;
@@ -1929,6 +2557,7 @@ int gmes_sim_set_tile(gmes_sim* s, int32_t bx, int32_t by) {
     return set_error(GMES_EINVAL, "bad tile: bx must be a power of two and bx*by <= 256");
   s->tile_bx = bx;
   s->tile_by = by;
+  s->tile_tuned = false;
   const char* ic = getenv("GMES_ICHUNK");
   s->tile_ic = ic ? atoi(ic) : 0;
   destroy_graph(s);
@@ -1951,6 +2580,7 @@ int gmes_sim_autotune(gmes_sim* s, int32_t* bx, int32_t* by) {
   if (tbx > 0) {
     s->tile_bx = tbx;
     s->tile_by = tby;
+    s->tile_tuned = true;
     destroy_graph(s);
   }
   if (bx) *bx = tbx;
@@ -2385,7 +3015,10 @@ int gmes_batch_step(gmes_batch* b, int64_t nsteps) {
     for (int64_t t = 0; t < nsteps; ++t) enqueue_batch_step(b, b->stream);
     HIP_TRY(hipGetLastError());
   }
-  for (gmes_sim* s : b->sims) advance_host_clock(s, nsteps);
+  for (gmes_sim* s : b->sims) {
+    s->clk_stale = true;
+    advance_host_clock(s, nsteps);
+  }
   return GMES_OK;
 }
 

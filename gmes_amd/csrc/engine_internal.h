@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <array>
 #include <string>
 #include <vector>
 
@@ -47,6 +48,16 @@ struct DevSrcOp {
   int32_t kind, wave, aux, aux_comp;
   int64_t i0, i1;
   R k, r0, r1;
+};
+
+// What a cell of a one-sweep step needs beyond its table entry (three per
+// entry): Const value, point source.
+struct StepRare {
+  int32_t keep;  // 1: Dummy, the old value stays; 2: Const
+  int32_t wave;  // waveform row, -1: none
+  int32_t kind;  // GMES_SRC_SET or GMES_SRC_SUB
+  int32_t pad_;
+  double re, im;
 };
 
 // Compact list of the cells of one ADE class in one component.
@@ -161,8 +172,34 @@ struct gmes_sim {
   bool use_graph = false;
   hipGraphExec_t graph_exec = nullptr;
   bool graph_dirty = true;
-  // launch shape
+  int graph_steps = 1, graph_par = 0;  // steps it holds, parity of the buffers it starts from
+  // launch shape; tile_tuned: set by the autotuner (the caller did not ask
+  // for it, so one-sweep steps still apply)
   int tile_bx = 0, tile_by = 0, tile_ic = 0;
+  bool tile_tuned = false;
+  // one-sweep steps (step3d.hip): a second set of field buffers and of E
+  // absorber state; f[] and pml_state[] are the current set, swapped by
+  // every such step (par: which one, counted from the first)
+  bool sweep_ok = false;     // tables built, buffers allocated (by commit)
+  bool sweep_src_ok = true;  // the sources can be applied inside the sweep
+  bool clk_stale = true;     // Ctl::clk lags Ctl::clock
+  int par = 0;
+  bool sweep_ghosts = true;  // the next one-sweep step writes the ghost planes
+  int sweep_absorber = 0;    // 0 none, 1 CPML, 2 UPML
+  int sweep_exact = 0;       // Step3Args::exact
+  int sweep_threads = 0, sweep_rows = 0, sweep_ch = 0;
+  void* f_alt[6] = {};
+  void* pml_alt[3] = {};
+  int32_t sweep_run_e[3] = {}, sweep_run_h[3] = {};  // Step3Args::run_e, run_h
+  uint32_t* d_step_ids = nullptr;  // entries of the E (low half) and H cells of (i, j, k), rows at the pitch of Ex
+  void* d_step_tab = nullptr;
+  gmes_engine::StepRare* d_rare = nullptr;
+  int64_t step_tab_cap = 0;   // entries the two tables hold room for
+  int64_t sweep_bytes = 0;
+  std::vector<std::array<uint16_t, 3>> step_e, step_h;  // record ids of each entry
+  std::vector<std::pair<int64_t, uint32_t>> src_ids;  // ids the sources replaced (element, old word)
+  int step_net = 0, step_nht = 0;
+  bool has_waves = false;     // a source in the sweep reads the waveforms
   gmes_engine::Timing timing;
   int64_t bytes = 0;
   // partial sums of gmes_sim_field_sum_sq (grown on demand)

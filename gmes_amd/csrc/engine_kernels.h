@@ -5,6 +5,8 @@
 
 namespace gmes_engine {
 
+typedef int i4_t __attribute__((ext_vector_type(4)));
+
 constexpr int kDm2Max = 8;    // transitions per DM2 cell held in registers
 constexpr int kRecLds = 128;  // records staged in LDS by the 3-D main kernel
 
@@ -19,6 +21,7 @@ struct Ctl {
   int64_t dft_n;       // rows of DFT weights
   int32_t err;         // deferred device error (1 NaN, 2 no convergence)
   int32_t pad_;
+  int64_t clk[2];      // the clock as the one-sweep steps pass it on (StepArgs::par)
 };
 
 constexpr int kPad = 32;  // elements before row 0 of every device array
@@ -101,6 +104,89 @@ struct MainArgs {
   cplx<R> hzph[2];
   cplx<R> hyxph;
 };
+
+// ---- one-sweep steps
+// A whole leapfrog step of one sim in one kernel (step3d.hip): the
+// fields are read from one set of buffers (fi) and written to another (fo),
+// so E can be computed again where a neighbouring block needs it and H
+// follows from it at once.  A cell's three E components (and the three H
+// components the same thread owns) share one table entry.
+// Dummy, Const and source cells are flagged (StepRare has the details);
+// every other cell of a sim without UPML runs one formula: at a coordinate
+// without live state the CPML update is the Dielectric one.
+constexpr uint32_t kStepRareCell = 1, kStepUpmlCells = 14;  // UPML: bit 1 + t for component t
+template <class R>
+struct alignas(16) StepEnt {
+  R c[3];         // dt/eps; UPML cells: 1/eps (FP32) or eps (FP64)
+  uint32_t meta;  // kStepRareCell | 2 << t per UPML component
+};
+
+template <class T>
+struct Step3Args {
+  using R = typename real_of<T>::type;
+  // buffer resources (base address, bytes): each starts at the array's
+  // logical element (0, 0, 0)
+  i4_t ei[3], hi[3];  // old E, H
+  i4_t eo[3], ho[3];  // new E, H
+  i4_t si[3], so[3];  // E absorber state, read and written
+  i4_t sh[3];         // H absorber state (in place: only its owner touches a word)
+  i4_t ids;           // [i][j][k] table entries of the E (low half) and H cells of thread (i, j, k)
+  int W0, W2;      // row pitch of Ex, Ey, Hx, Hy and of Ez, Hz
+  int n[3];
+  const void* tab;      // StepEnt<R>[net + nht]: E entries, then H entries
+  const StepRare* rare;  // [3 * (net + nht)]
+  int net, nht;
+  unsigned ds[6];  // CPML: bytes from the first word of a component's state to the second
+  R d[3], inv_d[3];
+  const R* re[3];  // absorber rows of E along x, y, z (CPML: b, c, kappa; UPML: c1..c6 of the shared row)
+  const R* rh[3];  // the same of H
+  const R* oe[3];  // UPML: rows of the component whose own axis it is
+  const R* oh[3];
+  int run_e[3], run_h[3];  // CPML: per axis the coordinates lo | hi << 16 without live state; UPML: the UPML-free box
+  cplx<R> pe[3][3];  // ghost phase of E component c along axis a
+  cplx<R> ph[3][3];  // of H
+  int rows;        // (j) rows per block, the last one a rim
+  int ch;          // i planes per block
+  int nj, nblk;    // tiles along j, blocks
+  const double* waves;
+  Ctl* ctl;
+  int par;
+  int exact;       // FP64: every division is by a power of two
+  int ghosts;      // write the ghost planes: the last step of a call, unless a monitor reads them
+};
+// The entry ids of a sim, looked up from its material ids on the device.
+struct StepKey {
+  uint64_t key, id;  // key ~0: empty slot
+};
+__host__ __device__ inline uint64_t step_key(uint16_t a, uint16_t b, uint16_t c) {
+  return a | (uint64_t)b << 16 | (uint64_t)c << 32;
+}
+__host__ __device__ inline uint32_t step_hash(uint64_t key, uint32_t mask) {
+  return (uint32_t)((key * 0x9E3779B97F4A7C15ull) >> 40) & mask;
+}
+struct StepIdArgs {
+  const uint16_t* ids[6];
+  int64_t first[6], plane[6], row[6];  // element of thread (0, 0, 0), strides along i and j
+  const StepKey* tab[2];               // E, H; open addressing, at most a quarter full
+  uint32_t mask[2];
+  int n[3];
+  int pitch;       // of out's rows
+  uint32_t* out;
+};
+void launch_step_ids(const StepIdArgs& a, hipStream_t st);
+// threads of a block at most, the stride of its LDS exchange planes
+constexpr int kStepMaxThreads = 1024;
+template <class T> constexpr int kStepThreads = kStepMaxThreads;
+// bytes of LDS of a block: exchange buffers, entries, absorber rows
+template <class T>
+inline size_t step3_lds(int nthreads, int nent, int rows, int nz, int absorber) {
+  using R = typename real_of<T>::type;
+  const size_t stride = absorber == 2 ? 8 : absorber == 1 ? 4 : 0;
+  const size_t exchange = sizeof(T) == 4 ? (2 * (2 * (size_t)nz + 9 * (size_t)nthreads) + 3) / 4 * 4 * sizeof(T)
+                                         : (size_t)12 * kStepThreads<T> * sizeof(T);
+  return exchange + (size_t)nent * sizeof(StepEnt<R>) +
+         2 * (size_t)(rows + nz) * stride * sizeof(R);
+}
 
 template <class T>
 struct AdeArgs {
@@ -229,6 +315,8 @@ void launch_sum_sq(const SqBox<T>& b, double* partial, hipStream_t st);
 // to rows spaced dpitch apart (field reads and writes of padded layouts)
 void launch_pitch_copy(const void* src, void* dst, int64_t rows, int n2, int spitch, int dpitch, int esize,
                        hipStream_t st);
+// out[x] = (uint8_t)ids[x]
+void launch_narrow_ids(const uint16_t* ids, uint8_t* out, int64_t n, hipStream_t st);
 template <class T>
 void launch_main(bool electric, const MainArgs<T>& m, int ext[3], int bx, int by, hipStream_t st);
 // flat blocks over packed rows (3-D; see k_main3d_flat)
@@ -260,6 +348,11 @@ template <class T>
 void launch_main2z(bool electric, const MainArgs<T>& m, int ext[3], hipStream_t st);
 template <class T>
 void launch_main3d(bool electric, const MainArgs<T>& m, int bx, int by, int ichunk, hipStream_t st);
+// absorber: 0 none, 1 CPML, 2 UPML
+template <class T>
+void launch_step3d(const Step3Args<T>& m, int absorber, int nthreads, hipStream_t st);
+// clk[0] = clk[1] = clock: before the first one-sweep step after others
+void launch_clock_copy(Ctl* ctl, hipStream_t st);
 template <class T>
 void launch_ade(int cls, int c, const AdeArgs<T>& m, hipStream_t st);
 template <class T>
