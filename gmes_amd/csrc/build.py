@@ -12,15 +12,16 @@ import tempfile
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "lib", "libgmes_engine.so")
-# (file, extra flags): kernels.hip is compiled once per storage type
-SOURCES = [("engine.hip", [])] + [("kernels.hip", ["-DGMES_TYPE=%d" % t]) for t in range(4)] + [("step3d.hip", [])]
+# (file, extra flags): kernels.hip and step2d.hip are compiled once per storage type
+SOURCES = [("engine.hip", []), ("step3d.hip", [])] + [
+    (src, ["-DGMES_TYPE=%d" % t]) for src in ("kernels.hip", "step2d.hip") for t in range(4)]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("GMES_OFFLOAD_ARCH", "gfx950")
 
 FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared", "--offload-arch=" + ARCH,
          "-ffp-contract=off", "-fno-fast-math",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-         "-Wno-unused-result", "-Wno-unused-command-line-argument"]
+         "-Wno-unused-result", "-Wno-unused-command-line-argument", "-Wno-inline-asm"]
 
 
 def build(verbose=True):

@@ -85,11 +85,13 @@ struct CaptureGuard {
   }
 };
 
-// f(0) .. f(n - 1) on a few threads (passes over all cells of a sim while it
-// is being set up); f writes only what is its own.
+// f(0) .. f(n - 1) on a few threads (passes over all `cells` of a sim while
+// it is being set up); f writes only what is its own.  Starting the threads
+// takes 0.1 ms, a pass over 2^18 cells about as long.
 template <class F>
-void host_parallel(int n, F f) {
-  const int nt = std::min<int>(n, std::min(8u, std::max(1u, std::thread::hardware_concurrency())));
+void host_parallel(int n, int64_t cells, F f) {
+  const int most = cells < (1 << 18) ? 1 : 8;
+  const int nt = std::min<int>(n, std::min<unsigned>(most, std::max(1u, std::thread::hardware_concurrency())));
   std::atomic<int> next{0};
   std::atomic<bool> failed{false};
   auto work = [&] {
@@ -137,7 +139,7 @@ bool is_2z(const gmes_sim* s) {
 
 // device element of logical (i,j,k) / of a logical C-order flat index
 int64_t dev_index(const gmes_sim* s, int c, int64_t i, int64_t j, int64_t k) {
-  return kPad + (i * s->shape[c][1] + j) * s->pitch[c] + k - s->koff[c];
+  return kPad + i * s->pi[c] + j * s->pitch[c] + k * s->pk[c] - s->koff[c];
 }
 int64_t dev_flat(const gmes_sim* s, int c, int64_t flat) {
   const int64_t sz = s->shape[c][2], sy = s->shape[c][1];
@@ -447,7 +449,9 @@ FieldArgs<T> field_args(const gmes_sim* s) {
   for (int c = 0; c < 6; ++c) {
     a.f[c] = static_cast<T*>(s->f[c]);
     for (int d = 0; d < 3; ++d) a.s[c][d] = (int)s->shape[c][d];
+    a.pi[c] = s->pi[c];
     a.p[c] = s->pitch[c];
+    a.pk[c] = s->pk[c];
     a.koff[c] = s->koff[c];
   }
   a.active = s->g.active;
@@ -716,8 +720,9 @@ void dft_jobs(const gmes_sim* s, std::vector<DftJob<T>>& out, int64_t& block0) {
   for (const auto& d : s->dfts) {
     DftJob<T> J{};
     J.f = static_cast<T*>(s->f[d.comp]);
-    J.s1 = (int)s->shape[d.comp][1];
+    J.pi = s->pi[d.comp];
     J.p = s->pitch[d.comp];
+    J.pk = s->pk[d.comp];
     J.koff = s->koff[d.comp];
     J.comp = d.comp;
     for (int a = 0; a < 3; ++a) { J.lo[a] = (int)d.lo[a]; J.n[a] = (int)d.n[a]; }
@@ -743,7 +748,7 @@ int upload_dft_jobs_t(gmes_sim* s) {
     int64_t nb = 0;
     std::vector<DftJob<T>> half;
     dft_jobs<T>(s, half, nb);
-    if (p != s->par && s->f_alt[0])
+    if (p != s->par && s->sweep_ok)
       for (auto& J : half) J.f = static_cast<T*>(s->f_alt[J.comp]);
     s->dft_blocks = nb;
     jobs.insert(jobs.end(), half.begin(), half.end());
@@ -906,7 +911,7 @@ bool sweep_live_cells_cpml(const gmes_sim* s) {
     ok[r] = cls == GMES_CLS_CPML || cls == GMES_CLS_DUMMY || cls == GMES_CLS_CONST;
   }
   std::atomic<bool> all{true};
-  host_parallel(12, [&](int q) {
+  host_parallel(12, s->ncell[0], [&](int q) {
     const int c = q / 2, a = q % 2 ? kAx2[c] : kAx1[c];
     const int64_t* n = s->shape[c];
     const int run = c < 3 ? s->sweep_run_e[a] : s->sweep_run_h[a], lo = run & 0xFFFF, hi = run >> 16;
@@ -934,7 +939,7 @@ bool sweep_triples(const gmes_sim* s, bool electric, size_t most, std::vector<st
   const int64_t nx = s->g.nx, ny = s->g.ny, nz = s->g.nz;
   constexpr int kParts = 16;
   std::vector<uint64_t> found[kParts];  // in the order of the cells
-  host_parallel(kParts, [&](int part) {
+  host_parallel(kParts, s->ncell[0], [&](int part) {
     std::unordered_set<uint64_t> seen;
     uint64_t last = ~0ull;
     const uint16_t* src[3];
@@ -967,21 +972,31 @@ bool sweep_triples(const gmes_sim* s, bool electric, size_t most, std::vector<st
 // Writes the entry ids of every cell on the device, from the material ids
 // there and hash tables of the triples (building them on the host and
 // copying them took 40 ms at 256^3).
-int sweep_ids(gmes_sim* s) {
-  std::vector<StepKey> tab[2];
-  for (int h = 0; h < 2; ++h) {
-    const auto& ent = h ? s->step_h : s->step_e;
-    size_t cap = 64;
-    while (cap < 4 * ent.size()) cap *= 2;
-    tab[h].assign(cap, StepKey{~0ull, 0});
-    for (size_t e = 0; e < ent.size(); ++e) {
-      const uint64_t key = step_key(ent[e][0], ent[e][1], ent[e][2]);
-      uint32_t at = step_hash(key, (uint32_t)cap - 1);
-      while (tab[h][at].key != ~0ull) at = (at + 1) & ((uint32_t)cap - 1);
-      tab[h][at] = StepKey{key, (uint64_t)e};
-    }
+std::vector<StepKey> sweep_keys(const std::vector<std::array<uint16_t, 3>>& ent) {
+  size_t cap = 64;
+  while (cap < 4 * ent.size()) cap *= 2;
+  std::vector<StepKey> tab(cap, StepKey{~0ull, 0});
+  for (size_t e = 0; e < ent.size(); ++e) {
+    const uint64_t key = step_key(ent[e][0], ent[e][1], ent[e][2]);
+    uint32_t at = step_hash(key, (uint32_t)cap - 1);
+    while (tab[at].key != ~0ull) at = (at + 1) & ((uint32_t)cap - 1);
+    tab[at] = StepKey{key, (uint64_t)e};
   }
+  return tab;
+}
+
+int sweep_ids(gmes_sim* s) {
   StepIdArgs a{};
+  for (int c = 0; c < 6; ++c) {
+    a.ids[c] = s->ids[c];
+    a.first[c] = dev_index(s, c, c >= 3 && c != 3, c >= 3 && c != 4, c >= 3 && c != 5);
+    a.plane[c] = s->pi[c];
+    a.row[c] = s->pitch[c];
+  }
+  a.n[0] = s->g.nx; a.n[1] = s->g.ny; a.n[2] = s->g.nz;
+  a.pitch = s->pitch[0];
+  a.out = s->d_step_ids;
+  const std::vector<StepKey> tab[2] = {sweep_keys(s->step_e), sweep_keys(s->step_h)};
   const size_t b0 = tab[0].size() * sizeof(StepKey), b1 = tab[1].size() * sizeof(StepKey);
   char* d = nullptr;
   HIP_TRY(hipMalloc((void**)&d, b0 + b1));
@@ -991,15 +1006,6 @@ int sweep_ids(gmes_sim* s) {
     a.tab[h] = reinterpret_cast<const StepKey*>(d + (h ? b0 : 0));
     a.mask[h] = (uint32_t)tab[h].size() - 1;
   }
-  for (int c = 0; c < 6; ++c) {
-    a.ids[c] = s->ids[c];
-    a.first[c] = dev_index(s, c, c >= 3 && c != 3, c >= 3 && c != 4, c >= 3 && c != 5);
-    a.plane[c] = s->shape[c][1] * s->pitch[c];
-    a.row[c] = s->pitch[c];
-  }
-  a.n[0] = s->g.nx; a.n[1] = s->g.ny; a.n[2] = s->g.nz;
-  a.pitch = s->pitch[0];
-  a.out = s->d_step_ids;
   if (e == hipSuccess) {
     launch_step_ids(a, s->stream);
     e = hipGetLastError();
@@ -1078,6 +1084,15 @@ void sweep_release(gmes_sim* s) {
       (void)dev_release(*b);
       *b = nullptr;
     }
+  for (int c = 0; c < 3; ++c) {
+    if (s->d_adeq[c]) (void)dev_release(s->d_adeq[c]);
+    s->d_adeq[c] = nullptr;
+    for (void*& p : s->ade_alt[c]) {
+      if (p) (void)dev_release(p);
+      p = nullptr;
+    }
+  }
+  s->sweep_2d = false;
   s->bytes -= s->sweep_bytes;
   s->sweep_bytes = 0;
   s->sweep_ok = false;
@@ -1120,10 +1135,315 @@ int sweep_upload_tab(gmes_sim* s, const std::vector<std::array<int, 3>>& se, con
   return GMES_OK;
 }
 
+// ---- one-sweep steps of collapsed-z 2-D modes (step2d.hip)
+//
+// Taken when
+//   * all absorber cells are of one kind and one profile set, in every
+//     component or none, and CPML has no live state along z,
+//   * no cell is of the DM2 class,
+//   * the distinct triples of records fit a block's LDS (kSweepMaxTab) and a
+//     component 4 GiB (32-bit byte offsets),
+//   * every source is a point operation off the ghost planes, at most
+//     kStep2Src of them, and no E probe sits on a ghost plane, and
+//   * the caller asked for no tile and did not turn ghost fusion off.
+bool step2_tm(const gmes_sim* s) { return active(s, 2); }
+// component of direction a of the mode
+int step2_comp(const gmes_sim* s, int a) { return step2_tm(s) ? (a == 2 ? 2 : 3 + a) : (a == 2 ? 5 : a); }
+// storage coordinate along axis x of thread coordinate 0
+int step2_first(int c, int x) { return c >= 3 && c - 3 != x; }
+
+// Columns per block and rows per block.  Whole rows up to 512 columns;
+// longer ones in stretches of 224 columns (whole lines of 128 bytes; 226
+// lanes of 256), which beat 448 (1200^2 FP32 14.2 against 14.9 us) and whole
+// rows of 640 (7.5 against 8.2).  Rows: a block pays one more than it owns,
+// and fewer, longer blocks leave the last ones running alone: the best
+// count grew with the square root of the tiles per CU (us per step at 1, 2,
+// 3, 4, 6 rows: 640^2 FP32 8.6, 7.5, 8.4; 1200^2 FP32 18.6, 15.2, 14.2,
+// 15.5, 14.5; 2048^2 FP32 5 rows 30.3, 4 31.7, 10 33.2; 300^2 5.6, 6.8;
+// 512^2 complex FP64 7.7, 6.2, 7.1).
+void sweep2_shape(gmes_sim* s) {
+  const int nx = s->g.nx, ny = s->g.ny;
+  s->sweep_whole = ny <= 512;
+  s->sweep_w = s->sweep_whole ? ny : 224;
+  const double waves = (double)nx * ((ny + s->sweep_w - 1) / s->sweep_w) * step2_threads(s->sweep_w, s->sweep_whole) / 64;
+  s->sweep_ch = std::max(1, std::min(nx, (int)std::ceil(std::sqrt(waves / 4096))));
+}
+
+// Entries, their cells' details, the key table of the entry ids and the ids
+// themselves share one allocation, filled by one copy and one launch.
+template <class R>
+int sweep2_tables(gmes_sim* s) {
+  const size_t n = s->step_e.size();
+  const std::vector<StepKey> keys = sweep_keys(s->step_e);
+  const size_t cells_at = n * sizeof(Step2Ent<R>), keys_at = cells_at + 3 * n * sizeof(Step2Cell),
+               ids_at = keys_at + keys.size() * sizeof(StepKey);
+  static_assert(sizeof(Step2Ent<R>) % 16 == 0 && sizeof(Step2Cell) % 8 == 0 && sizeof(StepKey) % 16 == 0, "alignment");
+  std::vector<char> host(ids_at, 0);
+  Step2Ent<R>* tab = reinterpret_cast<Step2Ent<R>*>(host.data());
+  Step2Cell* cells = reinterpret_cast<Step2Cell*>(host.data() + cells_at);
+  for (size_t e = 0; e < n; ++e)
+    for (int t = 0; t < 3; ++t) {
+      const gmes_mat_rec& r = s->recs[s->step_e[e][t]];
+      const bool absorber = r.cls == GMES_CLS_CPML || r.cls == GMES_CLS_UPML;
+      const int kind = r.cls == GMES_CLS_DUMMY ? 1 : r.cls == GMES_CLS_CONST ? 2 : r.cls >= GMES_CLS_DRUDE ? 3 : 0;
+      cells[3 * e + t] = Step2Cell{kind, s->step_e[e][t], r.value[0], r.value[1]};
+      if (kind) tab[e].meta |= 2u << (2 * t);
+      else if (absorber) tab[e].meta |= 1u << (2 * t);
+      if (!kind)
+        tab[e].c[t] = r.cls == GMES_CLS_UPML ? (s->fp64 ? (R)r.eps_mu : (R)(1.0 / r.eps_mu)) : (R)(s->g.dt / r.eps_mu);
+    }
+  memcpy(host.data() + keys_at, keys.data(), keys.size() * sizeof(StepKey));
+  const int64_t pi = s->pi[step2_comp(s, 0)];
+  if (int rc = sweep_alloc(s, &s->d_step_tab, ids_at + (size_t)(s->g.nx * pi) * sizeof(uint16_t))) return rc;
+  char* d = static_cast<char*>(s->d_step_tab);
+  s->step2_cells = d + cells_at;
+  s->step2_ids = reinterpret_cast<uint16_t*>(d + ids_at);
+  HIP_TRY(hipMemcpy(d, host.data(), ids_at, hipMemcpyHostToDevice));
+  StepIdArgs a{};
+  for (int x = 0; x < 3; ++x) {
+    const int c = step2_comp(s, x);
+    a.ids[x] = s->ids[c];
+    a.first[x] = dev_index(s, c, step2_first(c, 0), step2_first(c, 1), s->shape[c][2] == 2 ? step2_first(c, 2) : 0);
+    a.plane[x] = s->pi[c];
+  }
+  a.tab[0] = reinterpret_cast<const StepKey*>(d + keys_at);
+  a.mask[0] = (uint32_t)keys.size() - 1;
+  a.n[0] = s->g.nx; a.n[1] = 1; a.n[2] = s->g.ny;
+  a.pitch = (int)pi;
+  a.out16 = s->step2_ids;
+  launch_step_ids(a, s->stream);
+  for (int c = 0; c < 3; ++c)
+    for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2; ++k) {
+      const AdeList& L = s->ade[c][k];
+      if (!L.n) continue;
+      launch_list_places({L.cell, (int)L.n, (int)s->shape[c][1], (int)s->shape[c][2], s->pi[c], s->pitch[c], s->pk[c],
+                          s->d_adeq[c] + (kPad - s->koff[c])}, s->stream);
+    }
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipStreamSynchronize(s->stream));
+  return GMES_OK;
+}
+
+int sweep2_build(gmes_sim* s) {
+  const int64_t nx = s->g.nx, ny = s->g.ny;
+  const bool tm = step2_tm(s);
+  if (s->g.nz != 1 || s->g.active != (tm ? 0x1Cu : 0x23u)) return GMES_OK;
+  for (int a = 0; a < 3; ++a)  // 32-bit byte offsets
+    if (s->dsize[step2_comp(s, a)] * s->esize > (int64_t)0xFFFFFFFF) return GMES_OK;
+  bool cpml = false, upml = false;
+  for (int a = 0; a < 3; ++a) {
+    const int c = step2_comp(s, a);
+    cpml |= s->has_cls[c][GMES_CLS_CPML];
+    upml |= s->has_cls[c][GMES_CLS_UPML];
+    if (s->has_cls[c][GMES_CLS_DM2]) return GMES_OK;
+  }
+  if ((cpml && upml) || ((cpml || upml) && s->nprof != 1)) return GMES_OK;
+  s->sweep_absorber = cpml ? 1 : upml ? 2 : 0;
+  const uint16_t* ids[3];
+  for (int a = 0; a < 3; ++a) {
+    const int c = step2_comp(s, a);
+    if (s->sweep_absorber) {
+      if (!s->pml_state[c]) return GMES_OK;
+      for (int x = 0; x < 3; ++x)
+        if (s->prof_w[0][c][x] != (cpml ? 3 : 6) ||
+            (int64_t)s->prof_host[0][c][x].size() != s->shape[c][x] * (cpml ? 3 : 6))
+          return GMES_OK;
+    }
+    if (cpml) {
+      for (size_t q = 1; q < s->prof_host[0][c][2].size(); q += 3)
+        if (s->prof_host[0][c][2][q] != 0.0) return GMES_OK;
+      for (int x = 0; x < 2; ++x) {  // the longest run with c = 0
+        const std::vector<double>& v = s->prof_host[0][c][x];
+        const int len = (int)(v.size() / 3);
+        int lo = 0, hi = 0;
+        for (int q = 0; q < len;) {
+          if (v[3 * (size_t)q + 1] != 0.0) { ++q; continue; }
+          int e = q;
+          while (e < len && v[3 * (size_t)e + 1] == 0.0) ++e;
+          if (e - q > hi - lo) { lo = q; hi = e; }
+          q = e;
+        }
+        lo = std::max(0, lo - step2_first(c, x));
+        hi = std::max(0, hi - step2_first(c, x));
+        s->sweep_run2[a][x] = hi > 0x7FFF ? 0 : lo | (hi << 16);
+      }
+    }
+    // record of thread (i, j): [(i * s1 + j) * s2] from here
+    ids[a] = s->host_ids[c].data() + (step2_first(c, 0) * s->shape[c][1] + step2_first(c, 1)) * s->shape[c][2] +
+             (s->shape[c][2] == 2 ? step2_first(c, 2) : 0);
+  }
+  auto rec = [&](int a, int64_t i, int64_t j) {
+    const int64_t* n = s->shape[step2_comp(s, a)];
+    return ids[a][(i * n[1] + j) * n[2]];
+  };
+  if (upml) {
+    // a box without UPML cells: the free runs through the centre, if no cell
+    // inside is one
+    std::vector<char> is(s->recs.size());
+    for (size_t r = 0; r < is.size(); ++r) is[r] = s->recs[r].cls == GMES_CLS_UPML;
+    auto at = [&](int64_t i, int64_t j) { return is[rec(0, i, j)] || is[rec(1, i, j)] || is[rec(2, i, j)]; };
+    int64_t lo[2] = {nx / 2, ny / 2}, hi[2] = {nx / 2, ny / 2};
+    while (lo[0] > 0 && !at(lo[0] - 1, ny / 2)) --lo[0];
+    while (hi[0] < nx && !at(hi[0], ny / 2)) ++hi[0];
+    while (lo[1] > 0 && !at(nx / 2, lo[1] - 1)) --lo[1];
+    while (hi[1] < ny && !at(nx / 2, hi[1])) ++hi[1];
+    bool free = hi[0] <= 0x7FFF && hi[1] <= 0x7FFF;
+    for (int64_t i = lo[0]; free && i < hi[0]; ++i)
+      for (int64_t j = lo[1]; free && j < hi[1]; ++j) free = !at(i, j);
+    for (int x = 0; x < 2; ++x) s->sweep_run2[0][x] = free ? (int32_t)(lo[x] | (hi[x] << 16)) : 0;
+  }
+  auto pow2 = [](double v) { int e; return std::frexp(v, &e) == 0.5; };
+  bool exact = pow2(s->g.dx) && pow2(s->g.dy) && pow2(s->g.dz);
+  for (int a = 0; a < 3 && cpml; ++a)
+    for (int x = 0; x < 3; ++x) {
+      const std::vector<double>& v = s->prof_host[0][step2_comp(s, a)][x];
+      for (size_t q = 2; q < v.size(); q += 3) exact = exact && v[q] == 1.0;
+    }
+  s->sweep_exact = exact;
+  s->step_e.clear();
+  s->step_h.clear();
+  const size_t most = (size_t)kSweepMaxTab / (s->fp64 ? sizeof(Step2Ent<double>) : sizeof(Step2Ent<float>));
+  std::unordered_set<uint64_t> seen;
+  uint64_t last = ~0ull;
+  int64_t step[3];
+  for (int a = 0; a < 3; ++a) step[a] = s->shape[step2_comp(s, a)][2];
+  for (int64_t i = 0; i < nx; ++i) {
+    const uint16_t* r[3];
+    for (int a = 0; a < 3; ++a) r[a] = ids[a] + i * s->shape[step2_comp(s, a)][1] * step[a];
+    for (int64_t j = 0; j < ny; ++j) {
+      const uint16_t x = r[0][j * step[0]], y = r[1][j * step[1]], z = r[2][j * step[2]];
+      const uint64_t key = step_key(x, y, z);
+      if (key == last) continue;
+      last = key;
+      if (!seen.insert(key).second) continue;
+      if (s->step_e.size() >= most) return GMES_OK;
+      s->step_e.push_back({x, y, z});
+    }
+  }
+  sweep2_shape(s);
+  int rc = GMES_OK;
+  for (int a = 0; a < 3 && !rc; ++a) {
+    const int c = step2_comp(s, a);
+    rc = sweep_alloc(s, &s->f_alt[c], (size_t)s->dsize[c] * s->esize);
+    if (rc || c >= 3) continue;
+    if (s->pml_state[c]) {
+      const size_t b = (size_t)(cpml ? 2 : 1) * s->dsize[c] * s->esize;
+      rc = sweep_alloc(s, &s->pml_alt[c], b);
+      if (!rc) HIP_TRY(hipMemsetAsync(s->pml_alt[c], 0, b, s->stream));
+    }
+    bool any = false;
+    for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2 && !rc; ++k) {
+      const AdeList& L = s->ade[c][k];
+      if (!L.n) continue;
+      any = true;
+      const size_t b = std::max<size_t>(1, (size_t)L.nstate * L.n * ade_word(s, k));
+      rc = sweep_alloc(s, &s->ade_alt[c][k], b);
+      if (!rc) HIP_TRY(hipMemsetAsync(s->ade_alt[c][k], 0, b, s->stream));
+    }
+    if (any && !rc) rc = sweep_alloc(s, (void**)&s->d_adeq[c], (size_t)s->dsize[c] * sizeof(int32_t));
+  }
+  if (!rc) rc = s->fp64 ? sweep2_tables<double>(s) : sweep2_tables<float>(s);
+  if (rc) {  // no room for a second set of buffers
+    (void)hipGetLastError();
+    sweep_release(s);
+    return GMES_OK;
+  }
+  s->sweep_2d = true;
+  s->sweep_ok = true;
+  return GMES_OK;
+}
+
+int sweep2_sources(gmes_sim* s) {
+  s->step2_src.clear();
+  s->sweep_src_ok = (int)s->ops.size() <= kStep2Src;
+  s->has_waves = !s->ops.empty();
+  const int64_t n[3] = {s->g.nx, s->g.ny, 1};
+  for (size_t q = 0; s->sweep_src_ok && q < s->ops.size(); ++q) {
+    const gmes_src_op& o = s->ops[q];
+    const int64_t sy = s->shape[o.comp][1], sz = s->shape[o.comp][2];
+    int64_t ix[3] = {o.cell / (sy * sz), (o.cell / sz) % sy, o.cell % sz};
+    bool ok = o.kind == GMES_SRC_SET || o.kind == GMES_SRC_SUB;
+    for (int a = 0; a < 3; ++a) {
+      if (s->shape[o.comp][a] > n[a]) ix[a] -= step2_first(o.comp, a);
+      if (ix[a] < 0 || ix[a] >= n[a]) ok = false;  // a ghost cell
+    }
+    if (!ok) s->sweep_src_ok = false;
+    s->step2_src.push_back({o.comp % 3, (int)ix[0], (int)ix[1], o.wave, o.kind});
+  }
+  return GMES_OK;
+}
+
+template <class T>
+Step2Args<T> step2_args(const gmes_sim* s) {
+  using R = typename real_of<T>::type;
+  Step2Args<T> m{};
+  const int width = s->sweep_absorber == 1 ? 3 : 6;
+  for (int a = 0; a < 3; ++a) {
+    const int c = step2_comp(s, a);
+    const bool two = s->shape[c][2] == 2;
+    const int64_t o = dev_index(s, c, step2_first(c, 0), step2_first(c, 1), two ? step2_first(c, 2) : 0);
+    m.fi[a] = static_cast<const T*>(s->f[c]) + o;
+    m.fo[a] = static_cast<T*>(s->f_alt[c]) + o;
+    m.pi = s->pi[c];
+    m.pk[a] = two ? (c < 3 ? (int64_t)s->pk[c] : -(int64_t)s->pk[c]) : 0;
+    if (s->sweep_absorber) {
+      const T* in = static_cast<const T*>(s->pml_state[c]) + o;
+      T* out = static_cast<T*>(c < 3 ? s->pml_alt[c] : s->pml_state[c]) + o;
+      for (int x = 0; x < 2; ++x) {
+        // CPML: the first word goes with the first curl axis
+        const int64_t w = s->sweep_absorber == 1 && kAx2[c] == x ? s->dsize[c] : 0;
+        m.si[a][x] = in + w;
+        m.so[a][x] = out + w;
+      }
+      for (int x = 0; x < 3; ++x)
+        m.row[a][x] = static_cast<const R*>(s->d_prof) + s->prof_off0[c][x] +
+                      (s->shape[c][x] > (x == 2 ? 1 : 0) ? step2_first(c, x) * width : 0);
+    }
+    for (int x = 0; x < 2; ++x) m.run[a][x] = s->sweep_run2[a][x];
+    for (int x = 0; x < 3; ++x) m.ph[a][x] = cplx<R>{(R)s->g.phase[c][x][0], (R)s->g.phase[c][x][1]};
+    if (c < 3) {
+      m.adeq[a] = s->d_adeq[c] ? s->d_adeq[c] + o : nullptr;
+      for (int k = 0; k < 3; ++k) {
+        m.ade_in[a][k] = s->ade[c][GMES_CLS_DRUDE + k].state;
+        m.ade_out[a][k] = s->ade_alt[c][GMES_CLS_DRUDE + k];
+        m.ade_n[a][k] = (int)s->ade[c][GMES_CLS_DRUDE + k].n;
+      }
+    }
+  }
+  m.ids = s->step2_ids;
+  m.n[0] = s->g.nx; m.n[1] = s->g.ny;
+  m.tab = static_cast<const Step2Ent<R>*>(s->d_step_tab);
+  m.cells = static_cast<const Step2Cell*>(s->step2_cells);
+  m.nent = (int)s->step_e.size();
+  m.d[0] = (R)s->g.dx; m.d[1] = (R)s->g.dy; m.d[2] = (R)s->g.dz;
+  m.inv_d[0] = (R)(1.0 / s->g.dx); m.inv_d[1] = (R)(1.0 / s->g.dy); m.inv_d[2] = (R)(1.0 / s->g.dz);
+  m.recs = static_cast<const DevRec<R>*>(s->d_recs);
+  m.coef = static_cast<const R*>(s->d_coef);
+  m.nsrc = (int)s->step2_src.size();
+  for (int q = 0; q < m.nsrc; ++q) {
+    const auto& v = s->step2_src[q];
+    m.src[q] = {v[0], v[1], v[2], v[3], v[4]};
+  }
+  m.w = s->sweep_w;
+  m.whole = s->sweep_whole;
+  m.ch = s->sweep_ch;
+  m.nj = (s->g.ny + m.w - 1) / m.w;
+  m.nblk = m.nj * ((s->g.nx + m.ch - 1) / m.ch);
+  m.waves = s->d_waves;
+  m.ctl = reinterpret_cast<Ctl*>(s->d_clock);
+  m.par = s->par;
+  m.exact = s->sweep_exact;
+  m.ghosts = s->sweep_ghosts;
+  return m;
+}
+
+bool step2_ade(const gmes_sim* s) { return s->d_adeq[0] || s->d_adeq[1] || s->d_adeq[2]; }
+
 // Marks the cells of the sim's source operations in the sweep's ids, when
 // all of them can be applied there (sweep_src_ok).
 int sweep_sources(gmes_sim* s) {
   if (!s->sweep_ok) return GMES_OK;
+  if (s->sweep_2d) return sweep2_sources(s);
   HIP_TRY(sync_exec(s));
   for (const auto& x : s->src_ids)
     HIP_TRY(hipMemcpy(s->d_step_ids + x.first, &x.second, sizeof(uint32_t), hipMemcpyHostToDevice));
@@ -1167,6 +1487,7 @@ int sweep_sources(gmes_sim* s) {
 // the sim does not qualify.
 int sweep_build(gmes_sim* s) {
   sweep_release(s);
+  if (is_2z(s)) return sweep2_build(s);
   if (!is3d(s) || s->g.dtype == GMES_C128) return GMES_OK;
   const int nz = s->g.nz;
   if (kSweepMinRows * nz > kStepMaxThreads || s->g.ny < 2) return GMES_OK;
@@ -1327,20 +1648,26 @@ Step3Args<T> step3_args(const gmes_sim* s) {
 
 // The current buffers become the other set.
 void sweep_swap(gmes_sim* s) {
-  for (int c = 0; c < 6; ++c) std::swap(s->f[c], s->f_alt[c]);
+  for (int c = 0; c < 6; ++c)
+    if (s->f_alt[c]) std::swap(s->f[c], s->f_alt[c]);
   for (int c = 0; c < 3; ++c)
     if (s->pml_alt[c]) std::swap(s->pml_state[c], s->pml_alt[c]);
+  for (int c = 0; c < 3; ++c)
+    for (int k = 0; k < GMES_NCLS; ++k)
+      if (s->ade_alt[c][k]) std::swap(s->ade[c][k].state, s->ade_alt[c][k]);
   s->par ^= 1;
 }
 
 template <class T>
 void enqueue_sweep(gmes_sim* s, hipStream_t st) {
-  if constexpr (!std::is_same<T, cplx<double>>::value) {
-    time_begin(s, 0, st);
+  time_begin(s, 0, st);
+  if (s->sweep_2d) {
+    launch_step2d<T>(step2_args<T>(s), step2_tm(s), s->sweep_absorber, step2_ade(s), st);
+  } else if constexpr (!std::is_same<T, cplx<double>>::value) {
     launch_step3d<T>(step3_args<T>(s), s->sweep_absorber, s->sweep_threads, st);
-    time_end(s, st);
-    sweep_swap(s);
   }
+  time_end(s, st);
+  sweep_swap(s);
 }
 
 template <class T>
@@ -1712,8 +2039,9 @@ template <class T>
 static void sq_launch(const gmes_sim* s, int c, const int64_t lo[3], const int64_t hi[3], double* partial) {
   SqBox<T> b;
   b.f = static_cast<const T*>(s->f[c]);
-  b.s1 = (int)s->shape[c][1];
+  b.pi = s->pi[c];
   b.p = s->pitch[c];
+  b.pk = s->pk[c];
   b.koff = s->koff[c];
   b.ncells = 1;
   for (int a = 0; a < 3; ++a) {
@@ -1800,11 +2128,26 @@ int gmes_sim_create(const gmes_grid_desc* desc, gmes_sim** out) {
       s->shape[c][c % 3] = n[c % 3];
     }
     s->ncell[c] = s->shape[c][0] * s->shape[c][1] * s->shape[c][2];
-    const int64_t s2 = s->shape[c][2];
-    const bool padded = s2 >= 32 && !s->packed;
-    s->pitch[c] = (int32_t)(padded ? (s2 + 31) / 32 * 32 : s2);
-    s->koff[c] = padded && (c == GMES_HX || c == GMES_HY) ? 1 : 0;
-    s->dsize[c] = 2 * kPad + s->shape[c][0] * s->shape[c][1] * s->pitch[c];
+  }
+  for (int c = 0; c < 6; ++c) {
+    const int64_t s0 = s->shape[c][0], s1 = s->shape[c][1], s2 = s->shape[c][2];
+    if (is_2z(s) && active(s, c)) {  // one piece per z plane
+      const bool padded = n[1] >= 31;
+      const int64_t row = padded ? (n[1] + 32) / 32 * 32 : n[1] + 1;  // the same for every component
+      s->pitch[c] = 1;
+      s->pi[c] = (int32_t)row;
+      s->pk[c] = (int32_t)std::min<int64_t>(s0 * row, INT32_MAX);
+      s->koff[c] = padded && (c == GMES_HX || c == GMES_HZ) ? 1 : 0;
+      s->dsize[c] = 2 * kPad + s0 * row * s2;
+    } else {
+      const bool padded = s2 >= 32 && !s->packed;
+      const int64_t row = padded ? (s2 + 31) / 32 * 32 : s2;
+      s->pitch[c] = (int32_t)row;
+      s->pi[c] = (int32_t)std::min<int64_t>(s1 * row, INT32_MAX);
+      s->pk[c] = 1;
+      s->koff[c] = padded && (c == GMES_HX || c == GMES_HY) ? 1 : 0;
+      s->dsize[c] = 2 * kPad + s0 * s1 * row;
+    }
     if (s->dsize[c] >= (int64_t(1) << 31)) {
       delete s;
       return set_error(GMES_EINVAL, "component %d has more than 2^31 cells", c);
@@ -1935,9 +2278,13 @@ int gmes_sim_set_material_ids(gmes_sim* s, int32_t c, const uint16_t* ids, int64
   // in one contiguous transfer: a strided 2-D copy would wait for every
   // kernel running on the device, including other sims' batches
   std::vector<uint16_t> dev((size_t)s->dsize[c], 0);
-  const int64_t rows = s->shape[c][0] * s->shape[c][1], n2 = s->shape[c][2];
-  for (int64_t r = 0; r < rows; ++r)
-    memcpy(dev.data() + kPad - s->koff[c] + r * s->pitch[c], ids + r * n2, (size_t)n2 * sizeof(uint16_t));
+  const int64_t n1 = s->shape[c][1], n2 = s->shape[c][2], rows = s->shape[c][0] * n1;
+  for (int64_t r = 0; r < rows; ++r) {
+    uint16_t* d = dev.data() + dev_index(s, c, r / n1, r % n1, 0);
+    if (s->pk[c] == 1) memcpy(d, ids + r * n2, (size_t)n2 * sizeof(uint16_t));
+    else
+      for (int64_t k = 0; k < n2; ++k) d[k * s->pk[c]] = ids[r * n2 + k];
+  }
   HIP_TRY(hipMemcpy(s->ids[c], dev.data(), dev.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
   s->committed = false;
   return GMES_OK;
@@ -1966,7 +2313,7 @@ int gmes_sim_commit(gmes_sim* s) {
   free_ade(s);
   s->ade_on_ghost_source = false;
   std::vector<int64_t> counts[6];  // cells per record; empty: an id is out of range
-  host_parallel(6, [&](int c) {
+  host_parallel(6, s->ncell[0] + s->ncell[2] + s->ncell[5], [&](int c) {
     if (!active(s, c)) return;
     counts[c].assign(s->recs.size(), 0);
     for (const uint16_t id : s->host_ids[c]) {
@@ -2286,6 +2633,16 @@ int gmes_sim_read_dft(gmes_sim* s, int32_t id, double* out, int64_t count) {
   return GMES_OK;
 }
 
+// Whether a component's device layout is the host's, after kPad elements.
+static bool dense_layout(const gmes_sim* s, int c) {
+  const int64_t s1 = s->shape[c][1], s2 = s->shape[c][2];
+  return s->koff[c] == 0 && (s2 == 1 || s->pk[c] == 1) && s->pitch[c] == s2 && s->pi[c] == s1 * s2;
+}
+
+static LayoutArgs layout_of(const gmes_sim* s, int c) {
+  return {s->ncell[c], (int)s->shape[c][1], (int)s->shape[c][2], s->pi[c], s->pitch[c], s->pk[c]};
+}
+
 // The staging buffer of field reads and writes of padded rows, at least
 // `bytes` long (grown on demand; the sim's stream is idle when it grows).
 static int stage_reserve(gmes_sim* s, int64_t bytes) {
@@ -2294,6 +2651,7 @@ static int stage_reserve(gmes_sim* s, int64_t bytes) {
   if (s->d_stage) dev_free(s, s->d_stage, (size_t)s->stage_cap);
   s->d_stage = nullptr;
   s->stage_cap = 0;
+  for (int c = 0; c < 6; ++c) bytes = std::max(bytes, s->ncell[c] * s->esize);  // once for all components
   int rc = dev_alloc(s, &s->d_stage, (size_t)bytes);
   if (rc) return rc;
   s->stage_cap = bytes;
@@ -2307,7 +2665,7 @@ int gmes_sim_write_field(gmes_sim* s, int32_t c, const void* host, int64_t bytes
   if (bytes != s->ncell[c] * s->esize) return set_error(GMES_EINVAL, "size mismatch");
   HIP_TRY(hipSetDevice(s->device));
   HIP_TRY(sync_exec(s));  // steps queued on the sim's (or its batch's) stream come first
-  if (s->pitch[c] == s->shape[c][2] && s->koff[c] == 0) {
+  if (dense_layout(s, c)) {
     HIP_TRY(hipMemcpyAsync(static_cast<char*>(s->f[c]) + (size_t)kPad * s->esize, host, (size_t)bytes,
                            hipMemcpyHostToDevice, s->stream));
     HIP_TRY(sync_exec(s));
@@ -2317,9 +2675,8 @@ int gmes_sim_write_field(gmes_sim* s, int32_t c, const void* host, int64_t bytes
   int rc = stage_reserve(s, bytes);
   if (rc) return rc;
   HIP_TRY(hipMemcpyAsync(s->d_stage, host, (size_t)bytes, hipMemcpyHostToDevice, s->stream));
-  launch_pitch_copy(s->d_stage, static_cast<char*>(s->f[c]) + (size_t)(kPad - s->koff[c]) * s->esize,
-                    s->shape[c][0] * s->shape[c][1], (int)s->shape[c][2], (int)s->shape[c][2], s->pitch[c], s->esize,
-                    s->stream);
+  launch_layout_copy(true, s->d_stage, static_cast<char*>(s->f[c]) + (size_t)(kPad - s->koff[c]) * s->esize,
+                     layout_of(s, c), s->esize, s->stream);
   HIP_TRY(hipGetLastError());
   HIP_TRY(sync_exec(s));
   return GMES_OK;
@@ -2332,7 +2689,7 @@ int gmes_sim_read_field(gmes_sim* s, int32_t c, void* host, int64_t bytes) {
   if (bytes != s->ncell[c] * s->esize) return set_error(GMES_EINVAL, "size mismatch");
   HIP_TRY(hipSetDevice(s->device));
   HIP_TRY(sync_exec(s));  // steps queued on the sim's (or its batch's) stream come first
-  if (s->pitch[c] == s->shape[c][2] && s->koff[c] == 0) {
+  if (dense_layout(s, c)) {
     HIP_TRY(hipMemcpyAsync(host, static_cast<const char*>(s->f[c]) + (size_t)kPad * s->esize, (size_t)bytes,
                            hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(sync_exec(s));
@@ -2341,9 +2698,8 @@ int gmes_sim_read_field(gmes_sim* s, int32_t c, void* host, int64_t bytes) {
   // rows packed on the device, then one contiguous download
   int rc = stage_reserve(s, bytes);
   if (rc) return rc;
-  launch_pitch_copy(static_cast<const char*>(s->f[c]) + (size_t)(kPad - s->koff[c]) * s->esize, s->d_stage,
-                    s->shape[c][0] * s->shape[c][1], (int)s->shape[c][2], s->pitch[c], (int)s->shape[c][2], s->esize,
-                    s->stream);
+  launch_layout_copy(false, s->d_stage, static_cast<char*>(s->f[c]) + (size_t)(kPad - s->koff[c]) * s->esize,
+                     layout_of(s, c), s->esize, s->stream);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpyAsync(host, s->d_stage, (size_t)bytes, hipMemcpyDeviceToHost, s->stream));
   HIP_TRY(sync_exec(s));
@@ -2359,28 +2715,73 @@ int gmes_sim_read_field(gmes_sim* s, int32_t c, void* host, int64_t bytes) {
 // probe values, so the next step records and injects at the restored time.
 constexpr int64_t kSnapMagic = 0x31504e5353454d47LL;  // "GMESSNP1"
 
-static void state_blocks(gmes_sim* s, std::vector<std::pair<void*, size_t>>& out) {
-  for (int c = 0; c < 6; ++c) {
-    if (s->pml_state[c]) {
-      const int pw = s->has_cls[c][GMES_CLS_CPML] ? 2 : 1;
-      out.push_back({s->pml_state[c], (size_t)pw * s->dsize[c] * s->esize});
-    }
-    for (int k = GMES_CLS_DRUDE; k < GMES_NCLS; ++k)
-      if (s->ade[c][k].n) out.push_back({s->ade[c][k].state, (size_t)s->ade[c][k].nstate * s->ade[c][k].n * ade_word(s, k)});
+// Arrays laid out like a component are in it in the order of (i, j, k): as
+// one piece of device memory, except that collapsed-z modes keep k fastest
+// (their device layout is converted), with kPad elements before and after.
+struct StateBlock {
+  void* dev;
+  size_t bytes;  // in the blob
+  int comp;      // component whose layout it has, -1: plain bytes
+  int words;
+};
+
+static void grid_block(const gmes_sim* s, std::vector<StateBlock>& out, void* dev, int c, int words) {
+  if (is_2z(s)) out.push_back({dev, (size_t)words * (2 * kPad + s->ncell[c]) * s->esize, c, words});
+  else out.push_back({dev, (size_t)words * s->dsize[c] * s->esize, -1, words});
+}
+
+static int block_copy(const gmes_sim* s, const StateBlock& b, char* p, bool save) {
+  if (b.comp < 0) {
+    if (save) HIP_TRY(hipMemcpy(p, b.dev, b.bytes, hipMemcpyDeviceToHost));
+    else HIP_TRY(hipMemcpy(b.dev, p, b.bytes, hipMemcpyHostToDevice));
+    return GMES_OK;
   }
-  for (auto& d : s->dfts) out.push_back({d.acc, 2 * (size_t)d.nfreq * d.ncells * 2 * sizeof(double)});
+  const int c = b.comp;
+  const size_t e = (size_t)s->esize;
+  const int64_t n1 = s->shape[c][1], n2 = s->shape[c][2];
+  std::vector<char> dev((size_t)b.words * s->dsize[c] * e, 0);
+  if (save) {
+    HIP_TRY(hipMemcpy(dev.data(), b.dev, dev.size(), hipMemcpyDeviceToHost));
+    memset(p, 0, b.bytes);
+  }
+  for (int w = 0; w < b.words; ++w)
+    for (int64_t x = 0; x < s->ncell[c]; ++x) {
+      char* d = dev.data() + (w * s->dsize[c] + dev_index(s, c, x / (n1 * n2), x / n2 % n1, x % n2)) * e;
+      char* h = p + (w * (2 * kPad + s->ncell[c]) + kPad + x) * e;
+      if (save) memcpy(h, d, e);
+      else memcpy(d, h, e);
+    }
+  if (!save) HIP_TRY(hipMemcpy(b.dev, dev.data(), dev.size(), hipMemcpyHostToDevice));
+  return GMES_OK;
+}
+
+static void state_blocks(gmes_sim* s, std::vector<StateBlock>& out) {
+  for (int c = 0; c < 6; ++c) {
+    if (s->pml_state[c]) grid_block(s, out, s->pml_state[c], c, s->has_cls[c][GMES_CLS_CPML] ? 2 : 1);
+    for (int k = GMES_CLS_DRUDE; k < GMES_NCLS; ++k)
+      if (s->ade[c][k].n)
+        out.push_back({s->ade[c][k].state, (size_t)s->ade[c][k].nstate * s->ade[c][k].n * ade_word(s, k), -1, 0});
+  }
+  for (auto& d : s->dfts) out.push_back({d.acc, 2 * (size_t)d.nfreq * d.ncells * 2 * sizeof(double), -1, 0});
+}
+
+// the fields of an auxiliary grid
+static void field_blocks(gmes_sim* a, std::vector<StateBlock>& out) {
+  for (int c = 0; c < 6; ++c) {
+    if (active(a, c)) grid_block(a, out, a->f[c], c, 1);
+    else out.push_back({a->f[c], (size_t)a->dsize[c] * a->esize, -1, 1});
+  }
 }
 
 static int64_t blob_bytes(gmes_sim* s) {
-  std::vector<std::pair<void*, size_t>> b;
+  std::vector<StateBlock> b;
   state_blocks(s, b);
+  for (int i = 0; i < s->naux; ++i)
+    if (s->aux[i]) field_blocks(s->aux[i], b);
   int64_t t = 2 * sizeof(int64_t);
-  for (auto& x : b) t += (int64_t)x.second;
-  for (int i = 0; i < s->naux; ++i) {
-    if (!s->aux[i]) continue;
-    for (int c = 0; c < 6; ++c) t += s->aux[i]->dsize[c] * s->aux[i]->esize;
-    t += blob_bytes(s->aux[i]);
-  }
+  for (auto& x : b) t += (int64_t)x.bytes;
+  for (int i = 0; i < s->naux; ++i)
+    if (s->aux[i]) t += blob_bytes(s->aux[i]);
   return t;
 }
 
@@ -2395,21 +2796,20 @@ static int blob_copy(gmes_sim* s, char* p, bool save, int64_t& done) {
     if (head[0] != kSnapMagic || head[1] < 0) return set_error(GMES_EINVAL, "not a snapshot of this engine");
   }
   done = sizeof head;
-  std::vector<std::pair<void*, size_t>> b;
+  std::vector<StateBlock> b;
   state_blocks(s, b);
   for (auto& x : b) {
-    if (save) HIP_TRY(hipMemcpy(p + done, x.first, x.second, hipMemcpyDeviceToHost));
-    else HIP_TRY(hipMemcpy(x.first, p + done, x.second, hipMemcpyHostToDevice));
-    done += (int64_t)x.second;
+    if (int rc = block_copy(s, x, p + done, save)) return rc;
+    done += (int64_t)x.bytes;
   }
   for (int i = 0; i < s->naux; ++i) {
     gmes_sim* a = s->aux[i];
     if (!a) continue;
-    for (int c = 0; c < 6; ++c) {
-      const size_t fb = (size_t)a->dsize[c] * a->esize;
-      if (save) HIP_TRY(hipMemcpy(p + done, a->f[c], fb, hipMemcpyDeviceToHost));
-      else HIP_TRY(hipMemcpy(a->f[c], p + done, fb, hipMemcpyHostToDevice));
-      done += (int64_t)fb;
+    b.clear();
+    field_blocks(a, b);
+    for (auto& x : b) {
+      if (int rc = block_copy(a, x, p + done, save)) return rc;
+      done += (int64_t)x.bytes;
     }
     int64_t sub = 0;
     int rc = blob_copy(a, p + done, save, sub);

@@ -88,7 +88,8 @@ struct gmes_sim {
   bool fp64 = true;
   int64_t shape[6][3];
   int64_t ncell[6];
-  int32_t pitch[6];          // device row pitch (elements)
+  int32_t pitch[6];          // device row pitch (elements): the stride along j
+  int32_t pi[6], pk[6];      // strides along i and k
   bool packed = false;       // rows unpadded: 3-D sims with rows under 256 cells
   int32_t koff[6];           // device k offset (see FieldArgs)
   int64_t dsize[6];          // device elements per component
@@ -196,6 +197,16 @@ struct gmes_sim {
   gmes_engine::StepRare* d_rare = nullptr;
   int64_t step_tab_cap = 0;   // entries the two tables hold room for
   int64_t sweep_bytes = 0;
+  // 2-D (step2d.hip): columns per block, whole rows or not; places of the
+  // dispersive cells in their lists, the other set of their state
+  bool sweep_2d = false;
+  int sweep_w = 0, sweep_whole = 0;
+  int32_t sweep_run2[3][2] = {};   // Step2Args::run
+  uint16_t* step2_ids = nullptr;   // inside d_step_tab, as are the
+  void* step2_cells = nullptr;     // Step2Cell[3 * entries]
+  int32_t* d_adeq[3] = {};
+  void* ade_alt[3][GMES_NCLS] = {};
+  std::vector<std::array<int, 5>> step2_src;  // direction, i, j, wave, kind
   std::vector<std::array<uint16_t, 3>> step_e, step_h;  // record ids of each entry
   std::vector<std::pair<int64_t, uint32_t>> src_ids;  // ids the sources replaced (element, old word)
   int step_net = 0, step_nht = 0;

@@ -32,20 +32,24 @@ constexpr int kPad = 32;  // elements before row 0 of every device array
 // koff = 1 for Hx and Hy on a padded layout, so that the first updated
 // cell of every row (k = 0 for E and Hz, k = 1 for Hx, Hy) starts a
 // 128-byte line.  3-D sims with rows under 256 cells keep p = s2 and
-// koff = 0 (gmes_sim::packed).  Material ids and CPML/UPML state use the
-// same layout.
+// koff = 0 (gmes_sim::packed).  Collapsed-z 2-D modes (TMz, TEz) keep each z
+// plane of a component in one piece: element kPad + i*pi + j + k*pk - koff,
+// with rows along j padded the same way (koff = 1 for Hx and Hz, updated
+// from j = 1).  With k fastest, every second element of Hx, Hy (TMz) or Ex,
+// Ey (TEz) is a ghost, and the launches move twice the bytes they use.
+// Material ids and CPML/UPML state use the same layout.
 template <class T>
 struct FieldArgs {
   T* f[6];
   int s[6][3];
-  int p[6];
+  int pi[6], p[6], pk[6];  // strides along i, j, k
   int koff[6];
   unsigned active;
 };
 
 template <class T>
 __host__ __device__ __forceinline__ int didx(const FieldArgs<T>& a, int c, int i, int j, int k) {
-  return kPad + (i * a.s[c][1] + j) * a.p[c] + k - a.koff[c];
+  return kPad + i * a.pi[c] + j * a.p[c] + k * a.pk[c] - a.koff[c];
 }
 
 template <class T>
@@ -154,6 +158,66 @@ struct Step3Args {
   int exact;       // FP64: every division is by a power of two
   int ghosts;      // write the ghost planes: the last step of a call, unless a monitor reads them
 };
+// The same for a collapsed-z 2-D mode (TMz: Ez, Hx, Hy; TEz: Ex, Ey, Hz).
+// Arrays are indexed by the direction of the component; thread (i, j) owns
+// one cell of each, at element off + i * pi + j of its arrays.
+constexpr int kStep2Src = 16;
+struct Step2Cell {
+  int32_t kind;  // 0 the update of its entry, 1 Dummy, 2 Const, 3 dispersive
+  int32_t rec;   // dispersive: its record
+  double re, im; // Const value
+};
+template <class R>
+struct Step2Ent {
+  R c[3];         // dt/eps; UPML: 1/eps (FP32) or eps (FP64)
+  uint32_t meta;  // 2 bits a component: 0 Dielectric, 1 absorber, 2 see Step2Cell
+};
+template <class T>
+struct Step2Args {
+  using R = typename real_of<T>::type;
+  const T* fi[3];       // old fields, at thread (0, 0)'s cells
+  T* fo[3];             // new ones
+  // absorber words: CPML [x word, y word] of E and of H, UPML the component's
+  const T* si[3][2];
+  T* so[3][2];          // (H: the same arrays, only the owner touches a word)
+  int pi;               // stride along i, of every array
+  int64_t pk[3];        // from the updated z plane to its ghost plane (0: none)
+  const uint16_t* ids;  // [i * pi + j] entries
+  int n[2];
+  const Step2Ent<R>* tab;
+  const Step2Cell* cells;  // [3 * entry + direction]
+  int nent;
+  R d[3], inv_d[3];
+  const R* row[3][3];   // absorber rows of component c along axis a, at thread (0, 0)'s coordinate
+  int run[3][2];        // CPML: thread coordinates lo | hi << 16 without live state, x and y; UPML: [0] the UPML-free box
+  cplx<R> ph[3][3];     // ghost phase of component c along axis a
+  const DevRec<R>* recs;
+  const R* coef;
+  const int32_t* adeq[3];  // place of a dispersive cell in its list, at thread (0, 0)'s cell
+  const void* ade_in[3][3];
+  void* ade_out[3][3];
+  int ade_n[3][3];
+  int nsrc;
+  struct { int c, i, j, wave, kind; } src[kStep2Src];
+  int w;                // columns a block owns; n[1] when whole (neighbours wrap inside the block)
+  int whole;
+  int ch;               // rows per block
+  int nj, nblk;
+  const double* waves;
+  Ctl* ctl;
+  int par;
+  int exact;
+  int ghosts;
+};
+// threads of a block at most: 8-byte and wider words need more than 64 registers
+template <class T> constexpr int kStep2Threads = sizeof(T) == 4 ? 1024 : 512;
+// threads of a block: its columns and, unless rows are whole, two rim lanes
+inline int step2_threads(int w, int whole) { return ((whole ? w : w + 2) + 63) / 64 * 64; }
+template <class T>
+inline size_t step2_lds(int nthreads, int nent) {
+  return (size_t)nent * sizeof(Step2Ent<typename real_of<T>::type>) + 4 * (size_t)nthreads * sizeof(T);
+}
+
 // The entry ids of a sim, looked up from its material ids on the device.
 struct StepKey {
   uint64_t key, id;  // key ~0: empty slot
@@ -172,8 +236,16 @@ struct StepIdArgs {
   int n[3];
   int pitch;       // of out's rows
   uint32_t* out;
+  uint16_t* out16;  // one field type's: 2-D modes, whose three components make one triple
 };
 void launch_step_ids(const StepIdArgs& a, hipStream_t st);
+// out[element of cell[q]] = q, for the cells of a list
+struct PlaceArgs {
+  const int32_t* cell;
+  int n, s1, s2, pi, p, pk;
+  int32_t* out;  // at element (0, 0, 0)
+};
+void launch_list_places(const PlaceArgs& a, hipStream_t st);
 // threads of a block at most, the stride of its LDS exchange planes
 constexpr int kStepMaxThreads = 1024;
 template <class T> constexpr int kStepThreads = kStepMaxThreads;
@@ -276,9 +348,9 @@ struct GhostJob {
 template <class T>
 struct DftJob {
   T* f;
-  int s1, p, koff, comp;
+  int pi, p, pk, koff, comp;
   int lo[3], n[3];
-  int nfreq, decim, electric, pad_;
+  int nfreq, decim, electric;
   int64_t ncells;
   double* acc;      // [nfreq][ncells][re, im]
   const double* w;  // [row][nfreq][2: E, H][re, im]
@@ -303,7 +375,7 @@ constexpr int kSqBlockCells = 2048;  // 256 threads x 8 cells
 template <class T>
 struct SqBox {
   const T* f;    // element 0 of the device array
-  int s1, p, koff;
+  int pi, p, pk, koff;
   int lo[3], n[3];
   int ncells;    // < 2^31 (a component holds < 2^31 elements)
 };
@@ -311,10 +383,15 @@ inline int64_t sq_blocks(int64_t ncells) { return (ncells + kSqBlockCells - 1) /
 template <class T>
 void launch_sum_sq(const SqBox<T>& b, double* partial, hipStream_t st);
 
-// rows x n2 elements of esize bytes from rows spaced spitch elements apart
-// to rows spaced dpitch apart (field reads and writes of padded layouts)
-void launch_pitch_copy(const void* src, void* dst, int64_t rows, int n2, int spitch, int dpitch, int esize,
-                       hipStream_t st);
+// Elements of esize bytes of a component between the host's dense (i, j, k)
+// order and its device layout (field reads and writes): dev points at the
+// element of (0, 0, 0).
+struct LayoutArgs {
+  int64_t total;
+  int n1, n2;      // extents along j, k
+  int pi, p, pk;
+};
+void launch_layout_copy(bool to_device, void* dense, void* dev, const LayoutArgs& a, int esize, hipStream_t st);
 // out[x] = (uint8_t)ids[x]
 void launch_narrow_ids(const uint16_t* ids, uint8_t* out, int64_t n, hipStream_t st);
 template <class T>
@@ -351,6 +428,8 @@ void launch_main3d(bool electric, const MainArgs<T>& m, int bx, int by, int ichu
 // absorber: 0 none, 1 CPML, 2 UPML
 template <class T>
 void launch_step3d(const Step3Args<T>& m, int absorber, int nthreads, hipStream_t st);
+template <class T>
+void launch_step2d(const Step2Args<T>& m, bool tm, int absorber, bool ade, hipStream_t st);
 // clk[0] = clk[1] = clock: before the first one-sweep step after others
 void launch_clock_copy(Ctl* ctl, hipStream_t st);
 template <class T>

@@ -178,6 +178,128 @@ __device__ __forceinline__ void fused_ghost(const MainArgs<T>& m, int C, T* __re
   }
 }
 
+// Dispersive (ADE) cells: the new value of cell q of a list of n cells from
+// its old value e_now and the curl cu = D1/d1 - D2/d2.  State words are read
+// from st and the new ones written to so (the same array, or the other set
+// of a one-sweep step; `keep` false: not at all).  a: the record's
+// coefficients, P1 and P2 its pole counts.
+//
+// Drude and Lorentz poles: src/pw_drude.hh:90-101,145-150; src/pw_lorentz.hh:96-107,150-156
+template <class T>
+__device__ __forceinline__ T ade_drude_value(const typename real_of<T>::type* a, int P, const T* st, T* so, int n,
+                                             int q, bool keep, T e_now, T cu) {
+  const auto* cc = a + 3 * P;
+  T sum = vzero<T>();
+  for (int p = 0; p < P; ++p) {
+    const T q_old = ld_nt(st + p * n + q);
+    const T q_now = ld_nt(st + (P + p) * n + q);
+    const T q_new = vadd(vadd(vscl(gld(a + 3 * p), q_old), vscl(gld(a + 3 * p + 1), q_now)), vscl(gld(a + 3 * p + 2), e_now));
+    if (keep) {
+      st_nt(so + p * n + q, q_now);
+      st_nt(so + (P + p) * n + q, q_new);
+    }
+    sum = vadd(sum, vsub(q_new, q_now));
+  }
+  return vadd(vadd(vscl(gld(cc), cu), vscl(gld(cc + 1), sum)), vscl(gld(cc + 2), e_now));
+}
+
+// Drude-critical-points, ADE form: src/pw_dcp.hh:105-167,200-225
+// words: 0 e_old | 1..D q_old | D+1..2D q_now | 2D+1.. p_old | 2D+C+1.. p_now
+template <class T>
+__device__ __forceinline__ T ade_dcp_value(const typename real_of<T>::type* a, int D, int NC, const T* st, T* so,
+                                           int n, int q, bool keep, T e_now, T cu) {
+  using R = typename real_of<T>::type;
+  const R* b = a + 3 * D;
+  const R* cc = b + 5 * NC;
+  const T e_old = gld(st + q);
+  T ds = vzero<T>(), cs = vzero<T>();
+  for (int p = 0; p < D; ++p)
+    ds = vadd(ds, vsub(vscl(R(1) - gld(a + 3 * p + 1), gld(st + (1 + D + p) * n + q)),
+                       vscl(gld(a + 3 * p), gld(st + (1 + p) * n + q))));
+  for (int p = 0; p < NC; ++p)
+    cs = vadd(cs, vsub(vscl(R(1) - gld(b + 5 * p + 1), gld(st + (1 + 2 * D + NC + p) * n + q)),
+                       vscl(gld(b + 5 * p), gld(st + (1 + 2 * D + p) * n + q))));
+  const T e_new = vadd(vadd(vadd(vscl(gld(cc), cu), vscl(gld(cc + 1), vadd(ds, cs))), vscl(gld(cc + 2), e_old)),
+                       vscl(gld(cc + 3), e_now));
+  if (!keep) return e_new;
+  const T mix = vadd(vadd(e_old, vscl(R(2), e_now)), e_new);
+  for (int p = 0; p < D; ++p) {
+    const T qo = gld(st + (1 + p) * n + q), qn = gld(st + (1 + D + p) * n + q);
+    const T qq = vadd(vadd(vscl(gld(a + 3 * p), qo), vscl(gld(a + 3 * p + 1), qn)), vscl(gld(a + 3 * p + 2), mix));
+    st_nt(so + (1 + p) * n + q, qn);
+    st_nt(so + (1 + D + p) * n + q, qq);
+  }
+  for (int p = 0; p < NC; ++p) {
+    const T po = gld(st + (1 + 2 * D + p) * n + q), pn = gld(st + (1 + 2 * D + NC + p) * n + q);
+    const T pp = vadd(vadd(vadd(vadd(vscl(gld(b + 5 * p), po), vscl(gld(b + 5 * p + 1), pn)),
+                                vscl(gld(b + 5 * p + 2), e_old)),
+                           vscl(gld(b + 5 * p + 3), e_now)),
+                      vscl(gld(b + 5 * p + 4), e_new));
+    st_nt(so + (1 + 2 * D + p) * n + q, pn);
+    st_nt(so + (1 + 2 * D + NC + p) * n + q, pp);
+  }
+  st_nt(so + q, e_now);
+  return e_new;
+}
+
+// Drude-critical-points, PLRC/RC form: src/pw_dcp.hh:467-518,564-586.
+// State words are complex for any field type: psi_dp (re part = psi_dp_re,
+// im part = psi_dp_im), psi_cp_re, psi_cp_im.
+template <class T>
+__device__ __forceinline__ T ade_plrc_value(const typename real_of<T>::type* a, int D, int NC,
+                                            const cplx<typename real_of<T>::type>* st,
+                                            cplx<typename real_of<T>::type>* so, int n, int q, bool keep, T fv, T cu) {
+  using R = typename real_of<T>::type;
+  using Z = cplx<R>;
+  const R* b = a + 3 * D;
+  const R* cc = b + 6 * NC;
+  const Z e_now = {re_of(fv), im_of(fv)};
+  R sdr = R(0), sdi = R(0);
+  for (int p = 0; p < D; ++p) {
+    const Z v = gld(st + p * n + q);
+    sdr = sdr + v.re;
+    sdi = sdi + v.im;
+  }
+  Z scr = {R(0), R(0)}, sci = {R(0), R(0)};
+  for (int p = 0; p < NC; ++p) scr = vadd(scr, gld(st + (D + p) * n + q));
+  for (int p = 0; p < NC; ++p) sci = vadd(sci, gld(st + (D + NC + p) * n + q));
+  const Z psi = {sdr + scr.re, sdi + sci.re};  // .real() of the imaginary-part sum
+  Z e_new;
+  if constexpr (is_cplx<T>::value) {
+    e_new = vadd(vadd(vscl(gld(cc), Z{cu.re, cu.im}), vscl(gld(cc + 1), e_now)), vscl(gld(cc + 2), psi));
+  } else {
+    e_new.re = (gld(cc) * cu + gld(cc + 1) * e_now.re) + gld(cc + 2) * psi.re;
+    e_new.im = gld(cc + 1) * e_now.im + gld(cc + 2) * psi.im;
+  }
+  if (keep) {
+    for (int p = 0; p < D; ++p) {
+      Z v = gld(st + p * n + q);
+      v.re = (gld(a + 3 * p) * e_new.re + gld(a + 3 * p + 1) * e_now.re) + gld(a + 3 * p + 2) * v.re;
+      v.im = (gld(a + 3 * p) * e_new.im + gld(a + 3 * p + 1) * e_now.im) + gld(a + 3 * p + 2) * v.im;
+      gst(so + p * n + q, v);
+    }
+    for (int p = 0; p < NC; ++p) {
+      const Z b0 = {gld(b + 6 * p), gld(b + 6 * p + 1)}, b1 = {gld(b + 6 * p + 2), gld(b + 6 * p + 3)},
+              b2 = {gld(b + 6 * p + 4), gld(b + 6 * p + 5)};
+      const Z vr = gld(st + (D + p) * n + q), vi = gld(st + (D + NC + p) * n + q);
+      gst(so + (D + p) * n + q, vadd(vadd(vscl(e_new.re, b0), vscl(e_now.re, b1)), cmul(b2, vr)));
+      gst(so + (D + NC + p) * n + q, vadd(vadd(vscl(e_new.im, b0), vscl(e_now.im, b1)), cmul(b2, vi)));
+    }
+  }
+  return make_val<T>(e_new.re, e_new.im);
+}
+
+template <class T>
+__device__ __forceinline__ T ade_value(int cls, const typename real_of<T>::type* a, int P1, int P2, const void* st,
+                                       void* so, int n, int q, bool keep, T e_now, T cu) {
+  using Z = cplx<typename real_of<T>::type>;
+  if (cls == GMES_CLS_DRUDE)
+    return ade_drude_value<T>(a, P1, static_cast<const T*>(st), static_cast<T*>(so), n, q, keep, e_now, cu);
+  if (cls == GMES_CLS_DCP_ADE)
+    return ade_dcp_value<T>(a, P1, P2, static_cast<const T*>(st), static_cast<T*>(so), n, q, keep, e_now, cu);
+  return ade_plrc_value<T>(a, P1, P2, static_cast<const Z*>(st), static_cast<Z*>(so), n, q, keep, e_now, cu);
+}
+
 // Batched launches: block -> job by binary search on the jobs' first
 // blocks (uniform across a block).
 template <class J>

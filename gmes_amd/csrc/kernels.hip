@@ -849,147 +849,36 @@ __device__ __forceinline__ void cell_ijk(const FieldArgs<T>& a, int c, int flat,
   i = t / sy;
 }
 
-// Drude and Lorentz poles: src/pw_drude.hh:90-101,145-150; src/pw_lorentz.hh:96-107,150-156
+// One cell of an ADE list: its update from AdeArgs' arrays, in place.
 template <int C, class T>
-__device__ __forceinline__ void ade_drude_cell(const AdeArgs<T>& m, int q) {
+__device__ __forceinline__ void ade_cell(const AdeArgs<T>& m, int q, int cls) {
   using R = typename real_of<T>::type;
   if (q >= m.n) return;
-  const int flat = m.cell[q];
   int i, j, k;
-  cell_ijk(m.fa, C, flat, i, j, k);
+  cell_ijk(m.fa, C, m.cell[q], i, j, k);
   const DevRec<R>& rec = m.recs[m.rec[q]];
-  const R* a = m.coef + rec.coef_off;
-  const int P = rec.n1;
-  const R* cc = a + 3 * P;
-  T* st = static_cast<T*>(m.state);
   T* F = m.fa.f[C] + didx(m.fa, C, i, j, k);
   const T e_now = ld_nt(F);
-  T sum = vzero<T>();
-  for (int p = 0; p < P; ++p) {
-    const T q_old = ld_nt(st + p * m.n + q);
-    const T q_now = ld_nt(st + (P + p) * m.n + q);
-    const T q_new = vadd(vadd(vscl(a[3 * p], q_old), vscl(a[3 * p + 1], q_now)), vscl(a[3 * p + 2], e_now));
-    st_nt(st + p * m.n + q, q_now);
-    st_nt(st + (P + p) * m.n + q, q_new);
-    sum = vadd(sum, vsub(q_new, q_now));
-  }
   T D1, D2;
   curl_terms<C>(m.fa, i, j, k, D1, D2);
-  const R d1 = m.d[Ax<C>::a1], d2 = m.d[Ax<C>::a2];
-  T cu = vsub(vdiv(D1, d1), vdiv(D2, d2));
-  st_nt(F, vadd(vadd(vscl(cc[0], cu), vscl(cc[1], sum)), vscl(cc[2], e_now)));
+  const T cu = vsub(vdiv(D1, m.d[Ax<C>::a1]), vdiv(D2, m.d[Ax<C>::a2]));
+  st_nt(F, ade_value<T>(cls, m.coef + rec.coef_off, rec.n1, rec.n2, m.state, m.state, m.n, q, true, e_now, cu));
 }
+template <int C, class T>
+__device__ __forceinline__ void ade_drude_cell(const AdeArgs<T>& m, int q) { ade_cell<C, T>(m, q, GMES_CLS_DRUDE); }
+template <int C, class T>
+__device__ __forceinline__ void ade_dcp_cell(const AdeArgs<T>& m, int q) { ade_cell<C, T>(m, q, GMES_CLS_DCP_ADE); }
+template <int C, class T>
+__device__ __forceinline__ void ade_plrc_cell(const AdeArgs<T>& m, int q) { ade_cell<C, T>(m, q, GMES_CLS_DCP_PLRC); }
 
 template <int C, class T>
 __global__ void __launch_bounds__(256) k_ade_drude(AdeArgs<T> m) {
   ade_drude_cell<C, T>(m, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
-// Drude-critical-points, ADE form: src/pw_dcp.hh:105-167,200-225
-template <int C, class T>
-__device__ __forceinline__ void ade_dcp_cell(const AdeArgs<T>& m, int q) {
-  using R = typename real_of<T>::type;
-  if (q >= m.n) return;
-  const int flat = m.cell[q];
-  int i, j, k;
-  cell_ijk(m.fa, C, flat, i, j, k);
-  const DevRec<R>& rec = m.recs[m.rec[q]];
-  const int D = rec.n1, NC = rec.n2;
-  const R* a = m.coef + rec.coef_off;
-  const R* b = a + 3 * D;
-  const R* cc = b + 5 * NC;
-  T* st = static_cast<T*>(m.state);
-  const int n = m.n;
-  // words: 0 e_old | 1..D q_old | D+1..2D q_now | 2D+1.. p_old | 2D+C+1.. p_now
-  T* F = m.fa.f[C] + didx(m.fa, C, i, j, k);
-  const T e_now = *F;
-  const T e_old = st[q];
-  T ds = vzero<T>(), cs = vzero<T>();
-  for (int p = 0; p < D; ++p)
-    ds = vadd(ds, vsub(vscl(R(1) - a[3 * p + 1], st[(1 + D + p) * n + q]), vscl(a[3 * p], st[(1 + p) * n + q])));
-  for (int p = 0; p < NC; ++p)
-    cs = vadd(cs, vsub(vscl(R(1) - b[5 * p + 1], st[(1 + 2 * D + NC + p) * n + q]),
-                       vscl(b[5 * p], st[(1 + 2 * D + p) * n + q])));
-  T D1, D2;
-  curl_terms<C>(m.fa, i, j, k, D1, D2);
-  const R d1 = m.d[Ax<C>::a1], d2 = m.d[Ax<C>::a2];
-  T cu = vsub(vdiv(D1, d1), vdiv(D2, d2));
-  T e_new = vadd(vadd(vadd(vscl(cc[0], cu), vscl(cc[1], vadd(ds, cs))), vscl(cc[2], e_old)), vscl(cc[3], e_now));
-  T mix = vadd(vadd(e_old, vscl(R(2), e_now)), e_new);
-  for (int p = 0; p < D; ++p) {
-    T qo = st[(1 + p) * n + q], qn = st[(1 + D + p) * n + q];
-    T qq = vadd(vadd(vscl(a[3 * p], qo), vscl(a[3 * p + 1], qn)), vscl(a[3 * p + 2], mix));
-    st_nt(st + (1 + p) * n + q, qn);
-    st_nt(st + (1 + D + p) * n + q, qq);
-  }
-  for (int p = 0; p < NC; ++p) {
-    T po = st[(1 + 2 * D + p) * n + q], pn = st[(1 + 2 * D + NC + p) * n + q];
-    T pp = vadd(vadd(vadd(vadd(vscl(b[5 * p], po), vscl(b[5 * p + 1], pn)), vscl(b[5 * p + 2], e_old)),
-                     vscl(b[5 * p + 3], e_now)),
-                vscl(b[5 * p + 4], e_new));
-    st_nt(st + (1 + 2 * D + p) * n + q, pn);
-    st_nt(st + (1 + 2 * D + NC + p) * n + q, pp);
-  }
-  st_nt(st + q, e_now);
-  st_nt(F, e_new);
-}
-
 template <int C, class T>
 __global__ void __launch_bounds__(256) k_ade_dcp(AdeArgs<T> m) {
   ade_dcp_cell<C, T>(m, blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-// Drude-critical-points, PLRC/RC form: src/pw_dcp.hh:467-518,564-586.
-// State words are complex for any field type: psi_dp (re part = psi_dp_re,
-// im part = psi_dp_im), psi_cp_re, psi_cp_im.
-template <int C, class T>
-__device__ __forceinline__ void ade_plrc_cell(const AdeArgs<T>& m, int q) {
-  using R = typename real_of<T>::type;
-  using Z = cplx<R>;
-  if (q >= m.n) return;
-  const int flat = m.cell[q];
-  int i, j, k;
-  cell_ijk(m.fa, C, flat, i, j, k);
-  const DevRec<R>& rec = m.recs[m.rec[q]];
-  const int D = rec.n1, NC = rec.n2;
-  const R* a = m.coef + rec.coef_off;
-  const R* b = a + 3 * D;
-  const R* cc = b + 6 * NC;
-  Z* st = static_cast<Z*>(m.state);
-  const int n = m.n;
-  T* F = m.fa.f[C] + didx(m.fa, C, i, j, k);
-  const T fv = *F;
-  const Z e_now = {re_of(fv), im_of(fv)};
-  R sdr = R(0), sdi = R(0);
-  for (int p = 0; p < D; ++p) sdr = sdr + st[p * n + q].re;
-  for (int p = 0; p < D; ++p) sdi = sdi + st[p * n + q].im;
-  Z scr = {R(0), R(0)}, sci = {R(0), R(0)};
-  for (int p = 0; p < NC; ++p) scr = vadd(scr, st[(D + p) * n + q]);
-  for (int p = 0; p < NC; ++p) sci = vadd(sci, st[(D + NC + p) * n + q]);
-  const Z psi = {sdr + scr.re, sdi + sci.re};  // .real() of the imaginary-part sum
-  T D1, D2;
-  curl_terms<C>(m.fa, i, j, k, D1, D2);
-  const R d1 = m.d[Ax<C>::a1], d2 = m.d[Ax<C>::a2];
-  const T cu = vsub(vdiv(D1, d1), vdiv(D2, d2));
-  Z e_new;
-  if constexpr (is_cplx<T>::value) {
-    e_new = vadd(vadd(vscl(cc[0], Z{cu.re, cu.im}), vscl(cc[1], e_now)), vscl(cc[2], psi));
-  } else {
-    e_new.re = (cc[0] * cu + cc[1] * e_now.re) + cc[2] * psi.re;
-    e_new.im = cc[1] * e_now.im + cc[2] * psi.im;
-  }
-  for (int p = 0; p < D; ++p) {
-    Z v = st[p * n + q];
-    v.re = (a[3 * p] * e_new.re + a[3 * p + 1] * e_now.re) + a[3 * p + 2] * v.re;
-    v.im = (a[3 * p] * e_new.im + a[3 * p + 1] * e_now.im) + a[3 * p + 2] * v.im;
-    st[p * n + q] = v;
-  }
-  for (int p = 0; p < NC; ++p) {
-    const Z b0 = {b[6 * p], b[6 * p + 1]}, b1 = {b[6 * p + 2], b[6 * p + 3]}, b2 = {b[6 * p + 4], b[6 * p + 5]};
-    st[(D + p) * n + q] = vadd(vadd(vscl(e_new.re, b0), vscl(e_now.re, b1)), cmul(b2, st[(D + p) * n + q]));
-    st[(D + NC + p) * n + q] = vadd(vadd(vscl(e_new.im, b0), vscl(e_now.im, b1)), cmul(b2, st[(D + NC + p) * n + q]));
-  }
-  *F = make_val<T>(e_new.re, e_new.im);
 }
 
 template <int C, class T>
@@ -1120,7 +1009,7 @@ __global__ void __launch_bounds__(256) k_dft_batch(const DftJob<T>* jobs, int nj
   const int k = (int)(q % J.n[2]);
   const int j = (int)((q / J.n[2]) % J.n[1]);
   const int i = (int)(q / ((int64_t)J.n[2] * J.n[1]));
-  const T v = gld(J.f + (kPad + ((i + J.lo[0]) * J.s1 + (j + J.lo[1])) * J.p + (k + J.lo[2]) - J.koff));
+  const T v = gld(J.f + (kPad + (i + J.lo[0]) * J.pi + (j + J.lo[1]) * J.p + (k + J.lo[2]) * J.pk - J.koff));
   const double vr = (double)re_of(v), vi = (double)im_of(v);
   // the job table's pointers are global memory: address them as such
   const GMES_GLOBAL double* w = (const GMES_GLOBAL double*)J.w + row * J.nfreq * 4 + (J.electric ? 0 : 2);
@@ -1374,19 +1263,19 @@ void launch_main3d_flat(bool electric, const MainArgs<T>& m, hipStream_t st) {
   }
 }
 
-// Row repacking for field reads and writes of padded layouts: element k of
-// row r moves from src[r * sp + k] to dst[r * dp + k].  A 2-D copy from
-// the pitched device rows straight to pageable host memory ran at 0.2 GB/s
-// (256^3 FP32: 0.3 s per component); packing on the device and copying
-// one contiguous block is limited by the host link instead.
-template <class W>
-__global__ void __launch_bounds__(256) k_pitch_copy(const W* __restrict__ src, W* __restrict__ dst, int64_t total,
-                                                    int n2, int sp, int dp) {
+// Field reads and writes of layouts that differ from the host's.  A 2-D copy
+// from the pitched device rows straight to pageable host memory ran at
+// 0.2 GB/s (256^3 FP32: 0.3 s per component); packing on the device and
+// copying one contiguous block is limited by the host link instead.
+template <class W, bool TO>
+__global__ void __launch_bounds__(256) k_layout_copy(W* __restrict__ dense, W* __restrict__ dev, LayoutArgs a) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (t >= total) return;
-  const int64_t r = t / n2;
-  const int64_t k = t - r * n2;
-  dst[r * dp + k] = src[r * sp + k];
+  if (t >= a.total) return;
+  const int64_t r = t / a.n2;
+  const int64_t i = r / a.n1;
+  const int64_t x = i * a.pi + (r - i * a.n1) * a.p + (t - r * a.n2) * a.pk;
+  if (TO) dev[x] = dense[t];
+  else dense[t] = dev[x];
 }
 
 #if GMES_TYPE == 0
@@ -1400,22 +1289,20 @@ void launch_narrow_ids(const uint16_t* ids, uint8_t* out, int64_t n, hipStream_t
   hipLaunchKernelGGL(k_narrow_ids, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, ids, out, n);
 }
 
-void launch_pitch_copy(const void* src, void* dst, int64_t rows, int n2, int spitch, int dpitch, int esize,
-                       hipStream_t st) {
-  const int64_t total = rows * n2;
-  if (total <= 0) return;
-  const dim3 grid((unsigned)((total + 255) / 256)), block(256);
+void launch_layout_copy(bool to, void* dense, void* dev, const LayoutArgs& a, int esize, hipStream_t st) {
+  if (a.total <= 0) return;
+  const dim3 grid((unsigned)((a.total + 255) / 256)), block(256);
   typedef unsigned long long u64_t;
   typedef int w16_t __attribute__((ext_vector_type(4)));
-  if (esize == 4)
-    hipLaunchKernelGGL((k_pitch_copy<uint32_t>), grid, block, 0, st, (const uint32_t*)src, (uint32_t*)dst, total, n2,
-                       spitch, dpitch);
-  else if (esize == 8)
-    hipLaunchKernelGGL((k_pitch_copy<u64_t>), grid, block, 0, st, (const u64_t*)src, (u64_t*)dst, total, n2, spitch,
-                       dpitch);
-  else
-    hipLaunchKernelGGL((k_pitch_copy<w16_t>), grid, block, 0, st, (const w16_t*)src, (w16_t*)dst, total, n2, spitch,
-                       dpitch);
+#define GMES_LAYOUT(W)                                                                                     \
+  {                                                                                                        \
+    if (to) hipLaunchKernelGGL((k_layout_copy<W, true>), grid, block, 0, st, (W*)dense, (W*)dev, a);       \
+    else hipLaunchKernelGGL((k_layout_copy<W, false>), grid, block, 0, st, (W*)dense, (W*)dev, a);         \
+  }
+  if (esize == 4) GMES_LAYOUT(uint32_t)
+  else if (esize == 8) GMES_LAYOUT(u64_t)
+  else GMES_LAYOUT(w16_t)
+#undef GMES_LAYOUT
 }
 #endif
 
@@ -1538,7 +1425,7 @@ __global__ void __launch_bounds__(256) k_sum_sq(SqBox<T> b, double* __restrict__
     if (q < b.ncells) {
       const int k = q % b.n[2], t = q / b.n[2];
       const int j = t % b.n[1], i = t / b.n[1];
-      acc = acc + sq_of(b.f[kPad + ((i + b.lo[0]) * b.s1 + (j + b.lo[1])) * b.p + (k + b.lo[2]) - b.koff]);
+      acc = acc + sq_of(b.f[kPad + (i + b.lo[0]) * b.pi + (j + b.lo[1]) * b.p + (k + b.lo[2]) * b.pk - b.koff]);
     }
   }
   const double tot = block_sum_256(acc);

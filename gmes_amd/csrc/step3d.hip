@@ -37,16 +37,9 @@
 // the values and products of the separate copies (k_ghost): E's from the
 // new E, H's from the old H, as the copies at the two places of a step
 // leave them.
-#include "kernel_common.h"
+#include "step_common.h"
 
 namespace gmes_engine {
-
-#define GMES_CONST __attribute__((address_space(4)))
-// uniform reads of data no kernel writes meanwhile: scalar loads
-template <class V>
-__device__ __forceinline__ V cld(const V* p) {
-  return *(const GMES_CONST V*)(uintptr_t)p;
-}
 
 // Buffer accesses: a resource (base, size) per array, the plane as scalar
 // offset, the lane's place in the plane as vector offset.  One scalar offset
@@ -95,30 +88,11 @@ __device__ __forceinline__ void bst(const GMES_CONST i4_t& r, unsigned v, unsign
   else raw_store_v2f32(__builtin_bit_cast(vec2_t<float>, x), r, (int)v, (int)s, kAuxNt);
 }
 
-// Division by a cell size or a CPML kappa.  EXACT: every divisor of the sim
-// is a power of two (kappa: 1), so multiplying by the reciprocal rounds the
-// same real number and gives the quotient's bits.
-template <bool EXACT, class T, class R>
-__device__ __forceinline__ T by_size(T x, R d, R inv_d) {
-  if constexpr (EXACT) return vscl(inv_d, x);
-  else return vdiv(x, d);
-}
-template <bool EXACT, class T, class R>
-__device__ __forceinline__ T by_kappa(T x, R k) {
-  if constexpr (EXACT) return x;
-  else return vdiv(x, k);
-}
-
 // Absorber rows of one axis: CPML b, c, kappa (FP32: 1/kappa); UPML c1..c4
 // of the row two components share, c5, c6 of the third's.  Those of the
 // block's j and k live in LDS: held in registers for the whole march they
 // cost 12 (CPML) to 24 (UPML) of them, twice that in FP64.
 template <int PML> struct RowStride { static constexpr int v = PML == 2 ? 8 : 4; };
-template <class R, int PML>
-struct Rows {
-  R v[PML == 2 ? 6 : 3];
-};
-
 // A CPML coordinate without live state: c = 0, kappa = 1, and b multiplies a
 // word that is +0, so the CPML update below is the Dielectric one.
 template <class R, int PML>
@@ -158,54 +132,6 @@ __device__ __forceinline__ Rows<R, PML> x_row(const R* shared, const R* own, int
   return r;
 }
 
-// New value of one component, with the formulas and operand order of
-// update_value (kernels.hip).  plain: Dielectric; cpml: CPML with rows r1, r2
-// of the curl axes, old words o1, o2 and new ones n1, n2; upml: rows r1, r2
-// of the curl axes and r0 of the own one.
-template <bool E, bool X, class T, class R>
-__device__ __forceinline__ T plain_value(R c, T f, T D1, T D2, R d1, R i1, R d2, R i2) {
-  if constexpr (std::is_same<R, float>::value) {
-    const T a = vscl(i1, D1), b = vscl(i2, D2);
-    return E ? fma_(c, vsub(a, b), f) : fma_(c, vsub(b, a), f);
-  } else {
-    const T a = by_size<X>(D1, d1, i1), b = by_size<X>(D2, d2, i2);
-    return vadd(f, vscl(c, E ? vsub(a, b) : vsub(b, a)));
-  }
-}
-
-template <bool E, bool X, class T, class R>
-__device__ __forceinline__ T cpml_value(R c, T f, T D1, T D2, R d1, R i1, R d2, R i2, const Rows<R, 1>& r1,
-                                        const Rows<R, 1>& r2, T o1, T o2, T& n1, T& n2) {
-  if constexpr (std::is_same<R, float>::value) {
-    const T a = vscl(i1, D1), b = vscl(i2, D2);
-    n1 = fma_(r1.v[1], a, vscl(r1.v[0], o1));
-    n2 = fma_(r2.v[1], b, vscl(r2.v[0], o2));
-    const T t = vsub(vadd(fma_(-r2.v[2], b, vscl(r1.v[2], a)), n1), n2);
-    return E ? fma_(c, t, f) : fma_(-c, t, f);
-  } else {
-    n1 = vadd(vscl(r1.v[0], o1), by_size<X>(vscl(r1.v[1], D1), d1, i1));
-    n2 = vadd(vscl(r2.v[0], o2), by_size<X>(vscl(r2.v[1], D2), d2, i2));
-    const T t = vsub(vadd(vsub(by_kappa<X>(by_size<X>(D1, d1, i1), r1.v[2]),
-                               by_kappa<X>(by_size<X>(D2, d2, i2), r2.v[2])), n1), n2);
-    return E ? vadd(f, vscl(c, t)) : vsub(f, vscl(c, t));
-  }
-}
-
-// c: dt / eps; q: 1 / eps (FP32) or eps (FP64)
-template <bool E, bool X, class T, class R>
-__device__ __forceinline__ T upml_value(R q, T f, T D1, T D2, R d1, R i1, R d2, R i2, const Rows<R, 2>& r1,
-                                        const Rows<R, 2>& r2, const Rows<R, 2>& r0, T o, T& n) {
-  if constexpr (std::is_same<R, float>::value) {
-    const T cu = vsub(vscl(i1, D1), vscl(i2, D2));
-    n = E ? fma_(r1.v[1], cu, vscl(r1.v[0], o)) : fma_(-r1.v[1], cu, vscl(r1.v[0], o));
-    return fma_(r2.v[3] * q, fma_(-r0.v[5], o, vscl(r0.v[4], n)), vscl(r2.v[2], f));
-  } else {
-    const T cu = vsub(by_size<X>(D1, d1, i1), by_size<X>(D2, d2, i2));
-    n = E ? vadd(vscl(r1.v[0], o), vscl(r1.v[1], cu)) : vsub(vscl(r1.v[0], o), vscl(r1.v[1], cu));
-    return vadd(vscl(r2.v[2], f), vdiv(vscl(r2.v[3], vsub(vscl(r0.v[4], n), vscl(r0.v[5], o))), q));
-  }
-}
-
 // The arguments stay in constant memory (the kernel's own argument block, or
 // a job of a batch) and are read where they are used, through a pointer the
 // compiler cannot see through: hoisted out of the march their ~60 pointers
@@ -218,33 +144,6 @@ __device__ __forceinline__ StepPtr<T> fresh(StepPtr<T> p) {
   asm("" : "+s"(p));
   return p;
 }
-template <class R>
-__device__ __forceinline__ cplx<R> phase_of(const GMES_CONST cplx<R>& p) {
-  return {p.re, p.im};
-}
-// x times the phase (real fields: x)
-template <class T>
-__device__ __forceinline__ T phased(const GMES_CONST cplx<typename real_of<T>::type>& p, T x) {
-  if constexpr (is_cplx<T>::value) return cmul(phase_of(p), x);
-  else return x;
-}
-
-// Dummy and Const cells and cells with a point source: a handful per sim.
-// f is the cell's old value, v its updated one.
-template <class T>
-__device__ __forceinline__ T step_rare(const StepRare* q, const double* waves, int64_t wave_n, int64_t row, T f, T v) {
-  using R = typename real_of<T>::type;
-  const int keep = gld(&q->keep), wave = gld(&q->wave);
-  if (keep == 1) v = f;
-  if (keep == 2) v = make_val<T>((R)gld(&q->re), (R)gld(&q->im));
-  if (wave >= 0) {
-    const double* w = waves + (wave * wave_n + row) * 2;
-    const T wv = make_val<T>((R)gld(w), (R)gld(w + 1));
-    v = gld(&q->kind) == GMES_SRC_SET ? wv : vsub(v, wv);
-  }
-  return v;
-}
-
 // The operands a thread loads for one plane, a plane ahead.
 template <class T, int PML>
 struct StepOps {
@@ -769,6 +668,7 @@ __global__ void __launch_bounds__(256) k_step_ids(StepIdArgs a) {
   uint32_t v = 0;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
+    if (h && a.out16) continue;
     uint16_t id[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
@@ -784,12 +684,24 @@ __global__ void __launch_bounds__(256) k_step_ids(StepIdArgs a) {
       at = (at + 1) & a.mask[h];
     }
   }
-  gst(a.out + (int64_t)r * a.pitch + k, v);
+  if (a.out16) gst(a.out16 + (int64_t)r * a.pitch + k, (uint16_t)v);
+  else gst(a.out + (int64_t)r * a.pitch + k, v);
 }
 
 void launch_step_ids(const StepIdArgs& a, hipStream_t st) {
   const int64_t n = (int64_t)a.n[0] * a.n[1] * a.n[2];
   hipLaunchKernelGGL(k_step_ids, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a);
+}
+
+__global__ void __launch_bounds__(256) k_list_places(PlaceArgs a) {
+  const int q = blockIdx.x * 256 + threadIdx.x;
+  if (q >= a.n) return;
+  const int x = a.cell[q], k = x % a.s2, r = x / a.s2, j = r % a.s1, i = r / a.s1;
+  a.out[i * a.pi + j * a.p + k * a.pk] = q;
+}
+
+void launch_list_places(const PlaceArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(k_list_places, dim3((unsigned)(a.n + 255) / 256), dim3(256), 0, st, a);
 }
 
 __global__ void k_clock_copy(Ctl* ctl) { ctl->clk[0] = ctl->clk[1] = ctl->clock; }
