@@ -802,18 +802,17 @@ hipError_t sync_exec(gmes_sim* s);
 // ---- one-sweep steps (step3d.hip)
 //
 // A real FP32 or FP64, or complex FP32, 3-D sim takes them when
-//   * it holds only Dummy, Const and Dielectric cells and, in real FP32, one
-//     kind of absorber with one profile set, whose two rows per axis agree (a
-//     single Shell).  (With 8-byte words the absorber kernels need more than
-//     128 registers: FP64 171 x 150 x 139 CPML 230 us per step, 188 us with
-//     two kernels.)
-//   * three whole (j, k) rows fit a block (nz <= 341), so that at most half of
-//     the E work is done twice,
+//   * it holds only Dummy, Const and Dielectric cells and one kind of absorber
+//     with one profile set, whose two rows per axis agree (a single Shell),
+//   * three whole (j, k) rows fit a block (nz <= 341; 256 with 8-byte words and
+//     an absorber along x or y), so that at most half of the E work is done
+//     twice,
 //   * its distinct triples of records fit a block's LDS,
 //   * every source is a single point operation per cell, on few cells, off
 //     the ghost planes, and no E probe sits on a ghost plane (it reads the
 //     plane before the copy),
-//   * a component's CPML state is under 4 GiB (32-bit byte offsets), and
+//   * a component's CPML state is under 4 GiB (32-bit byte offsets),
+//   * it has no auxiliary grid (its sources lie between E and H), and
 //   * the caller asked for no tile and did not turn ghost fusion off.
 // Other sims keep the two-kernel step.
 constexpr int kSweepMinRows = 3;
@@ -1030,49 +1029,117 @@ void sweep_entry(const gmes_sim* s, const std::array<uint16_t, 3>& rec, StepEnt<
   }
 }
 
-// Rows per block and planes per block.  A block's march costs its planes and
-// two more (the rim plane, the prologue); blocks run in rounds over the 256
-// CUs, a last incomplete round costing about half of one; a CU with few
-// waves still pays the latency of a plane (kSweepFloor).  256^3 CPML, rows
-// of 256, blocks of 3 rows: 64 planes (one full round) 285 us, 32 planes 303,
-// 16 planes 312; 181 x 203 x 225 UPML: 3 rows 190 us, 4 rows (one block per
-// CU) 204.
+// CPML with live state along x or y: blocks without it take a body without
+// those words, blocks with one of the two a body that loads its words a plane
+// ahead, in one launch; from 5 MB a component (us per step, one body for all
+// against this: 96^3 FP32 26.6, 34; 112^3 39, 36; 256^3 293, 255; FP64 80^3
+// 31, 35; 96^3 58, 50; 160^3 177, 153; 171 x 150 x 139 153, 145).  Few planes
+// per block: a plane takes its loads' latency, which only more blocks hide
+// (256^3, planes of blocks with and without x or y words: 6 and 9 255, 16 and
+// 29 259, 24 and 39 277; 128^3 6 and 9 49, 16 and 29 61).
+constexpr int64_t kSweepSplitBytes = 5 << 20;
+constexpr int kSweepOuterPlanes = 6, kSweepInnerPlanes = 9;
+
+// The launches of a step.  A block's march costs its planes and two more (the
+// rim plane, the prologue); blocks run in rounds over the 256 CUs, a last
+// incomplete round costing about half of one; a CU with few waves still pays
+// the latency of a plane (kSweepFloor).  256^3 CPML, rows of 256, blocks of 3
+// rows: 64 planes (one full round) 285 us, 32 planes 303, 16 planes 312; 181 x
+// 203 x 225 UPML: 3 rows 190 us, 4 rows (one block per CU) 204.
+//
+// Rows and planes per block of a launch over ni planes of nj rows; returns its
+// cost (0: no shape fits).
 template <class T>
-void sweep_shape_t(gmes_sim* s, int nent) {
-  const int nx = s->g.nx, ny = s->g.ny, nz = s->g.nz;
-  double best = 1e300;
-  for (int rows = 2; rows <= ny + 1; ++rows) {
-    const int threads = (rows * nz + 63) / 64 * 64;
-    if (threads > kStepMaxThreads) break;
-    if (rows < kSweepMinRows && kSweepMinRows * nz <= kStepMaxThreads && ny + 1 >= kSweepMinRows) continue;
-    const int64_t lds = (int64_t)step3_lds<T>(threads, nent, rows, nz, s->sweep_absorber);
+double sweep_shape(const gmes_sim* s, int nent, int absorber, int ni, int nj, gmes_sim::SweepPart& part, int& ch_out) {
+  const int nz = s->g.nz;
+  double best = 0;
+  part.absorber = absorber;
+  for (int rows = 2; rows <= nj + 1; ++rows) {
+    const int threads = (rows * nz + 63) / 64 * 64, most = step3_max_threads<T>(absorber);
+    if (threads > most) break;
+    if (rows < kSweepMinRows && kSweepMinRows * nz <= most && nj + 1 >= kSweepMinRows) continue;
+    const int64_t lds = (int64_t)step3_lds<T>(threads, nent, rows, nz, absorber);
     if (lds > kSweepLds) break;
-    const int waves = threads / 64, held = s->sweep_absorber ? 24 : sizeof(T) == 4 ? 32 : 20;
+    // waves a CU holds: registers (see StepWaves)
+    const bool full = absorber != kPmlNone && absorber != kPmlZ;
+    const int waves = threads / 64, held = sizeof(T) == 4 ? (absorber ? 24 : 32) : full ? 12 : absorber ? 16 : 20;
     const int per_cu = std::max<int>(1, (int)std::min<int64_t>(held / waves, kSweepLds / lds));
-    const int nj = (ny + rows - 2) / (rows - 1);
+    const int tiles = (nj + rows - 2) / (rows - 1);
     const double plane = std::max(per_cu * waves, kSweepFloor);
-    for (int nch = 1; nch <= nx; ++nch) {
-      const int ch = (nx + nch - 1) / nch;
-      const double x = (double)nj * ((nx + ch - 1) / ch) / (256.0 * per_cu);
+    for (int nch = 1; nch <= ni; ++nch) {
+      const int ch = (ni + nch - 1) / nch;
+      const double x = (double)tiles * ((ni + ch - 1) / ch) / (256.0 * per_cu);
       const double rounds = x <= 1 ? 1 : x + (std::ceil(x) > x ? 0.5 : 0);
       const double cost = rounds * (ch + 2.0) * plane;
-      if (cost < best * 0.999) {
+      if (best == 0 || cost < best * 0.999) {
         best = cost;
-        s->sweep_rows = rows;
-        s->sweep_threads = threads;
-        s->sweep_ch = ch;
+        part.rows = rows;
+        part.threads = threads;
+        ch_out = ch;
       }
     }
   }
+  return best;
 }
 
-void sweep_shape(gmes_sim* s) {
+// The longest run of thread coordinates along axis a (0 x, 1 y), n of them,
+// whose E, H and the E after the last have no live CPML state: lo, hi.
+void sweep_quiet(const gmes_sim* s, int a, int n, int& lo, int& hi) {
+  const int re = s->sweep_run_e[a], rh = s->sweep_run_h[a];
+  auto dead_e = [&](int q) { q = q == n ? 0 : q; return q >= (re & 0xFFFF) && q < (re >> 16); };
+  auto dead_h = [&](int q) { return q + 1 >= (rh & 0xFFFF) && q + 1 < (rh >> 16); };  // storage index
+  lo = hi = 0;
+  for (int q = 0; q < n;) {
+    if (!dead_e(q) || !dead_h(q)) { ++q; continue; }
+    int e = q;
+    while (e < n && dead_e(e) && dead_h(e)) ++e;
+    while (e > q && !dead_e(e)) --e;
+    if (e - q > hi - lo) { lo = q; hi = e; }
+    q = std::max(e, q + 1);
+  }
+}
+
+template <class T>
+void sweep_plan_t(gmes_sim* s, int nent) {
+  const int nx = s->g.nx, ny = s->g.ny;
+  gmes_sim::SweepPart& part = s->sweep_part;
+  part = gmes_sim::SweepPart{};
+  int ia = 0, ib = 0, ja = 0, jb = 0, ch = 0, kind = s->sweep_absorber;
+  if (kind == 1) {
+    sweep_quiet(s, 0, nx, ia, ib);
+    sweep_quiet(s, 1, ny, ja, jb);
+    if (ib - ia == nx && jb - ja == ny) kind = kPmlZ;
+    else if (s->ncell[0] * s->esize >= kSweepSplitBytes && ib > ia && jb > ja) kind = kPmlMixed;
+  }
+  if (sweep_shape<T>(s, nent, kind, nx, ny, part, ch) == 0) {
+    part.rows = 0;
+    return;
+  }
+  auto rect = [&](int i0, int i1, int j0, int j1, int most, int k) {
+    if (i0 >= i1 || j0 >= j1) return;
+    const int len = i1 - i0, n = (len + most - 1) / most;
+    const int r[6] = {i0, i1, j0, j1, (len + n - 1) / n, k};
+    std::copy(r, r + 6, part.rect[part.nrect++]);
+  };
+  if (kind != kPmlMixed) {
+    rect(0, nx, 0, ny, ch, kind);
+    return;
+  }
+  const int xs[4] = {0, ia, ib, nx}, ys[4] = {0, ja, jb, ny};
+  const int cho = kSweepOuterPlanes;
+  for (int x : {0, 2})
+    for (int y : {0, 2}) rect(xs[x], xs[x + 1], ys[y], ys[y + 1], cho, kPmlXYZ);
+  for (int x : {0, 2}) rect(xs[x], xs[x + 1], ja, jb, cho, kPmlXZ);
+  for (int y : {0, 2}) rect(ia, ib, ys[y], ys[y + 1], cho, kPmlYZ);
+  rect(ia, ib, ja, jb, kSweepInnerPlanes, kPmlZ);
+}
+
+void sweep_plan(gmes_sim* s) {
   const int nent = (int)(s->step_e.size() + s->step_h.size()) + 2 * kSweepMaxSrc;
-  s->sweep_rows = 0;
   switch (s->g.dtype) {
-    case GMES_F32: sweep_shape_t<float>(s, nent); break;
-    case GMES_F64: sweep_shape_t<double>(s, nent); break;
-    default: sweep_shape_t<cplx<float>>(s, nent); break;
+    case GMES_F32: sweep_plan_t<float>(s, nent); break;
+    case GMES_F64: sweep_plan_t<double>(s, nent); break;
+    default: sweep_plan_t<cplx<float>>(s, nent); break;
   }
 }
 
@@ -1487,8 +1554,8 @@ int sweep_sources(gmes_sim* s) {
 // the sim does not qualify.
 int sweep_build(gmes_sim* s) {
   sweep_release(s);
-  if (is_2z(s)) return sweep2_build(s);
-  if (!is3d(s) || s->g.dtype == GMES_C128) return GMES_OK;
+  if (is_2z(s)) return s->naux ? GMES_OK : sweep2_build(s);
+  if (!is3d(s) || s->g.dtype == GMES_C128 || s->naux) return GMES_OK;
   const int nz = s->g.nz;
   if (kSweepMinRows * nz > kStepMaxThreads || s->g.ny < 2) return GMES_OK;
   for (int c = 0; c < 6; ++c)  // 32-bit byte offsets, both state words included
@@ -1503,7 +1570,6 @@ int sweep_build(gmes_sim* s) {
   if ((cpml && upml) || ((cpml || upml) && s->nprof != 1)) return GMES_OK;
   // the kernels keep every component's absorber state
   if (cpml || upml) {
-    if (s->esize > 4) return GMES_OK;
     for (int c = 0; c < 6; ++c)
       if (!s->pml_state[c]) return GMES_OK;
   }
@@ -1533,8 +1599,8 @@ int sweep_build(gmes_sim* s) {
   if (!sweep_triples(s, true, most, s->step_e) || !sweep_triples(s, false, most, s->step_h) ||
       s->step_e.size() + s->step_h.size() > most)
     return GMES_OK;
-  sweep_shape(s);
-  if (!s->sweep_rows) return GMES_OK;
+  sweep_plan(s);
+  if (!s->sweep_part.rows) return GMES_OK;
   int rc = GMES_OK;
   for (int c = 0; c < 6 && !rc; ++c) rc = sweep_alloc(s, &s->f_alt[c], (size_t)s->dsize[c] * s->esize);
   for (int c = 0; c < 3 && !rc; ++c) {
@@ -1636,10 +1702,15 @@ Step3Args<T> step3_args(const gmes_sim* s) {
     m.run_e[a] = s->sweep_run_e[a];
     m.run_h[a] = s->sweep_run_h[a];
   }
-  m.rows = s->sweep_rows;
-  m.ch = s->sweep_ch;
-  m.nj = (s->g.ny + m.rows - 2) / (m.rows - 1);
-  m.nblk = m.nj * ((s->g.nx + m.ch - 1) / m.ch);
+  const gmes_sim::SweepPart& part = s->sweep_part;
+  m.rows = part.rows;
+  m.nrect = part.nrect;
+  for (int q = 0; q < part.nrect; ++q) {
+    const int* r = part.rect[q];
+    const int tiles = (r[3] - r[2] + m.rows - 2) / (m.rows - 1), nblk = tiles * ((r[1] - r[0] + r[4] - 1) / r[4]);
+    m.rect[q] = {r[0], r[1], r[2], r[3], r[4], tiles, nblk, (nblk + 7) / 8, m.slots, r[5]};
+    m.slots += (nblk + 7) / 8;
+  }
   m.waves = s->has_waves ? s->d_waves : nullptr;
   m.ctl = reinterpret_cast<Ctl*>(s->d_clock);
   m.par = s->par;
@@ -1664,7 +1735,7 @@ void enqueue_sweep(gmes_sim* s, hipStream_t st) {
   if (s->sweep_2d) {
     launch_step2d<T>(step2_args<T>(s), step2_tm(s), s->sweep_absorber, step2_ade(s), st);
   } else if constexpr (!std::is_same<T, cplx<double>>::value) {
-    launch_step3d<T>(step3_args<T>(s), s->sweep_absorber, s->sweep_threads, st);
+    launch_step3d<T>(step3_args<T>(s), s->sweep_part.absorber, s->sweep_part.threads, st);
   }
   time_end(s, st);
   sweep_swap(s);
@@ -2501,6 +2572,9 @@ int gmes_sim_attach_aux(gmes_sim* s, gmes_sim* aux, int32_t* slot) {
   if (aux->device != s->device) return set_error(GMES_EINVAL, "aux sim on another device");
   if (aux->naux) return set_error(GMES_EINVAL, "an auxiliary grid cannot have its own");
   if (aux->parent) return set_error(GMES_EINVAL, "auxiliary grid already attached");
+  HIP_TRY(hipSetDevice(s->device));
+  HIP_TRY(sync_exec(s));
+  sweep_release(s);  // a sim with an auxiliary grid takes two-kernel steps: no second buffers
   s->aux[s->naux] = aux;
   aux->parent = s;
   void* ptrs[6];

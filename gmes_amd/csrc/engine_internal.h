@@ -188,7 +188,14 @@ struct gmes_sim {
   bool sweep_ghosts = true;  // the next one-sweep step writes the ghost planes
   int sweep_absorber = 0;    // 0 none, 1 CPML, 2 UPML
   int sweep_exact = 0;       // Step3Args::exact
-  int sweep_threads = 0, sweep_rows = 0, sweep_ch = 0;
+  int sweep_ch = 0;          // 2-D: rows per block
+  // 3-D: its launch
+  struct SweepPart {
+    int absorber = 0, threads = 0, rows = 0;  // as launch_step3d's
+    int nrect = 0;
+    int rect[9][6] = {};                      // i0, i1, j0, j1, planes per block, absorber
+  };
+  SweepPart sweep_part;
   void* f_alt[6] = {};
   void* pml_alt[3] = {};
   int32_t sweep_run_e[3] = {}, sweep_run_h[3] = {};  // Step3Args::run_e, run_h

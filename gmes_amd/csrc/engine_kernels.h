@@ -125,6 +125,16 @@ struct alignas(16) StepEnt {
   uint32_t meta;  // kStepRareCell | 2 << t per UPML component
 };
 
+// Absorbers of a one-sweep step: none, CPML with state along x, y and z, UPML,
+// CPML with state along z only, a launch with blocks of several kinds, CPML
+// along x and z, along y and z.
+constexpr int kPmlNone = 0, kPmlXYZ = 1, kUpml = 2, kPmlZ = 3, kPmlMixed = 4, kPmlXZ = 5, kPmlYZ = 6;
+// cells [i0, i1) x [j0, j1) of a launch: ch planes per block, nj tiles along
+// j, nblk blocks; per: blocks of it per XCD, first: those of the rectangles before
+struct StepRect {
+  int i0, i1, j0, j1, ch, nj, nblk, per, first, kind;
+};
+
 template <class T>
 struct Step3Args {
   using R = typename real_of<T>::type;
@@ -150,8 +160,8 @@ struct Step3Args {
   cplx<R> pe[3][3];  // ghost phase of E component c along axis a
   cplx<R> ph[3][3];  // of H
   int rows;        // (j) rows per block, the last one a rim
-  int ch;          // i planes per block
-  int nj, nblk;    // tiles along j, blocks
+  int nrect, slots;  // rectangles, blocks per XCD
+  StepRect rect[9];
   const double* waves;
   Ctl* ctl;
   int par;
@@ -246,16 +256,20 @@ struct PlaceArgs {
   int32_t* out;  // at element (0, 0, 0)
 };
 void launch_list_places(const PlaceArgs& a, hipStream_t st);
-// threads of a block at most, the stride of its LDS exchange planes
+// threads of a block at most: with 8-byte words the kernels of a full
+// absorber need 150 to 172 registers, three waves a SIMD
 constexpr int kStepMaxThreads = 1024;
-template <class T> constexpr int kStepThreads = kStepMaxThreads;
+template <class T>
+constexpr int step3_max_threads(int absorber) {
+  return sizeof(T) == 8 && absorber != kPmlNone && absorber != kPmlZ ? 768 : kStepMaxThreads;
+}
 // bytes of LDS of a block: exchange buffers, entries, absorber rows
 template <class T>
 inline size_t step3_lds(int nthreads, int nent, int rows, int nz, int absorber) {
   using R = typename real_of<T>::type;
-  const size_t stride = absorber == 2 ? 8 : absorber == 1 ? 4 : 0;
+  const size_t stride = absorber == kUpml ? 8 : absorber ? 4 : 0;
   const size_t exchange = sizeof(T) == 4 ? (2 * (2 * (size_t)nz + 9 * (size_t)nthreads) + 3) / 4 * 4 * sizeof(T)
-                                         : (size_t)12 * kStepThreads<T> * sizeof(T);
+                                         : (size_t)12 * nthreads * sizeof(T);
   return exchange + (size_t)nent * sizeof(StepEnt<R>) +
          2 * (size_t)(rows + nz) * stride * sizeof(R);
 }
@@ -425,7 +439,6 @@ template <class T>
 void launch_main2z(bool electric, const MainArgs<T>& m, int ext[3], hipStream_t st);
 template <class T>
 void launch_main3d(bool electric, const MainArgs<T>& m, int bx, int by, int ichunk, hipStream_t st);
-// absorber: 0 none, 1 CPML, 2 UPML
 template <class T>
 void launch_step3d(const Step3Args<T>& m, int absorber, int nthreads, hipStream_t st);
 template <class T>

@@ -22,15 +22,21 @@
 // Rows are whole so that every load starts on a line and the periodic wrap
 // along k stays inside the block.
 //
-// Measured per step, two-kernel step first: FP32 256^3 CPML 344 -> 293 us,
-// 181 x 203 x 225 UPML 210 -> 173, 96^3 CPML 39 -> 26, 64^3 UPML 24 -> 11;
-// FP64 171 x 150 x 139 without an absorber 89 (3.8 TB/s).  What bounds it: without an
-// absorber the bytes (256^3: 188 us, 4.3 TB/s); with one the latency of the
-// absorber words that are loaded in the plane that uses them.  The same
-// kernel takes 185 us with the absorber's arithmetic but none of its memory,
-// 240 with its stores, 243 with the z words a plane ahead, and the rest
-// with the x and y words; holding those a plane ahead too takes 98 registers,
-// one block per CU, and 386 us.
+// Blocks differ in the absorber words they hold: a body with none, with CPML
+// words along z (every row has those at both ends), along x and z, along y and
+// z, with all, with UPML.  The words of a body are loaded a plane ahead,
+// except in the body with all of them (blocks at the edges; every block of a
+// small sim), which loads those along x and y in the plane that uses them:
+// ahead they cost 98 registers and one block per CU in FP32.
+//
+// Measured per step, two-kernel step first: FP32 256^3 CPML 344 -> 255 us (one
+// body for all blocks 293), 181 x 203 x 225 UPML 210 -> 171, 96^3 CPML 39 ->
+// 26, 64^3 UPML 24 -> 11; FP64 CPML 171 x 150 x 139 189 -> 145, 64^3 31 -> 19;
+// complex FP32 with z layers 192 x 192 x 128 190 -> 136, 112^3 72 -> 46.  What
+// bounds it: without an absorber the bytes (256^3 FP32 188 us, 4.3 TB/s); with
+// one the latency of a plane, 1 to 2 us, of which a CU has few in flight (24
+// waves in FP32, 12 to 16 with 8-byte words, by their registers: held to 128
+// registers the 8-byte bodies with all words spill, 171 x 150 x 139 320 us).
 //
 // Ghost planes: operands wrap by index (with the Bloch phase), and the
 // owners of source-plane cells write the ghost images of both types with
@@ -97,11 +103,11 @@ template <int PML> struct RowStride { static constexpr int v = PML == 2 ? 8 : 4;
 // word that is +0, so the CPML update below is the Dielectric one.
 template <class R, int PML>
 __device__ __forceinline__ void stage_row(R* dst, const R* shared, const R* own, int xs, int xo, bool live) {
-  if constexpr (PML == 1) {
+  if constexpr (PML != 2) {
     dst[0] = live ? gld(shared + xs * 3) : R(0);
     dst[1] = live ? gld(shared + xs * 3 + 1) : R(0);
     dst[2] = live ? gld(shared + xs * 3 + 2) : R(1);
-  } else if constexpr (PML == 2) {
+  } else {
 #pragma unroll
     for (int q = 0; q < 4; ++q) dst[q] = gld(shared + xs * 6 + q);
     dst[4] = gld(own + xo * 6 + 4);
@@ -110,18 +116,26 @@ __device__ __forceinline__ void stage_row(R* dst, const R* shared, const R* own,
 }
 
 template <class R, int PML>
-__device__ __forceinline__ Rows<R, PML> lds_row(const R* p) {
-  Rows<R, PML> r;
+__device__ __forceinline__ Rows<R, PML == 2 ? 2 : 1> lds_row(const R* p) {
+  Rows<R, PML == 2 ? 2 : 1> r;
 #pragma unroll
   for (int q = 0; q < (PML == 2 ? 6 : 3); ++q) r.v[q] = p[q];
   return r;
 }
 
+// the row of a CPML coordinate without live state
+template <class R, int PML>
+__device__ __forceinline__ Rows<R, PML == 2 ? 2 : 1> dead_row() {
+  Rows<R, PML == 2 ? 2 : 1> r{};
+  r.v[2] = R(1);
+  return r;
+}
+
 // a row along x, the same for the whole block
 template <class R, int PML>
-__device__ __forceinline__ Rows<R, PML> x_row(const R* shared, const R* own, int xs, int xo, bool live) {
-  Rows<R, PML> r;
-  if constexpr (PML == 1) {
+__device__ __forceinline__ Rows<R, PML == 2 ? 2 : 1> x_row(const R* shared, const R* own, int xs, int xo, bool live) {
+  Rows<R, PML == 2 ? 2 : 1> r;
+  if constexpr (PML != 2) {
     r.v[0] = live ? cld(shared + xs * 3) : R(0);
     r.v[1] = live ? cld(shared + xs * 3 + 1) : R(0);
     r.v[2] = live ? cld(shared + xs * 3 + 2) : R(1);
@@ -154,9 +168,22 @@ struct StepOps {
   // two that live along z, which every row has at both ends; those along x
   // and y are read where they are used, by the few planes and rows that
   // have them (all twelve ahead took 98 registers and one block per CU).
-  T s[PML == 1 ? 2 : 3], g[PML == 1 ? 2 : 3];
+  T s[PML == 2 ? 3 : PML >= kPmlXZ ? 4 : 2], g[PML == 2 ? 3 : PML >= kPmlXZ ? 4 : 2];
   uint32_t id;
 };
+
+// Rectangle rc and its block rb of a launch's block.  Consecutive blocks go to
+// consecutive XCDs: each XCD gets a contiguous run of a rectangle's tiles, so
+// that the rim rows two blocks share meet in one L2 (256^3 without an
+// absorber: 189 to 180 us).
+template <class T>
+__device__ __forceinline__ bool step3d_block(StepPtr<T> m, unsigned blk, int& rc, unsigned& rb) {
+  const int slot = (int)(blk >> 3);
+  rc = m->nrect - 1;
+  while (rc > 0 && slot < m->rect[rc].first) --rc;
+  rb = (blk & 7u) * (unsigned)m->rect[rc].per + (unsigned)(slot - m->rect[rc].first);
+  return rb < (unsigned)m->rect[rc].nblk && slot - m->rect[rc].first < m->rect[rc].per;
+}
 
 // X: see by_size (FP64 only)
 template <class T, int PML, bool X>
@@ -164,7 +191,6 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
   using R = typename real_of<T>::type;
   StepPtr<T> m = fresh<T>(mp);
   constexpr unsigned S = sizeof(T);
-  constexpr int NT = kStepThreads<T>;  // LDS stride of the exchange planes
   const int t = threadIdx.x;
   const int nx = m->n[0], ny = m->n[1], nz = m->n[2];
   // 4-byte words: operands of a plane arrive in LDS by themselves (lds_load);
@@ -172,8 +198,10 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
   // first), hy and old Ex, Ey, Ez, then the exchange of new E.  8-byte words
   // arrive in registers and H is put there.
   constexpr bool DMA = sizeof(T) == 4;
+  // CPML; with live words along x, along y
+  constexpr bool CP = PML != 0 && PML != 2, LX = PML == 1 || PML == kPmlXZ, LY = PML == 1 || PML == kPmlYZ;
+  const int nt = (int)blockDim.x, NT = nt;
   T* const xb = reinterpret_cast<T*>(lds);  // DMA: [2][3 NT] new E after the operands; else [2][hx, hy, hz, ex, ey, ez][NT]
-  const int nt = (int)blockDim.x;
   const int slot = DMA ? 2 * nz + 6 * nt : 6 * NT;   // words of a parity's operands
   T* const eb = DMA ? xb + 2 * slot : xb + 3 * NT;   // new E: + parity * eslot + component * est
   const int eslot = DMA ? 3 * nt : 6 * NT, est = DMA ? nt : NT;
@@ -184,20 +212,18 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
     const i4_t* src = static_cast<const i4_t*>(m->tab);
     for (int e = t; e < (m->net + m->nht) * kq; e += (int)blockDim.x) dst[e] = gld(src + e);
   }
-  // consecutive blocks go to consecutive XCDs: give each XCD a contiguous
-  // run of tiles, so that the rim rows two blocks share meet in one L2
-  // (256^3 without an absorber: 189 to 180 us)
-  const unsigned per = ((unsigned)m->nblk + 7u) / 8u;
-  const unsigned b = (blk & 7u) * per + (blk >> 3);
-  if ((blk >> 3) >= per || b >= (unsigned)m->nblk) return;
-  const int c = (int)(b / (unsigned)m->nj), tile = (int)(b - (unsigned)c * (unsigned)m->nj);
-  const int i0 = c * m->ch, i1 = min(i0 + m->ch, nx);
-  const int jw = m->rows - 1, j0 = tile * jw;
+  int rc;
+  unsigned rb;
+  if (!step3d_block<T>(m, blk, rc, rb)) return;
+  const unsigned rnj = (unsigned)m->rect[rc].nj;
+  const int c = (int)(rb / rnj), tile = (int)(rb - (unsigned)c * rnj);
+  const int i0 = m->rect[rc].i0 + c * m->rect[rc].ch, i1 = min(i0 + m->rect[rc].ch, m->rect[rc].i1);
+  const int j0 = m->rect[rc].j0 + tile * (m->rows - 1), jw = min(m->rows - 1, m->rect[rc].j1 - j0);  // own rows
   // lanes past the last row repeat a row of the block and store nothing
   const int tr = (int)((unsigned)t / (unsigned)nz), k = t - tr * nz;
-  const int tj = min(tr, min(jw, ny - j0));
+  const int tj = min(tr, jw);
   const int j = j0 + tj == ny ? 0 : j0 + tj;
-  const bool own = tr < jw && j0 + tr < ny;
+  const bool own = tr < jw;
   const bool edge = tj == 0;
   const unsigned W0 = (unsigned)m->W0 * S, W2 = (unsigned)m->W2 * S;  // bytes of a row
   const unsigned PX = (unsigned)(ny + 1) * W0, PY = (unsigned)ny * W0, PZ = (unsigned)(ny + 1) * W2;  // of a plane
@@ -208,7 +234,7 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
   const int tm = k ? t - 1 : t + nz - 1, tp = k == nz - 1 ? t + 1 - nz : t + 1;
 
   // absorber rows of the block: E along y, H along y, E along z, H along z
-  using RowT = Rows<R, PML>;
+  using RowT = Rows<R, PML == 2 ? 2 : 1>;
   constexpr int rs = RowStride<PML>::v;
   bool ly = false, lz = false, lyh = false, lzh = false;  // live state along y, z (CPML); outside the box (UPML)
   R* const rows_y = reinterpret_cast<R*>(et + m->net + m->nht);
@@ -222,8 +248,9 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
     lz = live(m->run_e[2], k);
     lyh = live(m->run_h[1], j + 1);
     lzh = live(m->run_h[2], k + 1);
+    if (CP && !LY) ly = lyh = false;
     wave_live = __any(ly || lz || lyh || lzh);
-    if (k == 0 && tr == tj) {
+    if ((!CP || LY) && k == 0 && tr == tj) {
       stage_row<R, PML>(rows_y + tj * rs, m->re[1], m->oe[1], j, j, ly);
       stage_row<R, PML>(rows_yh + tj * rs, m->rh[1], m->oh[1], j + 1, j, lyh);
     }
@@ -237,8 +264,8 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
   auto xlive_h = [&](int x) { return x < (run_h & 0xFFFF) || x >= (run_h >> 16); };
   // live state along x: E at plane q; H at x = q (Hy, Hz of plane q - 1;
   // UPML: any of its three)
-  auto x_of_e = [&](int q) { return PML != 0 && xlive_e(q == nx ? 0 : q); };
-  auto x_of_h = [&](int q) { return PML != 0 && (xlive_h(q) || (PML == 2 && xlive_h(q - 1))); };
+  auto x_of_e = [&](int q) { return (LX || PML == 2) && xlive_e(q == nx ? 0 : q); };
+  auto x_of_h = [&](int q) { return (LX || PML == 2) && (xlive_h(q) || (PML == 2 && xlive_h(q - 1))); };
   const bool out_e = ly || lz, out_h = ly || lz || lyh || lzh;  // UPML: outside the box whatever x
 
   const unsigned wave0 = (unsigned)__builtin_amdgcn_readfirstlane(t) * 4u;  // LDS bytes before the wave's lanes
@@ -278,11 +305,11 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
     if constexpr (PML != 0) {
       const bool lx = x_of_e(q), lxh = x_of_h(q);
 #pragma unroll
-      for (int c = 0; c < (PML == 1 ? 2 : 3); ++c) l.s[c] = l.g[c] = T{};
+      for (int c = 0; c < (int)(sizeof(l.s) / sizeof(T)); ++c) l.s[c] = l.g[c] = T{};
       if (wave_live || lx || lxh) {
         const StepPtr<T> m = fresh<T>(mp);
         const unsigned px = (unsigned)(q - 1) * PX + W0 + S, py = (unsigned)q * PY + S, pz = (unsigned)q * PZ + W2;
-        if constexpr (PML == 1) {
+        if constexpr (CP) {
           if (lz) {
             l.s[0] = bld<T>(m->si[0], b0, ox + m->ds[0]);
             l.s[1] = bld<T>(m->si[1], b0, oy);
@@ -290,6 +317,25 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
           if (q > i0 && lzh && own) {
             l.g[0] = bld<T>(m->sh[0], b0, px + m->ds[3]);
             l.g[1] = bld<T>(m->sh[1], b0, py);
+          }
+          if constexpr (PML == kPmlXZ) {
+            if (lx) {
+              l.s[2] = bld<T>(m->si[1], b0, oy + m->ds[1]);
+              l.s[3] = bld<T>(m->si[2], b2, oz);
+            }
+            if (lxh && q > i0 && own) {
+              l.g[2] = bld<T>(m->sh[1], b0, py + m->ds[4]);
+              l.g[3] = bld<T>(m->sh[2], b2, pz);
+            }
+          } else if constexpr (PML == kPmlYZ) {
+            if (ly) {
+              l.s[2] = bld<T>(m->si[0], b0, ox);
+              l.s[3] = bld<T>(m->si[2], b2, oz + m->ds[2]);
+            }
+            if (lyh && q > i0 && own) {
+              l.g[2] = bld<T>(m->sh[0], b0, px);
+              l.g[3] = bld<T>(m->sh[2], b2, pz + m->ds[5]);
+            }
           }
         } else {
           if (out_e || lx) {
@@ -325,7 +371,7 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
   // - x side of this plane's E); new H of the plane before that
   T ex{}, ey{}, ez{}, hx{}, hy = bld<T>(m->hi[1], b0, ip * PY + S), hz = bld<T>(m->hi[2], b2, ip * PZ + W2);
   T nhx{}, nhy{}, nhz{};
-  T n[3][PML == 1 ? 2 : 1] = {}, r[3][PML == 1 ? 2 : 1] = {};  // their new absorber words
+  T n[3][CP ? 2 : 1] = {}, r[3][CP ? 2 : 1] = {};  // their new absorber words
   uint32_t hid = 0, meta_e = 0, meta_h = 0;  // UPML: which components those words belong to
   const double* const waves = m->waves;
   const StepRare* const rare = m->rare;
@@ -341,7 +387,7 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
     if constexpr (PML != 0) {
       const bool lx = x_of_e(p);
       if (wave_live || lx) {
-        if constexpr (PML == 1) {
+        if constexpr (CP) {
           if (ly) {
             bst<T>(m->so[0], b0, ox, n[0][0]);
             bst<T>(m->so[2], b2, oz + m->ds[2], n[2][1]);
@@ -371,7 +417,7 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
     if constexpr (PML != 0) {
       const bool lxh = x_of_h(p + 1);
       if (wave_live || lxh) {
-        if constexpr (PML == 1) {
+        if constexpr (CP) {
           if (lyh) {
             bst<T>(m->sh[0], b0, ox, r[0][0]);
             bst<T>(m->sh[2], b2, oz + m->ds[5], r[2][1]);
@@ -423,6 +469,17 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
       }
     }
     StepOps<T, PML> l = ahead;
+    if constexpr (PML == kPmlXZ) {
+      s11 = l.s[2];
+      s20 = l.s[3];
+      g11 = l.g[2];
+      g20 = l.g[3];
+    } else if constexpr (PML == kPmlYZ) {
+      s00 = l.s[2];
+      s21 = l.s[3];
+      g00 = l.g[2];
+      g21 = l.g[3];
+    }
     const T* const ob = xb + (q & 1) * slot;
     T* const we = eb + (q & 1) * eslot;
     const T* const re = eb + (1 - (q & 1)) * eslot;
@@ -499,14 +556,16 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
       plain_e();
       meta_e = 0;
     } else {
-      const RowT rx = x_row<R, PML>(m->re[0], m->oe[0], qe, qe, lx), ry = lds_row<R, PML>(rows_y + tj * rs),
+      const RowT rx = CP && !LX ? dead_row<R, PML>() : x_row<R, PML>(m->re[0], m->oe[0], qe, qe, lx),
+                  ry = CP && !LY ? dead_row<R, PML>() : lds_row<R, PML>(rows_y + tj * rs),
                  rz = lds_row<R, PML>(rows_z + k * rs);
-      if constexpr (PML == 1) {
+      if constexpr (CP) {
         nex = cpml_value<true, X>(en.c[0], l.e0, vsub(l.hz, hzj), vsub(l.hy, hyk), d1, v1, d2, v2, ry, rz, s00, l.s[0],
                                   n[0][0], n[0][1]);
         ney = cpml_value<true, X>(en.c[1], l.e1, vsub(l.hx, hxk), vsub(l.hz, hzp), d2, v2, d0, v0, rz, rx, l.s[1], s11,
                                   n[1][0], n[1][1]);
-        nez = cpml_value<true, X>(en.c[2], l.e2, vsub(l.hy, hyp), vsub(l.hx, hxj), d0, v0, d1, v1, rx, ry, s20, s21,
+        if constexpr (!LX && !LY) nez = plain_value<true, X>(en.c[2], l.e2, vsub(l.hy, hyp), vsub(l.hx, hxj), d0, v0, d1, v1);
+        else nez = cpml_value<true, X>(en.c[2], l.e2, vsub(l.hy, hyp), vsub(l.hx, hxj), d0, v0, d1, v1, rx, ry, s20, s21,
                                   n[2][0], n[2][1]);
       } else {
         plain_e();
@@ -610,14 +669,16 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
         plain_h();
         meta_h = 0;
       } else {
-        const RowT rx = x_row<R, PML>(m->rh[0], m->oh[0], q, q - 1, lxh), ry = lds_row<R, PML>(rows_yh + tj * rs),
+        const RowT rx = CP && !LX ? dead_row<R, PML>() : x_row<R, PML>(m->rh[0], m->oh[0], q, q - 1, lxh),
+                    ry = CP && !LY ? dead_row<R, PML>() : lds_row<R, PML>(rows_yh + tj * rs),
                    rz = lds_row<R, PML>(rows_zh + k * rs);
-        if constexpr (PML == 1) {
+        if constexpr (CP) {
           nhx = cpml_value<false, X>(eh.c[0], hx, vsub(ezj, ez), vsub(eyk, ey), d1, v1, d2, v2, ry, rz, g00, l.g[0],
                                      r[0][0], r[0][1]);
           nhy = cpml_value<false, X>(eh.c[1], hy, vsub(exk, ex), vsub(ezi, ez), d2, v2, d0, v0, rz, rx, l.g[1], g11,
                                      r[1][0], r[1][1]);
-          nhz = cpml_value<false, X>(eh.c[2], hz, vsub(eyi, ey), vsub(exj, ex), d0, v0, d1, v1, rx, ry, g20, g21,
+          if constexpr (!LX && !LY) nhz = plain_value<false, X>(eh.c[2], hz, vsub(eyi, ey), vsub(exj, ex), d0, v0, d1, v1);
+          else nhz = cpml_value<false, X>(eh.c[2], hz, vsub(eyi, ey), vsub(exj, ex), d0, v0, d1, v1, rx, ry, g20, g21,
                                      r[2][0], r[2][1]);
         } else {
           plain_h();
@@ -651,13 +712,25 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
   if (own) store_h(i1 - 1);
 }
 
-template <class T, int PML> struct StepWaves { static constexpr int v = 4; };
+template <class T, int PML> struct StepWaves { static constexpr int v = PML == 0 || PML == kPmlZ ? 4 : 3; };
 template <int PML> struct StepWaves<float, PML> { static constexpr int v = PML ? 6 : 8; };
 
 template <class T, int PML, bool X>
-__global__ void __launch_bounds__(kStepThreads<T>) __attribute__((amdgpu_waves_per_eu(StepWaves<T, PML>::v))) k_step3d(Step3Args<T>) {
+__global__ void __launch_bounds__(step3_max_threads<T>(PML)) __attribute__((amdgpu_waves_per_eu(StepWaves<T, PML>::v))) k_step3d(Step3Args<T>) {
   extern __shared__ __attribute__((aligned(16))) char step_lds[];
-  step3d_tile<T, PML, X>((StepPtr<T>)__builtin_amdgcn_kernarg_segment_ptr(), blockIdx.x, step_lds);
+  const StepPtr<T> m = (StepPtr<T>)__builtin_amdgcn_kernarg_segment_ptr();
+  if constexpr (PML == kPmlMixed) {
+    int rc;
+    unsigned rb;
+    (void)step3d_block<T>(m, blockIdx.x, rc, rb);
+    const int kind = m->rect[rc].kind;
+    if (kind == kPmlZ) step3d_tile<T, kPmlZ, X>(m, blockIdx.x, step_lds);
+    else if (kind == kPmlXZ) step3d_tile<T, kPmlXZ, X>(m, blockIdx.x, step_lds);
+    else if (kind == kPmlYZ) step3d_tile<T, kPmlYZ, X>(m, blockIdx.x, step_lds);
+    else step3d_tile<T, 1, X>(m, blockIdx.x, step_lds);
+  } else {
+    step3d_tile<T, PML, X>(m, blockIdx.x, step_lds);
+  }
 }
 
 __global__ void __launch_bounds__(256) k_step_ids(StepIdArgs a) {
@@ -710,12 +783,14 @@ void launch_clock_copy(Ctl* ctl, hipStream_t st) { hipLaunchKernelGGL(k_clock_co
 
 template <class T>
 void launch_step3d(const Step3Args<T>& m, int absorber, int nthreads, hipStream_t st) {
-  const dim3 grid(((unsigned)m.nblk + 7u) / 8u * 8u), block(nthreads);
+  const dim3 grid(8u * (unsigned)m.slots), block(nthreads);
   const unsigned lds = (unsigned)step3_lds<T>(nthreads, m.net + m.nht, m.rows, m.n[2], absorber);
 #define GMES_STEP(X)                                                                              \
   {                                                                                               \
     if (absorber == 0) hipLaunchKernelGGL((k_step3d<T, 0, X>), grid, block, lds, st, m);          \
     else if (absorber == 1) hipLaunchKernelGGL((k_step3d<T, 1, X>), grid, block, lds, st, m);     \
+    else if (absorber == kPmlZ) hipLaunchKernelGGL((k_step3d<T, kPmlZ, X>), grid, block, lds, st, m);     \
+    else if (absorber == kPmlMixed) hipLaunchKernelGGL((k_step3d<T, kPmlMixed, X>), grid, block, lds, st, m);     \
     else hipLaunchKernelGGL((k_step3d<T, 2, X>), grid, block, lds, st, m);                        \
   }
   if constexpr (std::is_same<T, double>::value) {

@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
 FP64_TOL = 1e-12
 
 
-def box(lib, n, precision="fp32", bound=None, bloch=None, comps=(g.Ex,), over_shell=False, res=1, dft=False):
+def box(lib, n, precision="fp32", bound=None, bloch=None, comps=(g.Ex,), over_shell=False, res=1, axes="xyz"):
     """A box of n cells with two dielectric objects, an absorber of 3 cells,
     waves everywhere and a source on each of comps."""
     space = g.Cartesian(size=tuple(v / res for v in n), resolution=res)
@@ -28,7 +28,10 @@ def box(lib, n, precision="fp32", bound=None, bloch=None, comps=(g.Ex,), over_sh
             g.Block(g.Dielectric(5.0, 1.5), center=(s, -s, s), size=(2.2 * s, 3.1 * s, 4.3 * s)),
             g.Block(g.Const(0.25), center=(-s, s, 0), size=(1.1 * s, 1.1 * s, 1.1 * s))]
     if bound is not None:
-        geom.append(g.Shell(bound(), thickness=3 * s))
+        # layers on the named axes: elsewhere the shell lies outside the box
+        size = [v * s if a in axes else (v + 8) * s for a, v in zip("xyz", n)]
+        faces = {"%s_%s" % (side, a): a in axes for side in ("plus", "minus") for a in "xyz"}
+        geom.append(g.Shell(bound(), size=size, thickness=3 * s, **faces))
     if over_shell:  # a medium on top of the absorber: its cells are not CPML
         geom.append(g.Block(g.Dielectric(2.0), center=(-n[0] * s / 2, 0, 0), size=(4 * s, 2 * s, 2 * s)))
     src = [g.PointSource(g.Continuous(freq=0.05 * res, width=5 * s), center=(q * s, 0, 0), component=c)
@@ -72,13 +75,30 @@ def test_fp32(engine_lib, n, bound):
     run_pair(engine_lib, n=n, bound=bound if min(n) >= 8 else None)
 
 
-@pytest.mark.parametrize("n", SIZES, ids=lambda n: "x".join(map(str, n)))
-@pytest.mark.parametrize("kw", [dict(precision="fp64"), dict(bloch=(0.3, -0.2, 0.1)),
-                                dict(precision="fp64", bound=g.Cpml)], ids=["fp64", "c64", "fp64_cpml"])
-def test_eight_byte_words(engine_lib, n, kw):
-    if "bound" in kw and min(n) < 8:
-        kw = dict(kw, bound=None)
-    run_pair(engine_lib, n=n, **kw)
+@pytest.mark.parametrize("n", SIZES + [(10, 11, 256), (9, 9, 257)], ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("kw", [dict(precision="fp64"), dict(bloch=(0.3, -0.2, 0.1))], ids=["fp64", "c64"])
+@pytest.mark.parametrize("bound", [None, g.Cpml, g.Upml], ids=["none", "cpml", "upml"])
+def test_eight_byte_words(engine_lib, n, kw, bound):
+    run_pair(engine_lib, n=n, bound=bound if min(n) >= 8 else None, **kw)
+
+
+AXES = ["x", "y", "z", "xy", "xz", "yz"]
+
+
+@pytest.mark.parametrize("axes", AXES)
+@pytest.mark.parametrize("kw", [dict(), dict(precision="fp64", res=3), dict(bloch=(0.3, -0.2, 0.1))],
+                         ids=["fp32", "fp64", "c64"])
+def test_layers_on_some_axes(engine_lib, axes, kw):
+    """No live absorber words along the other axes."""
+    run_pair(engine_lib, n=(13, 12, 15), bound=g.Cpml, axes=axes, **kw)
+
+
+# from 5 MB a component the launch has blocks of several kinds
+@pytest.mark.parametrize("n,kw", [((110, 113, 107), dict()), ((80, 91, 93), dict(precision="fp64")),
+                                  ((91, 80, 93), dict(bloch=(0.3, -0.2, 0.1)))], ids=["fp32", "fp64", "c64"])
+@pytest.mark.parametrize("axes", ["xyz"] + AXES)
+def test_blocks_of_several_kinds(engine_lib, n, kw, axes):
+    run_pair(engine_lib, n=n, steps=(1, 4), bound=g.Cpml, axes=axes, **kw)
 
 
 @pytest.mark.parametrize("res", [1, 3], ids=["exact_division", "division"])
