@@ -12,9 +12,10 @@ import tempfile
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "lib", "libgmes_engine.so")
-# (file, extra flags): kernels.hip and step2d.hip are compiled once per storage type
+# (file, extra flags): the kernel files but step3d.hip are compiled once per storage type
 SOURCES = [("engine.hip", []), ("step3d.hip", [])] + [
-    (src, ["-DGMES_TYPE=%d" % t]) for src in ("kernels.hip", "step2d.hip") for t in range(4)]
+    (src, ["-DGMES_TYPE=%d" % t])
+    for src, n in (("kernels.hip", 4), ("step1d.hip", 4), ("step2d.hip", 4), ("stepfix.hip", 3)) for t in range(n)]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("GMES_OFFLOAD_ARCH", "gfx950")
 

@@ -786,33 +786,27 @@ void enqueue_dft(gmes_sim* s, hipStream_t st) {
 void enqueue_step(gmes_sim* s, hipStream_t st);
 
 // One whole step of each auxiliary (TFSF) grid of s, between the E and H
-// half steps of s.
-void enqueue_aux_steps(gmes_sim* s, hipStream_t st) {
-  for (int i = 0; i < s->naux; ++i) {
-    if (!s->aux[i]) continue;
-    time_begin(s, 5, st);
-    enqueue_step(s->aux[i], st);
-    time_end(s, st);
-  }
-}
+// half steps of s; sweep: the step of s is a one-sweep step.
+void enqueue_aux_steps(gmes_sim* s, bool sweep, hipStream_t st);
 
 bool on_ghost_copy_plane(const gmes_sim* s, int c, int64_t x, bool source, bool ghost);
+int sweep_sources(gmes_sim* s);
 hipError_t sync_exec(gmes_sim* s);
 
 // ---- one-sweep steps (step3d.hip)
 //
 // A real FP32 or FP64, or complex FP32, 3-D sim takes them when
-//   * it holds only Dummy, Const and Dielectric cells and one kind of absorber
-//     with one profile set, whose two rows per axis agree (a single Shell),
+//   * it holds no DM2 cells, and one kind of absorber with one profile set,
+//     whose two rows per axis agree (a single Shell),
 //   * three whole (j, k) rows fit a block (nz <= 341; 256 with 8-byte words and
 //     an absorber along x or y), so that at most half of the E work is done
 //     twice,
 //   * its distinct triples of records fit a block's LDS,
-//   * every source is a single point operation per cell, on few cells, off
-//     the ghost planes, and no E probe sits on a ghost plane (it reads the
-//     plane before the copy),
-//   * a component's CPML state is under 4 GiB (32-bit byte offsets),
-//   * it has no auxiliary grid (its sources lie between E and H), and
+//   * its sources are off the ghost planes, and no E probe sits on a ghost
+//     plane (it reads the plane before the copy),
+//   * with dispersive cells, an auxiliary grid or sources on more than
+//     kSweepMaxSrc cells: what stepfix.hip and sweep_fix_build ask,
+//   * a component's CPML state is under 4 GiB (32-bit byte offsets), and
 //   * the caller asked for no tile and did not turn ghost fusion off.
 // Other sims keep the two-kernel step.
 constexpr int kSweepMinRows = 3;
@@ -1023,7 +1017,8 @@ void sweep_entry(const gmes_sim* s, const std::array<uint16_t, 3>& rec, StepEnt<
     const bool upml = r.cls == GMES_CLS_UPML;
     rare[t] = StepRare{r.cls == GMES_CLS_DUMMY ? 1 : r.cls == GMES_CLS_CONST ? 2 : 0, -1, GMES_SRC_SET, 0,
                        r.value[0], r.value[1]};
-    if (rare[t].keep) e.meta |= kStepRareCell;
+    if (r.cls >= GMES_CLS_DRUDE) e.c[t] = 0;  // keeps its value: see stepfix.hip
+    else if (rare[t].keep) e.meta |= kStepRareCell;
     else e.c[t] = upml ? (s->fp64 ? (R)r.eps_mu : (R)(1.0 / r.eps_mu)) : (R)(s->g.dt / r.eps_mu);
     if (upml) e.meta |= 2u << t;
   }
@@ -1159,7 +1154,10 @@ void sweep_release(gmes_sim* s) {
       p = nullptr;
     }
   }
-  s->sweep_2d = false;
+  if (s->d_fix_items) (void)dev_release(s->d_fix_items);
+  s->d_fix_items = nullptr;
+  s->sweep_fix = false;
+  s->sweep_1d = s->sweep_2d = false;
   s->bytes -= s->sweep_bytes;
   s->sweep_bytes = 0;
   s->sweep_ok = false;
@@ -1200,6 +1198,162 @@ int sweep_upload_tab(gmes_sim* s, const std::vector<std::array<int, 3>>& se, con
   s->step_net = net;
   s->step_nht = nht;
   return GMES_OK;
+}
+
+// ---- one-sweep steps of TEM lines (step1d.hip)
+//
+// Taken when every absorber cell is of one kind and one profile set, in both
+// components or none, CPML has no live state along the collapsed axes, no cell
+// is of the DM2 class, and for sources and probes what the 2-D modes ask.
+// Direction e of the E component of a line of components e and e + 1 along
+// axis e + 2; -1: not such a line.
+int line_dir(const gmes_sim* s) {
+  const int64_t n[3] = {s->g.nx, s->g.ny, s->g.nz};
+  for (int e = 0; e < 3; ++e) {
+    const int h = (e + 1) % 3, l = (e + 2) % 3;
+    if (s->g.active == ((1u << e) | (8u << h)) && n[e] == 1 && n[h] == 1 && n[l] > 1) return e;
+  }
+  return -1;
+}
+int64_t stride_of(const gmes_sim* s, int c, int axis) {
+  return axis == 0 ? s->pi[c] : axis == 1 ? s->pitch[c] : s->pk[c];
+}
+
+int sweep1_build(gmes_sim* s) {
+  const int e = line_dir(s), comp[2] = {e, 3 + (e + 1) % 3}, line = (e + 2) % 3;
+  if (s->naux) return GMES_OK;
+  bool cpml = false, upml = false;
+  for (const int c : comp) {
+    cpml |= s->has_cls[c][GMES_CLS_CPML];
+    upml |= s->has_cls[c][GMES_CLS_UPML];
+    if (s->has_cls[c][GMES_CLS_DM2]) return GMES_OK;
+  }
+  if ((cpml && upml) || ((cpml || upml) && s->nprof != 1)) return GMES_OK;
+  s->sweep_absorber = cpml ? 1 : upml ? 2 : 0;
+  for (const int c : comp) {
+    if (!s->sweep_absorber) break;
+    if (!s->pml_state[c]) return GMES_OK;
+    for (int a = 0; a < 3; ++a) {
+      const std::vector<double>& v = s->prof_host[0][c][a];
+      const int w = cpml ? 3 : 6;
+      if (s->prof_w[0][c][a] != w || (int64_t)v.size() != s->shape[c][a] * w) return GMES_OK;
+      for (size_t q = 1; cpml && a != line && q < v.size(); q += 3)
+        if (v[q] != 0.0) return GMES_OK;
+    }
+  }
+  int rc = GMES_OK;
+  for (const int c : comp) {
+    if (!rc) rc = sweep_alloc(s, &s->f_alt[c], (size_t)s->dsize[c] * s->esize);
+  }
+  if (!rc && s->pml_state[e]) {
+    const size_t b = (size_t)(cpml ? 2 : 1) * s->dsize[e] * s->esize;
+    rc = sweep_alloc(s, &s->pml_alt[e], b);
+    if (!rc) HIP_TRY(hipMemsetAsync(s->pml_alt[e], 0, b, s->stream));
+  }
+  bool any = false;
+  for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2 && !rc; ++k) {
+    const AdeList& L = s->ade[e][k];
+    if (!L.n) continue;
+    any = true;
+    const size_t b = std::max<size_t>(1, (size_t)L.nstate * L.n * ade_word(s, k));
+    rc = sweep_alloc(s, &s->ade_alt[e][k], b);
+    if (!rc) HIP_TRY(hipMemsetAsync(s->ade_alt[e][k], 0, b, s->stream));
+  }
+  if (any && !rc) rc = sweep_alloc(s, (void**)&s->d_adeq[e], (size_t)s->dsize[e] * sizeof(int32_t));
+  if (rc) {
+    (void)hipGetLastError();
+    sweep_release(s);
+    return GMES_OK;
+  }
+  for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2; ++k) {
+    const AdeList& L = s->ade[e][k];
+    if (L.n)
+      launch_list_places({L.cell, (int)L.n, (int)s->shape[e][1], (int)s->shape[e][2], s->pi[e], s->pitch[e], s->pk[e],
+                          s->d_adeq[e] + (kPad - s->koff[e])}, s->stream);
+  }
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipStreamSynchronize(s->stream));
+  s->sweep_1d = true;
+  s->sweep_ok = true;
+  return GMES_OK;
+}
+
+int sweep1_sources(gmes_sim* s) {
+  const int e = line_dir(s), line = (e + 2) % 3;
+  s->step2_src.clear();
+  s->sweep_src_ok = (int)s->ops.size() <= kStep2Src;
+  const int64_t n[3] = {s->g.nx, s->g.ny, s->g.nz};
+  for (const gmes_src_op& o : s->ops) {
+    const int64_t sy = s->shape[o.comp][1], sz = s->shape[o.comp][2];
+    const int64_t ix[3] = {o.cell / (sy * sz), (o.cell / sz) % sy, o.cell % sz};
+    int64_t q = 0;
+    if (o.kind != GMES_SRC_SET && o.kind != GMES_SRC_SUB) s->sweep_src_ok = false;
+    for (int a = 0; a < 3; ++a) {
+      const int64_t x = ix[a] - (o.comp >= 3 && a != o.comp - 3);
+      if (x < 0 || x >= n[a]) s->sweep_src_ok = false;  // a ghost cell
+      if (a == line) q = x;
+    }
+    s->step2_src.push_back({o.comp >= 3, (int)q, 0, o.wave, o.kind});
+  }
+  return GMES_OK;
+}
+
+template <class T>
+Step1Args<T> step1_args(const gmes_sim* s) {
+  using R = typename real_of<T>::type;
+  Step1Args<T> m{};
+  const int e = line_dir(s), hd = (e + 1) % 3, line = (e + 2) % 3, comp[2] = {e, 3 + hd};
+  const int w = s->sweep_absorber == 1 ? 3 : 6;
+  for (int f = 0; f < 2; ++f) {
+    const int c = comp[f], collapsed = f ? e : hd;
+    int64_t x[3] = {0, 0, 0};  // storage of cell 0
+    if (f) x[collapsed] = x[line] = 1;
+    const int64_t o = dev_index(s, c, x[0], x[1], x[2]);
+    m.fi[f] = static_cast<const T*>(s->f[c]) + o;
+    m.fo[f] = static_cast<T*>(s->f_alt[c]) + o;
+    m.st[f] = (int)stride_of(s, c, line);
+    m.gc[f] = (f ? -1 : 1) * stride_of(s, c, collapsed);
+    m.ids[f] = s->ids[c] + o;
+    if (s->sweep_absorber) {
+      // CPML: E's line is its second curl axis, H's its first
+      const int64_t word = s->sweep_absorber == 1 && f == 0 ? s->dsize[c] : 0;
+      m.si[f] = static_cast<const T*>(s->pml_state[c]) + o + word;
+      m.so[f] = static_cast<T*>(f ? s->pml_state[c] : s->pml_alt[c]) + o + word;
+      const int axes[3] = {kAx1[c], kAx2[c], c % 3};
+      for (int a = 0; a < 3; ++a)
+        m.row[f][a] = static_cast<const R*>(s->d_prof) + s->prof_off0[c][axes[a]] + x[axes[a]] * w;
+    }
+    m.ph[f][0] = cplx<R>{(R)s->g.phase[c][collapsed][0], (R)s->g.phase[c][collapsed][1]};
+    m.ph[f][1] = cplx<R>{(R)s->g.phase[c][line][0], (R)s->g.phase[c][line][1]};
+  }
+  const double d[3] = {s->g.dx, s->g.dy, s->g.dz};
+  const int axes[3] = {e, hd, line};
+  for (int a = 0; a < 3; ++a) {
+    m.d[a] = (R)d[axes[a]];
+    m.inv_d[a] = (R)(1.0 / d[axes[a]]);
+  }
+  const int64_t n[3] = {s->g.nx, s->g.ny, s->g.nz};
+  m.n = (int)n[line];
+  m.recs = static_cast<const DevRec<R>*>(s->d_recs);
+  m.coef = static_cast<const R*>(s->d_coef);
+  if (s->d_adeq[e]) m.adeq = s->d_adeq[e] + dev_index(s, e, 0, 0, 0);
+  for (int k = 0; k < 3; ++k) {
+    m.ade_in[k] = s->ade[e][GMES_CLS_DRUDE + k].state;
+    m.ade_out[k] = s->ade_alt[e][GMES_CLS_DRUDE + k];
+    m.ade_n[k] = (int)s->ade[e][GMES_CLS_DRUDE + k].n;
+  }
+  m.nsrc = (int)s->step2_src.size();
+  for (int q = 0; q < m.nsrc; ++q) {
+    const auto& v = s->step2_src[q];
+    m.src[q] = {v[0], v[1], v[3], v[4]};
+  }
+  m.waves = s->d_waves;
+  m.ctl = reinterpret_cast<Ctl*>(s->d_clock);
+  m.par = s->par;
+  // the operations of a parent may sample ghost cells
+  m.ghosts = s->sweep_ghosts || s->parent;
+  m.absorber = s->sweep_absorber;
+  return m;
 }
 
 // ---- one-sweep steps of collapsed-z 2-D modes (step2d.hip)
@@ -1506,17 +1660,174 @@ Step2Args<T> step2_args(const gmes_sim* s) {
 
 bool step2_ade(const gmes_sim* s) { return s->d_adeq[0] || s->d_adeq[1] || s->d_adeq[2]; }
 
+// Lists the H cells that a step finishes after the sweep (stepfix.hip).
+// sweep_src_ok is false, and the sim keeps the two-kernel step, when an
+// operation acts on a ghost cell or on a dispersive one (its order after the
+// medium's update would need another launch), or when one of those H cells has
+// live absorber state.
+int sweep_fix_build(gmes_sim* s) {
+  HIP_TRY(sync_exec(s));
+  if (s->d_fix_items) {
+    (void)dev_release(s->d_fix_items);
+    s->d_fix_items = nullptr;
+  }
+  for (int& n : s->fix_nitem) n = 0;
+  s->sweep_src_ok = false;
+  const int64_t n[3] = {s->g.nx, s->g.ny, s->g.nz};
+  for (const gmes_src_op& o : s->ops) {
+    const int64_t sy = s->shape[o.comp][1], sz = s->shape[o.comp][2];
+    const int64_t ix[3] = {o.cell / (sy * sz), (o.cell / sz) % sy, o.cell % sz};
+    for (int a = 0; a < 3; ++a) {
+      const int64_t x = ix[a] - (o.comp >= 3 && a != o.comp - 3);
+      if (x < 0 || x >= n[a]) return GMES_OK;  // a ghost cell
+    }
+    if (o.comp < 3 && s->recs[s->host_ids[o.comp][o.cell]].cls >= GMES_CLS_DRUDE) return GMES_OK;
+  }
+  FixBuild b{};
+  for (int a = 0; a < 3; ++a) {
+    b.n[a] = (int)n[a];
+    // storage coordinates of H lie one up
+    const int lo = s->sweep_run_h[a] & 0xFFFF, hi = s->sweep_run_h[a] >> 16;
+    b.run_h[a] = std::max(0, lo - 1) | (std::max(0, hi - 1) << 16);
+  }
+  b.cells = n[0] * n[1] * n[2];
+  b.nblk = (int)((b.cells + kFixMark - 1) / kFixMark);
+  for (int c = 0; c < 6; ++c) {
+    b.base[c] = dev_index(s, c, 0, 0, 0);
+    b.pi[c] = s->pi[c];
+    b.p[c] = s->pitch[c];
+    if (c >= 3) b.hid[c - 3] = s->ids[c] + dev_index(s, c, c != 3, c != 4, c != 5);
+  }
+  b.groups = s->d_groups;
+  b.nge = s->ngroups_e;
+  b.ngroups = s->ngroups_e + s->ngroups_h;
+  std::vector<int32_t> cls(s->recs.size());
+  for (size_t r = 0; r < cls.size(); ++r) cls[r] = s->recs[r].cls;
+  const size_t mark = ((size_t)(3 * b.cells) + 15) / 16 * 16, count = (size_t)3 * b.nblk * sizeof(int32_t),
+               rec = cls.size() * sizeof(int32_t);
+  char* tmp = nullptr;
+  HIP_TRY(hipMalloc((void**)&tmp, mark + count + rec + 16));
+  b.mark = reinterpret_cast<uint8_t*>(tmp);
+  b.count = reinterpret_cast<int32_t*>(tmp + mark);
+  b.cls = reinterpret_cast<int32_t*>(tmp + mark + count);
+  b.bad = reinterpret_cast<int*>(tmp + mark + count + rec);
+  std::vector<int32_t> counts((size_t)3 * b.nblk);
+  int bad = 0;
+  auto build = [&]() -> hipError_t {
+    hipError_t e = hipMemset(tmp, 0, mark + count + rec + 16);
+    if (e != hipSuccess) return e;
+    if ((e = hipMemcpy(const_cast<int32_t*>(b.cls), cls.data(), rec, hipMemcpyHostToDevice)) != hipSuccess) return e;
+    for (int c = 0; c < 3; ++c)
+      for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2; ++k) {
+        const AdeList& L = s->ade[c][k];
+        if (!L.n) continue;
+        b.ade_cell = L.cell;
+        b.ade_n = (int)L.n;
+        b.comp = c;
+        b.s1 = (int)s->shape[c][1];
+        b.s2 = (int)s->shape[c][2];
+        launch_fix_mark_ade(b, nullptr);
+      }
+    if (b.ngroups) launch_fix_mark_src(b, nullptr);
+    launch_fix_count(b, nullptr);
+    if ((e = hipMemcpy(counts.data(), b.count, count, hipMemcpyDeviceToHost)) != hipSuccess) return e;
+    int total = 0;
+    for (int c = 0; c < 3; ++c) {
+      b.first_item[c] = total;
+      for (int q = 0; q < b.nblk; ++q) {
+        const int m = counts[(size_t)c * b.nblk + q];
+        counts[(size_t)c * b.nblk + q] = total;
+        total += m;
+      }
+      b.nitem[c] = total - b.first_item[c];
+    }
+    if (!total) return hipSuccess;
+    if ((e = hipMalloc(&s->d_fix_items, (size_t)total * sizeof(FixItem))) != hipSuccess) return e;
+    b.items = static_cast<FixItem*>(s->d_fix_items);
+    if ((e = hipMemcpy(b.count, counts.data(), count, hipMemcpyHostToDevice)) != hipSuccess) return e;
+    launch_fix_fill(b, nullptr);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    return hipMemcpy(&bad, b.bad, sizeof bad, hipMemcpyDeviceToHost);
+  };
+  const hipError_t e = b.cells < INT32_MAX / 4 ? build() : hipErrorOutOfMemory;
+  (void)dev_release(tmp);
+  if (e == hipErrorOutOfMemory) {  // no room for the lists: the two-kernel step needs none
+    (void)hipGetLastError();
+    return GMES_OK;
+  }
+  HIP_TRY(e);
+  for (int c = 0; c < 3; ++c) s->fix_nitem[c] = b.nitem[c];
+  s->sweep_src_ok = !bad;
+  return GMES_OK;
+}
+
+template <class T>
+FixArgs<T> fix_args(const gmes_sim* s) {
+  using R = typename real_of<T>::type;
+  FixArgs<T> m{};
+  for (int c = 0; c < 6; ++c) {
+    const int64_t o = dev_index(s, c, c >= 3 && c != 3, c >= 3 && c != 4, c >= 3 && c != 5);
+    const T* old = static_cast<const T*>(s->f_alt[c]) + o;  // the sweep has swapped the sets
+    T* now = static_cast<T*>(s->f[c]) + o;
+    const int a = c % 3;
+    (c < 3 ? m.ei : m.hi)[a] = old;
+    (c < 3 ? m.eo : m.ho)[a] = now;
+    (c < 3 ? m.pe : m.ph)[a] = s->pi[c];
+    (c < 3 ? m.re : m.rh)[a] = s->pitch[c];
+    for (int x = 0; x < 3; ++x)
+      (c < 3 ? m.phe : m.phh)[a][x] = cplx<R>{(R)s->g.phase[c][x][0], (R)s->g.phase[c][x][1]};
+    m.base[c] = static_cast<T*>(s->f[c]);
+    if (c >= 3) m.hid[a] = s->ids[c] + o;
+  }
+  m.n[0] = s->g.nx; m.n[1] = s->g.ny; m.n[2] = s->g.nz;
+  m.d[0] = (R)s->g.dx; m.d[1] = (R)s->g.dy; m.d[2] = (R)s->g.dz;
+  m.inv_d[0] = (R)(1.0 / s->g.dx); m.inv_d[1] = (R)(1.0 / s->g.dy); m.inv_d[2] = (R)(1.0 / s->g.dz);
+  m.recs = static_cast<const DevRec<R>*>(s->d_recs);
+  m.coef = static_cast<const R*>(s->d_coef);
+  for (int c = 0; c < 3; ++c)
+    for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2; ++k) {
+      const AdeList& L = s->ade[c][k];
+      if (!L.n) continue;
+      m.ade[m.nade++] = {L.cell, L.rec, L.state, (int)L.n, c, k, m.eblocks, (int)s->shape[c][1], (int)s->shape[c][2]};
+      m.eblocks += (int)((L.n + kFixBlock - 1) / kFixBlock);
+    }
+  m.first_src = m.eblocks;
+  m.groups = s->d_groups;
+  m.nge = s->ngroups_e;
+  m.eblocks += (m.nge + kFixBlock - 1) / kFixBlock;
+  m.ops = static_cast<const DevSrcOp<R>*>(s->d_ops);
+  m.waves = s->d_waves;
+  for (int i = 0; i < s->naux; ++i)
+    for (int c = 0; c < 6; ++c) m.aux[i][c] = s->aux[i] ? s->aux[i]->f[c] : nullptr;
+  m.ctl = reinterpret_cast<Ctl*>(s->d_clock);
+  m.items = static_cast<const FixItem*>(s->d_fix_items);
+  for (int c = 0, at = 0; c < 3; ++c) {
+    m.nitem[c] = s->fix_nitem[c];
+    m.first_item[c] = at;
+    m.item_blk[c] = m.hblocks;
+    at += m.nitem[c];
+    m.hblocks += (m.nitem[c] + kFixBlock - 1) / kFixBlock;
+  }
+  return m;
+}
+
 // Marks the cells of the sim's source operations in the sweep's ids, when
 // all of them can be applied there (sweep_src_ok).
 int sweep_sources(gmes_sim* s) {
   if (!s->sweep_ok) return GMES_OK;
+  if (s->sweep_1d) return sweep1_sources(s);
   if (s->sweep_2d) return sweep2_sources(s);
   HIP_TRY(sync_exec(s));
   for (const auto& x : s->src_ids)
     HIP_TRY(hipMemcpy(s->d_step_ids + x.first, &x.second, sizeof(uint32_t), hipMemcpyHostToDevice));
   s->src_ids.clear();
-  s->sweep_src_ok = (int)s->ops.size() <= kSweepMaxSrc;
   s->has_waves = false;
+  s->sweep_fix = s->sweep_ade || s->naux || (int)s->ops.size() > kSweepMaxSrc;
+  if (s->sweep_fix) {
+    if (int rc = sweep_fix_build(s)) return rc;
+    return s->fp64 ? sweep_upload_tab<double>(s, {}, {}) : sweep_upload_tab<float>(s, {}, {});
+  }
+  s->sweep_src_ok = true;
   std::vector<std::array<int, 3>> src[2];
   std::vector<int64_t> cell(s->ops.size());
   const int64_t n[3] = {s->g.nx, s->g.ny, s->g.nz};
@@ -1554,18 +1865,20 @@ int sweep_sources(gmes_sim* s) {
 // the sim does not qualify.
 int sweep_build(gmes_sim* s) {
   sweep_release(s);
+  if (line_dir(s) >= 0) return sweep1_build(s);
   if (is_2z(s)) return s->naux ? GMES_OK : sweep2_build(s);
-  if (!is3d(s) || s->g.dtype == GMES_C128 || s->naux) return GMES_OK;
+  if (!is3d(s) || s->g.dtype == GMES_C128) return GMES_OK;
   const int nz = s->g.nz;
   if (kSweepMinRows * nz > kStepMaxThreads || s->g.ny < 2) return GMES_OK;
   for (int c = 0; c < 6; ++c)  // 32-bit byte offsets, both state words included
     if (2 * s->dsize[c] * s->esize >= (int64_t)0xFFFFFF00) return GMES_OK;
   bool cpml = false, upml = false;
+  s->sweep_ade = false;
   for (int c = 0; c < 6; ++c) {
     cpml |= s->has_cls[c][GMES_CLS_CPML];
     upml |= s->has_cls[c][GMES_CLS_UPML];
-    for (int k = GMES_CLS_DRUDE; k < GMES_NCLS; ++k)
-      if (s->has_cls[c][k]) return GMES_OK;
+    if (s->has_cls[c][GMES_CLS_DM2]) return GMES_OK;
+    for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2; ++k) s->sweep_ade |= s->has_cls[c][k];
   }
   if ((cpml && upml) || ((cpml || upml) && s->nprof != 1)) return GMES_OK;
   // the kernels keep every component's absorber state
@@ -1625,8 +1938,13 @@ int sweep_build(gmes_sim* s) {
 }
 
 // Whether the next step of s is a one-sweep step.
+// Whether an auxiliary grid takes one-sweep steps when its parent does.
+bool aux_sweeps(const gmes_sim* a) {
+  return a->sweep_1d && a->sweep_ok && a->sweep_src_ok && a->allow_fuse && a->probes.empty() && a->dfts.empty();
+}
+
 bool sweeps(const gmes_sim* s) {
-  if (!s->sweep_ok || !s->sweep_src_ok || !s->allow_fuse || s->naux || s->parent) return false;
+  if (!s->sweep_ok || !s->sweep_src_ok || !s->allow_fuse || (s->naux && !s->sweep_fix) || s->parent) return false;
   if (s->tile_bx > 0 && !s->tile_tuned) return false;
   for (const auto& p : s->probes)
     if (p.comp < 3 && on_ghost_copy_plane(s, p.comp, p.cell, false, true)) return false;
@@ -1732,7 +2050,9 @@ void sweep_swap(gmes_sim* s) {
 template <class T>
 void enqueue_sweep(gmes_sim* s, hipStream_t st) {
   time_begin(s, 0, st);
-  if (s->sweep_2d) {
+  if (s->sweep_1d) {
+    launch_step1d<T>(step1_args<T>(s), st);
+  } else if (s->sweep_2d) {
     launch_step2d<T>(step2_args<T>(s), step2_tm(s), s->sweep_absorber, step2_ade(s), st);
   } else if constexpr (!std::is_same<T, cplx<double>>::value) {
     launch_step3d<T>(step3_args<T>(s), s->sweep_part.absorber, s->sweep_part.threads, st);
@@ -1745,6 +2065,22 @@ template <class T>
 void enqueue_step_t(gmes_sim* s, hipStream_t st) {
   if (sweeps(s)) {
     enqueue_sweep<T>(s, st);
+    if constexpr (!std::is_same<T, cplx<double>>::value) {
+      if (s->sweep_fix) {
+        time_begin(s, 2, st);
+        launch_fix_e<T>(fix_args<T>(s), st);  // reads the auxiliary grids before their step
+        time_end(s, st);
+        enqueue_probe<T>(s, true, st);
+        enqueue_aux_steps(s, true, st);
+        if (s->sweep_ghosts) enqueue_ghost<T>(s, true, 0, st);
+        time_begin(s, 3, st);
+        launch_fix_h<T>(fix_args<T>(s), st);
+        time_end(s, st);
+        enqueue_probe<T>(s, false, st);
+        enqueue_dft<T>(s, st);
+        return;
+      }
+    }
     enqueue_probe<T>(s, true, st);
     enqueue_probe<T>(s, false, st);
     enqueue_dft<T>(s, st);
@@ -1755,12 +2091,31 @@ void enqueue_step_t(gmes_sim* s, hipStream_t st) {
   enqueue_ade<T>(s, st);
   enqueue_src<T>(s, true, st);
   enqueue_probe<T>(s, true, st);
-  enqueue_aux_steps(s, st);
+  enqueue_aux_steps(s, false, st);
   if (!s->fuse_e) enqueue_ghost<T>(s, true, 0, st);
   enqueue_main<T>(s, false, st);
   enqueue_src<T>(s, false, st);
   enqueue_probe<T>(s, false, st);
   enqueue_dft<T>(s, st);
+}
+
+void enqueue_aux_steps(gmes_sim* s, bool sweep, hipStream_t st) {
+  for (int i = 0; i < s->naux; ++i) {
+    gmes_sim* a = s->aux[i];
+    if (!a) continue;
+    time_begin(s, 5, st);
+    if (!(sweep && aux_sweeps(a))) {
+      enqueue_step(a, st);
+    } else {
+      switch (a->g.dtype) {
+        case GMES_F32: enqueue_sweep<float>(a, st); break;
+        case GMES_F64: enqueue_sweep<double>(a, st); break;
+        case GMES_C64: enqueue_sweep<cplx<float>>(a, st); break;
+        default: enqueue_sweep<cplx<double>>(a, st); break;
+      }
+    }
+    time_end(s, st);
+  }
 }
 
 void enqueue_step(gmes_sim* s, hipStream_t st) {
@@ -1890,6 +2245,25 @@ int collect_timing(gmes_sim* s) {
 
 bool any_graph_blocker(gmes_sim* s) { return s->timing.on; }
 
+// The clock as one-sweep steps pass it on (Ctl::clk), brought up to date before
+// the first of them after other steps.
+void sweep_clock(gmes_sim* s, bool sweep, hipStream_t st) {
+  if (sweep && s->clk_stale) launch_clock_copy(reinterpret_cast<Ctl*>(s->d_clock), st);
+  s->clk_stale = !sweep;
+}
+
+// The table of the auxiliary grids' buffers that source launches read; their
+// one-sweep steps swap those.
+int aux_pointers(gmes_sim* s) {
+  for (int i = 0; i < s->naux; ++i) {
+    if (!s->aux[i] || !memcmp(s->aux_ptr[i], s->aux[i]->f, sizeof s->aux_ptr[i])) continue;
+    HIP_TRY(sync_exec(s));
+    memcpy(s->aux_ptr[i], s->aux[i]->f, sizeof s->aux_ptr[i]);
+    HIP_TRY(hipMemcpy(static_cast<void**>(s->d_aux_ptrs) + i * 6, s->aux_ptr[i], sizeof s->aux_ptr[i], hipMemcpyHostToDevice));
+  }
+  return GMES_OK;
+}
+
 int do_step(gmes_sim* s, int64_t n) {
   if (!s->committed) return set_error(GMES_EINVAL, "sim is not committed");
   if (n < 0) return set_error(GMES_EINVAL, "negative step count");
@@ -1901,11 +2275,11 @@ int do_step(gmes_sim* s, int64_t n) {
   if ((rc = ensure_probe_capacity(s, n))) return rc;
   HIP_TRY(hipSetDevice(s->device));
   const bool sweep = sweeps(s);
-  if (!sweep) {
-    s->clk_stale = true;
-  } else if (s->clk_stale && n > 0) {
-    launch_clock_copy(reinterpret_cast<Ctl*>(s->d_clock), s->stream);
-    s->clk_stale = false;
+  if (n > 0) {
+    sweep_clock(s, sweep, s->stream);
+    for (int i = 0; i < s->naux; ++i)
+      if (s->aux[i]) sweep_clock(s->aux[i], sweep && aux_sweeps(s->aux[i]), s->stream);
+    if (!sweep && (rc = aux_pointers(s))) return rc;
   }
   const int par = s->par;
   if (s->use_graph && !any_graph_blocker(s)) {
@@ -2574,16 +2948,13 @@ int gmes_sim_attach_aux(gmes_sim* s, gmes_sim* aux, int32_t* slot) {
   if (aux->parent) return set_error(GMES_EINVAL, "auxiliary grid already attached");
   HIP_TRY(hipSetDevice(s->device));
   HIP_TRY(sync_exec(s));
-  sweep_release(s);  // a sim with an auxiliary grid takes two-kernel steps: no second buffers
+  if (s->sweep_1d || s->sweep_2d) sweep_release(s);  // a 1-D or 2-D sim with one takes two-kernel steps: no second buffers
   s->aux[s->naux] = aux;
   aux->parent = s;
-  void* ptrs[6];
-  for (int c = 0; c < 6; ++c) ptrs[c] = aux->f[c];
-  HIP_TRY(hipSetDevice(s->device));
-  HIP_TRY(hipMemcpy(static_cast<void**>(s->d_aux_ptrs) + s->naux * 6, ptrs, sizeof ptrs, hipMemcpyHostToDevice));
   *slot = s->naux++;
+  if (int rc = aux_pointers(s)) return rc;
   destroy_graph(s);
-  return GMES_OK;
+  return sweep_sources(s);
 }
 
 int gmes_sim_add_probe(gmes_sim* s, int32_t c, int64_t cell, int32_t* id) {
@@ -3412,6 +3783,11 @@ int gmes_batch_step(gmes_batch* b, int64_t nsteps) {
     int rc = check_windows(s, nsteps);
     if (rc) return rc;
     if ((rc = ensure_probe_capacity(s, nsteps))) return rc;
+    HIP_TRY(hipSetDevice(b->device));
+    if ((rc = aux_pointers(s))) return rc;
+    sweep_clock(s, false, b->stream);
+    for (int i = 0; i < s->naux; ++i)
+      if (s->aux[i]) sweep_clock(s->aux[i], false, b->stream);
   }
   HIP_TRY(hipSetDevice(b->device));
   // the job tables are read by kernels still in flight: wait before rewriting
@@ -3489,10 +3865,7 @@ int gmes_batch_step(gmes_batch* b, int64_t nsteps) {
     for (int64_t t = 0; t < nsteps; ++t) enqueue_batch_step(b, b->stream);
     HIP_TRY(hipGetLastError());
   }
-  for (gmes_sim* s : b->sims) {
-    s->clk_stale = true;
-    advance_host_clock(s, nsteps);
-  }
+  for (gmes_sim* s : b->sims) advance_host_clock(s, nsteps);
   return GMES_OK;
 }
 

@@ -213,6 +213,13 @@ struct gmes_sim {
   void* step2_cells = nullptr;     // Step2Cell[3 * entries]
   int32_t* d_adeq[3] = {};
   void* ade_alt[3][GMES_NCLS] = {};
+  bool sweep_1d = false;           // a TEM line (step1d.hip)
+  void* aux_ptr[8][6] = {};        // what d_aux_ptrs holds
+  // 3-D, cells finished after the sweep (stepfix.hip): dispersive ones, sources
+  // on many cells
+  bool sweep_ade = false, sweep_fix = false;
+  void* d_fix_items = nullptr;    // FixItem[], of Hx, Hy, Hz in turn
+  int fix_nitem[3] = {};
   std::vector<std::array<int, 5>> step2_src;  // direction, i, j, wave, kind
   std::vector<std::array<uint16_t, 3>> step_e, step_h;  // record ids of each entry
   std::vector<std::pair<int64_t, uint32_t>> src_ids;  // ids the sources replaced (element, old word)

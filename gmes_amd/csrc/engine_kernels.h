@@ -168,6 +168,71 @@ struct Step3Args {
   int exact;       // FP64: every division is by a power of two
   int ghosts;      // write the ghost planes: the last step of a call, unless a monitor reads them
 };
+// Cells a one-sweep 3-D step leaves to two launches after it (stepfix.hip):
+// dispersive E cells and E cells with sources that do not fit its table, then
+// the H cells whose curl reads those, and H cells with such sources.
+constexpr int kFixBlock = 256, kFixMark = 1024;
+struct FixItem {
+  int32_t cell;  // thread (i * ny + j) * nz + k
+  int32_t grp;   // source group, -1: none
+};
+template <class T>
+struct FixArgs {
+  using R = typename real_of<T>::type;
+  // by direction, at thread (0, 0, 0)'s cell
+  const T* ei[3];  // old E, H
+  const T* hi[3];
+  T* eo[3];        // new ones
+  T* ho[3];
+  T* base[6];      // new arrays from element 0 (source groups)
+  int pe[3], re[3], ph[3], rh[3];  // strides along i and j of E, H
+  int n[3];
+  cplx<R> phe[3][3], phh[3][3];    // ghost phases of component c along axis a
+  R d[3], inv_d[3];
+  const DevRec<R>* recs;
+  const R* coef;
+  const uint16_t* hid[3];
+  struct { const int32_t* cell; const uint16_t* rec; void* state; int n, comp, cls, first, s1, s2; } ade[9];
+  int nade;
+  const SrcGroup* groups;  // E's, then H's
+  int nge, first_src;      // E groups, their first block
+  const DevSrcOp<R>* ops;
+  const double* waves;
+  const void* aux[8][6];   // current fields of the auxiliary grids
+  Ctl* ctl;
+  const FixItem* items;
+  int nitem[3], first_item[3], item_blk[3];  // of Hx, Hy, Hz; first item, first block
+  int eblocks, hblocks;
+};
+template <class T> void launch_fix_e(const FixArgs<T>& a, hipStream_t st);
+template <class T> void launch_fix_h(const FixArgs<T>& a, hipStream_t st);
+// Marks the H cells of the lists (phase 0: dispersive cells and E groups, the
+// H cells that read them; H groups, themselves), counts them per kFixMark
+// cells, writes the items, and their groups.
+struct FixBuild {
+  int n[3];
+  int64_t cells;           // n[0] * n[1] * n[2]
+  uint8_t* mark;           // [3][cells]
+  int32_t* count;          // [3][blocks]: marked cells, then their first item
+  int nblk;
+  FixItem* items;
+  int nitem[3], first_item[3];
+  const int32_t* ade_cell; // one list
+  int ade_n, comp, s1, s2;
+  const SrcGroup* groups;
+  int ngroups, nge;
+  int64_t base[6];         // element of logical (0, 0, 0)
+  int pi[6], p[6];
+  const uint16_t* hid[3];  // at thread (0, 0, 0)
+  const int32_t* cls;      // class of each record
+  int run_h[3];            // thread coordinates without live CPML state
+  int* bad;                // an absorber cell with live state is among them
+};
+void launch_fix_mark_ade(const FixBuild& b, hipStream_t st);
+void launch_fix_mark_src(const FixBuild& b, hipStream_t st);
+void launch_fix_count(const FixBuild& b, hipStream_t st);
+void launch_fix_fill(const FixBuild& b, hipStream_t st);
+
 // The same for a collapsed-z 2-D mode (TMz: Ez, Hx, Hy; TEz: Ex, Ey, Hz).
 // Arrays are indexed by the direction of the component; thread (i, j) owns
 // one cell of each, at element off + i * pi + j of its arrays.
@@ -227,6 +292,38 @@ template <class T>
 inline size_t step2_lds(int nthreads, int nent) {
   return (size_t)nent * sizeof(Step2Ent<typename real_of<T>::type>) + 4 * (size_t)nthreads * sizeof(T);
 }
+
+// The same for a 1-D line (TEM modes; also the auxiliary grids of total-field
+// boxes): component e of E, h = e + 1 of H, along axis e + 2 (mod 3).
+template <class T>
+struct Step1Args {
+  using R = typename real_of<T>::type;
+  const T* fi[2];   // old E, H at cell 0
+  T* fo[2];
+  const T* si[2];   // absorber words: CPML along the line, UPML the component's
+  T* so[2];
+  int st[2];        // element strides along the line
+  int64_t gc[2];    // from a cell to its ghost image along the collapsed axis
+  const uint16_t* ids[2];
+  int n;
+  const DevRec<R>* recs;
+  const R* coef;
+  const R* row[2][3];  // absorber rows of E, H: first curl axis, second, own; the line's at cell 0
+  cplx<R> ph[2][2];    // ghost phase along the collapsed axis, along the line
+  R d[3], inv_d[3];    // of axes e, h, the line
+  const int32_t* adeq;
+  const void* ade_in[3];
+  void* ade_out[3];
+  int ade_n[3];
+  int nsrc;
+  struct { int c, q, wave, kind; } src[kStep2Src];
+  const double* waves;
+  Ctl* ctl;
+  int par, ghosts, absorber;
+};
+constexpr int kStep1Threads = 256;
+template <class T>
+void launch_step1d(const Step1Args<T>& m, hipStream_t st);
 
 // The entry ids of a sim, looked up from its material ids on the device.
 struct StepKey {

@@ -168,3 +168,73 @@ def test_monitors_see_each_step(engine_lib, tmp_path):
         assert len(x) == 9
         np.testing.assert_array_equal(x, y)
     np.testing.assert_array_equal(out[0][1], out[1][1])
+
+
+def media_box(lib, n, precision="fp32", bloch=None, media=True, wave=True, bound=None, point=(), seam=True):
+    """Dispersive objects (over the periodic edges with seam), a plane wave
+    through a total-field box, point sources."""
+    geom = [g.DefaultMedium(g.Dielectric())]
+    if media:
+        pole, crit = g.DrudePole(omega=0.5, gamma=0.05), g.CriticalPoint(amp=0.6, phi=-0.4, omega=0.4, gamma=0.05)
+        kinds = [g.Drude(eps_inf=2.0, dps=(pole,)),
+                 g.Lorentz(eps_inf=2.0, lps=(g.LorentzPole(amp=1.2, omega=0.4, gamma=0.02),)),
+                 g.DcpAde(eps_inf=2.0, sigma=0.01, dps=(pole,), cps=(crit,)),
+                 g.DcpPlrc(eps_inf=2.0, sigma=0.01, dps=(pole,), cps=(crit, crit))]
+        for q, kind in enumerate(kinds):
+            c = [(-0.5 if seam and q == 0 else 0.2 * q - 0.3) * v for v in n]
+            geom.append(g.Block(kind, center=c, size=[v / 5 for v in n]))
+        geom.append(g.Block(g.Const(0.25), center=(0.1 * n[0], 0, 0), size=(1.1, 1.1, 1.1)))
+    if bound is not None:
+        geom.append(g.Shell(bound(), thickness=2))
+    wf = g.Continuous(freq=0.05, width=5)
+    src = [g.PointSource(wf, center=(q, 1, 2), component=c) for q, c in enumerate(point)]
+    if wave:
+        src.append(g.TotalFieldScatteredField(wf, center=(0, 0, 0), size=(2 * n[0], 2 * n[1], n[2] - 7.3),
+                                              direction=(0, 0, -1), polarization=(1, 0, 0)))
+    sim = g.FDTD(g.Cartesian(size=n, resolution=1), geom, src, courant_ratio=0.5, verbose=False, precision=precision,
+                 bloch=bloch, _engine=lib)
+    sim.init()
+    rng = np.random.default_rng(5)
+    for c in g.constant.COMPONENTS:
+        a = sim.field[c]
+        a[...] = rng.standard_normal(a.shape)
+        if bloch is not None:
+            a[...] += 1j * rng.standard_normal(a.shape)
+    return sim
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(precision="fp64"), dict(bloch=(0.3, -0.2, 0.0))], ids=["fp32", "fp64", "c64"])
+@pytest.mark.parametrize("what", [dict(wave=False), dict(media=False), dict(), dict(wave=False, seam=False, bound=g.Cpml),
+                                  dict(wave=False, seam=False, bound=g.Upml), dict(wave=False, point=(g.Ez, g.Hx, g.Ey)),
+                                  dict(media=False, bound=g.Cpml)],
+                         ids=["media", "wave", "both", "media_cpml", "media_upml", "media_points", "wave_cpml"])
+@pytest.mark.parametrize("graph", [False, True], ids=["direct", "graph"])
+def test_cells_finished_after_the_sweep(engine_lib, kw, what, graph):
+    """Dispersive cells and sources on many cells, and the H cells next to
+    them, the periodic images included; in the last case some of those have
+    absorber state (the two-kernel step)."""
+    n = (22, 21, 24)
+    a, b = media_box(engine_lib, n, **kw, **what), media_box(engine_lib, n, **kw, **what)
+    engine_lib.set_ghost_fusion(b._sim, 0)
+    if graph:
+        engine_lib.set_graph(a._sim, 1)
+    for k in (1, 4, 7):
+        a._advance(k)
+        b._advance(k)
+        agree(a, b)
+    snap = a.snapshot()
+    a._advance(3)
+    want = {c: np.array(a.field[c]) for c in g.constant.COMPONENTS}
+    a.restore(snap)
+    a._advance(3)
+    for c, v in want.items():
+        np.testing.assert_array_equal(a.field[c], v)
+
+
+def test_finished_cells_match_the_oracle(engine_lib, oracle_lib):
+    a, b = (media_box(lib, (16, 15, 20), precision="fp64") for lib in (engine_lib, oracle_lib))
+    a._advance(12)
+    b._advance(12)
+    for c in g.constant.COMPONENTS:
+        x, y = np.array(a.field[c]), np.array(b.field[c])
+        assert np.linalg.norm(x - y) <= FP64_TOL * np.linalg.norm(y)
