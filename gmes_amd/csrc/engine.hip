@@ -111,6 +111,48 @@ void host_parallel(int n, int64_t cells, F f) {
   if (failed) throw std::bad_alloc();
 }
 
+// Pinned staging of large field reads and writes: at most kStageMax buffers,
+// leased for one transfer each and freed with the last sim.
+constexpr int64_t kStageBytes = 16 << 20;
+constexpr int kStageMax = 4, kStageThreads = 4;
+struct StagePool {
+  std::mutex mu;
+  std::vector<void*> idle;
+  int total = 0, sims = 0;
+} g_stage;
+
+void* stage_lease() {
+  std::lock_guard<std::mutex> lk(g_stage.mu);
+  if (!g_stage.idle.empty()) {
+    void* p = g_stage.idle.back();
+    g_stage.idle.pop_back();
+    return p;
+  }
+  if (g_stage.total == kStageMax) return nullptr;
+  void* p = nullptr;
+  if (hipHostMalloc(&p, kStageBytes, hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  ++g_stage.total;
+  return p;
+}
+
+void stage_return(void* p) {
+  std::lock_guard<std::mutex> lk(g_stage.mu);
+  g_stage.idle.push_back(p);
+}
+
+// a sim is created (1) or gone (-1)
+void stage_sims(int d) {
+  std::lock_guard<std::mutex> lk(g_stage.mu);
+  g_stage.sims += d;
+  if (g_stage.sims) return;
+  for (void* p : g_stage.idle) (void)hipHostFree(p);
+  g_stage.total -= (int)g_stage.idle.size();
+  g_stage.idle.clear();
+}
+
 hipError_t dev_release(void* p) { return hipFree(p); }
 hipError_t device_drain() { return hipDeviceSynchronize(); }
 hipError_t stream_release(hipStream_t st) { return hipStreamDestroy(st); }
@@ -2552,6 +2594,7 @@ int gmes_sim_create(const gmes_grid_desc* desc, gmes_sim** out) {
   if (desc->device < 0 || desc->device >= ndev) return set_error(GMES_EINVAL, "bad device ordinal");
   HIP_TRY(hipSetDevice(desc->device));
   gmes_sim* s = new gmes_sim();
+  stage_sims(1);
   s->g = *desc;
   s->device = desc->device;
   s->complex_ = desc->dtype == GMES_C64 || desc->dtype == GMES_C128;
@@ -2595,6 +2638,7 @@ int gmes_sim_create(const gmes_grid_desc* desc, gmes_sim** out) {
     }
     if (s->dsize[c] >= (int64_t(1) << 31)) {
       delete s;
+      stage_sims(-1);
       return set_error(GMES_EINVAL, "component %d has more than 2^31 cells", c);
     }
   }
@@ -2656,6 +2700,7 @@ int gmes_sim_destroy(gmes_sim* s) {
     if (b) (void)dev_release(b);
   if (s->stream) (void)stream_release(s->stream);
   delete s;
+  stage_sims(-1);
   return GMES_OK;
 }
 
@@ -3103,6 +3148,70 @@ static int stage_reserve(gmes_sim* s, int64_t bytes) {
   return GMES_OK;
 }
 
+// Copies contiguous device memory from or to the caller's array, on the stream
+// of s, and waits.  The caller's memory is pageable: the runtime copies it
+// through its own buffers on one thread.  Large copies go through pinned
+// buffers here, a few threads each moving a part of the array while the next
+// piece is on the link (67 MB: reading 17.3 -> 37 GB/s, writing 28 -> 36; 11 MB:
+// reading 17.2 -> 26, writing 27 -> 25.5; below, starting the threads costs as
+// much as it gains).
+constexpr int64_t kStageRead = 8 << 20, kStageWrite = 16 << 20;
+static int host_copy(gmes_sim* s, char* dev, char* host, int64_t bytes, bool to_device) {
+  void* const pinned = bytes >= (to_device ? kStageWrite : kStageRead) ? stage_lease() : nullptr;
+  if (!pinned) {
+    HIP_TRY(to_device ? hipMemcpyAsync(dev, host, (size_t)bytes, hipMemcpyHostToDevice, s->stream)
+                      : hipMemcpyAsync(host, dev, (size_t)bytes, hipMemcpyDeviceToHost, s->stream));
+    HIP_TRY(sync_exec(s));
+    return GMES_OK;
+  }
+  constexpr int64_t piece = kStageBytes / kStageThreads / 2;
+  std::atomic<int> error{(int)hipSuccess};
+  auto part = [&](int t) {
+    const int64_t lo = bytes / 64 * t / kStageThreads * 64,
+                  hi = t == kStageThreads - 1 ? bytes : bytes / 64 * (t + 1) / kStageThreads * 64;
+    char* const buf = static_cast<char*>(pinned) + 2 * piece * t;
+    hipEvent_t done[2] = {};
+    auto ok = [&](hipError_t e) {
+      if (e != hipSuccess) error = (int)e;
+      return e == hipSuccess;
+    };
+    auto move = [&](int64_t k) {  // piece k of the part over the link
+      const int64_t o = lo + k * piece, n = std::min(piece, hi - o);
+      char* const b = buf + (k & 1) * piece;
+      return ok(to_device ? hipMemcpyAsync(dev + o, b, (size_t)n, hipMemcpyHostToDevice, s->stream)
+                          : hipMemcpyAsync(b, dev + o, (size_t)n, hipMemcpyDeviceToHost, s->stream)) &&
+             ok(hipEventRecord(done[k & 1], s->stream));
+    };
+    const int64_t n = (hi - lo + piece - 1) / piece;
+    bool good = ok(hipSetDevice(s->device));
+    for (hipEvent_t& e : done) good = good && ok(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (good && !to_device && n > 0) good = move(0);
+    for (int64_t k = 0; k < n && good; ++k) {
+      char* const h = host + lo + k * piece;
+      const size_t m = (size_t)std::min(piece, hi - lo - k * piece);
+      if (to_device) {
+        if (k >= 2) good = ok(hipEventSynchronize(done[k & 1]));
+        if (good) memcpy(buf + (k & 1) * piece, h, m);
+        good = good && move(k);
+      } else {
+        if (k + 1 < n) good = move(k + 1);
+        good = good && ok(hipEventSynchronize(done[k & 1]));
+        if (good) memcpy(h, buf + (k & 1) * piece, m);
+      }
+    }
+    if (!good) (void)hipStreamSynchronize(s->stream);
+    for (hipEvent_t e : done)
+      if (e) (void)hipEventDestroy(e);
+  };
+  host_parallel(kStageThreads, bytes, part);
+  const hipError_t e = hipStreamSynchronize(s->stream);
+  stage_return(pinned);
+  if (e != hipSuccess) error = (int)e;
+  HIP_TRY((hipError_t)error.load());
+  HIP_TRY(sync_exec(s));
+  return GMES_OK;
+}
+
 int gmes_sim_write_field(gmes_sim* s, int32_t c, const void* host, int64_t bytes) {
   ApiGuard api;
   if (!s) return set_error(GMES_EINVAL, "null sim handle");
@@ -3111,15 +3220,14 @@ int gmes_sim_write_field(gmes_sim* s, int32_t c, const void* host, int64_t bytes
   HIP_TRY(hipSetDevice(s->device));
   HIP_TRY(sync_exec(s));  // steps queued on the sim's (or its batch's) stream come first
   if (dense_layout(s, c)) {
-    HIP_TRY(hipMemcpyAsync(static_cast<char*>(s->f[c]) + (size_t)kPad * s->esize, host, (size_t)bytes,
-                           hipMemcpyHostToDevice, s->stream));
-    HIP_TRY(sync_exec(s));
-    return GMES_OK;
+    return host_copy(s, static_cast<char*>(s->f[c]) + (size_t)kPad * s->esize,
+                     const_cast<char*>(static_cast<const char*>(host)), bytes, true);
   }
   // one contiguous upload, then rows moved to their pitched places
   int rc = stage_reserve(s, bytes);
   if (rc) return rc;
-  HIP_TRY(hipMemcpyAsync(s->d_stage, host, (size_t)bytes, hipMemcpyHostToDevice, s->stream));
+  if ((rc = host_copy(s, static_cast<char*>(s->d_stage), const_cast<char*>(static_cast<const char*>(host)), bytes, true)))
+    return rc;
   launch_layout_copy(true, s->d_stage, static_cast<char*>(s->f[c]) + (size_t)(kPad - s->koff[c]) * s->esize,
                      layout_of(s, c), s->esize, s->stream);
   HIP_TRY(hipGetLastError());
@@ -3135,10 +3243,7 @@ int gmes_sim_read_field(gmes_sim* s, int32_t c, void* host, int64_t bytes) {
   HIP_TRY(hipSetDevice(s->device));
   HIP_TRY(sync_exec(s));  // steps queued on the sim's (or its batch's) stream come first
   if (dense_layout(s, c)) {
-    HIP_TRY(hipMemcpyAsync(host, static_cast<const char*>(s->f[c]) + (size_t)kPad * s->esize, (size_t)bytes,
-                           hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(sync_exec(s));
-    return GMES_OK;
+    return host_copy(s, static_cast<char*>(s->f[c]) + (size_t)kPad * s->esize, static_cast<char*>(host), bytes, false);
   }
   // rows packed on the device, then one contiguous download
   int rc = stage_reserve(s, bytes);
@@ -3146,9 +3251,7 @@ int gmes_sim_read_field(gmes_sim* s, int32_t c, void* host, int64_t bytes) {
   launch_layout_copy(false, s->d_stage, static_cast<char*>(s->f[c]) + (size_t)(kPad - s->koff[c]) * s->esize,
                      layout_of(s, c), s->esize, s->stream);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(host, s->d_stage, (size_t)bytes, hipMemcpyDeviceToHost, s->stream));
-  HIP_TRY(sync_exec(s));
-  return GMES_OK;
+  return host_copy(s, static_cast<char*>(s->d_stage), static_cast<char*>(host), bytes, false);
 }
 
 // ---- snapshot / restore
