@@ -286,12 +286,14 @@ def batched_leg(steps, warm=5, alone_steps=50, prof_steps=50):
     b.profile(False)
     b.close()
     three = [s for s in sims if len(s._active) == 6]
+    # one-sweep members: whole steps under the E families, nothing under H
+    sweep = launches[1] == 0 and launches[3] == 0
     fam = {}
     for k, name, sel, el in ((0, "e_main3d", three, True), (1, "h_main3d", three, False),
                              (2, "e_main2d", [s for s in sims if s not in three], True),
                              (3, "h_main2d", [s for s in sims if s not in three], False)):
         avg = ms[k] / max(1, launches[k])
-        nb = sum(kernel_bytes(s, el) for s in sel)
+        nb = sum(sweep_bytes(s) if sweep else kernel_bytes(s, el) for s in sel)
         fam[name] = dict(avg_launch_ms=round(avg, 5), bytes_per_launch=int(nb),
                          gbps=round(nb / (avg * 1e-3) / 1e9, 1) if avg > 0 else None)
     split = {k: round(ms[i] / max(1, launches[i]), 4) for i, k in enumerate(
@@ -299,8 +301,9 @@ def batched_leg(steps, warm=5, alone_steps=50, prof_steps=50):
     dom = max(("e_main3d", "h_main3d"), key=lambda k: fam[k]["avg_launch_ms"])
     roof = dict(bound="hbm", achieved=fam[dom]["gbps"], peak=HBM_PEAK_GBPS, unit="GB/s",
                 frac=round(fam[dom]["gbps"] / HBM_PEAK_GBPS, 4),
-                traffic=measured_traffic_batch(dom),
-                kernel="k_main3d_batch<%s, float> (%d 3-D members, one launch per profile-row kind)" % (
+                traffic=None if sweep else measured_traffic_batch(dom),
+                kernel="k_step3d_batch<float, false> (%d 3-D members)" % len(three) if sweep else
+                "k_main3d_batch<%s, float> (%d 3-D members, one launch per profile-row kind)" % (
                     "true" if dom == "e_main3d" else "false", len(three)),
                 bytes_per_launch=fam[dom]["bytes_per_launch"], avg_launch_ms=fam[dom]["avg_launch_ms"],
                 families=fam)
@@ -446,14 +449,17 @@ def served_leg(nreq, budget_gb=64.0, max_active=16, chunk=250, policy="shortest"
     b.close()
     fam = 0 if ms[0] >= ms[1] else 1
     avg = ms[fam] / max(1, launches[fam])
-    nb = sum(kernel_bytes(sm, fam == 0) for sm in sims)
+    sweep = launches[1] == 0
+    nb = sum(sweep_bytes(sm) if sweep else kernel_bytes(sm, fam == 0) for sm in sims)
     for sm in sims:
         sm.close()
     gbps = nb / (avg * 1e-3) / 1e9
     roof = dict(bound="hbm", achieved=round(gbps, 1), peak=HBM_PEAK_GBPS, unit="GB/s",
                 frac=round(gbps / HBM_PEAK_GBPS, 4), traffic=None,
-                kernel="k_main3d_batch<%s, cplx<float>> on the stream's first 16 slabs (sides %s)"
-                       % ("true" if fam == 0 else "false", sorted(r.side for r in sample)),
+                kernel="%s on the stream's first 16 slabs (sides %s)"
+                       % ("k_step3d_batch<cplx<float>>" if sweep else
+                          "k_main3d_batch<%s, cplx<float>>" % ("true" if fam == 0 else "false"),
+                          sorted(r.side for r in sample)),
                 bytes_per_launch=int(nb), avg_launch_ms=round(avg, 5))
     log("served: %d requests (%d ok) in %.1f s, p50 %.2f s p99 %.2f s, %.1f Mcell/s, peak active %d; "
         "stream %.0f GB/s algorithmic; batch-16 main kernel %.0f GB/s"
@@ -592,7 +598,7 @@ def main():
     roofline = dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK_GBPS, unit="GB/s",
                     frac=round(achieved / HBM_PEAK_GBPS, 4),
                     traffic=measured_traffic(n, "step" if sweep else "E" if fam == 0 else "H"),
-                    kernel="k_step3d<float, 1, false>" if sweep else
+                    kernel="k_step3d<float, 4, false>" if sweep else
                     "k_main3d<%s, float, 1, false, true, true, false>" % ("true" if fam == 0 else "false"),
                     bytes_per_launch=int(nbytes), avg_launch_ms=round(avg_ms, 5),
                     other_kernel_gbps=other_gbps)

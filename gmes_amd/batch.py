@@ -2,13 +2,13 @@
 
 A ``Batch`` groups initialised FDTD objects of one precision and field type
 (real or complex).  Each keeps its own fields, materials, sources, probes
-and clock; a step of the batch runs the main, source and ghost kernels of
-every member as one launch each (the engine maps blocks to members through
-a device job table) and is replayed from one captured HIP graph.  Members
-may differ in size, mode and materials.  The batched main launches of 3-D
-and collapsed-z members run flat blocks of 256 consecutive cells, so they
-need no tile; autotune=True still tunes each 3-D member's tile for its own
-launches (when it is stepped alone).
+and clock; a step of the batch runs the members' kernels of one kind as one
+launch (the engine maps blocks to members through a device job table) and
+is replayed from one captured HIP graph.  Members may differ in size, mode
+and materials.  Members whose own step is a one-sweep step take it here too;
+the others run main, source and ghost kernels, whose main launches use flat
+blocks of 256 consecutive cells and need no tile; autotune=True still tunes
+each 3-D member's tile for its own launches (when it is stepped alone).
 
 This has no counterpart in the reference, which advances one FDTD at a
 time (gmes/fdtd.py:1099-1122); every member computes exactly what it would
@@ -67,7 +67,7 @@ class Batch(object):
 
     def read_profile(self):
         """(ms, launches) per family: E 3-D main, H 3-D main, E 2-D main,
-        H 2-D main, dispersive, the rest."""
+        H 2-D main, dispersive, the rest.  One-sweep steps count under E."""
         return self._lib.batch_read_profile(self._b)
 
     def close(self):

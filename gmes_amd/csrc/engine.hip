@@ -1136,6 +1136,49 @@ void sweep_quiet(const gmes_sim* s, int a, int n, int& lo, int& hi) {
   }
 }
 
+void sweep_rect(gmes_sim::SweepPart& part, int i0, int i1, int j0, int j1, int most, int kind) {
+  if (i0 >= i1 || j0 >= j1) return;
+  const int len = i1 - i0, n = (len + most - 1) / most;
+  const int r[6] = {i0, i1, j0, j1, (len + n - 1) / n, kind};
+  std::copy(r, r + 6, part.rect[part.nrect++]);
+}
+
+// Blocks by their CPML words; [ia, ib) x [ja, jb) has none along x and y.
+void sweep_rects(gmes_sim::SweepPart& part, int nx, int ny, int ia, int ib, int ja, int jb, int out, int in) {
+  const int xs[4] = {0, ia, ib, nx}, ys[4] = {0, ja, jb, ny};
+  for (int x : {0, 2})
+    for (int y : {0, 2}) sweep_rect(part, xs[x], xs[x + 1], ys[y], ys[y + 1], out, kPmlXYZ);
+  for (int x : {0, 2}) sweep_rect(part, xs[x], xs[x + 1], ja, jb, out, kPmlXZ);
+  for (int y : {0, 2}) sweep_rect(part, ia, ib, ys[y], ys[y + 1], out, kPmlYZ);
+  sweep_rect(part, ia, ib, ja, jb, in, kPmlZ);
+}
+
+// The shape of a member of a batch: blocks of one size for all, and at most ch
+// planes.  lean: as step3_batch_threads has it.
+bool sweep_lean(const gmes_sim* s, int& ia, int& ib, int& ja, int& jb) {
+  ia = ib = ja = jb = 0;
+  if (s->sweep_absorber == kPmlXYZ) {
+    sweep_quiet(s, 0, s->g.nx, ia, ib);
+    sweep_quiet(s, 1, s->g.ny, ja, jb);
+  }
+  return s->sweep_absorber == kPmlNone || (ib - ia == s->g.nx && jb - ja == s->g.ny);
+}
+
+bool sweep_batch_part(const gmes_sim* s, gmes_sim::SweepPart& part, bool& lean, int ch) {
+  const int nx = s->g.nx, ny = s->g.ny, nz = s->g.nz;
+  int ia, ib, ja, jb;
+  lean = sweep_lean(s, ia, ib, ja, jb);
+  part = gmes_sim::SweepPart{};
+  part.threads = s->esize == 8 ? step3_batch_threads<double>(lean) : step3_batch_threads<float>(lean);
+  part.rows = std::min(part.threads / nz, ny + 1);
+  if (kSweepMinRows * nz > part.threads || part.rows < 2) return false;
+  part.absorber = s->sweep_absorber;
+  if (lean) sweep_rect(part, 0, nx, 0, ny, ch, s->sweep_absorber ? kPmlZ : kPmlNone);
+  else if (ib > ia && jb > ja) sweep_rects(part, nx, ny, ia, ib, ja, jb, std::min(ch, kSweepOuterPlanes), ch);
+  else sweep_rect(part, 0, nx, 0, ny, ch, s->sweep_absorber);
+  return true;
+}
+
 template <class T>
 void sweep_plan_t(gmes_sim* s, int nent) {
   const int nx = s->g.nx, ny = s->g.ny;
@@ -1152,23 +1195,11 @@ void sweep_plan_t(gmes_sim* s, int nent) {
     part.rows = 0;
     return;
   }
-  auto rect = [&](int i0, int i1, int j0, int j1, int most, int k) {
-    if (i0 >= i1 || j0 >= j1) return;
-    const int len = i1 - i0, n = (len + most - 1) / most;
-    const int r[6] = {i0, i1, j0, j1, (len + n - 1) / n, k};
-    std::copy(r, r + 6, part.rect[part.nrect++]);
-  };
   if (kind != kPmlMixed) {
-    rect(0, nx, 0, ny, ch, kind);
+    sweep_rect(part, 0, nx, 0, ny, ch, kind);
     return;
   }
-  const int xs[4] = {0, ia, ib, nx}, ys[4] = {0, ja, jb, ny};
-  const int cho = kSweepOuterPlanes;
-  for (int x : {0, 2})
-    for (int y : {0, 2}) rect(xs[x], xs[x + 1], ys[y], ys[y + 1], cho, kPmlXYZ);
-  for (int x : {0, 2}) rect(xs[x], xs[x + 1], ja, jb, cho, kPmlXZ);
-  for (int y : {0, 2}) rect(ia, ib, ys[y], ys[y + 1], cho, kPmlYZ);
-  rect(ia, ib, ja, jb, kSweepInnerPlanes, kPmlZ);
+  sweep_rects(part, nx, ny, ia, ib, ja, jb, kSweepOuterPlanes, kSweepInnerPlanes);
 }
 
 void sweep_plan(gmes_sim* s) {
@@ -2012,7 +2043,7 @@ bool sweep_ghosts(const gmes_sim* s) {
 }
 
 template <class T>
-Step3Args<T> step3_args(const gmes_sim* s) {
+Step3Args<T> step3_args(const gmes_sim* s, const gmes_sim::SweepPart& part) {
   using R = typename real_of<T>::type;
   Step3Args<T> m{};
   auto rsrc = [](const void* p, int64_t bytes) {
@@ -2062,7 +2093,6 @@ Step3Args<T> step3_args(const gmes_sim* s) {
     m.run_e[a] = s->sweep_run_e[a];
     m.run_h[a] = s->sweep_run_h[a];
   }
-  const gmes_sim::SweepPart& part = s->sweep_part;
   m.rows = part.rows;
   m.nrect = part.nrect;
   for (int q = 0; q < part.nrect; ++q) {
@@ -2097,7 +2127,7 @@ void enqueue_sweep(gmes_sim* s, hipStream_t st) {
   } else if (s->sweep_2d) {
     launch_step2d<T>(step2_args<T>(s), step2_tm(s), s->sweep_absorber, step2_ade(s), st);
   } else if constexpr (!std::is_same<T, cplx<double>>::value) {
-    launch_step3d<T>(step3_args<T>(s), s->sweep_part.absorber, s->sweep_part.threads, st);
+    launch_step3d<T>(step3_args<T>(s, s->sweep_part), s->sweep_part.absorber, s->sweep_part.threads, st);
   }
   time_end(s, st);
   sweep_swap(s);
@@ -3588,7 +3618,15 @@ struct gmes_batch {
     Launch ade[GMES_NCLS];                                      // by dispersive class
     Launch dft;
   };
-  JobSet set;                      // the members
+  // one-sweep members: the launches of a step, for the first and second step
+  // of a call (their buffers swap), then the same writing the ghost planes
+  struct SweepSet {
+    Launch s3[4], s2, s1, aux, fix_e, fix_h, ghost, dft;  // s3: exact divisions (1), lean (2)
+    size_t lds3[4] = {}, lds2 = 0;
+  };
+  SweepSet sweep[4];
+  std::vector<gmes_sim*> sweepers, others;
+  JobSet set;                      // the other members
   JobSet aux_set;                  // their auxiliary (TFSF) grids, stepped inside the members' step
   std::vector<gmes_sim*> aux_sims;
   std::vector<int64_t> shape_sig;  // launch shapes the graph was captured with
@@ -3714,8 +3752,149 @@ const J* job_ptr(const gmes_batch* b, size_t off) {
   return reinterpret_cast<const J*>(static_cast<const char*>(b->d_jobs) + off);
 }
 
+// Whether a member takes one-sweep steps in a batch.
+bool batch_sweeps(const gmes_sim* s) {
+  if (!sweeps(s)) return false;
+  for (int i = 0; i < s->naux; ++i)
+    if (s->aux[i] && !aux_sweeps(s->aux[i])) return false;
+  gmes_sim::SweepPart part;
+  bool lean;
+  return s->sweep_1d || s->sweep_2d || sweep_batch_part(s, part, lean, kSweepInnerPlanes);
+}
+
+// A member's buffers, and those of its auxiliary grids, become the other set.
+void sweep_swap_aux(gmes_sim* s) {
+  for (int i = 0; i < s->naux; ++i)
+    if (s->aux[i]) sweep_swap(s->aux[i]);
+}
+
+// Planes (rows) per block of a batch's one-sweep members, from its tiles times
+// planes (rows).  As in sweep2_shape, fewer while they fill the chip badly (us
+// per step at 3, 5, 7, 9, 16 planes: 476 tile planes 36, 43, 48, 54, 63; 2199
+// 79, 89, 83, 93, 115; 4315 99, 99, 103, 111, 118; 12303 224, 217, 217, 223,
+// 237; at 1, 2, 3, 5 rows: 965 tile rows 107, 108, 111, 115; 5852 274, 266,
+// 264, 266).
+int batch_ch3(double work) { return std::max(3, std::min(9, (int)std::lround(std::sqrt(work / 300)))); }
+int batch_ch2(double work) { return std::max(1, std::min(5, (int)std::ceil(std::sqrt(work / 1500)))); }
+
+// Job tables of the one-sweep members.  The arguments of a step are taken
+// from the sims as that step finds them: the host's pointers are swapped
+// twice on the way and end where they were.
+template <class T>
+void build_sweep_jobs(gmes_batch* b) {
+  std::vector<Step3Job<T>> j3[2][4];
+  std::vector<Step2Job<T>> j2[2];
+  std::vector<Step1Job<T>> j1[2], ja;
+  // planes (rows in 2-D) per block: a few rounds of blocks over the chip
+  double work3 = 0, work2 = 0;
+  for (const gmes_sim* s : b->sweepers) {
+    if (s->sweep_2d) work2 += (double)s->g.nx * ((s->g.ny + 255) / 256);
+    else if (!s->sweep_1d) work3 += (double)s->g.nx * s->g.ny / std::max(1, 768 / s->g.nz - 1);
+  }
+  const int ch3 = batch_ch3(work3), ch2 = batch_ch2(work2);
+  for (int t = 0; t < 2; ++t) {
+    std::vector<FixJob<T>> je, jh;
+    std::vector<GhostJob<T>> jg[2];
+    std::vector<DftJob<T>> jd;
+    int64_t n3[4] = {}, n2 = 0, n1 = 0, na = 0, ne = 0, nh = 0, ng[2] = {0, 0}, nd = 0;
+    size_t lds3[4] = {}, lds2 = 0;
+    for (int g = 0; g < 2; ++g) {
+      for (auto& v : j3[g]) v.clear();
+      j2[g].clear();
+      j1[g].clear();
+    }
+    ja.clear();
+    for (gmes_sim* s : b->sweepers) {
+      const bool always = sweep_ghosts(s);
+      for (int g = 0; g < 2; ++g) {
+        s->sweep_ghosts = always || g;
+        if (s->sweep_1d) {
+          Step1Job<T> J{step1_args<T>(s), n1};
+          if (g) n1 += (J.a.n + kStep1Threads - 2) / (kStep1Threads - 1);
+          j1[g].push_back(J);
+        } else if (s->sweep_2d) {
+          Step2Job<T> J{step2_args<T>(s), step2_tm(s), s->sweep_absorber, n2};
+          // blocks of kStep2BatchThreads threads, a few rows each
+          J.a.whole = J.a.n[1] <= kStep2BatchThreads;
+          J.a.w = J.a.whole ? J.a.n[1] : 224;
+          J.a.ch = std::min(ch2, J.a.n[0]);
+          J.a.nj = (J.a.n[1] + J.a.w - 1) / J.a.w;
+          J.a.nblk = J.a.nj * ((J.a.n[0] + J.a.ch - 1) / J.a.ch);
+          if (g) n2 += (J.a.nblk + 7) / 8 * 8;
+          lds2 = std::max(lds2, step2_lds<T>(kStep2BatchThreads, J.a.nent));
+          j2[g].push_back(J);
+        } else if constexpr (!std::is_same<T, cplx<double>>::value) {
+          gmes_sim::SweepPart part;
+          bool lean;
+          (void)sweep_batch_part(s, part, lean, ch3);
+          Step3Job<T> J{step3_args<T>(s, part), 0};
+          const int x = (std::is_same<T, double>::value && J.a.exact) + 2 * lean;
+          J.block0 = n3[x];
+          if (g) n3[x] += 8 * (int64_t)J.a.slots;
+          lds3[x] = std::max(lds3[x], step3_lds<T>(part.threads, J.a.net + J.a.nht, part.rows, s->g.nz, s->sweep_absorber));
+          j3[g][x].push_back(J);
+        }
+      }
+      sweep_swap(s);
+      if constexpr (!std::is_same<T, cplx<double>>::value) {
+        if (s->sweep_fix && !s->sweep_1d && !s->sweep_2d) {
+          FixJob<T> F{fix_args<T>(s), ne};
+          ne += F.a.eblocks;
+          if (F.a.eblocks) je.push_back(F);
+          for (int i = 0; i < s->naux; ++i) {
+            if (!s->aux[i]) continue;
+            Step1Job<T> A{step1_args<T>(s->aux[i]), na};
+            na += (A.a.n + kStep1Threads - 2) / (kStep1Threads - 1);
+            ja.push_back(A);
+          }
+          sweep_swap_aux(s);
+          FixJob<T> H{fix_args<T>(s), nh};
+          nh += H.a.hblocks;
+          if (H.a.hblocks) jh.push_back(H);
+          for (int g = 0; g < 2; ++g) {
+            if (!always && !g) continue;
+            GhostJob<T> G{};
+            int64_t total = 0;
+            G.g = ghost_args<T>(s, true, 0, total);
+            G.block0 = ng[g];
+            ng[g] += std::max<int64_t>(1, (total + 255) / 256);
+            jg[g].push_back(G);
+          }
+        }
+      }
+      dft_jobs<T>(s, jd, nd);
+    }
+    auto put = [&](const auto& v, int64_t blocks) {
+      using J = typename std::decay<decltype(v[0])>::type;
+      return gmes_batch::Launch{append_table(b->h_jobs, v.data(), v.size() * sizeof(J)), (int)v.size(), blocks};
+    };
+    for (int g = 0; g < 2; ++g) {
+      gmes_batch::SweepSet& S = b->sweep[t + 2 * g];
+      for (int x = 0; x < 4; ++x) {
+        S.s3[x] = put(j3[g][x], n3[x]);
+        S.lds3[x] = lds3[x];
+      }
+      S.s2 = put(j2[g], n2);
+      S.s1 = put(j1[g], n1);
+      S.aux = put(ja, na);
+      S.fix_e = put(je, ne);
+      S.fix_h = put(jh, nh);
+      S.ghost = put(jg[g], ng[g]);
+      S.dft = put(jd, nd);
+      S.lds2 = lds2;
+    }
+  }
+}
+
 // One step of a group of sims (the members, or their auxiliary grids)
 // with one launch per kernel kind.
+template <class T>
+void build_tables(gmes_batch* b) {
+  build_sweep_jobs<T>(b);
+  build_jobs<T>(b, b->others, b->set);
+  build_jobs<T>(b, b->aux_sims, b->aux_set);
+}
+
 // HIP events around the launches of one kernel family of a batch step
 // (members only; the auxiliary grids count as "the rest").
 void btime_begin(gmes_batch* b, bool on, int fam, hipStream_t st) {
@@ -3784,19 +3963,54 @@ void enqueue_set_step_t(gmes_batch* b, const gmes_batch::JobSet& js, const std::
   btime_end(b, tm, st);
 }
 
-// One step of every member, in the single-sim order, with the main, source
-// and ghost kernels of all members batched into one launch each.
+// One step of the one-sweep members, in the order of their own step.
 template <class T>
-void enqueue_batch_step_t(gmes_batch* b, hipStream_t st) {
-  enqueue_set_step_t<T>(b, b->set, b->sims, true, st);
+void enqueue_sweep_set(gmes_batch* b, int variant, hipStream_t st) {
+  const gmes_batch::SweepSet& S = b->sweep[variant];
+  if constexpr (!std::is_same<T, cplx<double>>::value) {
+    btime_begin(b, true, 0, st);
+    for (int x = 0; x < 4; ++x)
+      launch_step3d_batch<T>(job_ptr<Step3Job<T>>(b, S.s3[x].off), S.s3[x].njobs, S.s3[x].nblocks, x & 1, x & 2,
+                             S.lds3[x], st);
+    btime_end(b, true, st);
+  }
+  btime_begin(b, true, 2, st);
+  launch_step2d_batch<T>(job_ptr<Step2Job<T>>(b, S.s2.off), S.s2.njobs, S.s2.nblocks, S.lds2, st);
+  launch_step1d_batch<T>(job_ptr<Step1Job<T>>(b, S.s1.off), S.s1.njobs, S.s1.nblocks, st);
+  btime_end(b, true, st);
+  for (gmes_sim* s : b->sweepers) sweep_swap(s);
+  btime_begin(b, true, 4, st);
+  if constexpr (!std::is_same<T, cplx<double>>::value)
+    launch_fix_batch<T>(true, job_ptr<FixJob<T>>(b, S.fix_e.off), S.fix_e.njobs, S.fix_e.nblocks, st);
+  btime_end(b, true, st);
+  btime_begin(b, true, 5, st);
+  for (gmes_sim* s : b->sweepers) enqueue_probe<T>(s, true, st);
+  launch_step1d_batch<T>(job_ptr<Step1Job<T>>(b, S.aux.off), S.aux.njobs, S.aux.nblocks, st);
+  for (gmes_sim* s : b->sweepers) sweep_swap_aux(s);
+  if (S.ghost.njobs)
+    launch_ghost_batch<T>(job_ptr<GhostJob<T>>(b, S.ghost.off), S.ghost.njobs, S.ghost.nblocks, 0, st);
+  if constexpr (!std::is_same<T, cplx<double>>::value)
+    launch_fix_batch<T>(false, job_ptr<FixJob<T>>(b, S.fix_h.off), S.fix_h.njobs, S.fix_h.nblocks, st);
+  for (gmes_sim* s : b->sweepers) enqueue_probe<T>(s, false, st);
+  if (S.dft.njobs) launch_dft_batch<T>(job_ptr<DftJob<T>>(b, S.dft.off), S.dft.njobs, S.dft.nblocks, st);
+  btime_end(b, true, st);
 }
 
-void enqueue_batch_step(gmes_batch* b, hipStream_t st) {
+// One step of every member, in the single-sim order, with the kernels of all
+// members batched into one launch of each kind.  variant: which tables of the
+// one-sweep members (gmes_batch::sweep).
+template <class T>
+void enqueue_batch_step_t(gmes_batch* b, int variant, hipStream_t st) {
+  if (!b->sweepers.empty()) enqueue_sweep_set<T>(b, variant, st);
+  if (!b->others.empty()) enqueue_set_step_t<T>(b, b->set, b->others, true, st);
+}
+
+void enqueue_batch_step(gmes_batch* b, int variant, hipStream_t st) {
   switch (b->dtype) {
-    case GMES_F32: enqueue_batch_step_t<float>(b, st); break;
-    case GMES_F64: enqueue_batch_step_t<double>(b, st); break;
-    case GMES_C64: enqueue_batch_step_t<cplx<float>>(b, st); break;
-    default: enqueue_batch_step_t<cplx<double>>(b, st); break;
+    case GMES_F32: enqueue_batch_step_t<float>(b, variant, st); break;
+    case GMES_F64: enqueue_batch_step_t<double>(b, variant, st); break;
+    case GMES_C64: enqueue_batch_step_t<cplx<float>>(b, variant, st); break;
+    default: enqueue_batch_step_t<cplx<double>>(b, variant, st); break;
   }
 }
 
@@ -3886,31 +4100,33 @@ int gmes_batch_step(gmes_batch* b, int64_t nsteps) {
     int rc = check_windows(s, nsteps);
     if (rc) return rc;
     if ((rc = ensure_probe_capacity(s, nsteps))) return rc;
+  }
+  if (nsteps == 0) return GMES_OK;
+  b->sweepers.clear();
+  b->others.clear();
+  for (gmes_sim* s : b->sims) {
+    const bool sweep = batch_sweeps(s);
     HIP_TRY(hipSetDevice(b->device));
-    if ((rc = aux_pointers(s))) return rc;
-    sweep_clock(s, false, b->stream);
+    if (!sweep)
+      if (int rc = aux_pointers(s)) return rc;
+    sweep_clock(s, sweep, b->stream);
     for (int i = 0; i < s->naux; ++i)
-      if (s->aux[i]) sweep_clock(s->aux[i], false, b->stream);
+      if (s->aux[i]) sweep_clock(s->aux[i], sweep, b->stream);
+    (sweep ? b->sweepers : b->others).push_back(s);
   }
   HIP_TRY(hipSetDevice(b->device));
   // the job tables are read by kernels still in flight: wait before rewriting
   HIP_TRY(hipStreamSynchronize(b->stream));
   b->aux_sims.clear();
-  for (gmes_sim* s : b->sims)
+  for (gmes_sim* s : b->others)
     for (int i = 0; i < s->naux; ++i)
       if (s->aux[i]) b->aux_sims.push_back(s->aux[i]);
   b->h_jobs.clear();
   switch (b->dtype) {
-    case GMES_F32: build_jobs<float>(b, b->sims, b->set); build_jobs<float>(b, b->aux_sims, b->aux_set); break;
-    case GMES_F64: build_jobs<double>(b, b->sims, b->set); build_jobs<double>(b, b->aux_sims, b->aux_set); break;
-    case GMES_C64:
-      build_jobs<cplx<float>>(b, b->sims, b->set);
-      build_jobs<cplx<float>>(b, b->aux_sims, b->aux_set);
-      break;
-    default:
-      build_jobs<cplx<double>>(b, b->sims, b->set);
-      build_jobs<cplx<double>>(b, b->aux_sims, b->aux_set);
-      break;
+    case GMES_F32: build_tables<float>(b); break;
+    case GMES_F64: build_tables<double>(b); break;
+    case GMES_C64: build_tables<cplx<float>>(b); break;
+    default: build_tables<cplx<double>>(b); break;
   }
   if (b->h_jobs.size() > b->jobs_cap) {
     destroy_batch_graph(b);
@@ -3941,6 +4157,15 @@ int gmes_batch_step(gmes_batch* b, int64_t nsteps) {
     sig.push_back(js->dft.njobs);
     sig.push_back(js->dft.nblocks);
   }
+  for (const gmes_batch::SweepSet& S : b->sweep) {
+    for (const auto* L : {&S.s3[0], &S.s3[1], &S.s3[2], &S.s3[3], &S.s2, &S.s1, &S.aux, &S.fix_e, &S.fix_h, &S.ghost, &S.dft}) {
+      sig.push_back((int64_t)L->off);
+      sig.push_back(L->njobs);
+      sig.push_back(L->nblocks);
+    }
+    for (const size_t l : S.lds3) sig.push_back((int64_t)l);
+    sig.push_back((int64_t)S.lds2);
+  }
   std::vector<uint64_t> gens;
   for (gmes_sim* s : b->sims) {
     gens.push_back(s->gen);
@@ -3950,24 +4175,29 @@ int gmes_batch_step(gmes_batch* b, int64_t nsteps) {
   if (sig != b->shape_sig || gens != b->gens) destroy_batch_graph(b);
   b->shape_sig = sig;
   b->gens = gens;
-  if (b->use_graph && !b->timing.on) {
+  // one-sweep members swap buffers: their graph holds two steps, and the last
+  // step, which writes the ghost planes, is launched by itself
+  const int per = b->sweepers.empty() ? 1 : 2, last = per - 1;
+  int64_t t = 0;
+  if (b->use_graph && !b->timing.on && nsteps >= per + last) {
     if (!b->graph_exec) {
       hipGraph_t graph;
       {
         CaptureGuard capture;
         HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-        enqueue_batch_step(b, b->stream);
+        for (int k = 0; k < per; ++k) enqueue_batch_step(b, k, b->stream);
         HIP_TRY(hipStreamEndCapture(b->stream, &graph));
       }
       hipError_t e = hipGraphInstantiate(&b->graph_exec, graph, nullptr, nullptr, 0);
       (void)hipGraphDestroy(graph);
       if (e != hipSuccess) return set_error(GMES_EDEVICE, "hipGraphInstantiate: %s", hipGetErrorString(e));
     }
-    for (int64_t t = 0; t < nsteps; ++t) HIP_TRY(hipGraphLaunch(b->graph_exec, b->stream));
-  } else {
-    for (int64_t t = 0; t < nsteps; ++t) enqueue_batch_step(b, b->stream);
-    HIP_TRY(hipGetLastError());
+    for (; t + per + last <= nsteps; t += per) HIP_TRY(hipGraphLaunch(b->graph_exec, b->stream));
   }
+  for (; t < nsteps; ++t) enqueue_batch_step(b, (int)(t & 1) + (t == nsteps - 1 ? 2 : 0), b->stream);
+  HIP_TRY(hipGetLastError());
+  if (nsteps & 1)
+    for (gmes_sim* s : b->sweepers) ++s->gen;  // captured arguments hold the other set's pointers
   for (gmes_sim* s : b->sims) advance_host_clock(s, nsteps);
   return GMES_OK;
 }

@@ -325,6 +325,26 @@ constexpr int kStep1Threads = 256;
 template <class T>
 void launch_step1d(const Step1Args<T>& m, hipStream_t st);
 
+// Batched one-sweep launches: job tables as those below.  3-D and 2-D jobs start
+// at a multiple of 8 blocks (their blocks go round the XCDs).
+template <class T> struct Step3Job { Step3Args<T> a; int64_t block0; };
+template <class T> struct Step2Job { Step2Args<T> a; int tm, absorber; int64_t block0; };
+template <class T> struct Step1Job { Step1Args<T> a; int64_t block0; };
+template <class T> struct FixJob { FixArgs<T> a; int64_t block0; };
+constexpr int kStep2BatchThreads = 256;
+// lean: jobs without CPML words along x and y and without UPML, whose 8-byte
+// bodies fit 128 registers
+template <class T> constexpr int step3_batch_threads(bool lean) { return sizeof(T) == 8 && lean ? 1024 : 768; }
+template <class T>
+void launch_step3d_batch(const Step3Job<T>* jobs, int njobs, int64_t nblocks, bool exact, bool lean, size_t lds,
+                         hipStream_t st);
+template <class T>
+void launch_step2d_batch(const Step2Job<T>* jobs, int njobs, int64_t nblocks, size_t lds, hipStream_t st);
+template <class T>
+void launch_step1d_batch(const Step1Job<T>* jobs, int njobs, int64_t nblocks, hipStream_t st);
+template <class T>
+void launch_fix_batch(bool electric, const FixJob<T>* jobs, int njobs, int64_t nblocks, hipStream_t st);
+
 // The entry ids of a sim, looked up from its material ids on the device.
 struct StepKey {
   uint64_t key, id;  // key ~0: empty slot

@@ -472,6 +472,29 @@ __global__ void __launch_bounds__(kStep2Threads<T>) k_step2d(Step2Args<T>) {
   step2d_tile<T, TM, PML, ADE, X>((Step2Ptr<T>)__builtin_amdgcn_kernarg_segment_ptr(), blockIdx.x, step2_lds_mem);
 }
 
+// Every member in one launch, by its mode and absorber.
+template <class T>
+__global__ void __launch_bounds__(kStep2BatchThreads) k_step2d_batch(const Step2Job<T>* jobs, int njobs) {
+  extern __shared__ __attribute__((aligned(16))) char step2_lds_mem[];
+  const GMES_CONST Step2Job<T>* J = step_job(jobs, njobs, (int64_t)blockIdx.x);
+  const Step2Ptr<T> m = &J->a;
+  const unsigned blk = (unsigned)((int64_t)blockIdx.x - J->block0);
+  const int kind = J->tm * 3 + J->absorber;
+  if (kind == 0) step2d_tile<T, false, 0, true, false>(m, blk, step2_lds_mem);
+  else if (kind == 1) step2d_tile<T, false, 1, true, false>(m, blk, step2_lds_mem);
+  else if (kind == 2) step2d_tile<T, false, 2, true, false>(m, blk, step2_lds_mem);
+  else if (kind == 3) step2d_tile<T, true, 0, true, false>(m, blk, step2_lds_mem);
+  else if (kind == 4) step2d_tile<T, true, 1, true, false>(m, blk, step2_lds_mem);
+  else step2d_tile<T, true, 2, true, false>(m, blk, step2_lds_mem);
+}
+
+template <class T>
+void launch_step2d_batch(const Step2Job<T>* jobs, int njobs, int64_t nblocks, size_t lds, hipStream_t st) {
+  if (njobs)
+    hipLaunchKernelGGL((k_step2d_batch<T>), dim3((unsigned)nblocks), dim3(kStep2BatchThreads), (unsigned)lds, st, jobs, njobs);
+}
+template void launch_step2d_batch<step2_t>(const Step2Job<step2_t>*, int, int64_t, size_t, hipStream_t);
+
 template <class T, bool TM, int PML, bool ADE>
 static void launch_step2d_x(const Step2Args<T>& m, hipStream_t st) {
   const dim3 grid(((unsigned)m.nblk + 7u) / 8u * 8u), block(step2_threads(m.w, m.whole));

@@ -781,6 +781,59 @@ __global__ void k_clock_copy(Ctl* ctl) { ctl->clk[0] = ctl->clk[1] = ctl->clock;
 
 void launch_clock_copy(Ctl* ctl, hipStream_t st) { hipLaunchKernelGGL(k_clock_copy, dim3(1), dim3(1), 0, st, ctl); }
 
+// Every block of every member, by its own kind; blocks of one size.  LEAN: see
+// step3_batch_threads (in the kernel of all kinds, complex FP32 slabs with z
+// layers run at 12 waves a CU, and no faster than two batched launches).  us
+// per step, two launches each for E and H before: 8 2-D and 6 3-D FP32 members
+// of 128 to 640 and 64 to 160 cells a side 329 -> 259 (3-D 243 -> 216); 8
+// complex FP32 slabs of 64 to 206 with plane waves 970 -> 855; 4 FP64 CPML
+// boxes of 64 to 128 274 -> 187.
+template <class T, bool X, bool LEAN>
+__global__ void __launch_bounds__(step3_batch_threads<T>(LEAN))
+    __attribute__((amdgpu_waves_per_eu(StepWaves<T, LEAN ? kPmlZ : kPmlMixed>::v))) k_step3d_batch(const Step3Job<T>* jobs, int njobs) {
+  extern __shared__ __attribute__((aligned(16))) char step_lds[];
+  const GMES_CONST Step3Job<T>* J = step_job(jobs, njobs, (int64_t)blockIdx.x);
+  const StepPtr<T> m = &J->a;
+  const unsigned blk = (unsigned)((int64_t)blockIdx.x - J->block0);
+  int rc;
+  unsigned rb;
+  (void)step3d_block<T>(m, blk, rc, rb);
+  const int kind = m->rect[rc].kind;
+  if constexpr (LEAN) {
+    if (kind == kPmlZ) step3d_tile<T, kPmlZ, X>(m, blk, step_lds);
+    else step3d_tile<T, kPmlNone, X>(m, blk, step_lds);
+  } else {
+    if (kind == kPmlZ) step3d_tile<T, kPmlZ, X>(m, blk, step_lds);
+    else if (kind == kPmlXZ) step3d_tile<T, kPmlXZ, X>(m, blk, step_lds);
+    else if (kind == kPmlYZ) step3d_tile<T, kPmlYZ, X>(m, blk, step_lds);
+    else if (kind == kPmlXYZ) step3d_tile<T, kPmlXYZ, X>(m, blk, step_lds);
+    else step3d_tile<T, kUpml, X>(m, blk, step_lds);
+  }
+}
+
+template <class T>
+void launch_step3d_batch(const Step3Job<T>* jobs, int njobs, int64_t nblocks, bool exact, bool lean, size_t lds,
+                         hipStream_t st) {
+  if (!njobs) return;
+  const dim3 grid((unsigned)nblocks), block(step3_batch_threads<T>(lean));
+#define GMES_BATCH3(X)                                                                                          \
+  {                                                                                                             \
+    if (lean) hipLaunchKernelGGL((k_step3d_batch<T, X, true>), grid, block, (unsigned)lds, st, jobs, njobs);    \
+    else hipLaunchKernelGGL((k_step3d_batch<T, X, false>), grid, block, (unsigned)lds, st, jobs, njobs);        \
+  }
+  if constexpr (std::is_same<T, double>::value) {
+    if (exact) {
+      GMES_BATCH3(true)
+      return;
+    }
+  }
+  GMES_BATCH3(false)
+#undef GMES_BATCH3
+}
+template void launch_step3d_batch<float>(const Step3Job<float>*, int, int64_t, bool, bool, size_t, hipStream_t);
+template void launch_step3d_batch<double>(const Step3Job<double>*, int, int64_t, bool, bool, size_t, hipStream_t);
+template void launch_step3d_batch<cplx<float>>(const Step3Job<cplx<float>>*, int, int64_t, bool, bool, size_t, hipStream_t);
+
 template <class T>
 void launch_step3d(const Step3Args<T>& m, int absorber, int nthreads, hipStream_t st) {
   const dim3 grid(8u * (unsigned)m.slots), block(nthreads);

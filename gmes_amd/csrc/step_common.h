@@ -12,6 +12,18 @@ __device__ __forceinline__ V cld(const V* p) {
   return *(const GMES_CONST V*)(uintptr_t)p;
 }
 
+// Block -> job of a batched launch, by scalar loads; the job in constant memory.
+template <class J>
+__device__ __forceinline__ const GMES_CONST J* step_job(const J* jobs, int njobs, int64_t b) {
+  int lo = 0, hi = njobs - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (cld(&jobs[mid].block0) <= b) lo = mid;
+    else hi = mid - 1;
+  }
+  return (const GMES_CONST J*)(uintptr_t)(jobs + lo);
+}
+
 // Division by a cell size or a CPML kappa.  EXACT: every divisor of the sim
 // is a power of two (kappa: 1), so multiplying by the reciprocal rounds the
 // same real number and gives the quotient's bits.

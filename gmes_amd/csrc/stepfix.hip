@@ -28,11 +28,14 @@ typedef double fix_t;
 typedef cplx<float> fix_t;
 #endif
 
+template <class T>
+using FixPtr = const GMES_CONST FixArgs<T>*;
+
 // Value of an array of one component at thread coordinates x moved by s along
 // axis a, wrapped with the ghost phase.
 template <class T, class R>
-__device__ __forceinline__ T moved(const T* f, int pi, int p, const int n[3], const int x[3], int a, int s,
-                                   const cplx<R>& ph) {
+__device__ __forceinline__ T moved(const T* f, int pi, int p, const GMES_CONST int* n, const int x[3], int a, int s,
+                                   const GMES_CONST cplx<R>& ph) {
   int y[3] = {x[0], x[1], x[2]};
   bool wrap = false;
 #pragma unroll
@@ -43,25 +46,25 @@ __device__ __forceinline__ T moved(const T* f, int pi, int p, const int n[3], co
       if (y[q] >= n[q]) { y[q] = 0; wrap = true; }
     }
   const T v = gld(f + y[0] * pi + y[1] * p + y[2]);
-  return wrap ? ghost_phase<T>(ph, v) : v;
+  return wrap ? phased<T>(ph, v) : v;
 }
 
 // The operations of a source group on value v (src_group, kernels.hip).
 template <class T>
-__device__ __forceinline__ T fix_source(const FixArgs<T>& m, const SrcGroup& grp, T v) {
+__device__ __forceinline__ T fix_source(FixPtr<T> m, const SrcGroup& grp, T v) {
   using R = typename real_of<T>::type;
-  const int64_t row = (m.ctl->clock - 1) - m.ctl->wave_step0;
+  const int64_t row = (m->ctl->clock - 1) - m->ctl->wave_step0;
   for (int o = grp.begin; o < grp.end; ++o) {
-    const DevSrcOp<R> op = m.ops[o];
+    const DevSrcOp<R> op = m->ops[o];
     if (op.kind == GMES_SRC_SET || op.kind == GMES_SRC_SUB) {
-      const double* w = m.waves + (op.wave * m.ctl->wave_n + row) * 2;
+      const double* w = m->waves + (op.wave * m->ctl->wave_n + row) * 2;
       const T wv = make_val<T>((R)w[0], (R)w[1]);
       v = op.kind == GMES_SRC_SET ? wv : vsub(v, wv);
     } else {
-      const T* aux = static_cast<const T*>(m.aux[op.aux][op.aux_comp]);
+      const T* aux = static_cast<const T*>(m->aux[op.aux][op.aux_comp]);
       T a0 = gld(aux + op.i0), a1 = gld(aux + op.i1);
       if (op.wave >= 0) {
-        const R env = (R)m.waves[(op.wave * m.ctl->wave_n + row) * 2];
+        const R env = (R)m->waves[(op.wave * m->ctl->wave_n + row) * 2];
         a0 = vscl(env, a0);
         a1 = vscl(env, a1);
       }
@@ -73,63 +76,86 @@ __device__ __forceinline__ T fix_source(const FixArgs<T>& m, const SrcGroup& grp
 }
 
 template <class T>
-__global__ void __launch_bounds__(kFixBlock) k_fix_e(FixArgs<T> m) {
+__device__ __forceinline__ void fix_e(FixPtr<T> m, int b) {
   using R = typename real_of<T>::type;
-  const int b = blockIdx.x;
-  if (b >= m.first_src) {
-    const int g = (b - m.first_src) * kFixBlock + (int)threadIdx.x;
-    if (g >= m.nge) return;
-    const SrcGroup grp = m.groups[g];
-    T* F = m.base[grp.comp] + grp.cell;
+  if (b >= m->first_src) {
+    const int g = (b - m->first_src) * kFixBlock + (int)threadIdx.x;
+    if (g >= m->nge) return;
+    const SrcGroup grp = m->groups[g];
+    T* F = m->base[grp.comp] + grp.cell;
     gst(F, fix_source<T>(m, grp, gld(F)));
     return;
   }
-  int l = m.nade - 1;
-  while (l > 0 && b < m.ade[l].first) --l;
-  const int q = (b - m.ade[l].first) * kFixBlock + (int)threadIdx.x;
-  if (q >= m.ade[l].n) return;
-  const int c = m.ade[l].comp, a1 = c == 2 ? 0 : c + 1, a2 = c == 0 ? 2 : c - 1;
-  const int flat = gld(m.ade[l].cell + q), r = flat / m.ade[l].s2, i = r / m.ade[l].s1;
-  const int x[3] = {i, r - i * m.ade[l].s1, flat - r * m.ade[l].s2};
-  const DevRec<R>* rec = m.recs + gld(m.ade[l].rec + q);
-  const int e = x[0] * m.pe[c] + x[1] * m.re[c] + x[2];
-  const T e_now = gld(m.ei[c] + e);
-  const T h2 = gld(m.hi[a2] + x[0] * m.ph[a2] + x[1] * m.rh[a2] + x[2]);
-  const T h1 = gld(m.hi[a1] + x[0] * m.ph[a1] + x[1] * m.rh[a1] + x[2]);
-  const T D1 = vsub(h2, moved<T, R>(m.hi[a2], m.ph[a2], m.rh[a2], m.n, x, a1, -1, m.phh[a2][a1]));
-  const T D2 = vsub(h1, moved<T, R>(m.hi[a1], m.ph[a1], m.rh[a1], m.n, x, a2, -1, m.phh[a1][a2]));
-  const T cu = vsub(vdiv(D1, m.d[a1]), vdiv(D2, m.d[a2]));
-  gst(m.eo[c] + e, ade_value<T>(m.ade[l].cls, m.coef + gld(&rec->coef_off), gld(&rec->n1), gld(&rec->n2),
-                                m.ade[l].state, m.ade[l].state, m.ade[l].n, q, true, e_now, cu));
+  int l = m->nade - 1;
+  while (l > 0 && b < m->ade[l].first) --l;
+  const int q = (b - m->ade[l].first) * kFixBlock + (int)threadIdx.x;
+  if (q >= m->ade[l].n) return;
+  const int c = m->ade[l].comp, a1 = c == 2 ? 0 : c + 1, a2 = c == 0 ? 2 : c - 1;
+  const int flat = gld(m->ade[l].cell + q), r = flat / m->ade[l].s2, i = r / m->ade[l].s1;
+  const int x[3] = {i, r - i * m->ade[l].s1, flat - r * m->ade[l].s2};
+  const DevRec<R>* rec = m->recs + gld(m->ade[l].rec + q);
+  const int e = x[0] * m->pe[c] + x[1] * m->re[c] + x[2];
+  const T e_now = gld(m->ei[c] + e);
+  const T h2 = gld(m->hi[a2] + x[0] * m->ph[a2] + x[1] * m->rh[a2] + x[2]);
+  const T h1 = gld(m->hi[a1] + x[0] * m->ph[a1] + x[1] * m->rh[a1] + x[2]);
+  const T D1 = vsub(h2, moved<T, R>(m->hi[a2], m->ph[a2], m->rh[a2], m->n, x, a1, -1, m->phh[a2][a1]));
+  const T D2 = vsub(h1, moved<T, R>(m->hi[a1], m->ph[a1], m->rh[a1], m->n, x, a2, -1, m->phh[a1][a2]));
+  const T cu = vsub(vdiv(D1, m->d[a1]), vdiv(D2, m->d[a2]));
+  gst(m->eo[c] + e, ade_value<T>(m->ade[l].cls, m->coef + gld(&rec->coef_off), gld(&rec->n1), gld(&rec->n2),
+                                m->ade[l].state, m->ade[l].state, m->ade[l].n, q, true, e_now, cu));
 }
 
 template <class T>
-__global__ void __launch_bounds__(kFixBlock) k_fix_h(FixArgs<T> m) {
+__device__ __forceinline__ void fix_h(FixPtr<T> m, int b) {
   using R = typename real_of<T>::type;
-  const int b = blockIdx.x;
-  const int c = b >= m.item_blk[2] ? 2 : b >= m.item_blk[1] ? 1 : 0;
-  const int q = (b - m.item_blk[c]) * kFixBlock + (int)threadIdx.x;
-  if (q >= m.nitem[c]) return;
+  const int c = b >= m->item_blk[2] ? 2 : b >= m->item_blk[1] ? 1 : 0;
+  const int q = (b - m->item_blk[c]) * kFixBlock + (int)threadIdx.x;
+  if (q >= m->nitem[c]) return;
   const int a1 = c == 2 ? 0 : c + 1, a2 = c == 0 ? 2 : c - 1;
-  const int cell = gld(&m.items[m.first_item[c] + q].cell), grp = gld(&m.items[m.first_item[c] + q].grp);
-  const int r = cell / m.n[2], i = r / m.n[1];
-  const int x[3] = {i, r - i * m.n[1], cell - r * m.n[2]};
-  const int h = x[0] * m.ph[c] + x[1] * m.rh[c] + x[2];
-  const DevRec<R>* rec = m.recs + gld(m.hid[c] + h);
-  const T old = gld(m.hi[c] + h);
-  const T* const e2 = m.eo[a2];
-  const T* const e1 = m.eo[a1];
-  const T E2 = gld(e2 + x[0] * m.pe[a2] + x[1] * m.re[a2] + x[2]), E1 = gld(e1 + x[0] * m.pe[a1] + x[1] * m.re[a1] + x[2]);
-  const T D1 = vsub(moved<T, R>(e2, m.pe[a2], m.re[a2], m.n, x, a1, 1, m.phe[a2][a1]), E2);
-  const T D2 = vsub(moved<T, R>(e1, m.pe[a1], m.re[a1], m.n, x, a2, 1, m.phe[a1][a2]), E1);
+  const int cell = gld(&m->items[m->first_item[c] + q].cell), grp = gld(&m->items[m->first_item[c] + q].grp);
+  const int r = cell / m->n[2], i = r / m->n[1];
+  const int x[3] = {i, r - i * m->n[1], cell - r * m->n[2]};
+  const int h = x[0] * m->ph[c] + x[1] * m->rh[c] + x[2];
+  const DevRec<R>* rec = m->recs + gld(m->hid[c] + h);
+  const T old = gld(m->hi[c] + h);
+  const T* const e2 = m->eo[a2];
+  const T* const e1 = m->eo[a1];
+  const T E2 = gld(e2 + x[0] * m->pe[a2] + x[1] * m->re[a2] + x[2]), E1 = gld(e1 + x[0] * m->pe[a1] + x[1] * m->re[a1] + x[2]);
+  const T D1 = vsub(moved<T, R>(e2, m->pe[a2], m->re[a2], m->n, x, a1, 1, m->phe[a2][a1]), E2);
+  const T D2 = vsub(moved<T, R>(e1, m->pe[a1], m->re[a1], m->n, x, a2, 1, m->phe[a1][a2]), E1);
   const int cls = gld(&rec->cls);
   T v = cls == GMES_CLS_DUMMY ? old
         : cls == GMES_CLS_CONST
             ? make_val<T>(gld(&rec->val_re), gld(&rec->val_im))
-            : plain_value<false, false>(gld(&rec->c0), old, D1, D2, m.d[a1], m.inv_d[a1], m.d[a2], m.inv_d[a2]);
-  if (grp >= 0) v = fix_source<T>(m, m.groups[grp], v);
-  gst(m.ho[c] + h, v);
+            : plain_value<false, false>(gld(&rec->c0), old, D1, D2, m->d[a1], m->inv_d[a1], m->d[a2], m->inv_d[a2]);
+  if (grp >= 0) v = fix_source<T>(m, m->groups[grp], v);
+  gst(m->ho[c] + h, v);
 }
+
+template <class T>
+__global__ void __launch_bounds__(kFixBlock) k_fix_e(FixArgs<T>) {
+  fix_e<T>((FixPtr<T>)__builtin_amdgcn_kernarg_segment_ptr(), (int)blockIdx.x);
+}
+template <class T>
+__global__ void __launch_bounds__(kFixBlock) k_fix_h(FixArgs<T>) {
+  fix_h<T>((FixPtr<T>)__builtin_amdgcn_kernarg_segment_ptr(), (int)blockIdx.x);
+}
+template <class T, bool E>
+__global__ void __launch_bounds__(kFixBlock) k_fix_batch(const FixJob<T>* jobs, int njobs) {
+  const GMES_CONST FixJob<T>* J = step_job(jobs, njobs, (int64_t)blockIdx.x);
+  const int b = (int)((int64_t)blockIdx.x - J->block0);
+  if constexpr (E) fix_e<T>(&J->a, b);
+  else fix_h<T>(&J->a, b);
+}
+
+template <class T>
+void launch_fix_batch(bool electric, const FixJob<T>* jobs, int njobs, int64_t nblocks, hipStream_t st) {
+  if (!njobs || !nblocks) return;
+  const dim3 grid((unsigned)nblocks), block(kFixBlock);
+  if (electric) hipLaunchKernelGGL((k_fix_batch<T, true>), grid, block, 0, st, jobs, njobs);
+  else hipLaunchKernelGGL((k_fix_batch<T, false>), grid, block, 0, st, jobs, njobs);
+}
+template void launch_fix_batch<fix_t>(bool, const FixJob<fix_t>*, int, int64_t, hipStream_t);
 
 template <class T>
 void launch_fix_e(const FixArgs<T>& a, hipStream_t st) {
