@@ -848,7 +848,8 @@ hipError_t sync_exec(gmes_sim* s);
 //     plane (it reads the plane before the copy),
 //   * with dispersive cells, an auxiliary grid or sources on more than
 //     kSweepMaxSrc cells: what stepfix.hip and sweep_fix_build ask,
-//   * a component's CPML state is under 4 GiB (32-bit byte offsets), and
+//   * a component's CPML state is under 4 GiB (32-bit byte offsets),
+//   * its second buffers leave the device half empty (sweep_room), and
 //   * the caller asked for no tile and did not turn ghost fusion off.
 // Other sims keep the two-kernel step.
 constexpr int kSweepMinRows = 3;
@@ -1243,6 +1244,23 @@ int sweep_alloc(gmes_sim* s, void** p, size_t bytes) {
   return rc;
 }
 
+// Whether the second buffers of s leave the device at least half empty: sims
+// that fill it keep the two-kernel step, and sims made later find room.
+bool sweep_room(const gmes_sim* s) {
+  int64_t need = (int64_t)s->g.nx * s->g.ny * s->g.nz * 4;
+  for (int c = 0; c < 6; ++c) {
+    if (!active(s, c)) continue;
+    need += s->dsize[c] * s->esize;
+    if (c < 3 && s->pml_state[c]) need += (s->has_cls[c][GMES_CLS_CPML] ? 2 : 1) * s->dsize[c] * s->esize;
+  }
+  size_t idle = 0, total = 0;
+  if (hipMemGetInfo(&idle, &total) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return (int64_t)idle - need >= (int64_t)(total / 2);
+}
+
 // Uploads the entry tables, those of source cells (after the step_net /
 // step_nht plain ones) included.
 template <class R>
@@ -1314,6 +1332,7 @@ int sweep1_build(gmes_sim* s) {
         if (v[q] != 0.0) return GMES_OK;
     }
   }
+  if (!sweep_room(s)) return GMES_OK;
   int rc = GMES_OK;
   for (const int c : comp) {
     if (!rc) rc = sweep_alloc(s, &s->f_alt[c], (size_t)s->dsize[c] * s->esize);
@@ -1614,6 +1633,7 @@ int sweep2_build(gmes_sim* s) {
       s->step_e.push_back({x, y, z});
     }
   }
+  if (!sweep_room(s)) return GMES_OK;
   sweep2_shape(s);
   int rc = GMES_OK;
   for (int a = 0; a < 3 && !rc; ++a) {
@@ -1986,7 +2006,7 @@ int sweep_build(gmes_sim* s) {
       s->step_e.size() + s->step_h.size() > most)
     return GMES_OK;
   sweep_plan(s);
-  if (!s->sweep_part.rows) return GMES_OK;
+  if (!s->sweep_part.rows || !sweep_room(s)) return GMES_OK;
   int rc = GMES_OK;
   for (int c = 0; c < 6 && !rc; ++c) rc = sweep_alloc(s, &s->f_alt[c], (size_t)s->dsize[c] * s->esize);
   for (int c = 0; c < 3 && !rc; ++c) {

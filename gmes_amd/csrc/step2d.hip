@@ -190,10 +190,13 @@ __device__ __forceinline__ void step2d_tile(Step2Ptr<T> mp, unsigned blk, char* 
   }
   const bool wave_live = PML != 0 && __any(lye || lyh);
 
-  auto load = [&](int q, Step2Ops<T, PML>& l) {
+  // (past the last row, and in idle lanes, the operands are left undefined:
+  // keeping the old ones instead would move registers, behind a wait)
+  auto load = [&](int q) {
+    Step2Ops<T, PML> l;
     const int qe = q == nx ? 0 : q;
     const unsigned e = (unsigned)qe * pi + (unsigned)j, o = e * S;
-    if (used) {
+    if (used && q <= i1) {
       l.f[0] = at(f0, o);
       l.f[1] = at(f1, o);
       l.f[2] = at(f2, o);
@@ -203,7 +206,7 @@ __device__ __forceinline__ void step2d_tile(Step2Ptr<T> mp, unsigned blk, char* 
 #pragma unroll
       for (int a = 0; a < 4; ++a) l.s[a] = T{};
       const bool xe = live(rune, qe), xh = PML == 1 && live(runh, qe);
-      if (wave_live || xe || xh) {
+      if (q <= i1 && (wave_live || xe || xh)) {
         const Step2Ptr<T> m = fresh2<T>(mp);
         if constexpr (PML == 1) {
           if (used && xe) l.s[0] = at(m->si[EX][0], o);
@@ -221,6 +224,7 @@ __device__ __forceinline__ void step2d_tile(Step2Ptr<T> mp, unsigned blk, char* 
         }
       }
     }
+    return l;
   };
 
   int64_t row = 0, wave_n = 0;
@@ -234,11 +238,10 @@ __device__ __forceinline__ void step2d_tile(Step2Ptr<T> mp, unsigned blk, char* 
     }
   }
 
-  Step2Ops<T, PML> l0{}, l1{};
-  load(i0, l0);
+  Step2Ops<T, PML> l0 = load(i0);
   T hi_prev = T{};  // the H of the row before that E reads
   if (used) hi_prev = at(HI == 1 ? f1 : f2, ((unsigned)(i0 ? i0 - 1 : nx - 1) * pi + (unsigned)j) * S);
-  load(i0 + 1, l1);
+  Step2Ops<T, PML> l1 = load(i0 + 1);
 
   // values of the row before: new E, old H and their entry and absorber words
   T pe[3]{}, ph[3]{}, ps[4]{};
@@ -316,12 +319,20 @@ __device__ __forceinline__ void step2d_tile(Step2Ptr<T> mp, unsigned blk, char* 
     }
   };
 
-  auto body = [&](int q, int par, Step2Ops<T, PML>& ahead) {
-    const Step2Ops<T, PML> l = ahead;
+  // The operands of a row make way for those of the row after the next, early
+  // (for more time on their way) or once the row is done with them: replaced
+  // early, in other registers, they have to be moved, and waited for, at the end
+  // of every other row.  With UPML words or dispersive cells late is better (TEz
+  // 517 x 389 FP32 UPML with dispersive rods 13.3 -> 12.4 us, 1000 x 2000 53 ->
+  // 47) and with wider words a little (2048^2 FP64 CPML 57 -> 55); else early
+  // (1200^2 FP32 CPML 14.2 against 14.7).
+  constexpr bool LATE = PML == 2 || ADE || S > 4;
+  auto body = [&](int q, int par, Step2Ops<T, PML>& next) {
+    const Step2Ops<T, PML> l = next;
     const int qe = q == nx ? 0 : q;
     xb[par * nt + t] = l.f[HJ];
     __syncthreads();
-    if (q + 2 <= i1) load(q + 2, ahead);
+    if (!LATE) next = load(q + 2);
     T hj = xb[par * nt + tl], hi = hi_prev;
     if constexpr (is_cplx<T>::value) {
       const Step2Ptr<T> m = fresh2<T>(mp);
@@ -459,11 +470,14 @@ __device__ __forceinline__ void step2d_tile(Step2Ptr<T> mp, unsigned blk, char* 
     hi_prev = l.f[HI];
     pid = l.id;
     pen = en;
+    if (LATE) next = load(q + 2);
   };
-  for (int q = i0; q <= i1; q += 2) {
+  int q = i0;
+  for (; q < i1; q += 2) {
     body(__builtin_amdgcn_readfirstlane(q), 0, l0);
-    if (q + 1 <= i1) body(__builtin_amdgcn_readfirstlane(q + 1), 1, l1);
+    body(__builtin_amdgcn_readfirstlane(q + 1), 1, l1);
   }
+  if (q == i1) body(__builtin_amdgcn_readfirstlane(q), 0, l0);
 }
 
 template <class T, bool TM, int PML, bool ADE, bool X>
