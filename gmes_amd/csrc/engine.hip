@@ -1031,7 +1031,10 @@ int sweep_ids(gmes_sim* s) {
   }
   a.n[0] = s->g.nx; a.n[1] = s->g.ny; a.n[2] = s->g.nz;
   a.pitch = s->pitch[0];
-  a.out = s->d_step_ids;
+  a.types = 2;
+  a.shift = s->step_eb;
+  if (s->step_idw == 2) a.out16 = static_cast<uint16_t*>(s->d_step_ids);
+  else a.out = static_cast<uint32_t*>(s->d_step_ids);
   const std::vector<StepKey> tab[2] = {sweep_keys(s->step_e), sweep_keys(s->step_h)};
   const size_t b0 = tab[0].size() * sizeof(StepKey), b1 = tab[1].size() * sizeof(StepKey);
   char* d = nullptr;
@@ -1214,7 +1217,7 @@ void sweep_plan(gmes_sim* s) {
 
 void sweep_release(gmes_sim* s) {
   void** bufs[] = {&s->f_alt[0], &s->f_alt[1], &s->f_alt[2], &s->f_alt[3], &s->f_alt[4], &s->f_alt[5],
-                   &s->pml_alt[0], &s->pml_alt[1], &s->pml_alt[2], (void**)&s->d_step_ids, &s->d_step_tab, (void**)&s->d_rare};
+                   &s->pml_alt[0], &s->pml_alt[1], &s->pml_alt[2], &s->d_step_ids, &s->d_step_tab, (void**)&s->d_rare};
   for (void** b : bufs)
     if (*b) {
       (void)dev_release(*b);
@@ -1523,6 +1526,7 @@ int sweep2_tables(gmes_sim* s) {
   a.mask[0] = (uint32_t)keys.size() - 1;
   a.n[0] = s->g.nx; a.n[1] = 1; a.n[2] = s->g.ny;
   a.pitch = (int)pi;
+  a.types = 1;
   a.out16 = s->step2_ids;
   launch_step_ids(a, s->stream);
   for (int c = 0; c < 3; ++c)
@@ -1911,8 +1915,9 @@ int sweep_sources(gmes_sim* s) {
   if (s->sweep_1d) return sweep1_sources(s);
   if (s->sweep_2d) return sweep2_sources(s);
   HIP_TRY(sync_exec(s));
-  for (const auto& x : s->src_ids)
-    HIP_TRY(hipMemcpy(s->d_step_ids + x.first, &x.second, sizeof(uint32_t), hipMemcpyHostToDevice));
+  const size_t idw = (size_t)s->step_idw;
+  char* const ids = static_cast<char*>(s->d_step_ids);
+  for (const auto& x : s->src_ids) HIP_TRY(hipMemcpy(ids + x.first * idw, &x.second, idw, hipMemcpyHostToDevice));
   s->src_ids.clear();
   s->has_waves = false;
   s->sweep_fix = s->sweep_ade || s->naux || (int)s->ops.size() > kSweepMaxSrc;
@@ -1943,12 +1948,13 @@ int sweep_sources(gmes_sim* s) {
   for (size_t q = 0; q < s->ops.size(); ++q) {
     const int h = s->ops[q].comp >= 3;
     uint32_t w = 0;
-    HIP_TRY(hipMemcpy(&w, s->d_step_ids + cell[q], sizeof w, hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(&w, ids + cell[q] * idw, idw, hipMemcpyDeviceToHost));
     s->src_ids.push_back({cell[q], w});
     const uint32_t id = (uint32_t)((h ? s->step_h.size() : s->step_e.size()) + src[h].size());
-    src[h].push_back({(int)(h ? w >> 16 : w & 0xFFFFu), s->ops[q].comp % 3, (int)q});
-    w = h ? (w & 0xFFFFu) | id << 16 : (w & 0xFFFF0000u) | id;
-    HIP_TRY(hipMemcpy(s->d_step_ids + cell[q], &w, sizeof w, hipMemcpyHostToDevice));
+    const uint32_t low = (1u << s->step_eb) - 1u;
+    src[h].push_back({(int)(h ? w >> s->step_eb : w & low), s->ops[q].comp % 3, (int)q});
+    w = h ? (w & low) | id << s->step_eb : (w & ~low) | id;
+    HIP_TRY(hipMemcpy(ids + cell[q] * idw, &w, idw, hipMemcpyHostToDevice));
   }
   s->has_waves = !s->ops.empty();
   return s->fp64 ? sweep_upload_tab<double>(s, src[0], src[1]) : sweep_upload_tab<float>(s, src[0], src[1]);
@@ -2007,6 +2013,17 @@ int sweep_build(gmes_sim* s) {
     return GMES_OK;
   sweep_plan(s);
   if (!s->sweep_part.rows || !sweep_room(s)) return GMES_OK;
+  // E and H entries, those of source cells included, in one 16-bit word when
+  // they fit (256^3 FP32: at 4 bytes they are 67 of 1250 MB a step, 256 us; at 2
+  // 248.  181 x 203 x 225 UPML 173, 168)
+  auto bits = [](size_t n) {
+    int b = 1;
+    while ((size_t(1) << b) < n) ++b;
+    return b;
+  };
+  const int eb = bits(s->step_e.size() + kSweepMaxSrc), hb = bits(s->step_h.size() + kSweepMaxSrc);
+  s->step_idw = eb + hb <= 16 ? 2 : 4;
+  s->step_eb = eb + hb <= 16 ? eb : 16;
   int rc = GMES_OK;
   for (int c = 0; c < 6 && !rc; ++c) rc = sweep_alloc(s, &s->f_alt[c], (size_t)s->dsize[c] * s->esize);
   for (int c = 0; c < 3 && !rc; ++c) {
@@ -2015,7 +2032,7 @@ int sweep_build(gmes_sim* s) {
     rc = sweep_alloc(s, &s->pml_alt[c], b);
     if (!rc) HIP_TRY(hipMemset(s->pml_alt[c], 0, b));
   }
-  if (!rc) rc = sweep_alloc(s, (void**)&s->d_step_ids, (size_t)s->g.nx * s->g.ny * s->pitch[0] * sizeof(uint32_t));
+  if (!rc) rc = sweep_alloc(s, &s->d_step_ids, (size_t)s->g.nx * s->g.ny * s->pitch[0] * s->step_idw);
   s->step_tab_cap = (int64_t)(s->step_e.size() + s->step_h.size()) + 2 * kSweepMaxSrc;
   if (!rc) rc = sweep_alloc(s, &s->d_step_tab, (size_t)s->step_tab_cap * ent);
   if (!rc) rc = sweep_alloc(s, (void**)&s->d_rare, (size_t)s->step_tab_cap * 3 * sizeof(StepRare));
@@ -2093,7 +2110,9 @@ Step3Args<T> step3_args(const gmes_sim* s, const gmes_sim::SweepPart& part) {
   m.W0 = s->pitch[0];
   m.W2 = s->pitch[2];
   m.n[0] = s->g.nx; m.n[1] = s->g.ny; m.n[2] = s->g.nz;
-  m.ids = rsrc(s->d_step_ids, (int64_t)s->g.nx * s->g.ny * s->pitch[0] * 4);
+  m.ids = rsrc(s->d_step_ids, (int64_t)s->g.nx * s->g.ny * s->pitch[0] * s->step_idw);
+  m.idw = s->step_idw;
+  m.eb = s->step_eb;
   m.exact = s->sweep_exact;
   m.ghosts = s->sweep_ghosts;
   m.tab = s->d_step_tab;
@@ -4108,8 +4127,9 @@ int gmes_batch_set_graph(gmes_batch* b, int32_t enable) {
   return GMES_OK;
 }
 
-// Advance every member by nsteps: one batched launch per kernel kind and
-// half step, replayed from one captured graph per step.
+// Advance every member by nsteps: one batched launch per kernel kind (and half
+// step, for members that take those), replayed from a captured graph of a step
+// or, with one-sweep members, of two.
 int gmes_batch_step(gmes_batch* b, int64_t nsteps) {
   ApiGuard api;
   if (!b) return set_error(GMES_EINVAL, "null batch handle");

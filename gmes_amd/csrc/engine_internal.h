@@ -199,7 +199,8 @@ struct gmes_sim {
   void* f_alt[6] = {};
   void* pml_alt[3] = {};
   int32_t sweep_run_e[3] = {}, sweep_run_h[3] = {};  // Step3Args::run_e, run_h
-  uint32_t* d_step_ids = nullptr;  // entries of the E (low half) and H cells of (i, j, k), rows at the pitch of Ex
+  void* d_step_ids = nullptr;      // Step3Args::ids, rows at the pitch of Ex
+  int step_eb = 16, step_idw = 4;  // Step3Args::eb, idw
   void* d_step_tab = nullptr;
   gmes_engine::StepRare* d_rare = nullptr;
   int64_t step_tab_cap = 0;   // entries the two tables hold room for

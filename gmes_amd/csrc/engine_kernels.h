@@ -144,7 +144,8 @@ struct Step3Args {
   i4_t eo[3], ho[3];  // new E, H
   i4_t si[3], so[3];  // E absorber state, read and written
   i4_t sh[3];         // H absorber state (in place: only its owner touches a word)
-  i4_t ids;           // [i][j][k] table entries of the E (low half) and H cells of thread (i, j, k)
+  i4_t ids;           // [i][j][k] table entries of the E and H cells of thread (i, j, k): E | H << eb,
+  int eb, idw;        // in words of idw bytes (2 when both fit, else 4 and eb = 16)
   int W0, W2;      // row pitch of Ex, Ey, Hx, Hy and of Ez, Hz
   int n[3];
   const void* tab;      // StepEnt<R>[net + nht]: E entries, then H entries
@@ -362,8 +363,10 @@ struct StepIdArgs {
   uint32_t mask[2];
   int n[3];
   int pitch;       // of out's rows
-  uint32_t* out;
-  uint16_t* out16;  // one field type's: 2-D modes, whose three components make one triple
+  int types;       // 1: one triple per cell (2-D modes), 2: E | H << shift
+  int shift;
+  uint32_t* out;   // or, when out16
+  uint16_t* out16;
 };
 void launch_step_ids(const StepIdArgs& a, hipStream_t st);
 // out[element of cell[q]] = q, for the cells of a list

@@ -29,9 +29,9 @@
 // small sim), which loads those along x and y in the plane that uses them:
 // ahead they cost 98 registers and one block per CU in FP32.
 //
-// Measured per step, two-kernel step first: FP32 256^3 CPML 344 -> 255 us (one
-// body for all blocks 293), 181 x 203 x 225 UPML 210 -> 171, 96^3 CPML 39 ->
-// 26, 64^3 UPML 24 -> 11; FP64 CPML 171 x 150 x 139 189 -> 145, 64^3 31 -> 19;
+// Measured per step, two-kernel step first: FP32 256^3 CPML 344 -> 248 us (one
+// body for all blocks 293), 181 x 203 x 225 UPML 210 -> 168, 96^3 CPML 39 ->
+// 26, 64^3 UPML 24 -> 11; FP64 CPML 171 x 150 x 139 189 -> 143, 64^3 31 -> 19;
 // complex FP32 with z layers 192 x 192 x 128 190 -> 136, 112^3 72 -> 46.  What
 // bounds it: without an absorber the bytes (256^3 FP32 188 us, 4.3 TB/s); with
 // one the latency of a plane, 1 to 2 us, of which a CU has few in flight (24
@@ -57,6 +57,7 @@ __device__ float raw_load_f32(i4_t r, int v, int s, int aux) __asm("llvm.amdgcn.
 __device__ vec2_t<float> raw_load_v2f32(i4_t r, int v, int s, int aux) __asm("llvm.amdgcn.raw.buffer.load.v2f32");
 __device__ void raw_store_f32(float x, i4_t r, int v, int s, int aux) __asm("llvm.amdgcn.raw.buffer.store.f32");
 __device__ void raw_store_v2f32(vec2_t<float> x, i4_t r, int v, int s, int aux) __asm("llvm.amdgcn.raw.buffer.store.v2f32");
+__device__ short raw_load_i16(i4_t r, int v, int s, int aux) __asm("llvm.amdgcn.raw.buffer.load.i16");
 __device__ int raw_load_i32(i4_t r, int v, int s, int aux) __asm("llvm.amdgcn.raw.buffer.load.i32");
 
 constexpr unsigned kNowhere = 0xFFFFFFF0u;
@@ -230,7 +231,7 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
   const unsigned b0 = (unsigned)j * W0 + (unsigned)k * S, b2 = (unsigned)j * W2 + (unsigned)k * S;
   const int jm = j ? j - 1 : ny - 1;  // row of the H below, one row up
   const unsigned bj0 = (unsigned)jm * W0 + (unsigned)k * S, bj2 = (unsigned)jm * W2 + (unsigned)k * S;
-  const unsigned PI = (unsigned)ny * W0 / S * 4u;  // ids: rows at the pitch of Ex
+  const unsigned PI = (unsigned)ny * W0 / S * (unsigned)m->idw;  // ids: rows at the pitch of Ex
   const int tm = k ? t - 1 : t + nz - 1, tp = k == nz - 1 ? t + 1 - nz : t + 1;
 
   // absorber rows of the block: E along y, H along y, E along z, H along z
@@ -301,7 +302,8 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
       l.e1 = bld<T>(m->ei[1], b0, oy, kAuxNt);
       l.e2 = bld<T>(m->ei[2], b2, oz, kAuxNt);
     }
-    l.id = (uint32_t)raw_load_i32(m->ids, (int)(b0 / S * 4u), (int)(qe * PI), kAuxNt);
+    if (m->idw == 2) l.id = (uint16_t)raw_load_i16(m->ids, (int)(b0 / S * 2u), (int)(qe * PI), kAuxNt);
+    else l.id = (uint32_t)raw_load_i32(m->ids, (int)(b0 / S * 4u), (int)(qe * PI), kAuxNt);
     if constexpr (PML != 0) {
       const bool lx = x_of_e(q), lxh = x_of_h(q);
 #pragma unroll
@@ -542,7 +544,8 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
         hyk = phased<T>(m->ph[1][2], hyk);
       }
     }
-    const StepEnt<R> en = et[l.id & 0xFFFFu];
+    const unsigned eid = l.id & ((1u << m->eb) - 1u);
+    const StepEnt<R> en = et[eid];
     const R d0 = m->d[0], d1 = m->d[1], d2 = m->d[2], v0 = m->inv_d[0], v1 = m->inv_d[1], v2 = m->inv_d[2];
     T nex, ney, nez;
     auto plain_e = [&]() {
@@ -582,7 +585,7 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
       }
     }
     if (en.meta & kStepRareCell) {
-      const StepRare* x = rare + (l.id & 0xFFFFu) * 3;
+      const StepRare* x = rare + eid * 3;
       nex = step_rare<T>(x, waves, wave_n, row, l.e0, nex);
       ney = step_rare<T>(x + 1, waves, wave_n, row, l.e1, ney);
       nez = step_rare<T>(x + 2, waves, wave_n, row, l.e2, nez);
@@ -707,7 +710,7 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
     hx = l.hx;
     hy = l.hy;
     hz = l.hz;
-    hid = l.id >> 16;
+    hid = l.id >> m->eb;
   }
   if (own) store_h(i1 - 1);
 }
@@ -741,7 +744,7 @@ __global__ void __launch_bounds__(256) k_step_ids(StepIdArgs a) {
   uint32_t v = 0;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    if (h && a.out16) continue;
+    if (h >= a.types) continue;
     uint16_t id[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
@@ -751,7 +754,7 @@ __global__ void __launch_bounds__(256) k_step_ids(StepIdArgs a) {
     for (uint32_t n = 0; n <= a.mask[h]; ++n) {  // every cell's triple is in the table
       const uint64_t got = gld(&a.tab[h][at].key);
       if (got == key) {
-        v |= (uint32_t)gld(&a.tab[h][at].id) << (16 * h);
+        v |= (uint32_t)gld(&a.tab[h][at].id) << (h ? a.shift : 0);
         break;
       }
       at = (at + 1) & a.mask[h];

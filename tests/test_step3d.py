@@ -238,3 +238,31 @@ def test_finished_cells_match_the_oracle(engine_lib, oracle_lib):
     for c in g.constant.COMPONENTS:
         x, y = np.array(a.field[c]), np.array(b.field[c])
         assert np.linalg.norm(x - y) <= FP64_TOL * np.linalg.norm(y)
+
+
+@pytest.mark.parametrize("precision,media", [("fp32", 9), ("fp64", 7), ("fp32", 3)])
+def test_many_media(engine_lib, precision, media):
+    """Entry ids of 32 bits: more distinct triples of E and of H cells than 16
+    hold together (and, with 3 media, fewer)."""
+    rng = np.random.default_rng(8)
+    n = (14, 13, 15)
+    kinds = [g.Dielectric(1.0 + 0.3 * q, 1.0 + 0.1 * q) for q in range(media)]
+    geom = [g.DefaultMedium(g.Dielectric())]
+    for _ in range(900):
+        c = [rng.uniform(-v / 2, v / 2) for v in n]
+        geom.append(g.Block(kinds[rng.integers(media)], center=c, size=rng.uniform(0.8, 2.6, 3)))
+    src = [g.PointSource(g.Continuous(freq=0.05, width=5), center=(0, 0, 0), component=c) for c in (g.Ex, g.Hy)]
+    sims = []
+    for fuse in (1, 0):
+        sim = g.FDTD(g.Cartesian(size=n, resolution=1), geom, src, courant_ratio=0.4, verbose=False,
+                     precision=precision, _engine=engine_lib)
+        sim.init()
+        r = np.random.default_rng(5)
+        for c in g.constant.COMPONENTS:
+            sim.field[c][...] = r.standard_normal(sim.field[c].shape)
+        engine_lib.set_ghost_fusion(sim._sim, fuse)
+        sims.append(sim)
+    for k in (1, 6):
+        for sim in sims:
+            sim._advance(k)
+        agree(*sims)
