@@ -84,6 +84,17 @@ def sweep_bytes(sim):
     return kernel_bytes(sim, True) + kernel_bytes(sim, False) - s * n
 
 
+def takes_sweep(sim, lib):
+    """Whether the sim's step is a one-sweep step (two steps are run: such a
+    step launches no H kernel)."""
+    lib.profile(sim._sim, 1)
+    sim._advance(2)
+    lib.sync(sim._sim)
+    launches = lib.read_profile(sim._sim)[1]
+    lib.profile(sim._sim, 0)
+    return launches[1] == 0
+
+
 def measured_traffic(n, fam):
     """HBM bytes per launch of the dominant kernel from the committed
     rocprofv3 FETCH_SIZE/WRITE_SIZE summary (copy-kernel scaled), for the
@@ -261,10 +272,11 @@ def batched_leg(steps, warm=5, alone_steps=50, prof_steps=50):
     sims = workloads.batch_instances(precision="fp32")
     setup = time.perf_counter() - t
     cells = sum(int(np.prod(s.space.whole_field_size)) for s in sims)
-    nbytes = sum(kernel_bytes(s, True) + kernel_bytes(s, False) for s in sims)
     log("batch: %d instances, %.1f M cells, setup %.1f s" % (len(sims), cells / 1e6, setup))
     # one at a time (each on its own stream, synchronised per instance)
     lib = sims[0]._lib
+    swept = [s for s in sims if takes_sweep(s, lib)]
+    nbytes = sum(sweep_bytes(s) if s in swept else kernel_bytes(s, True) + kernel_bytes(s, False) for s in sims)
     t0 = time.perf_counter()
     for s in sims:
         s._advance(alone_steps)
@@ -287,22 +299,26 @@ def batched_leg(steps, warm=5, alone_steps=50, prof_steps=50):
     b.close()
     three = [s for s in sims if len(s._active) == 6]
     # one-sweep members: whole steps under the E families, nothing under H
-    sweep = launches[1] == 0 and launches[3] == 0
+    sweep = any(s in swept for s in three)
     fam = {}
     for k, name, sel, el in ((0, "e_main3d", three, True), (1, "h_main3d", three, False),
                              (2, "e_main2d", [s for s in sims if s not in three], True),
                              (3, "h_main2d", [s for s in sims if s not in three], False)):
         avg = ms[k] / max(1, launches[k])
-        nb = sum(sweep_bytes(s) if sweep else kernel_bytes(s, el) for s in sel)
+        # a family's time is per launch, its bytes per step: where both kinds
+        # of members are there, E has two launches a step
+        avg *= max(1, round(launches[k] / prof_steps))
+        nb = sum(kernel_bytes(s, el) if s not in swept else sweep_bytes(s) if el else 0 for s in sel)
         fam[name] = dict(avg_launch_ms=round(avg, 5), bytes_per_launch=int(nb),
-                         gbps=round(nb / (avg * 1e-3) / 1e9, 1) if avg > 0 else None)
+                         gbps=round(nb / (avg * 1e-3) / 1e9, 1) if avg > 0 and nb else None)
     split = {k: round(ms[i] / max(1, launches[i]), 4) for i, k in enumerate(
         ("e_main3d", "h_main3d", "e_main2d", "h_main2d", "ade", "rest"))}
     dom = max(("e_main3d", "h_main3d"), key=lambda k: fam[k]["avg_launch_ms"])
     roof = dict(bound="hbm", achieved=fam[dom]["gbps"], peak=HBM_PEAK_GBPS, unit="GB/s",
                 frac=round(fam[dom]["gbps"] / HBM_PEAK_GBPS, 4),
                 traffic=None if sweep else measured_traffic_batch(dom),
-                kernel="k_step3d_batch<float, false> (%d 3-D members)" % len(three) if sweep else
+                kernel="k_step3d_batch<float, false> (%d of %d 3-D members, the others in k_main3d_batch)" % (
+                    sum(s in swept for s in three), len(three)) if sweep else
                 "k_main3d_batch<%s, float> (%d 3-D members, one launch per profile-row kind)" % (
                     "true" if dom == "e_main3d" else "false", len(three)),
                 bytes_per_launch=fam[dom]["bytes_per_launch"], avg_launch_ms=fam[dom]["avg_launch_ms"],
@@ -418,7 +434,7 @@ def served_leg(nreq, budget_gb=64.0, max_active=16, chunk=250, policy="shortest"
 
         def wrapped():
             sim, fn = build()
-            step_bytes[r.rid] = kernel_bytes(sim, True) + kernel_bytes(sim, False)
+            step_bytes[r.rid] = (kernel_bytes(sim, True) + kernel_bytes(sim, False), sweep_bytes(sim))
             return sim, fn
         return wrapped
     for r in reqs:
@@ -436,7 +452,6 @@ def served_leg(nreq, budget_gb=64.0, max_active=16, chunk=250, policy="shortest"
     ok = [r for r in done if r.error is None]
     st = latency_stats(done)
     value = work / srv.elapsed / 1e6
-    moved = sum(step_bytes[r.rid] * r.steps for r in ok)
     sims = [sim for sim, _ in built]
     b = Batch(sims)
     b.advance(5)
@@ -450,6 +465,7 @@ def served_leg(nreq, budget_gb=64.0, max_active=16, chunk=250, policy="shortest"
     fam = 0 if ms[0] >= ms[1] else 1
     avg = ms[fam] / max(1, launches[fam])
     sweep = launches[1] == 0
+    moved = sum(step_bytes[r.rid][int(sweep)] * r.steps for r in ok)
     nb = sum(sweep_bytes(sm) if sweep else kernel_bytes(sm, fam == 0) for sm in sims)
     for sm in sims:
         sm.close()
