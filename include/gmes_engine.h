@@ -154,7 +154,8 @@ int gmes_sim_create(const gmes_grid_desc* desc, gmes_sim** sim);
 int gmes_sim_destroy(gmes_sim* sim);
 /* Shape of component comp (inactive -> 1,1,1). */
 int gmes_sim_shape(const gmes_sim* sim, int32_t comp, int64_t shape[3]);
-/* Bytes of device memory held by the sim (fields, state, tables). */
+/* Bytes of device memory held by the sim (fields, state, tables; a sim that
+ * takes one-sweep steps holds its fields and E state twice). */
 int gmes_sim_footprint(const gmes_sim* sim, int64_t* bytes);
 
 /* ---- materials (replace PwMaterial attach/merge) ---------------------- */
@@ -253,9 +254,11 @@ int gmes_sim_step(gmes_sim* sim, int64_t nsteps);
 int gmes_sim_sync(gmes_sim* sim);
 /* Number of completed steps enqueued so far. */
 int gmes_sim_get_step(const gmes_sim* sim, int64_t* step);
-/* 1: capture one step as a HIP graph and replay it; 0: launch directly. */
+/* 1: capture a step (one-sweep steps: two) as a HIP graph and replay it; 0:
+ * launch directly. */
 int gmes_sim_set_graph(gmes_sim* sim, int32_t enable);
-/* Launch-shape override (0 = autotuned default) for the main E/H kernels:
+/* Launch-shape override (0 = autotuned default) for the main E/H kernels
+ * (a sim with one takes separate E and H launches, not one-sweep steps):
  * a bx x by tile of one plane (bx along k, a power of two, bx * by <= 256).
  * On a 3-D sim whose rows are under 256 cells (stored unpadded) 256 x 1,
  * the default there, means flat blocks of 256 consecutive (j, k) points.
@@ -277,21 +280,24 @@ int gmes_sim_autotune(gmes_sim* sim, int32_t* bx, int32_t* by);
  * operation on a source or ghost plane, no E probe on a ghost plane.  In
  * TMz it lets the 2-D E kernel write the z ghost plane of Hx and Hy (read
  * by no E update) in place of that part of the H copy at the start of the
- * step (gmes/fdtd.py:955-1097).  enable = 0 keeps the separate copies.
+ * step (gmes/fdtd.py:955-1097).  enable = 0 keeps the separate copies,
+ * and separate E and H launches: one-sweep steps, which run a whole step
+ * in one kernel with the same values, write the ghost planes themselves.
  * *fused (may be NULL) reports whether either fusion is in effect now.
  * No reference counterpart. */
 int gmes_sim_set_ghost_fusion(gmes_sim* sim, int32_t enable, int32_t* fused);
 /* Kernel timing on the sim's stream: enable accumulates HIP-event time per
  * kernel family; read returns ms and launch counts for
- * [E main, H main, E ADE, sources, ghost, aux].  */
+ * [E main, H main, E ADE, sources, ghost, aux].  One-sweep steps count
+ * under E main, the cells finished after them under E ADE and sources. */
 int gmes_sim_profile(gmes_sim* sim, int32_t enable);
 int gmes_sim_read_profile(gmes_sim* sim, double ms[6], int64_t launches[6]);
 
-/* ---- batches (many sims, one launch per kernel kind per half step) ------
- * Members keep their own fields, tables and clocks; the main, source and
- * ghost kernels of all members run as one launch each (a device job table
- * maps blocks to members), and a step of the whole batch is one captured
- * HIP graph.  A member is not stepped on its own while in a batch.  No
+/* ---- batches (many sims, one launch per kernel kind) ---------------------
+ * Members keep their own fields, tables and clocks; the members' kernels of
+ * one kind run as one launch (a device job table maps blocks to members),
+ * and a step of the whole batch (two, when members take one-sweep steps) is
+ * one captured HIP graph.  A member is not stepped on its own while in a batch.  No
  * reference counterpart: the reference advances one FDTD at a time
  * (gmes/fdtd.py:1099-1122). */
 
@@ -305,7 +311,8 @@ int gmes_batch_set_graph(gmes_batch* batch, int32_t enable);
 /* Kernel timing of a batch's own stream (HIP events; steps run without the
  * graph while it is on): read returns ms and launch counts for
  * [E 3-D main, H 3-D main, E 2-D/1-D main, H 2-D/1-D main, dispersive,
- * the rest (ghosts, sources, probes, auxiliary grids, DFT)]. */
+ * the rest (ghosts, sources, probes, auxiliary grids, DFT)].  One-sweep
+ * steps count under E. */
 int gmes_batch_profile(gmes_batch* batch, int32_t enable);
 int gmes_batch_read_profile(gmes_batch* batch, double ms[6], int64_t launches[6]);
 
