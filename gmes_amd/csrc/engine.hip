@@ -2047,12 +2047,12 @@ int sweep_build(gmes_sim* s) {
   return GMES_OK;
 }
 
-// Whether the next step of s is a one-sweep step.
 // Whether an auxiliary grid takes one-sweep steps when its parent does.
 bool aux_sweeps(const gmes_sim* a) {
   return a->sweep_1d && a->sweep_ok && a->sweep_src_ok && a->allow_fuse && a->probes.empty() && a->dfts.empty();
 }
 
+// Whether the next step of s is a one-sweep step.
 bool sweeps(const gmes_sim* s) {
   if (!s->sweep_ok || !s->sweep_src_ok || !s->allow_fuse || (s->naux && !s->sweep_fix) || s->parent) return false;
   if (s->tile_bx > 0 && !s->tile_tuned) return false;
