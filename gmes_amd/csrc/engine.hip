@@ -1909,7 +1909,9 @@ FixArgs<T> fix_args(const gmes_sim* s) {
 }
 
 // Marks the cells of the sim's source operations in the sweep's ids, when
-// all of them can be applied there (sweep_src_ok).
+// all of them can be applied there (sweep_src_ok).  Of a committed sim only
+// (commit itself calls it): records or material ids set since are neither
+// checked nor those that the tables were built from.
 int sweep_sources(gmes_sim* s) {
   if (!s->sweep_ok) return GMES_OK;
   if (s->sweep_1d) return sweep1_sources(s);
@@ -3023,7 +3025,7 @@ int gmes_sim_set_sources(gmes_sim* s, const gmes_src_op* ops, int64_t nops, int3
   s->ops.assign(ops, ops + nops);
   s->nwaves = nwaves;
   int rc = s->fp64 ? upload_sources<double>(s) : upload_sources<float>(s);
-  if (!rc) rc = sweep_sources(s);
+  if (!rc && s->committed) rc = sweep_sources(s);
   destroy_graph(s);
   decide_fusion(s);
   return rc;
@@ -3068,7 +3070,7 @@ int gmes_sim_attach_aux(gmes_sim* s, gmes_sim* aux, int32_t* slot) {
   *slot = s->naux++;
   if (int rc = aux_pointers(s)) return rc;
   destroy_graph(s);
-  return sweep_sources(s);
+  return s->committed ? sweep_sources(s) : GMES_OK;
 }
 
 int gmes_sim_add_probe(gmes_sim* s, int32_t c, int64_t cell, int32_t* id) {
