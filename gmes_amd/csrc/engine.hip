@@ -1215,6 +1215,13 @@ void sweep_plan(gmes_sim* s) {
   }
 }
 
+void fix_release(gmes_sim* s) {
+  dev_free(s, s->d_fix_items, (size_t)s->fix_bytes);
+  s->sweep_bytes -= s->fix_bytes;
+  s->d_fix_items = nullptr;
+  s->fix_bytes = 0;
+}
+
 void sweep_release(gmes_sim* s) {
   void** bufs[] = {&s->f_alt[0], &s->f_alt[1], &s->f_alt[2], &s->f_alt[3], &s->f_alt[4], &s->f_alt[5],
                    &s->pml_alt[0], &s->pml_alt[1], &s->pml_alt[2], &s->d_step_ids, &s->d_step_tab, (void**)&s->d_rare};
@@ -1231,8 +1238,7 @@ void sweep_release(gmes_sim* s) {
       p = nullptr;
     }
   }
-  if (s->d_fix_items) (void)dev_release(s->d_fix_items);
-  s->d_fix_items = nullptr;
+  fix_release(s);
   s->sweep_fix = false;
   s->sweep_1d = s->sweep_2d = false;
   s->bytes -= s->sweep_bytes;
@@ -1764,13 +1770,11 @@ bool step2_ade(const gmes_sim* s) { return s->d_adeq[0] || s->d_adeq[1] || s->d_
 // live absorber state.
 int sweep_fix_build(gmes_sim* s) {
   HIP_TRY(sync_exec(s));
-  if (s->d_fix_items) {
-    (void)dev_release(s->d_fix_items);
-    s->d_fix_items = nullptr;
-  }
+  fix_release(s);
   for (int& n : s->fix_nitem) n = 0;
   s->sweep_src_ok = false;
   const int64_t n[3] = {s->g.nx, s->g.ny, s->g.nz};
+  if (n[0] * n[1] * n[2] >= INT32_MAX / 4) return GMES_OK;  // 32-bit items
   for (const gmes_src_op& o : s->ops) {
     const int64_t sy = s->shape[o.comp][1], sz = s->shape[o.comp][2];
     const int64_t ix[3] = {o.cell / (sy * sz), (o.cell / sz) % sy, o.cell % sz};
@@ -1803,16 +1807,16 @@ int sweep_fix_build(gmes_sim* s) {
   const size_t mark = ((size_t)(3 * b.cells) + 15) / 16 * 16, count = (size_t)3 * b.nblk * sizeof(int32_t),
                rec = cls.size() * sizeof(int32_t);
   char* tmp = nullptr;
-  HIP_TRY(hipMalloc((void**)&tmp, mark + count + rec + 16));
-  b.mark = reinterpret_cast<uint8_t*>(tmp);
-  b.count = reinterpret_cast<int32_t*>(tmp + mark);
-  b.cls = reinterpret_cast<int32_t*>(tmp + mark + count);
-  b.bad = reinterpret_cast<int*>(tmp + mark + count + rec);
   std::vector<int32_t> counts((size_t)3 * b.nblk);
   int bad = 0;
   auto build = [&]() -> hipError_t {
-    hipError_t e = hipMemset(tmp, 0, mark + count + rec + 16);
+    hipError_t e = hipMalloc((void**)&tmp, mark + count + rec + 16);
     if (e != hipSuccess) return e;
+    b.mark = reinterpret_cast<uint8_t*>(tmp);
+    b.count = reinterpret_cast<int32_t*>(tmp + mark);
+    b.cls = reinterpret_cast<int32_t*>(tmp + mark + count);
+    b.bad = reinterpret_cast<int*>(tmp + mark + count + rec);
+    if ((e = hipMemset(tmp, 0, mark + count + rec + 16)) != hipSuccess) return e;
     if ((e = hipMemcpy(const_cast<int32_t*>(b.cls), cls.data(), rec, hipMemcpyHostToDevice)) != hipSuccess) return e;
     for (int c = 0; c < 3; ++c)
       for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2; ++k) {
@@ -1840,14 +1844,17 @@ int sweep_fix_build(gmes_sim* s) {
     }
     if (!total) return hipSuccess;
     if ((e = hipMalloc(&s->d_fix_items, (size_t)total * sizeof(FixItem))) != hipSuccess) return e;
+    s->fix_bytes = (int64_t)total * sizeof(FixItem);
+    s->bytes += s->fix_bytes;
+    s->sweep_bytes += s->fix_bytes;
     b.items = static_cast<FixItem*>(s->d_fix_items);
     if ((e = hipMemcpy(b.count, counts.data(), count, hipMemcpyHostToDevice)) != hipSuccess) return e;
     launch_fix_fill(b, nullptr);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     return hipMemcpy(&bad, b.bad, sizeof bad, hipMemcpyDeviceToHost);
   };
-  const hipError_t e = b.cells < INT32_MAX / 4 ? build() : hipErrorOutOfMemory;
-  (void)dev_release(tmp);
+  const hipError_t e = build();
+  if (tmp) (void)dev_release(tmp);
   if (e == hipErrorOutOfMemory) {  // no room for the lists: the two-kernel step needs none
     (void)hipGetLastError();
     return GMES_OK;
@@ -2043,7 +2050,12 @@ int sweep_build(gmes_sim* s) {
     sweep_release(s);
     return GMES_OK;
   }
-  if ((rc = sweep_ids(s))) return rc;
+  if ((rc = sweep_ids(s))) {
+    const bool room = rc != GMES_ENOMEM;
+    (void)hipGetLastError();
+    sweep_release(s);
+    return room ? rc : GMES_OK;
+  }
   s->src_ids.clear();
   s->sweep_ok = true;
   return GMES_OK;

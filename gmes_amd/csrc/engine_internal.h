@@ -220,6 +220,7 @@ struct gmes_sim {
   // on many cells
   bool sweep_ade = false, sweep_fix = false;
   void* d_fix_items = nullptr;    // FixItem[], of Hx, Hy, Hz in turn
+  int64_t fix_bytes = 0;          // (part of sweep_bytes)
   int fix_nitem[3] = {};
   std::vector<std::array<int, 5>> step2_src;  // direction, i, j, wave, kind
   std::vector<std::array<uint16_t, 3>> step_e, step_h;  // record ids of each entry
