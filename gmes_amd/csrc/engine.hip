@@ -189,9 +189,20 @@ int64_t dev_flat(const gmes_sim* s, int c, int64_t flat) {
 }
 
 
+// Device memory.  When there is none left, the second buffers of the one-sweep
+// steps on the device make room: sims that have them never keep out what
+// would fit without them.
+bool sweep_reclaim(int device);
+hipError_t dev_malloc(int device, void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  return sweep_reclaim(device) ? hipMalloc(p, bytes) : e;
+}
+
 int dev_alloc(gmes_sim* s, void** p, size_t bytes) {
   if (bytes == 0) bytes = 16;
-  HIP_TRY(hipMalloc(p, bytes));
+  HIP_TRY(dev_malloc(s->device, p, bytes));
   s->bytes += (int64_t)bytes;
   return GMES_OK;
 }
@@ -802,7 +813,7 @@ int upload_dft_jobs_t(gmes_sim* s) {
   if (need > s->dft_jobs_cap) {
     if (s->d_dft_jobs) HIP_TRY(dev_release(s->d_dft_jobs));
     s->d_dft_jobs = nullptr;
-    HIP_TRY(hipMalloc(&s->d_dft_jobs, (size_t)need * sizeof(DftJob<T>)));
+    HIP_TRY(dev_malloc(s->device, &s->d_dft_jobs, (size_t)need * sizeof(DftJob<T>)));
     s->dft_jobs_cap = need;
   }
   HIP_TRY(hipMemcpy(s->d_dft_jobs, jobs.data(), jobs.size() * sizeof(DftJob<T>), hipMemcpyHostToDevice));
@@ -833,6 +844,7 @@ void enqueue_aux_steps(gmes_sim* s, bool sweep, hipStream_t st);
 
 bool on_ghost_copy_plane(const gmes_sim* s, int c, int64_t x, bool source, bool ghost);
 int sweep_sources(gmes_sim* s);
+void destroy_graph(gmes_sim* s);
 hipError_t sync_exec(gmes_sim* s);
 
 // ---- one-sweep steps (step3d.hip)
@@ -1247,14 +1259,47 @@ void sweep_release(gmes_sim* s) {
   s->step_tab_cap = 0;
 }
 
+// (plain hipMalloc: a sim that finds no room does without)
 int sweep_alloc(gmes_sim* s, void** p, size_t bytes) {
-  const int rc = dev_alloc(s, p, bytes);
-  if (!rc) s->sweep_bytes += (int64_t)std::max<size_t>(16, bytes);
-  return rc;
+  if (bytes == 0) bytes = 16;
+  HIP_TRY(hipMalloc(p, bytes));
+  s->bytes += (int64_t)bytes;
+  s->sweep_bytes += (int64_t)bytes;
+  return GMES_OK;
+}
+
+// Every sim, for sweep_reclaim.
+std::mutex g_sims_mu;
+std::unordered_set<gmes_sim*> g_sims;
+void known_sim(gmes_sim* s, bool there) {
+  std::lock_guard<std::mutex> lk(g_sims_mu);
+  if (there) g_sims.insert(s);
+  else g_sims.erase(s);
+}
+
+// Releases the second buffers of every sim on a device, with no other thread
+// inside the engine: between two calls, and where a call has let go of its
+// hold (it captures a graph, or is here itself), the current buffers hold the
+// whole state, and the two-kernel step goes on from there.  False: there were
+// none.
+bool sweep_reclaim(int device) {
+  CaptureGuard alone;
+  std::lock_guard<std::mutex> lk(g_sims_mu);
+  bool any = false;
+  for (gmes_sim* s : g_sims) {
+    if (s->device != device || s->sweep_bytes == 0) continue;
+    (void)sync_exec(s);
+    destroy_graph(s);
+    sweep_release(s);
+    any = true;
+  }
+  return any;
 }
 
 // Whether the second buffers of s leave the device at least half empty: sims
-// that fill it keep the two-kernel step, and sims made later find room.
+// that fill it keep the two-kernel step, and other users of the device find
+// room (the engine's own sims take it from here when there is none left, see
+// sweep_reclaim).
 bool sweep_room(const gmes_sim* s) {
   int64_t need = (int64_t)s->g.nx * s->g.ny * s->g.nz * 4;
   for (int c = 0; c < 6; ++c) {
@@ -1969,10 +2014,9 @@ int sweep_sources(gmes_sim* s) {
   return s->fp64 ? sweep_upload_tab<double>(s, src[0], src[1]) : sweep_upload_tab<float>(s, src[0], src[1]);
 }
 
-// Builds what one-sweep steps need (at commit); leaves sweep_ok false when
-// the sim does not qualify.
+// Builds what one-sweep steps need (at commit, which has released the old);
+// leaves sweep_ok false when the sim does not qualify.
 int sweep_build(gmes_sim* s) {
-  sweep_release(s);
   if (line_dir(s) >= 0) return sweep1_build(s);
   if (is_2z(s)) return s->naux ? GMES_OK : sweep2_build(s);
   if (!is3d(s) || s->g.dtype == GMES_C128) return GMES_OK;
@@ -2337,6 +2381,7 @@ void destroy_graph(gmes_sim* s) {
 int build_graph(gmes_sim* s) {
   destroy_graph(s);
   hipGraph_t graph;
+  hipError_t e;
   {
     CaptureGuard capture;
     HIP_TRY(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
@@ -2346,11 +2391,11 @@ int build_graph(gmes_sim* s) {
     s->sweep_ghosts = sweep_ghosts(s);
     for (int t = 0; t < s->graph_steps; ++t) enqueue_step(s, s->stream);
     HIP_TRY(hipStreamEndCapture(s->stream, &graph));
+    e = hipGraphInstantiate(&s->graph_exec, graph, nullptr, nullptr, 0);
+    s->graph_dirty = e != hipSuccess;
   }
-  hipError_t e = hipGraphInstantiate(&s->graph_exec, graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
   if (e != hipSuccess) return set_error(GMES_EDEVICE, "hipGraphInstantiate: %s", hipGetErrorString(e));
-  s->graph_dirty = false;
   return GMES_OK;
 }
 
@@ -2399,6 +2444,11 @@ int do_step(gmes_sim* s, int64_t n) {
   if (rc) return rc;
   if ((rc = ensure_probe_capacity(s, n))) return rc;
   HIP_TRY(hipSetDevice(s->device));
+  // a capture waits until it is alone in the engine: what another thread does
+  // before or after it (sweep_reclaim) may call for another graph
+  const bool graph = s->use_graph && !any_graph_blocker(s);
+  while (graph && (s->graph_dirty || !s->graph_exec || s->graph_steps != (sweeps(s) ? 2 : 1)))
+    if ((rc = build_graph(s))) return rc;
   const bool sweep = sweeps(s);
   if (n > 0) {
     sweep_clock(s, sweep, s->stream);
@@ -2407,9 +2457,7 @@ int do_step(gmes_sim* s, int64_t n) {
     if (!sweep && (rc = aux_pointers(s))) return rc;
   }
   const int par = s->par;
-  if (s->use_graph && !any_graph_blocker(s)) {
-    if (s->graph_dirty || !s->graph_exec || s->graph_steps != (sweep ? 2 : 1))
-      if ((rc = build_graph(s))) return rc;
+  if (graph) {
     int64_t t = 0;
     const int64_t last = sweep ? 1 : 0;  // the step that writes the ghost planes
     if (s->par != s->graph_par && t + last < n) { enqueue_step(s, s->stream); ++t; }
@@ -2483,13 +2531,13 @@ int autotune_t(gmes_sim* s, int& best_bx, int& best_by) {
     if (!active(s, c)) continue;
     const size_t fb = (size_t)s->dsize[c] * s->esize;
     void* tmp = nullptr;
-    HIP_TRY(hipMalloc(&tmp, fb));
+    HIP_TRY(dev_malloc(s->device, &tmp, fb));
     HIP_TRY(hipMemcpy(tmp, s->f[c], fb, hipMemcpyDeviceToDevice));
     saved.push_back({tmp, {s->f[c], fb}});
     if (s->pml_state[c]) {
       const int pw = s->has_cls[c][GMES_CLS_CPML] ? 2 : 1;
       const size_t pb = (size_t)pw * s->dsize[c] * s->esize;
-      HIP_TRY(hipMalloc(&tmp, pb));
+      HIP_TRY(dev_malloc(s->device, &tmp, pb));
       HIP_TRY(hipMemcpy(tmp, s->pml_state[c], pb, hipMemcpyDeviceToDevice));
       saved.push_back({tmp, {s->pml_state[c], pb}});
     }
@@ -2678,6 +2726,7 @@ int gmes_sim_create(const gmes_grid_desc* desc, gmes_sim** out) {
   HIP_TRY(hipSetDevice(desc->device));
   gmes_sim* s = new gmes_sim();
   stage_sims(1);
+  known_sim(s, true);
   s->g = *desc;
   s->device = desc->device;
   s->complex_ = desc->dtype == GMES_C64 || desc->dtype == GMES_C128;
@@ -2720,6 +2769,7 @@ int gmes_sim_create(const gmes_grid_desc* desc, gmes_sim** out) {
       s->dsize[c] = 2 * kPad + s0 * s1 * row;
     }
     if (s->dsize[c] >= (int64_t(1) << 31)) {
+      known_sim(s, false);
       delete s;
       stage_sims(-1);
       return set_error(GMES_EINVAL, "component %d has more than 2^31 cells", c);
@@ -2782,6 +2832,7 @@ int gmes_sim_destroy(gmes_sim* s) {
   for (void* b : bufs)
     if (b) (void)dev_release(b);
   if (s->stream) (void)stream_release(s->stream);
+  known_sim(s, false);
   delete s;
   stage_sims(-1);
   return GMES_OK;
@@ -2883,6 +2934,8 @@ int gmes_sim_commit(gmes_sim* s) {
   if (s->recs.empty()) return set_error(GMES_EINVAL, "materials not set");
   HIP_TRY(hipSetDevice(s->device));
   HIP_TRY(sync_exec(s));
+  s->committed = false;
+  sweep_release(s);
   free_ade(s);
   s->ade_on_ghost_source = false;
   std::vector<int64_t> counts[6];  // cells per record; empty: an id is out of range
@@ -2968,10 +3021,10 @@ int gmes_sim_commit(gmes_sim* s) {
       L.n = (int64_t)cells[k].size();
       if (!L.n) continue;
       L.nstate = words[k];
-      HIP_TRY(hipMalloc((void**)&L.cell, L.n * sizeof(int32_t)));
-      HIP_TRY(hipMalloc((void**)&L.rec, L.n * sizeof(uint16_t)));
+      HIP_TRY(dev_malloc(s->device, (void**)&L.cell, L.n * sizeof(int32_t)));
+      HIP_TRY(dev_malloc(s->device, (void**)&L.rec, L.n * sizeof(uint16_t)));
       const size_t sb = std::max<size_t>(1, (size_t)L.nstate * L.n * ade_word(s, k));
-      HIP_TRY(hipMalloc(&L.state, sb));
+      HIP_TRY(dev_malloc(s->device, &L.state, sb));
       s->bytes += L.n * 6 + (int64_t)sb;
       HIP_TRY(hipMemcpy(L.cell, cells[k].data(), L.n * sizeof(int32_t), hipMemcpyHostToDevice));
       HIP_TRY(hipMemcpy(L.rec, recs[k].data(), L.n * sizeof(uint16_t), hipMemcpyHostToDevice));
@@ -3102,8 +3155,8 @@ int gmes_sim_add_probe(gmes_sim* s, int32_t c, int64_t cell, int32_t* id) {
   if (s->d_probe_buf) (void)dev_release(s->d_probe_buf);
   s->d_probe_buf = nullptr;
   s->probe_cap = 0;
-  HIP_TRY(hipMalloc((void**)&s->d_probe_cells, cells.size() * sizeof(int64_t)));
-  HIP_TRY(hipMalloc((void**)&s->d_probe_comps, comps.size() * sizeof(int32_t)));
+  HIP_TRY(dev_malloc(s->device, (void**)&s->d_probe_cells, cells.size() * sizeof(int64_t)));
+  HIP_TRY(dev_malloc(s->device, (void**)&s->d_probe_comps, comps.size() * sizeof(int32_t)));
   HIP_TRY(hipMemcpy(s->d_probe_cells, cells.data(), cells.size() * sizeof(int64_t), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(s->d_probe_comps, comps.data(), comps.size() * sizeof(int32_t), hipMemcpyHostToDevice));
   *id = (int32_t)s->probes.size() - 1;
@@ -3161,7 +3214,7 @@ int gmes_sim_add_dft(gmes_sim* s, int32_t c, const int64_t lo[3], const int64_t 
   HIP_TRY(sync_exec(s));
   // sums [nfreq][ncells][re, im], then their compensations, same layout
   const size_t bytes = 2 * (size_t)nfreq * d.ncells * 2 * sizeof(double);
-  HIP_TRY(hipMalloc((void**)&d.acc, bytes));
+  HIP_TRY(dev_malloc(s->device, (void**)&d.acc, bytes));
   HIP_TRY(hipMemset(d.acc, 0, bytes));
   s->dfts.push_back(d);
   s->dft_nfreq = nfreq;
@@ -3182,7 +3235,7 @@ int gmes_sim_set_dft_weights(gmes_sim* s, int64_t step0, int64_t nsteps, const d
   if (need > s->dft_w_cap) {
     if (s->d_dft_w) HIP_TRY(dev_release(s->d_dft_w));
     s->d_dft_w = nullptr;
-    HIP_TRY(hipMalloc((void**)&s->d_dft_w, (size_t)need * sizeof(double)));
+    HIP_TRY(dev_malloc(s->device, (void**)&s->d_dft_w, (size_t)need * sizeof(double)));
     s->dft_w_cap = need;
     int rc = upload_dft_jobs(s);  // the jobs hold the weight pointer
     if (rc) return rc;
@@ -3652,6 +3705,7 @@ struct gmes_batch {
   bool use_graph = true;
   hipGraphExec_t graph_exec = nullptr;
   std::vector<uint64_t> gens;  // member generations the graph was captured with
+  int per = 1;                 // steps it holds
   // job tables: one device buffer, rebuilt on the host for every call
   void* d_jobs = nullptr;
   size_t jobs_cap = 0;
@@ -4074,6 +4128,107 @@ void destroy_batch_graph(gmes_batch* b) {
   }
 }
 
+std::vector<uint64_t> batch_gens(const gmes_batch* b) {
+  std::vector<uint64_t> gens;
+  for (const gmes_sim* s : b->sims) {
+    gens.push_back(s->gen);
+    for (int i = 0; i < s->naux; ++i)
+      if (s->aux[i]) gens.push_back(s->aux[i]->gen);
+  }
+  return gens;
+}
+
+// The job tables of a call of nsteps on the device, and its graph; ready is
+// false when a member changed meanwhile, where this call waited to be alone
+// in the engine (dev_malloc, the capture).
+int batch_ready(gmes_batch* b, int64_t nsteps, bool& ready) {
+  const std::vector<uint64_t> gens = batch_gens(b);
+  b->sweepers.clear();
+  b->others.clear();
+  for (gmes_sim* s : b->sims) {
+    const bool sweep = batch_sweeps(s);
+    if (!sweep)
+      if (int rc = aux_pointers(s)) return rc;
+    sweep_clock(s, sweep, b->stream);
+    for (int i = 0; i < s->naux; ++i)
+      if (s->aux[i]) sweep_clock(s->aux[i], sweep, b->stream);
+    (sweep ? b->sweepers : b->others).push_back(s);
+  }
+  // the job tables are read by kernels still in flight: wait before rewriting
+  HIP_TRY(hipStreamSynchronize(b->stream));
+  b->aux_sims.clear();
+  for (gmes_sim* s : b->others)
+    for (int i = 0; i < s->naux; ++i)
+      if (s->aux[i]) b->aux_sims.push_back(s->aux[i]);
+  b->h_jobs.clear();
+  switch (b->dtype) {
+    case GMES_F32: build_tables<float>(b); break;
+    case GMES_F64: build_tables<double>(b); break;
+    case GMES_C64: build_tables<cplx<float>>(b); break;
+    default: build_tables<cplx<double>>(b); break;
+  }
+  if (b->h_jobs.size() > b->jobs_cap) {
+    destroy_batch_graph(b);
+    if (b->d_jobs) HIP_TRY(dev_release(b->d_jobs));
+    b->d_jobs = nullptr;
+    b->jobs_cap = 0;
+    HIP_TRY(dev_malloc(b->device, &b->d_jobs, b->h_jobs.size()));
+    b->jobs_cap = b->h_jobs.size();
+  }
+  HIP_TRY(hipMemcpy(b->d_jobs, b->h_jobs.data(), b->h_jobs.size(), hipMemcpyHostToDevice));
+  // launch shapes and per-member captured arguments decide whether the
+  // graph is still valid; table contents are read at run time
+  std::vector<int64_t> sig;
+  for (const gmes_batch::JobSet* js : {&b->set, &b->aux_set}) {
+    for (int e = 0; e < 2; ++e)
+      for (const auto* L : {&js->main3d[e], &js->main3d_pp[e], &js->main3d_ur[e], &js->main2z[e], &js->mainnd[e], &js->src[e],
+                            &js->ghost[e]}) {
+        sig.push_back((int64_t)L->off);
+        sig.push_back(L->njobs);
+        sig.push_back(L->nblocks);
+      }
+    for (const auto& L : js->ade) {
+      sig.push_back((int64_t)L.off);
+      sig.push_back(L.njobs);
+      sig.push_back(L.nblocks);
+    }
+    sig.push_back((int64_t)js->dft.off);
+    sig.push_back(js->dft.njobs);
+    sig.push_back(js->dft.nblocks);
+  }
+  for (const gmes_batch::SweepSet& S : b->sweep) {
+    for (const auto* L : {&S.s3[0], &S.s3[1], &S.s3[2], &S.s3[3], &S.s2, &S.s1, &S.aux, &S.fix_e, &S.fix_h, &S.ghost, &S.dft}) {
+      sig.push_back((int64_t)L->off);
+      sig.push_back(L->njobs);
+      sig.push_back(L->nblocks);
+    }
+    for (const size_t l : S.lds3) sig.push_back((int64_t)l);
+    sig.push_back((int64_t)S.lds2);
+  }
+  if (sig != b->shape_sig || gens != b->gens) destroy_batch_graph(b);
+  b->shape_sig = sig;
+  b->gens = gens;
+  // one-sweep members swap buffers: their graph holds two steps, and the last
+  // step, which writes the ghost planes, is launched by itself
+  b->per = b->sweepers.empty() ? 1 : 2;
+  if (b->use_graph && !b->timing.on && !b->graph_exec && nsteps >= 2 * b->per - 1) {
+    hipGraph_t graph;
+    hipError_t e;
+    {
+      CaptureGuard capture;
+      if (gens != batch_gens(b)) return GMES_OK;
+      HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+      for (int k = 0; k < b->per; ++k) enqueue_batch_step(b, k, b->stream);
+      HIP_TRY(hipStreamEndCapture(b->stream, &graph));
+      e = hipGraphInstantiate(&b->graph_exec, graph, nullptr, nullptr, 0);
+    }
+    (void)hipGraphDestroy(graph);
+    if (e != hipSuccess) return set_error(GMES_EDEVICE, "hipGraphInstantiate: %s", hipGetErrorString(e));
+  }
+  ready = gens == batch_gens(b);
+  return GMES_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -4156,98 +4311,15 @@ int gmes_batch_step(gmes_batch* b, int64_t nsteps) {
     if ((rc = ensure_probe_capacity(s, nsteps))) return rc;
   }
   if (nsteps == 0) return GMES_OK;
-  b->sweepers.clear();
-  b->others.clear();
-  for (gmes_sim* s : b->sims) {
-    const bool sweep = batch_sweeps(s);
-    HIP_TRY(hipSetDevice(b->device));
-    if (!sweep)
-      if (int rc = aux_pointers(s)) return rc;
-    sweep_clock(s, sweep, b->stream);
-    for (int i = 0; i < s->naux; ++i)
-      if (s->aux[i]) sweep_clock(s->aux[i], sweep, b->stream);
-    (sweep ? b->sweepers : b->others).push_back(s);
-  }
   HIP_TRY(hipSetDevice(b->device));
-  // the job tables are read by kernels still in flight: wait before rewriting
-  HIP_TRY(hipStreamSynchronize(b->stream));
-  b->aux_sims.clear();
-  for (gmes_sim* s : b->others)
-    for (int i = 0; i < s->naux; ++i)
-      if (s->aux[i]) b->aux_sims.push_back(s->aux[i]);
-  b->h_jobs.clear();
-  switch (b->dtype) {
-    case GMES_F32: build_tables<float>(b); break;
-    case GMES_F64: build_tables<double>(b); break;
-    case GMES_C64: build_tables<cplx<float>>(b); break;
-    default: build_tables<cplx<double>>(b); break;
-  }
-  if (b->h_jobs.size() > b->jobs_cap) {
-    destroy_batch_graph(b);
-    if (b->d_jobs) HIP_TRY(dev_release(b->d_jobs));
-    b->d_jobs = nullptr;
-    b->jobs_cap = 0;
-    HIP_TRY(hipMalloc(&b->d_jobs, b->h_jobs.size()));
-    b->jobs_cap = b->h_jobs.size();
-  }
-  HIP_TRY(hipMemcpy(b->d_jobs, b->h_jobs.data(), b->h_jobs.size(), hipMemcpyHostToDevice));
-  // launch shapes and per-member captured arguments decide whether the
-  // graph is still valid; table contents are read at run time
-  std::vector<int64_t> sig;
-  for (const gmes_batch::JobSet* js : {&b->set, &b->aux_set}) {
-    for (int e = 0; e < 2; ++e)
-      for (const auto* L : {&js->main3d[e], &js->main3d_pp[e], &js->main3d_ur[e], &js->main2z[e], &js->mainnd[e], &js->src[e],
-                            &js->ghost[e]}) {
-        sig.push_back((int64_t)L->off);
-        sig.push_back(L->njobs);
-        sig.push_back(L->nblocks);
-      }
-    for (const auto& L : js->ade) {
-      sig.push_back((int64_t)L.off);
-      sig.push_back(L.njobs);
-      sig.push_back(L.nblocks);
-    }
-    sig.push_back((int64_t)js->dft.off);
-    sig.push_back(js->dft.njobs);
-    sig.push_back(js->dft.nblocks);
-  }
-  for (const gmes_batch::SweepSet& S : b->sweep) {
-    for (const auto* L : {&S.s3[0], &S.s3[1], &S.s3[2], &S.s3[3], &S.s2, &S.s1, &S.aux, &S.fix_e, &S.fix_h, &S.ghost, &S.dft}) {
-      sig.push_back((int64_t)L->off);
-      sig.push_back(L->njobs);
-      sig.push_back(L->nblocks);
-    }
-    for (const size_t l : S.lds3) sig.push_back((int64_t)l);
-    sig.push_back((int64_t)S.lds2);
-  }
-  std::vector<uint64_t> gens;
-  for (gmes_sim* s : b->sims) {
-    gens.push_back(s->gen);
-    for (int i = 0; i < s->naux; ++i)
-      if (s->aux[i]) gens.push_back(s->aux[i]->gen);
-  }
-  if (sig != b->shape_sig || gens != b->gens) destroy_batch_graph(b);
-  b->shape_sig = sig;
-  b->gens = gens;
-  // one-sweep members swap buffers: their graph holds two steps, and the last
-  // step, which writes the ghost planes, is launched by itself
-  const int per = b->sweepers.empty() ? 1 : 2, last = per - 1;
+  // members that lose their second buffers meanwhile (sweep_reclaim) change
+  // the tables
+  bool ready = false;
+  while (!ready)
+    if (int rc = batch_ready(b, nsteps, ready)) return rc;
   int64_t t = 0;
-  if (b->use_graph && !b->timing.on && nsteps >= per + last) {
-    if (!b->graph_exec) {
-      hipGraph_t graph;
-      {
-        CaptureGuard capture;
-        HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-        for (int k = 0; k < per; ++k) enqueue_batch_step(b, k, b->stream);
-        HIP_TRY(hipStreamEndCapture(b->stream, &graph));
-      }
-      hipError_t e = hipGraphInstantiate(&b->graph_exec, graph, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(graph);
-      if (e != hipSuccess) return set_error(GMES_EDEVICE, "hipGraphInstantiate: %s", hipGetErrorString(e));
-    }
-    for (; t + per + last <= nsteps; t += per) HIP_TRY(hipGraphLaunch(b->graph_exec, b->stream));
-  }
+  if (b->graph_exec && !b->timing.on)
+    for (; t + b->per + b->per - 1 <= nsteps; t += b->per) HIP_TRY(hipGraphLaunch(b->graph_exec, b->stream));
   for (; t < nsteps; ++t) enqueue_batch_step(b, (int)(t & 1) + (t == nsteps - 1 ? 2 : 0), b->stream);
   HIP_TRY(hipGetLastError());
   if (nsteps & 1)

@@ -28,7 +28,7 @@ def case(f):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name", ["source_lists"])
+@pytest.mark.parametrize("name", ["source_lists", "commit", "many_sims"])
 def test_limited_memory(engine_lib, tmp_path, name):
     shim = str(tmp_path / "memory_shim.so")
     subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", shim, os.path.join(HERE, "memory_shim.c"), "-lpthread"],
@@ -38,6 +38,17 @@ def test_limited_memory(engine_lib, tmp_path, name):
     assert out.returncode == 0, out.stdout.decode()
 
 
+def builders():
+    import gmes_amd as g
+    from test_step1d import line
+    from test_step2d import plane
+    from test_step3d import box, media_box
+    return [lambda lib: box(lib, (22, 21, 24), bound=g.Cpml), lambda lib: media_box(lib, (22, 21, 24)),
+            lambda lib: box(lib, (22, 21, 24), precision="fp64", bound=g.Upml),
+            lambda lib: plane(lib, "tez", (41, 67), bound=g.Cpml, media=True),
+            lambda lib: line(lib, "z", 300, bound=g.Cpml, media=True)]
+
+
 def fields(sim):
     return [np.array(sim.field[c]) for c in sim._active]
 
@@ -45,6 +56,106 @@ def fields(sim):
 def agree(a, b):
     for x, y in zip(a, b):
         np.testing.assert_array_equal(x, y)
+
+
+@case
+def commit(lib, shim):
+    """Memory taken by others between the look at it and the allocation."""
+    for build in builders():
+        start = shim.shim_used()
+        shim.shim_peak(1)
+        sim = build(lib)
+        sim._advance(5)
+        want = fields(sim)
+        sim.close()
+        most = shim.shim_peak(1) - start
+        # on a device this small nothing is held twice: the two-kernel step
+        shim.shim_limit(start + int(1.1 * most), 1)
+        sim = build(lib)
+        sim._advance(5)
+        agree(fields(sim), want)
+        sim.close()
+        least = shim.shim_peak(1) - start
+        assert least < most
+        for q in range(13):
+            shim.shim_limit(start + least + (most - least) * q // 12 - (q == 12), 0)
+            sim = build(lib)
+            sim._advance(5)
+            agree(fields(sim), want)
+            sim.close()
+        shim.shim_limit(0, 0)
+
+
+@case
+def many_sims(lib, shim):
+    """A device that holds every sim once, but not twice: sims made later find
+    the room that the second buffers of earlier ones hold, while those are
+    being stepped."""
+    import threading
+
+    import gmes_amd as g
+    from gmes_amd.batch import Batch
+    from test_step3d import box, media_box
+
+    def made():
+        return box(lib, (40, 41, 42), bound=g.Cpml), media_box(lib, (44, 41, 42))
+
+    start = shim.shim_used()
+    pair = made()
+    twice = shim.shim_used() - start
+    for s in pair:
+        lib.set_graph(s._sim, 1)
+        s._advance(5)
+    want = [fields(s) for s in pair]
+    for s in pair:
+        s.close()
+    shim.shim_limit(start + int(1.2 * twice), 1)
+    pair = made()
+    once = shim.shim_used() - start
+    for s in pair:
+        s.close()
+    assert once < 0.8 * twice
+    shim.shim_limit(start + int(7.3 * once) + (4 << 20), 1)
+    batch = Batch([s for _ in range(2) for s in made()])
+    done = 3
+    batch.advance(done)
+    swept = [lib.footprint(s._sim) for s in batch.sims]
+    errors, sims = [], []
+
+    def work():
+        try:
+            mine = made()
+            for s in mine:
+                lib.set_graph(s._sim, 1)
+                s._advance(4)
+            sims.extend(mine)
+        except Exception as e:
+            errors.append(e)
+
+    threads = [threading.Thread(target=work) for _ in range(5)]
+    for t in threads:
+        t.start()
+    while any(t.is_alive() for t in threads):
+        k = 1 + done % 6
+        batch.advance(k)
+        done += k
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    assert [lib.footprint(s._sim) for s in batch.sims] < swept
+    for s in sims:
+        s._advance(1)
+    for q, s in enumerate(sims):
+        agree(fields(s), want[q % 2])
+    for s in sims:
+        s.close()
+    shim.shim_limit(0, 0)
+    alone = made()
+    for s in alone:
+        s._advance(done)
+    for q, s in enumerate(batch.sims):
+        agree(fields(s), fields(alone[q % 2]))
+    batch.close()
 
 
 @case
