@@ -192,12 +192,16 @@ int64_t dev_flat(const gmes_sim* s, int c, int64_t flat) {
 // Device memory.  When there is none left, the second buffers of the one-sweep
 // steps on the device make room: sims that have them never keep out what
 // would fit without them.
-bool sweep_reclaim(int device);
+void sweep_reclaim(int device);
 hipError_t dev_malloc(int device, void** p, size_t bytes) {
-  hipError_t e = hipMalloc(p, bytes);
+  const hipError_t e = hipMalloc(p, bytes);
   if (e != hipErrorOutOfMemory) return e;
   (void)hipGetLastError();
-  return sweep_reclaim(device) ? hipMalloc(p, bytes) : e;
+  // alone until it is allocated: another thread may have made room, or be
+  // about to take it
+  CaptureGuard alone;
+  sweep_reclaim(device);
+  return hipMalloc(p, bytes);
 }
 
 int dev_alloc(gmes_sim* s, void** p, size_t bytes) {
