@@ -865,7 +865,8 @@ hipError_t sync_exec(gmes_sim* s);
 //   * with dispersive cells, an auxiliary grid or sources on more than
 //     kSweepMaxSrc cells: what stepfix.hip and sweep_fix_build ask,
 //   * a component's CPML state is under 4 GiB (32-bit byte offsets),
-//   * its second buffers leave the device half empty (sweep_room), and
+//   * its second buffers leave the device half empty, or are a small part of
+//     what is idle (sweep_room), and
 //   * the caller asked for no tile and did not turn ghost fusion off.
 // Other sims keep the two-kernel step.
 constexpr int kSweepMinRows = 3;
@@ -1284,26 +1285,24 @@ void known_sim(gmes_sim* s, bool there) {
 // Releases the second buffers of every sim on a device, with no other thread
 // inside the engine: between two calls, and where a call has let go of its
 // hold (it captures a graph, or is here itself), the current buffers hold the
-// whole state, and the two-kernel step goes on from there.  False: there were
-// none.
-bool sweep_reclaim(int device) {
-  CaptureGuard alone;
+// whole state, and the two-kernel step goes on from there.
+void sweep_reclaim(int device) {
   std::lock_guard<std::mutex> lk(g_sims_mu);
-  bool any = false;
   for (gmes_sim* s : g_sims) {
     if (s->device != device || s->sweep_bytes == 0) continue;
     (void)sync_exec(s);
     destroy_graph(s);
     sweep_release(s);
-    any = true;
   }
-  return any;
 }
 
 // Whether the second buffers of s leave the device at least half empty: sims
 // that fill it keep the two-kernel step, and other users of the device find
 // room (the engine's own sims take it from here when there is none left, see
-// sweep_reclaim).
+// sweep_reclaim).  Lines and small planes take them on a fuller device too: at
+// most 1/256 of what is idle each, so never all of it.  Held until they are
+// allocated: sims set up at once count each other's.
+std::mutex g_room_mu;
 bool sweep_room(const gmes_sim* s) {
   int64_t need = (int64_t)s->g.nx * s->g.ny * s->g.nz * 4;
   for (int c = 0; c < 6; ++c) {
@@ -1316,7 +1315,7 @@ bool sweep_room(const gmes_sim* s) {
     (void)hipGetLastError();
     return false;
   }
-  return (int64_t)idle - need >= (int64_t)(total / 2);
+  return (int64_t)idle - need >= (int64_t)(total / 2) || need <= (int64_t)(idle / 256);
 }
 
 // Uploads the entry tables, those of source cells (after the step_net /
@@ -1390,6 +1389,7 @@ int sweep1_build(gmes_sim* s) {
         if (v[q] != 0.0) return GMES_OK;
     }
   }
+  std::unique_lock<std::mutex> room(g_room_mu);
   if (!sweep_room(s)) return GMES_OK;
   int rc = GMES_OK;
   for (const int c : comp) {
@@ -1410,6 +1410,7 @@ int sweep1_build(gmes_sim* s) {
     if (!rc) HIP_TRY(hipMemsetAsync(s->ade_alt[e][k], 0, b, s->stream));
   }
   if (any && !rc) rc = sweep_alloc(s, (void**)&s->d_adeq[e], (size_t)s->dsize[e] * sizeof(int32_t));
+  room.unlock();
   if (rc) {
     (void)hipGetLastError();
     sweep_release(s);
@@ -1692,6 +1693,7 @@ int sweep2_build(gmes_sim* s) {
       s->step_e.push_back({x, y, z});
     }
   }
+  std::unique_lock<std::mutex> room(g_room_mu);
   if (!sweep_room(s)) return GMES_OK;
   sweep2_shape(s);
   int rc = GMES_OK;
@@ -1715,6 +1717,7 @@ int sweep2_build(gmes_sim* s) {
     }
     if (any && !rc) rc = sweep_alloc(s, (void**)&s->d_adeq[c], (size_t)s->dsize[c] * sizeof(int32_t));
   }
+  room.unlock();
   if (!rc) rc = s->fp64 ? sweep2_tables<double>(s) : sweep2_tables<float>(s);
   if (rc) {  // no room for a second set of buffers
     (void)hipGetLastError();
@@ -2069,6 +2072,7 @@ int sweep_build(gmes_sim* s) {
       s->step_e.size() + s->step_h.size() > most)
     return GMES_OK;
   sweep_plan(s);
+  std::unique_lock<std::mutex> room(g_room_mu);
   if (!s->sweep_part.rows || !sweep_room(s)) return GMES_OK;
   // E and H entries, those of source cells included, in one 16-bit word when
   // they fit (256^3 FP32: at 4 bytes they are 67 of 1250 MB a step, 256 us; at 2
@@ -2093,6 +2097,7 @@ int sweep_build(gmes_sim* s) {
   s->step_tab_cap = (int64_t)(s->step_e.size() + s->step_h.size()) + 2 * kSweepMaxSrc;
   if (!rc) rc = sweep_alloc(s, &s->d_step_tab, (size_t)s->step_tab_cap * ent);
   if (!rc) rc = sweep_alloc(s, (void**)&s->d_rare, (size_t)s->step_tab_cap * 3 * sizeof(StepRare));
+  room.unlock();
   if (rc) {  // no room for a second set of buffers: the two-kernel step needs none
     (void)hipGetLastError();
     sweep_release(s);

@@ -3,11 +3,12 @@
  * runtime's in the engine's symbol lookup. */
 #include <pthread.h>
 #include <stddef.h>
+#include <unistd.h>
 
 enum { kSlots = 1 << 16, kOutOfMemory = 2 };
 static struct { void* p; size_t n; } slot[kSlots];
 static size_t used, peak, limit;
-static int report;
+static int report, wait_us;
 static int (*real_malloc)(void**, size_t);
 static int (*real_free)(void*);
 static int (*real_info)(size_t*, size_t*);
@@ -21,6 +22,8 @@ void shim_init(void* m, void* f, void* i) {
 /* bytes: of a device that the engine seems to have (0: no limit); r: whether
  * hipMemGetInfo says so too */
 void shim_limit(size_t bytes, int r) { limit = bytes; report = r; }
+/* hipMemGetInfo takes so long to answer */
+void shim_wait(int us) { wait_us = us; }
 size_t shim_used(void) { return used; }
 size_t shim_peak(int reset) {
   const size_t p = peak;
@@ -62,5 +65,6 @@ int hipMemGetInfo(size_t* idle, size_t* total) {
     *total = limit;
     *idle = limit > used ? limit - used : 0;
   }
+  if (wait_us) usleep(wait_us);
   return rc;
 }

@@ -28,7 +28,7 @@ def case(f):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name", ["source_lists", "commit", "many_sims"])
+@pytest.mark.parametrize("name", ["source_lists", "commit", "many_sims", "half_full", "set_up_at_once"])
 def test_limited_memory(engine_lib, tmp_path, name):
     shim = str(tmp_path / "memory_shim.so")
     subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", shim, os.path.join(HERE, "memory_shim.c"), "-lpthread"],
@@ -180,6 +180,59 @@ def source_lists(lib, shim):
             for s in (a, b):
                 s._advance(4)
             agree(fields(a), fields(b))
+
+
+def swept(lib, sim):
+    """Whether a step of sim is a one-sweep step (it launches no H kernel)."""
+    lib.profile(sim._sim, 1)
+    sim._advance(2)
+    lib.sync(sim._sim)
+    launches = lib.read_profile(sim._sim)[1]
+    lib.profile(sim._sim, 0)
+    return launches[1] == 0
+
+
+@case
+def half_full(lib, shim):
+    """Small sims take one-sweep steps however full the device is; large ones
+    do not when they would fill more than half of it."""
+    import gmes_amd as g
+    from test_step1d import line
+    from test_step2d import plane
+    from test_step3d import box
+    shim.shim_limit(shim.shim_used() + (16 << 20), 1)
+    large = [box(lib, (40, 41, 42), bound=g.Cpml) for _ in range(2)]
+    assert not swept(lib, large[1])
+    shim.shim_limit(shim.shim_used() + (10 << 20), 1)
+    small = [line(lib, "z", 300, bound=g.Cpml, media=True), plane(lib, "tmz", (20, 24))]
+    assert all(swept(lib, s) for s in small)
+
+
+@case
+def set_up_at_once(lib, shim):
+    """Sims committed by several threads together do not take the same room."""
+    import threading
+
+    import gmes_amd as g
+    from test_step3d import box
+    start = shim.shim_used()
+    sim = box(lib, (40, 41, 42), bound=g.Cpml)
+    twice = shim.shim_used() - start
+    shim.shim_limit(shim.shim_used() + 1, 1)
+    lib.commit(sim._sim)
+    once = shim.shim_used() - start
+    shim.shim_limit(shim.shim_used() + 4 * once, 1)
+    sims = [sim] + [box(lib, (40, 41, 42), bound=g.Cpml) for _ in range(3)]
+    assert not any(swept(lib, s) for s in sims)
+    shim.shim_limit(start + 2 * (4 * once + 5 * (twice - once) // 4), 1)
+    shim.shim_wait(50000)
+    threads = [threading.Thread(target=lib.commit, args=(s._sim,)) for s in sims]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    shim.shim_wait(0)
+    assert sum(swept(lib, s) for s in sims) == 1
 
 
 def main(path, name):
