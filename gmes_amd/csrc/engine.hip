@@ -1083,7 +1083,7 @@ void sweep_entry(const gmes_sim* s, const std::array<uint16_t, 3>& rec, StepEnt<
     if (r.cls >= GMES_CLS_DRUDE) e.c[t] = 0;  // keeps its value: see stepfix.hip
     else if (rare[t].keep) e.meta |= kStepRareCell;
     else e.c[t] = upml ? (s->fp64 ? (R)r.eps_mu : (R)(1.0 / r.eps_mu)) : (R)(s->g.dt / r.eps_mu);
-    if (upml) e.meta |= 2u << t;
+    if (upml || r.cls == GMES_CLS_CPML) e.meta |= 2u << t;
   }
 }
 

@@ -115,14 +115,12 @@ struct MainArgs {
 // so E can be computed again where a neighbouring block needs it and H
 // follows from it at once.  A cell's three E components (and the three H
 // components the same thread owns) share one table entry.
-// Dummy, Const and source cells are flagged (StepRare has the details);
-// every other cell of a sim without UPML runs one formula: at a coordinate
-// without live state the CPML update is the Dielectric one.
-constexpr uint32_t kStepRareCell = 1, kStepUpmlCells = 14;  // UPML: bit 1 + t for component t
+// Dummy, Const and source cells are flagged (StepRare has the details).
+constexpr uint32_t kStepRareCell = 1, kStepAbsorberCells = 14;  // CPML, UPML: bit 1 + t for component t
 template <class R>
 struct alignas(16) StepEnt {
   R c[3];         // dt/eps; UPML cells: 1/eps (FP32) or eps (FP64)
-  uint32_t meta;  // kStepRareCell | 2 << t per UPML component
+  uint32_t meta;  // kStepRareCell | 2 << t per absorber component
 };
 
 // Absorbers of a one-sweep step: none, CPML with state along x, y and z, UPML,

@@ -101,7 +101,7 @@ __device__ __forceinline__ void bst(const GMES_CONST i4_t& r, unsigned v, unsign
 // cost 12 (CPML) to 24 (UPML) of them, twice that in FP64.
 template <int PML> struct RowStride { static constexpr int v = PML == 2 ? 8 : 4; };
 // A CPML coordinate without live state: c = 0, kappa = 1, and b multiplies a
-// word that is +0, so the CPML update below is the Dielectric one.
+// word that is +0.
 template <class R, int PML>
 __device__ __forceinline__ void stage_row(R* dst, const R* shared, const R* own, int xs, int xo, bool live) {
   if constexpr (PML != 2) {
@@ -547,6 +547,9 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
     const unsigned eid = l.id & ((1u << m->eb) - 1u);
     const StepEnt<R> en = et[eid];
     const R d0 = m->d[0], d1 = m->d[1], d2 = m->d[2], v0 = m->inv_d[0], v1 = m->inv_d[1], v2 = m->inv_d[2];
+    // a wave without live words, but with CPML cells, takes their formula too
+    // (with words of 0): its value is not the Dielectric one where a difference
+    // is infinite
     T nex, ney, nez;
     auto plain_e = [&]() {
       nex = plain_value<true, X>(en.c[0], l.e0, vsub(l.hz, hzj), vsub(l.hy, hyk), d1, v1, d2, v2);
@@ -555,7 +558,7 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
     };
     if constexpr (PML == 0) {
       plain_e();
-    } else if (!pml) {
+    } else if (!pml && !(CP && __any(en.meta & kStepAbsorberCells))) {
       plain_e();
       meta_e = 0;
     } else {
@@ -563,13 +566,15 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
                   ry = CP && !LY ? dead_row<R, PML>() : lds_row<R, PML>(rows_y + tj * rs),
                  rz = lds_row<R, PML>(rows_z + k * rs);
       if constexpr (CP) {
+        T dead1, dead2;
         nex = cpml_value<true, X>(en.c[0], l.e0, vsub(l.hz, hzj), vsub(l.hy, hyk), d1, v1, d2, v2, ry, rz, s00, l.s[0],
-                                  n[0][0], n[0][1]);
+                                  n[0][0], n[0][1], en.meta & 2u);
         ney = cpml_value<true, X>(en.c[1], l.e1, vsub(l.hx, hxk), vsub(l.hz, hzp), d2, v2, d0, v0, rz, rx, l.s[1], s11,
-                                  n[1][0], n[1][1]);
-        if constexpr (!LX && !LY) nez = plain_value<true, X>(en.c[2], l.e2, vsub(l.hy, hyp), vsub(l.hx, hxj), d0, v0, d1, v1);
+                                  n[1][0], n[1][1], en.meta & 4u);
+        if constexpr (!LX && !LY) nez = cpml_value<true, X>(en.c[2], l.e2, vsub(l.hy, hyp), vsub(l.hx, hxj), d0, v0, d1, v1,
+                                  dead_row<R, PML>(), dead_row<R, PML>(), T{}, T{}, dead1, dead2, en.meta & 8u);
         else nez = cpml_value<true, X>(en.c[2], l.e2, vsub(l.hy, hyp), vsub(l.hx, hxj), d0, v0, d1, v1, rx, ry, s20, s21,
-                                  n[2][0], n[2][1]);
+                                  n[2][0], n[2][1], en.meta & 8u);
       } else {
         plain_e();
         meta_e = en.meta;
@@ -668,7 +673,7 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
       };
       if constexpr (PML == 0) {
         plain_h();
-      } else if (!pml) {
+      } else if (!pml && !(CP && __any(eh.meta & kStepAbsorberCells))) {
         plain_h();
         meta_h = 0;
       } else {
@@ -676,13 +681,15 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
                     ry = CP && !LY ? dead_row<R, PML>() : lds_row<R, PML>(rows_yh + tj * rs),
                    rz = lds_row<R, PML>(rows_zh + k * rs);
         if constexpr (CP) {
+          T dead1, dead2;
           nhx = cpml_value<false, X>(eh.c[0], hx, vsub(ezj, ez), vsub(eyk, ey), d1, v1, d2, v2, ry, rz, g00, l.g[0],
-                                     r[0][0], r[0][1]);
+                                     r[0][0], r[0][1], eh.meta & 2u);
           nhy = cpml_value<false, X>(eh.c[1], hy, vsub(exk, ex), vsub(ezi, ez), d2, v2, d0, v0, rz, rx, l.g[1], g11,
-                                     r[1][0], r[1][1]);
-          if constexpr (!LX && !LY) nhz = plain_value<false, X>(eh.c[2], hz, vsub(eyi, ey), vsub(exj, ex), d0, v0, d1, v1);
+                                     r[1][0], r[1][1], eh.meta & 4u);
+          if constexpr (!LX && !LY) nhz = cpml_value<false, X>(eh.c[2], hz, vsub(eyi, ey), vsub(exj, ex), d0, v0, d1, v1,
+                                  dead_row<R, PML>(), dead_row<R, PML>(), T{}, T{}, dead1, dead2, eh.meta & 8u);
           else nhz = cpml_value<false, X>(eh.c[2], hz, vsub(eyi, ey), vsub(exj, ex), d0, v0, d1, v1, rx, ry, g20, g21,
-                                     r[2][0], r[2][1]);
+                                     r[2][0], r[2][1], eh.meta & 8u);
         } else {
           plain_h();
           meta_h = eh.meta;

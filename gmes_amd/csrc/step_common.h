@@ -44,10 +44,25 @@ struct Rows {
   R v[PML == 2 ? 6 : 3];
 };
 
+__device__ __forceinline__ float vneg(float a) { return -a; }
+__device__ __forceinline__ double vneg(double a) { return -a; }
+template <class R>
+__device__ __forceinline__ cplx<R> vneg(cplx<R> a) {
+  return {-a.re, -a.im};
+}
+template <class T>
+__device__ __forceinline__ T vsel(bool c, T a, T b) {
+  if constexpr (is_cplx<T>::value) return {c ? a.re : b.re, c ? a.im : b.im};
+  else return c ? a : b;
+}
+
 // New value of one component, with the formulas and operand order of
 // update_value (kernels.hip).  plain: Dielectric; cpml: CPML with rows r1, r2
-// of the curl axes, old words o1, o2 and new ones n1, n2; upml: rows r1, r2
-// of the curl axes and r0 of the own one.
+// of the curl axes, old words o1, o2 and new ones n1, n2 (of a lane that is
+// no CPML cell, `is` false, the Dielectric value all the same: where both
+// words are dead the two agree in finite values but zeros' signs, and an
+// infinite difference times c = 0 is NaN); upml: rows r1, r2 of the curl axes
+// and r0 of the own one.
 template <bool E, bool X, class T, class R>
 __device__ __forceinline__ T plain_value(R c, T f, T D1, T D2, R d1, R i1, R d2, R i2) {
   if constexpr (std::is_same<R, float>::value) {
@@ -61,19 +76,19 @@ __device__ __forceinline__ T plain_value(R c, T f, T D1, T D2, R d1, R i1, R d2,
 
 template <bool E, bool X, class T, class R>
 __device__ __forceinline__ T cpml_value(R c, T f, T D1, T D2, R d1, R i1, R d2, R i2, const Rows<R, 1>& r1,
-                                        const Rows<R, 1>& r2, T o1, T o2, T& n1, T& n2) {
+                                        const Rows<R, 1>& r2, T o1, T o2, T& n1, T& n2, bool is = true) {
   if constexpr (std::is_same<R, float>::value) {
     const T a = vscl(i1, D1), b = vscl(i2, D2);
     n1 = fma_(r1.v[1], a, vscl(r1.v[0], o1));
     n2 = fma_(r2.v[1], b, vscl(r2.v[0], o2));
     const T t = vsub(vadd(fma_(-r2.v[2], b, vscl(r1.v[2], a)), n1), n2);
-    return E ? fma_(c, t, f) : fma_(-c, t, f);
+    return fma_(c, vsel(is, E ? t : vneg(t), E ? vsub(a, b) : vsub(b, a)), f);
   } else {
+    const T a = by_size<X>(D1, d1, i1), b = by_size<X>(D2, d2, i2);
     n1 = vadd(vscl(r1.v[0], o1), by_size<X>(vscl(r1.v[1], D1), d1, i1));
     n2 = vadd(vscl(r2.v[0], o2), by_size<X>(vscl(r2.v[1], D2), d2, i2));
-    const T t = vsub(vadd(vsub(by_kappa<X>(by_size<X>(D1, d1, i1), r1.v[2]),
-                               by_kappa<X>(by_size<X>(D2, d2, i2), r2.v[2])), n1), n2);
-    return E ? vadd(f, vscl(c, t)) : vsub(f, vscl(c, t));
+    const T t = vsub(vadd(vsub(by_kappa<X>(a, r1.v[2]), by_kappa<X>(b, r2.v[2])), n1), n2);
+    return vadd(f, vscl(c, vsel(is, E ? t : vneg(t), E ? vsub(a, b) : vsub(b, a))));
   }
 }
 

@@ -124,10 +124,17 @@ __device__ __forceinline__ void fix_h(FixPtr<T> m, int b) {
   const T D1 = vsub(moved<T, R>(e2, m->pe[a2], m->re[a2], m->n, x, a1, 1, m->phe[a2][a1]), E2);
   const T D2 = vsub(moved<T, R>(e1, m->pe[a1], m->re[a1], m->n, x, a2, 1, m->phe[a1][a2]), E1);
   const int cls = gld(&rec->cls);
-  T v = cls == GMES_CLS_DUMMY ? old
-        : cls == GMES_CLS_CONST
-            ? make_val<T>(gld(&rec->val_re), gld(&rec->val_im))
-            : plain_value<false, false>(gld(&rec->c0), old, D1, D2, m->d[a1], m->inv_d[a1], m->d[a2], m->inv_d[a2]);
+  T v;
+  if (cls == GMES_CLS_DUMMY) {
+    v = old;
+  } else if (cls == GMES_CLS_CONST) {
+    v = make_val<T>(gld(&rec->val_re), gld(&rec->val_im));
+  } else {  // Dielectric, or CPML at dead coordinates
+    const Rows<R, 1> dead{{R(0), R(0), R(1)}};
+    T w1, w2;
+    v = cpml_value<false, false>(gld(&rec->c0), old, D1, D2, m->d[a1], m->inv_d[a1], m->d[a2], m->inv_d[a2], dead, dead,
+                                 T{}, T{}, w1, w2, cls == GMES_CLS_CPML);
+  }
   if (grp >= 0) v = fix_source<T>(m, m->groups[grp], v);
   gst(m->ho[c] + h, v);
 }
