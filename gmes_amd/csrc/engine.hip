@@ -856,9 +856,9 @@ hipError_t sync_exec(gmes_sim* s);
 // A real FP32 or FP64, or complex FP32, 3-D sim takes them when
 //   * it holds no DM2 cells, and one kind of absorber with one profile set,
 //     whose two rows per axis agree (a single Shell),
-//   * three whole (j, k) rows fit a block (nz <= 341; 256 with 8-byte words and
-//     an absorber along x or y), so that at most half of the E work is done
-//     twice,
+//   * three whole (j, k) rows fit a block, with some absorbers more
+//     (sweep_min_rows): nz <= 341; 256 with 8-byte words and an absorber along
+//     x or y; at most half of the E work is done twice,
 //   * its distinct triples of records fit a block's LDS,
 //   * its sources are off the ghost planes, and no E probe sits on a ghost
 //     plane (it reads the plane before the copy),
@@ -1098,6 +1098,21 @@ void sweep_entry(const gmes_sim* s, const std::array<uint16_t, 3>& rec, StepEnt<
 constexpr int64_t kSweepSplitBytes = 5 << 20;
 constexpr int kSweepOuterPlanes = 6, kSweepInnerPlanes = 9;
 
+// Whole rows a block needs, so that the rim row, whose E it computes again, is
+// worth it: three; with UPML, or in complex sims CPML along x or y, whose
+// bodies hold few waves, five of 8-byte words and four of 4-byte ones, unless
+// the launches bound the two-kernel step (us per step, that one against this:
+// complex FP32 CPML 120 x 30 x 200 46, 58; 160^3 163, 168; 144^3, five rows,
+// 122, 116; UPML 160^3 FP64 182, 215; 144^3 136, 138; 96 x 96 x 256 FP64 106,
+// 119; FP32, three rows, 160 x 200 x 310 221, 240; 40 x 40 x 341 28, 23; FP64
+// CPML 96 x 96 x 256 118, 99).
+constexpr int64_t kSweepLongBytes = 4 << 20;
+int sweep_min_rows(const gmes_sim* s, int absorber) {
+  if (s->ncell[0] * s->esize < kSweepLongBytes || absorber == kPmlNone || absorber == kPmlZ) return kSweepMinRows;
+  if (absorber == kUpml) return s->esize == 8 ? 5 : 4;
+  return s->complex_ ? 5 : kSweepMinRows;
+}
+
 // The launches of a step.  A block's march costs its planes and two more (the
 // rim plane, the prologue); blocks run in rounds over the 256 CUs, a last
 // incomplete round costing about half of one; a CU with few waves still pays
@@ -1112,10 +1127,9 @@ double sweep_shape(const gmes_sim* s, int nent, int absorber, int ni, int nj, gm
   const int nz = s->g.nz;
   double best = 0;
   part.absorber = absorber;
-  for (int rows = 2; rows <= nj + 1; ++rows) {
+  for (int rows = sweep_min_rows(s, absorber); rows <= nj + 1; ++rows) {
     const int threads = (rows * nz + 63) / 64 * 64, most = step3_max_threads<T>(absorber);
     if (threads > most) break;
-    if (rows < kSweepMinRows && kSweepMinRows * nz <= most && nj + 1 >= kSweepMinRows) continue;
     const int64_t lds = (int64_t)step3_lds<T>(threads, nent, rows, nz, absorber);
     if (lds > kSweepLds) break;
     // waves a CU holds: registers (see StepWaves)
@@ -1192,7 +1206,7 @@ bool sweep_batch_part(const gmes_sim* s, gmes_sim::SweepPart& part, bool& lean, 
   part = gmes_sim::SweepPart{};
   part.threads = s->esize == 8 ? step3_batch_threads<double>(lean) : step3_batch_threads<float>(lean);
   part.rows = std::min(part.threads / nz, ny + 1);
-  if (kSweepMinRows * nz > part.threads || part.rows < 2) return false;
+  if (part.rows < kSweepMinRows) return false;
   part.absorber = s->sweep_absorber;
   if (lean) sweep_rect(part, 0, nx, 0, ny, ch, s->sweep_absorber ? kPmlZ : kPmlNone);
   else if (ib > ia && jb > ja) sweep_rects(part, nx, ny, ia, ib, ja, jb, std::min(ch, kSweepOuterPlanes), ch);
