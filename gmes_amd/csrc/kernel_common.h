@@ -179,15 +179,17 @@ __device__ __forceinline__ void fused_ghost(const MainArgs<T>& m, int C, T* __re
 }
 
 // Dispersive (ADE) cells: the new value of cell q of a list of n cells from
-// its old value e_now and the curl cu = D1/d1 - D2/d2.  State words are read
+// its old value e_now and the curl cu() = D1/d1 - D2/d2, which the two-kernel
+// step's lists load when the state words are on their way back (before them,
+// the Drude list of 160^3 FP64 took 82 us for 76).  State words are read
 // from st and the new ones written to so (the same array, or the other set
 // of a one-sweep step; `keep` false: not at all).  a: the record's
 // coefficients, P1 and P2 its pole counts.
 //
 // Drude and Lorentz poles: src/pw_drude.hh:90-101,145-150; src/pw_lorentz.hh:96-107,150-156
-template <class T>
+template <class T, class Cu>
 __device__ __forceinline__ T ade_drude_value(const typename real_of<T>::type* a, int P, const T* st, T* so, int n,
-                                             int q, bool keep, T e_now, T cu) {
+                                             int q, bool keep, T e_now, Cu cu) {
   const auto* cc = a + 3 * P;
   T sum = vzero<T>();
   for (int p = 0; p < P; ++p) {
@@ -200,14 +202,15 @@ __device__ __forceinline__ T ade_drude_value(const typename real_of<T>::type* a,
     }
     sum = vadd(sum, vsub(q_new, q_now));
   }
-  return vadd(vadd(vscl(gld(cc), cu), vscl(gld(cc + 1), sum)), vscl(gld(cc + 2), e_now));
+  const T c = cu();
+  return vadd(vadd(vscl(gld(cc), c), vscl(gld(cc + 1), sum)), vscl(gld(cc + 2), e_now));
 }
 
 // Drude-critical-points, ADE form: src/pw_dcp.hh:105-167,200-225
 // words: 0 e_old | 1..D q_old | D+1..2D q_now | 2D+1.. p_old | 2D+C+1.. p_now
-template <class T>
+template <class T, class Cu>
 __device__ __forceinline__ T ade_dcp_value(const typename real_of<T>::type* a, int D, int NC, const T* st, T* so,
-                                           int n, int q, bool keep, T e_now, T cu) {
+                                           int n, int q, bool keep, T e_now, Cu cu) {
   using R = typename real_of<T>::type;
   const R* b = a + 3 * D;
   const R* cc = b + 5 * NC;
@@ -219,7 +222,8 @@ __device__ __forceinline__ T ade_dcp_value(const typename real_of<T>::type* a, i
   for (int p = 0; p < NC; ++p)
     cs = vadd(cs, vsub(vscl(R(1) - gld(b + 5 * p + 1), gld(st + (1 + 2 * D + NC + p) * n + q)),
                        vscl(gld(b + 5 * p), gld(st + (1 + 2 * D + p) * n + q))));
-  const T e_new = vadd(vadd(vadd(vscl(gld(cc), cu), vscl(gld(cc + 1), vadd(ds, cs))), vscl(gld(cc + 2), e_old)),
+  const T c = cu();
+  const T e_new = vadd(vadd(vadd(vscl(gld(cc), c), vscl(gld(cc + 1), vadd(ds, cs))), vscl(gld(cc + 2), e_old)),
                        vscl(gld(cc + 3), e_now));
   if (!keep) return e_new;
   const T mix = vadd(vadd(e_old, vscl(R(2), e_now)), e_new);
@@ -245,10 +249,10 @@ __device__ __forceinline__ T ade_dcp_value(const typename real_of<T>::type* a, i
 // Drude-critical-points, PLRC/RC form: src/pw_dcp.hh:467-518,564-586.
 // State words are complex for any field type: psi_dp (re part = psi_dp_re,
 // im part = psi_dp_im), psi_cp_re, psi_cp_im.
-template <class T>
+template <class T, class Cu>
 __device__ __forceinline__ T ade_plrc_value(const typename real_of<T>::type* a, int D, int NC,
                                             const cplx<typename real_of<T>::type>* st,
-                                            cplx<typename real_of<T>::type>* so, int n, int q, bool keep, T fv, T cu) {
+                                            cplx<typename real_of<T>::type>* so, int n, int q, bool keep, T fv, Cu cu) {
   using R = typename real_of<T>::type;
   using Z = cplx<R>;
   const R* b = a + 3 * D;
@@ -265,10 +269,11 @@ __device__ __forceinline__ T ade_plrc_value(const typename real_of<T>::type* a, 
   for (int p = 0; p < NC; ++p) sci = vadd(sci, gld(st + (D + NC + p) * n + q));
   const Z psi = {sdr + scr.re, sdi + sci.re};  // .real() of the imaginary-part sum
   Z e_new;
+  const T c = cu();
   if constexpr (is_cplx<T>::value) {
-    e_new = vadd(vadd(vscl(gld(cc), Z{cu.re, cu.im}), vscl(gld(cc + 1), e_now)), vscl(gld(cc + 2), psi));
+    e_new = vadd(vadd(vscl(gld(cc), Z{c.re, c.im}), vscl(gld(cc + 1), e_now)), vscl(gld(cc + 2), psi));
   } else {
-    e_new.re = (gld(cc) * cu + gld(cc + 1) * e_now.re) + gld(cc + 2) * psi.re;
+    e_new.re = (gld(cc) * c + gld(cc + 1) * e_now.re) + gld(cc + 2) * psi.re;
     e_new.im = gld(cc + 1) * e_now.im + gld(cc + 2) * psi.im;
   }
   if (keep) {
@@ -289,9 +294,9 @@ __device__ __forceinline__ T ade_plrc_value(const typename real_of<T>::type* a, 
   return make_val<T>(e_new.re, e_new.im);
 }
 
-template <class T>
+template <class T, class Cu>
 __device__ __forceinline__ T ade_value(int cls, const typename real_of<T>::type* a, int P1, int P2, const void* st,
-                                       void* so, int n, int q, bool keep, T e_now, T cu) {
+                                       void* so, int n, int q, bool keep, T e_now, Cu cu) {
   using Z = cplx<typename real_of<T>::type>;
   if (cls == GMES_CLS_DRUDE)
     return ade_drude_value<T>(a, P1, static_cast<const T*>(st), static_cast<T*>(so), n, q, keep, e_now, cu);

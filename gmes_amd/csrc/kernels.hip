@@ -859,9 +859,11 @@ __device__ __forceinline__ void ade_cell(const AdeArgs<T>& m, int q, int cls) {
   const DevRec<R>& rec = m.recs[m.rec[q]];
   T* F = m.fa.f[C] + didx(m.fa, C, i, j, k);
   const T e_now = ld_nt(F);
-  T D1, D2;
-  curl_terms<C>(m.fa, i, j, k, D1, D2);
-  const T cu = vsub(vdiv(D1, m.d[Ax<C>::a1]), vdiv(D2, m.d[Ax<C>::a2]));
+  const auto cu = [&]() -> T {
+    T D1, D2;
+    curl_terms<C>(m.fa, i, j, k, D1, D2);
+    return vsub(vdiv(D1, m.d[Ax<C>::a1]), vdiv(D2, m.d[Ax<C>::a2]));
+  };
   st_nt(F, ade_value<T>(cls, m.coef + rec.coef_off, rec.n1, rec.n2, m.state, m.state, m.n, q, true, e_now, cu));
 }
 template <int C, class T>

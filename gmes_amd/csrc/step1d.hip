@@ -99,7 +99,8 @@ __device__ __forceinline__ T step1_value(Step1Ptr<T> m, int q, const Step1Ops<T,
     }
   }
   if (E && cls >= GMES_CLS_DRUDE) {
-    const T cu = vsub(vdiv(D1, m->d[a1]), vdiv(D2, m->d[a2]));
+    const T curl = vsub(vdiv(D1, m->d[a1]), vdiv(D2, m->d[a2]));
+    const auto cu = [curl] { return curl; };
     const int k = cls - GMES_CLS_DRUDE;
     return ade_value<T>(cls, m->coef + l.rec.coef_off, l.rec.n1, l.rec.n2, k == 0 ? m->ade_in[0] : k == 1 ? m->ade_in[1] : m->ade_in[2],
                         k == 0 ? m->ade_out[0] : k == 1 ? m->ade_out[1] : m->ade_out[2],

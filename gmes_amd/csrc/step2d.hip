@@ -261,7 +261,8 @@ __device__ __forceinline__ void step2d_tile(Step2Ptr<T> mp, unsigned blk, char* 
         const int cls = gld(&rec->cls), s = cls - GMES_CLS_DRUDE;
         const int q = gld(m->adeq[cc] + ((unsigned)qe * pi + (unsigned)j));
         const int a1 = cc == 2 ? 0 : cc + 1, a2 = cc == 0 ? 2 : cc - 1;
-        const T cu = vsub(vdiv(D1, m->d[a1]), vdiv(D2, m->d[a2]));
+        const T curl = vsub(vdiv(D1, m->d[a1]), vdiv(D2, m->d[a2]));
+        const auto cu = [curl] { return curl; };
         const bool keep = own && qe >= i0 && qe < i1;
         const R* a = m->coef + gld(&rec->coef_off);
         const int p1 = gld(&rec->n1), p2 = gld(&rec->n2);

@@ -100,7 +100,8 @@ __device__ __forceinline__ void fix_e(FixPtr<T> m, int b) {
   const T h1 = gld(m->hi[a1] + x[0] * m->ph[a1] + x[1] * m->rh[a1] + x[2]);
   const T D1 = vsub(h2, moved<T, R>(m->hi[a2], m->ph[a2], m->rh[a2], m->n, x, a1, -1, m->phh[a2][a1]));
   const T D2 = vsub(h1, moved<T, R>(m->hi[a1], m->ph[a1], m->rh[a1], m->n, x, a2, -1, m->phh[a1][a2]));
-  const T cu = vsub(vdiv(D1, m->d[a1]), vdiv(D2, m->d[a2]));
+  const T curl = vsub(vdiv(D1, m->d[a1]), vdiv(D2, m->d[a2]));
+  const auto cu = [curl] { return curl; };
   gst(m->eo[c] + e, ade_value<T>(m->ade[l].cls, m->coef + gld(&rec->coef_off), gld(&rec->n1), gld(&rec->n2),
                                 m->ade[l].state, m->ade[l].state, m->ade[l].n, q, true, e_now, cu));
 }
