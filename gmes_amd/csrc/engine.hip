@@ -863,7 +863,8 @@ hipError_t sync_exec(gmes_sim* s);
 //   * its sources are off the ghost planes, and no E probe sits on a ghost
 //     plane (it reads the plane before the copy),
 //   * with dispersive cells, an auxiliary grid or sources on more than
-//     kSweepMaxSrc cells: what stepfix.hip and sweep_fix_build ask,
+//     kSweepMaxSrc cells: what stepfix.hip and sweep_fix_build ask, and not too
+//     many of them (sweep_list_limit),
 //   * a component's CPML state is under 4 GiB (32-bit byte offsets),
 //   * its second buffers leave the device half empty, or are a small part of
 //     what is idle (sweep_room), and
@@ -1829,11 +1830,35 @@ Step2Args<T> step2_args(const gmes_sim* s) {
 
 bool step2_ade(const gmes_sim* s) { return s->d_adeq[0] || s->d_adeq[1] || s->d_adeq[2]; }
 
+// Bytes of the cells that a step may finish after the sweep (dispersive E, and
+// the H cells listed): those move twice, while the sweep saves a third of the
+// whole grid's, and more where the two-kernel step has absorber words to read
+// again.  us per step, that one against this, small Drude or critical-point
+// blocks all over: no absorber, FP64 160^3 41 MB 166, 161; 82 MB 185, 191;
+// 96^3 31 MB 63, 62; complex FP32 128^3 21 MB 102, 102; 37 MB 112, 119; FP32
+// 160^3 36 MB 129, 125; 59 MB 151, 162; CPML FP64 160^3 34 MB 234, 230; FP32
+// 192^3 30 MB 210, 191; CPML on z alone, complex FP32 384 x 384 x 192 173 MB
+// (13 % of the cells) 1489, 1450.
+double sweep_list_limit(const gmes_sim* s) {
+  switch (s->sweep_part.absorber) {
+    case kPmlNone: return s->esize == 8 ? 20e6 : 35e6;
+    case kUpml: return s->esize == 8 ? 12e6 : 35e6;
+    case kPmlZ: return std::max(72e6, 0.15 * 6 * s->ncell[0] * s->esize);
+    default: return 35e6;
+  }
+}
+int64_t ade_cells(const gmes_sim* s) {
+  int64_t n = 0;
+  for (int c = 0; c < 3; ++c)
+    for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2; ++k) n += s->ade[c][k].n;
+  return n;
+}
+
 // Lists the H cells that a step finishes after the sweep (stepfix.hip).
 // sweep_src_ok is false, and the sim keeps the two-kernel step, when an
 // operation acts on a ghost cell or on a dispersive one (its order after the
-// medium's update would need another launch), or when one of those H cells has
-// live absorber state.
+// medium's update would need another launch), when one of those H cells has
+// live absorber state, or when they are too many (sweep_list_limit).
 int sweep_fix_build(gmes_sim* s) {
   HIP_TRY(sync_exec(s));
   fix_release(s);
@@ -1909,6 +1934,10 @@ int sweep_fix_build(gmes_sim* s) {
       b.nitem[c] = total - b.first_item[c];
     }
     if (!total) return hipSuccess;
+    if ((double)(total + ade_cells(s)) * s->esize > sweep_list_limit(s)) {
+      bad = 1;
+      return hipSuccess;
+    }
     if ((e = hipMalloc(&s->d_fix_items, (size_t)total * sizeof(FixItem))) != hipSuccess) return e;
     s->fix_bytes = (int64_t)total * sizeof(FixItem);
     s->bytes += s->fix_bytes;
@@ -2086,8 +2115,11 @@ int sweep_build(gmes_sim* s) {
       s->step_e.size() + s->step_h.size() > most)
     return GMES_OK;
   sweep_plan(s);
+  if (!s->sweep_part.rows) return GMES_OK;
+  // (they are read by at least as many H cells)
+  if (2.0 * ade_cells(s) * s->esize > sweep_list_limit(s)) return GMES_OK;
   std::unique_lock<std::mutex> room(g_room_mu);
-  if (!s->sweep_part.rows || !sweep_room(s)) return GMES_OK;
+  if (!sweep_room(s)) return GMES_OK;
   // E and H entries, those of source cells included, in one 16-bit word when
   // they fit (256^3 FP32: at 4 bytes they are 67 of 1250 MB a step, 256 us; at 2
   // 248.  181 x 203 x 225 UPML 173, 168)

@@ -7,10 +7,13 @@
 // the E sources; k_fix_h computes the H cells next to those again, from the old
 // H and the new E, and applies the H sources.  The absorber state of such an H
 // cell would have advanced twice: sims that have one take the two-kernel step.
-// The lists are a small part of the cells, and each launch is bound by its
+// While the lists are a small part of the cells, each launch is bound by its
 // start and the latency of its few dependent loads (4 to 6 us; the two-kernel
 // step has one launch per dispersive class and component, two for sources, two
-// for ghosts).  Per step, two-kernel step first: complex FP32 192 x 192 x 128,
+// for ghosts); where media fill much of the grid they move most of E and H a
+// second time (complex FP32 384 x 384 x 192 with 12 % dispersive cells: 0.35 and
+// 0.29 ms beside the sweep's 0.785), and sims with more take the two-kernel step
+// (sweep_list_limit).  Per step, two-kernel step first: complex FP32 192 x 192 x 128,
 // dispersive objects and a plane wave, 252 -> 180 us (137 of them the sweep,
 // k_fix_h 24, k_fix_e 11); 112^3 slab with a plane wave and a flux plane 105 ->
 // 76 (46, 11, 5); FP32 96^3 CPML box with dispersive objects 64 -> 36.
