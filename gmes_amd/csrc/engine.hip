@@ -3758,9 +3758,11 @@ struct gmes_batch {
   int dtype = 0;
   hipStream_t stream = nullptr;
   bool use_graph = true;
-  hipGraphExec_t graph_exec = nullptr;
-  std::vector<uint64_t> gens;  // member generations the graph was captured with
-  int per = 1;                 // steps it holds
+  // Captured steps.  Without one-sweep members: one step ([0][0]).  With them,
+  // by the buffer set they start from (theirs swap with every step): two steps,
+  // and the last one or two of an odd or even call, which write the ghost planes.
+  hipGraphExec_t graphs[2][3] = {};
+  std::vector<uint64_t> gens;  // member generations they were captured with
   // job tables: one device buffer, rebuilt on the host for every call
   void* d_jobs = nullptr;
   size_t jobs_cap = 0;
@@ -4177,10 +4179,11 @@ void enqueue_batch_step(gmes_batch* b, int variant, hipStream_t st) {
 }
 
 void destroy_batch_graph(gmes_batch* b) {
-  if (b->graph_exec) {
-    (void)hipGraphExecDestroy(b->graph_exec);
-    b->graph_exec = nullptr;
-  }
+  for (auto& set : b->graphs)
+    for (hipGraphExec_t& g : set) {
+      if (g) (void)hipGraphExecDestroy(g);
+      g = nullptr;
+    }
 }
 
 std::vector<uint64_t> batch_gens(const gmes_batch* b) {
@@ -4193,7 +4196,25 @@ std::vector<uint64_t> batch_gens(const gmes_batch* b) {
   return gens;
 }
 
-// The job tables of a call of nsteps on the device, and its graph; ready is
+// The buffers of the one-sweep members become the other set.
+void batch_swap(gmes_batch* b) {
+  for (gmes_sim* s : b->sweepers) {
+    sweep_swap(s);
+    sweep_swap_aux(s);
+  }
+}
+
+hipGraphExec_t& batch_graph(gmes_batch* b, int kind) {
+  return b->graphs[b->sweepers.empty() ? 0 : b->sweepers[0]->par][kind];
+}
+
+// Whether a call of nsteps replays the graph of a kind (gmes_batch::graphs).
+bool batch_uses(const gmes_batch* b, int kind, int64_t nsteps) {
+  if (b->sweepers.empty()) return kind == 0;
+  return kind == 0 ? nsteps > 2 : kind == 1 ? nsteps % 2 == 1 : nsteps % 2 == 0;
+}
+
+// The job tables of a call of nsteps on the device, and its graphs; ready is
 // false when a member changed meanwhile, where this call waited to be alone
 // in the engine (dev_malloc, the capture).
 int batch_ready(gmes_batch* b, int64_t nsteps, bool& ready) {
@@ -4263,19 +4284,21 @@ int batch_ready(gmes_batch* b, int64_t nsteps, bool& ready) {
   if (sig != b->shape_sig || gens != b->gens) destroy_batch_graph(b);
   b->shape_sig = sig;
   b->gens = gens;
-  // one-sweep members swap buffers: their graph holds two steps, and the last
-  // step, which writes the ghost planes, is launched by itself
-  b->per = b->sweepers.empty() ? 1 : 2;
-  if (b->use_graph && !b->timing.on && !b->graph_exec && nsteps >= 2 * b->per - 1) {
+  for (int kind = 0; kind < 3 && b->use_graph && !b->timing.on; ++kind) {
+    hipGraphExec_t& exec = batch_graph(b, kind);
+    if (exec || !batch_uses(b, kind, nsteps)) continue;
     hipGraph_t graph;
     hipError_t e;
     {
       CaptureGuard capture;
       if (gens != batch_gens(b)) return GMES_OK;
       HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-      for (int k = 0; k < b->per; ++k) enqueue_batch_step(b, k, b->stream);
+      const int first = kind == 1 ? 2 : 0;  // the tables (gmes_batch::sweep) of its steps
+      enqueue_batch_step(b, first, b->stream);
+      if (!b->sweepers.empty() && kind != 1) enqueue_batch_step(b, kind == 0 ? 1 : 3, b->stream);
       HIP_TRY(hipStreamEndCapture(b->stream, &graph));
-      e = hipGraphInstantiate(&b->graph_exec, graph, nullptr, nullptr, 0);
+      if (kind == 1) batch_swap(b);
+      e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
     }
     (void)hipGraphDestroy(graph);
     if (e != hipSuccess) return set_error(GMES_EDEVICE, "hipGraphInstantiate: %s", hipGetErrorString(e));
@@ -4352,8 +4375,7 @@ int gmes_batch_set_graph(gmes_batch* b, int32_t enable) {
 }
 
 // Advance every member by nsteps: one batched launch per kernel kind (and half
-// step, for members that take those), replayed from a captured graph of a step
-// or, with one-sweep members, of two.
+// step, for members that take those), replayed from captured graphs.
 int gmes_batch_step(gmes_batch* b, int64_t nsteps) {
   ApiGuard api;
   if (!b) return set_error(GMES_EINVAL, "null batch handle");
@@ -4372,13 +4394,16 @@ int gmes_batch_step(gmes_batch* b, int64_t nsteps) {
   bool ready = false;
   while (!ready)
     if (int rc = batch_ready(b, nsteps, ready)) return rc;
-  int64_t t = 0;
-  if (b->graph_exec && !b->timing.on)
-    for (; t + b->per + b->per - 1 <= nsteps; t += b->per) HIP_TRY(hipGraphLaunch(b->graph_exec, b->stream));
-  for (; t < nsteps; ++t) enqueue_batch_step(b, (int)(t & 1) + (t == nsteps - 1 ? 2 : 0), b->stream);
-  HIP_TRY(hipGetLastError());
-  if (nsteps & 1)
-    for (gmes_sim* s : b->sweepers) ++s->gen;  // captured arguments hold the other set's pointers
+  if (!b->use_graph || b->timing.on) {
+    for (int64_t t = 0; t < nsteps; ++t) enqueue_batch_step(b, (int)(t & 1) + (t == nsteps - 1 ? 2 : 0), b->stream);
+    HIP_TRY(hipGetLastError());
+  } else if (b->sweepers.empty()) {
+    for (int64_t t = 0; t < nsteps; ++t) HIP_TRY(hipGraphLaunch(batch_graph(b, 0), b->stream));
+  } else {
+    for (int64_t t = 0; t + 2 < nsteps; t += 2) HIP_TRY(hipGraphLaunch(batch_graph(b, 0), b->stream));
+    HIP_TRY(hipGraphLaunch(batch_graph(b, nsteps % 2 ? 1 : 2), b->stream));
+    if (nsteps % 2) batch_swap(b);
+  }
   for (gmes_sim* s : b->sims) advance_host_clock(s, nsteps);
   return GMES_OK;
 }
