@@ -756,15 +756,17 @@ void enqueue_src(gmes_sim* s, bool electric, hipStream_t st) {
   time_end(s, st);
 }
 
+// Records the probes of one field type or, after a one-sweep step, of both.
+constexpr int kProbeH = 0, kProbeE = 1, kProbeBoth = 2;
 template <class T>
-void enqueue_probe(gmes_sim* s, bool electric, hipStream_t st) {
+void enqueue_probe(gmes_sim* s, int types, hipStream_t st) {
   if (s->probes.empty()) return;
   ProbeArgs<T> a{};
   a.fa = field_args<T>(s);
   a.cells = s->d_probe_cells;
   a.comps = s->d_probe_comps;
   a.n = (int)s->probes.size();
-  a.electric = electric;
+  a.types = types;
   a.buf = s->d_probe_buf;
   a.cap = s->probe_cap;
   a.ctl = reinterpret_cast<Ctl*>(s->d_clock);
@@ -2294,19 +2296,17 @@ void enqueue_step_t(gmes_sim* s, hipStream_t st) {
         time_begin(s, 2, st);
         launch_fix_e<T>(fix_args<T>(s), st);  // reads the auxiliary grids before their step
         time_end(s, st);
-        enqueue_probe<T>(s, true, st);
         enqueue_aux_steps(s, true, st);
         if (s->sweep_ghosts) enqueue_ghost<T>(s, true, 0, st);
         time_begin(s, 3, st);
         launch_fix_h<T>(fix_args<T>(s), st);
         time_end(s, st);
-        enqueue_probe<T>(s, false, st);
+        enqueue_probe<T>(s, kProbeBoth, st);
         enqueue_dft<T>(s, st);
         return;
       }
     }
-    enqueue_probe<T>(s, true, st);
-    enqueue_probe<T>(s, false, st);
+    enqueue_probe<T>(s, kProbeBoth, st);
     enqueue_dft<T>(s, st);
     return;
   }
@@ -2314,12 +2314,12 @@ void enqueue_step_t(gmes_sim* s, hipStream_t st) {
   enqueue_main<T>(s, true, st);
   enqueue_ade<T>(s, st);
   enqueue_src<T>(s, true, st);
-  enqueue_probe<T>(s, true, st);
+  enqueue_probe<T>(s, kProbeE, st);
   enqueue_aux_steps(s, false, st);
   if (!s->fuse_e) enqueue_ghost<T>(s, true, 0, st);
   enqueue_main<T>(s, false, st);
   enqueue_src<T>(s, false, st);
-  enqueue_probe<T>(s, false, st);
+  enqueue_probe<T>(s, kProbeH, st);
   enqueue_dft<T>(s, st);
 }
 
@@ -4148,14 +4148,13 @@ void enqueue_sweep_set(gmes_batch* b, int variant, hipStream_t st) {
     launch_fix_batch<T>(true, job_ptr<FixJob<T>>(b, S.fix_e.off), S.fix_e.njobs, S.fix_e.nblocks, st);
   btime_end(b, true, st);
   btime_begin(b, true, 5, st);
-  for (gmes_sim* s : b->sweepers) enqueue_probe<T>(s, true, st);
   launch_step1d_batch<T>(job_ptr<Step1Job<T>>(b, S.aux.off), S.aux.njobs, S.aux.nblocks, st);
   for (gmes_sim* s : b->sweepers) sweep_swap_aux(s);
   if (S.ghost.njobs)
     launch_ghost_batch<T>(job_ptr<GhostJob<T>>(b, S.ghost.off), S.ghost.njobs, S.ghost.nblocks, 0, st);
   if constexpr (!std::is_same<T, cplx<double>>::value)
     launch_fix_batch<T>(false, job_ptr<FixJob<T>>(b, S.fix_h.off), S.fix_h.njobs, S.fix_h.nblocks, st);
-  for (gmes_sim* s : b->sweepers) enqueue_probe<T>(s, false, st);
+  for (gmes_sim* s : b->sweepers) enqueue_probe<T>(s, kProbeBoth, st);
   if (S.dft.njobs) launch_dft_batch<T>(job_ptr<DftJob<T>>(b, S.dft.off), S.dft.njobs, S.dft.nblocks, st);
   btime_end(b, true, st);
 }

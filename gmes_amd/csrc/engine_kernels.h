@@ -425,7 +425,7 @@ struct ProbeArgs {
   const int64_t* cells;
   const int32_t* comps;
   int n;
-  int electric;
+  int types;  // 0: H, 1: E, 2: both
   double* buf;
   int64_t cap;
   Ctl* ctl;

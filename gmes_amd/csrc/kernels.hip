@@ -1089,7 +1089,7 @@ __global__ void k_probe(ProbeArgs<T> m) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= m.n) return;
   const int c = m.comps[p];
-  if ((c < 3) != m.electric) return;
+  if (m.types != 2 && (c < 3) != (m.types == 1)) return;
   const T v = m.fa.f[c][m.cells[p]];
   const int64_t pos = (m.ctl->clock - 1) - m.ctl->probe_base;
   double* out = m.buf + (p * m.cap + pos) * 2;
