@@ -4,7 +4,7 @@ A ``Batch`` groups initialised FDTD objects of one precision and field type
 (real or complex).  Each keeps its own fields, materials, sources, probes
 and clock; a step of the batch runs the members' kernels of one kind as one
 launch (the engine maps blocks to members through a device job table) and
-is replayed from one captured HIP graph.  Members may differ in size, mode
+is replayed from captured HIP graphs.  Members may differ in size, mode
 and materials.  Members whose own step is a one-sweep step take it here too;
 the others run main, source and ghost kernels, whose main launches use flat
 blocks of 256 consecutive cells and need no tile; autotune=True still tunes

@@ -3932,6 +3932,14 @@ void sweep_swap_aux(gmes_sim* s) {
     if (s->aux[i]) sweep_swap(s->aux[i]);
 }
 
+// The buffers of the one-sweep members become the other set.
+void batch_swap(gmes_batch* b) {
+  for (gmes_sim* s : b->sweepers) {
+    sweep_swap(s);
+    sweep_swap_aux(s);
+  }
+}
+
 // Planes (rows) per block of a batch's one-sweep members, from its tiles times
 // planes (rows).  As in sweep2_shape, fewer while they fill the chip badly (us
 // per step at 3, 5, 7, 9, 16 planes: 476 tile planes 36, 43, 48, 54, 63; 2199
@@ -3943,9 +3951,11 @@ int batch_ch2(double work) { return std::max(1, std::min(5, (int)std::ceil(std::
 
 // Job tables of the one-sweep members.  The arguments of a step are taken
 // from the sims as that step finds them: the host's pointers are swapped
-// twice on the way and end where they were.
+// on the way and end where they were.  A call of one step leaves out the second
+// one's (gmes_batch::sweep [1] and [3] stay as they were, at the end of the
+// tables).
 template <class T>
-void build_sweep_jobs(gmes_batch* b) {
+void build_sweep_jobs(gmes_batch* b, int64_t nsteps) {
   std::vector<Step3Job<T>> j3[2][4];
   std::vector<Step2Job<T>> j2[2];
   std::vector<Step1Job<T>> j1[2], ja;
@@ -3956,7 +3966,8 @@ void build_sweep_jobs(gmes_batch* b) {
     else if (!s->sweep_1d) work3 += (double)s->g.nx * s->g.ny / std::max(1, 768 / s->g.nz - 1);
   }
   const int ch3 = batch_ch3(work3), ch2 = batch_ch2(work2);
-  for (int t = 0; t < 2; ++t) {
+  const int steps = nsteps > 1 ? 2 : 1;
+  for (int t = 0; t < steps; ++t) {
     std::vector<FixJob<T>> je, jh;
     std::vector<GhostJob<T>> jg[2];
     std::vector<DftJob<T>> jd;
@@ -3970,34 +3981,39 @@ void build_sweep_jobs(gmes_batch* b) {
     ja.clear();
     for (gmes_sim* s : b->sweepers) {
       const bool always = sweep_ghosts(s);
-      for (int g = 0; g < 2; ++g) {
-        s->sweep_ghosts = always || g;
-        if (s->sweep_1d) {
-          Step1Job<T> J{step1_args<T>(s), n1};
-          if (g) n1 += (J.a.n + kStep1Threads - 2) / (kStep1Threads - 1);
-          j1[g].push_back(J);
-        } else if (s->sweep_2d) {
-          Step2Job<T> J{step2_args<T>(s), step2_tm(s), s->sweep_absorber, n2};
-          // blocks of kStep2BatchThreads threads, a few rows each
-          J.a.whole = J.a.n[1] <= kStep2BatchThreads;
-          J.a.w = J.a.whole ? J.a.n[1] : 224;
-          J.a.ch = std::min(ch2, J.a.n[0]);
-          J.a.nj = (J.a.n[1] + J.a.w - 1) / J.a.w;
-          J.a.nblk = J.a.nj * ((J.a.n[0] + J.a.ch - 1) / J.a.ch);
-          if (g) n2 += (J.a.nblk + 7) / 8 * 8;
-          lds2 = std::max(lds2, step2_lds<T>(kStep2BatchThreads, J.a.nent));
-          j2[g].push_back(J);
-        } else if constexpr (!std::is_same<T, cplx<double>>::value) {
-          gmes_sim::SweepPart part;
-          bool lean;
-          (void)sweep_batch_part(s, part, lean, ch3);
-          Step3Job<T> J{step3_args<T>(s, part), 0};
-          const int x = (std::is_same<T, double>::value && J.a.exact) + 2 * lean;
-          J.block0 = n3[x];
-          if (g) n3[x] += 8 * (int64_t)J.a.slots;
-          lds3[x] = std::max(lds3[x], step3_lds<T>(part.threads, J.a.net + J.a.nht, part.rows, s->g.nz, s->sweep_absorber));
-          j3[g][x].push_back(J);
-        }
+      s->sweep_ghosts = true;
+      auto add = [&](auto& v, auto& J) {  // with the ghost planes, and without
+        v[1].push_back(J);
+        J.a.ghosts = always;
+        v[0].push_back(J);
+      };
+      if (s->sweep_1d) {
+        Step1Job<T> J{step1_args<T>(s), n1};
+        n1 += (J.a.n + kStep1Threads - 2) / (kStep1Threads - 1);
+        add(j1, J);
+      } else if (s->sweep_2d) {
+        Step2Job<T> J{step2_args<T>(s), step2_tm(s), s->sweep_absorber, n2};
+        // blocks of kStep2BatchThreads threads, a few rows each
+        J.a.whole = J.a.n[1] <= kStep2BatchThreads;
+        J.a.w = J.a.whole ? J.a.n[1] : 224;
+        J.a.ch = std::min(ch2, J.a.n[0]);
+        J.a.nj = (J.a.n[1] + J.a.w - 1) / J.a.w;
+        J.a.nblk = J.a.nj * ((J.a.n[0] + J.a.ch - 1) / J.a.ch);
+        n2 += (J.a.nblk + 7) / 8 * 8;
+        lds2 = std::max(lds2, step2_lds<T>(kStep2BatchThreads, J.a.nent));
+        add(j2, J);
+      } else if constexpr (!std::is_same<T, cplx<double>>::value) {
+        gmes_sim::SweepPart part;
+        bool lean;
+        (void)sweep_batch_part(s, part, lean, ch3);
+        Step3Job<T> J{step3_args<T>(s, part), 0};
+        const int x = (std::is_same<T, double>::value && J.a.exact) + 2 * lean;
+        J.block0 = n3[x];
+        n3[x] += 8 * (int64_t)J.a.slots;
+        lds3[x] = std::max(lds3[x], step3_lds<T>(part.threads, J.a.net + J.a.nht, part.rows, s->g.nz, s->sweep_absorber));
+        j3[1][x].push_back(J);
+        J.a.ghosts = always;
+        j3[0][x].push_back(J);
       }
       sweep_swap(s);
       if constexpr (!std::is_same<T, cplx<double>>::value) {
@@ -4032,6 +4048,7 @@ void build_sweep_jobs(gmes_batch* b) {
       using J = typename std::decay<decltype(v[0])>::type;
       return gmes_batch::Launch{append_table(b->h_jobs, v.data(), v.size() * sizeof(J)), (int)v.size(), blocks};
     };
+    const gmes_batch::Launch la = put(ja, na), le = put(je, ne), lh = put(jh, nh), ld = put(jd, nd);
     for (int g = 0; g < 2; ++g) {
       gmes_batch::SweepSet& S = b->sweep[t + 2 * g];
       for (int x = 0; x < 4; ++x) {
@@ -4040,23 +4057,24 @@ void build_sweep_jobs(gmes_batch* b) {
       }
       S.s2 = put(j2[g], n2);
       S.s1 = put(j1[g], n1);
-      S.aux = put(ja, na);
-      S.fix_e = put(je, ne);
-      S.fix_h = put(jh, nh);
+      S.aux = la;
+      S.fix_e = le;
+      S.fix_h = lh;
       S.ghost = put(jg[g], ng[g]);
-      S.dft = put(jd, nd);
+      S.dft = ld;
       S.lds2 = lds2;
     }
   }
+  if (steps == 1) batch_swap(b);
 }
 
 // One step of a group of sims (the members, or their auxiliary grids)
 // with one launch per kernel kind.
 template <class T>
-void build_tables(gmes_batch* b) {
-  build_sweep_jobs<T>(b);
+void build_tables(gmes_batch* b, int64_t nsteps) {
   build_jobs<T>(b, b->others, b->set);
   build_jobs<T>(b, b->aux_sims, b->aux_set);
+  build_sweep_jobs<T>(b, nsteps);
 }
 
 // HIP events around the launches of one kernel family of a batch step
@@ -4195,14 +4213,6 @@ std::vector<uint64_t> batch_gens(const gmes_batch* b) {
   return gens;
 }
 
-// The buffers of the one-sweep members become the other set.
-void batch_swap(gmes_batch* b) {
-  for (gmes_sim* s : b->sweepers) {
-    sweep_swap(s);
-    sweep_swap_aux(s);
-  }
-}
-
 hipGraphExec_t& batch_graph(gmes_batch* b, int kind) {
   return b->graphs[b->sweepers.empty() ? 0 : b->sweepers[0]->par][kind];
 }
@@ -4237,10 +4247,10 @@ int batch_ready(gmes_batch* b, int64_t nsteps, bool& ready) {
       if (s->aux[i]) b->aux_sims.push_back(s->aux[i]);
   b->h_jobs.clear();
   switch (b->dtype) {
-    case GMES_F32: build_tables<float>(b); break;
-    case GMES_F64: build_tables<double>(b); break;
-    case GMES_C64: build_tables<cplx<float>>(b); break;
-    default: build_tables<cplx<double>>(b); break;
+    case GMES_F32: build_tables<float>(b, nsteps); break;
+    case GMES_F64: build_tables<double>(b, nsteps); break;
+    case GMES_C64: build_tables<cplx<float>>(b, nsteps); break;
+    default: build_tables<cplx<double>>(b, nsteps); break;
   }
   if (b->h_jobs.size() > b->jobs_cap) {
     destroy_batch_graph(b);

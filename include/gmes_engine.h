@@ -296,8 +296,8 @@ int gmes_sim_read_profile(gmes_sim* sim, double ms[6], int64_t launches[6]);
 /* ---- batches (many sims, one launch per kernel kind) ---------------------
  * Members keep their own fields, tables and clocks; the members' kernels of
  * one kind run as one launch (a device job table maps blocks to members),
- * and a step of the whole batch (two, when members take one-sweep steps) is
- * one captured HIP graph.  A member is not stepped on its own while in a batch.  No
+ * and steps of the whole batch (one; with one-sweep members two, and the last
+ * ones of a call) are captured HIP graphs.  A member is not stepped on its own while in a batch.  No
  * reference counterpart: the reference advances one FDTD at a time
  * (gmes/fdtd.py:1099-1122). */
 
