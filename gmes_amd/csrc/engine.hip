@@ -19,7 +19,7 @@
 #include <shared_mutex>
 #include <string>
 #include <unordered_set>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <atomic>
 #include <vector>
@@ -103,8 +103,9 @@ void host_parallel(int n, int64_t cells, F f) {
   };
   std::vector<std::thread> t;
   try {
+    t.reserve(nt);  // a vector that could not grow would take its threads with it
     for (int q = 1; q < nt; ++q) t.emplace_back(work);
-  } catch (const std::system_error&) {  // no more threads: the ones there do it
+  } catch (const std::exception&) {  // no more threads, or no memory for one: the ones there do it
   }
   work();
   for (auto& x : t) x.join();
