@@ -51,8 +51,7 @@ namespace gmes_engine {
 // offset, the lane's place in the plane as vector offset.  One scalar offset
 // serves every array of a stagger, so an access costs no address arithmetic
 // (with 64-bit pointers the march spent 236 scalar instructions a plane, and
-// a CU's one scalar unit was the bound).  A lane offset past the resource
-// (kNowhere) loads zero and stores nothing.
+// a CU's one scalar unit was the bound).
 __device__ float raw_load_f32(i4_t r, int v, int s, int aux) __asm("llvm.amdgcn.raw.buffer.load.f32");
 __device__ vec2_t<float> raw_load_v2f32(i4_t r, int v, int s, int aux) __asm("llvm.amdgcn.raw.buffer.load.v2f32");
 __device__ void raw_store_f32(float x, i4_t r, int v, int s, int aux) __asm("llvm.amdgcn.raw.buffer.store.f32");
@@ -60,7 +59,6 @@ __device__ void raw_store_v2f32(vec2_t<float> x, i4_t r, int v, int s, int aux) 
 __device__ short raw_load_i16(i4_t r, int v, int s, int aux) __asm("llvm.amdgcn.raw.buffer.load.i16");
 __device__ int raw_load_i32(i4_t r, int v, int s, int aux) __asm("llvm.amdgcn.raw.buffer.load.i32");
 
-constexpr unsigned kNowhere = 0xFFFFFFF0u;
 constexpr int kAuxNt = 2;  // non-temporal
 
 // One dword per active lane from memory straight into LDS, at lds (bytes
@@ -441,8 +439,9 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
     }
   };
 
-  // Results are stored one step late, behind the loads of the next plane:
-  // stores of a plane are not in the way of the loads it waits for.
+  // Results are stored one step late, behind the loads of the next plane, which
+  // are on their way before them.  (The wait for loads into LDS is for stores too:
+  // one counter, in order.)
   for (int qv = i0; qv <= i1; ++qv) {
     const int q = __builtin_amdgcn_readfirstlane(qv);
     // CPML words along x and y, where there are any, for E at this plane and

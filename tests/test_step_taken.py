@@ -194,3 +194,17 @@ def test_media_and_sources(engine_lib, kind, graph, wave):
     a._advance(3)
     for c, v in want.items():
         np.testing.assert_array_equal(a.field[c], v)
+
+
+@pytest.mark.parametrize("kind", sorted(KINDS3))
+@pytest.mark.parametrize("n", [(1, 8, 8), (2, 2, 2), (8, 9, 1), (1, 2, 1), (3, 1200, 1), (1, 40, 70), (2, 3, 341), (70, 2, 1)],
+                         ids=lambda n: "x".join(map(str, n)))
+def test_thin_boxes(engine_lib, kind, n):
+    """Boxes of one or two cells along an axis."""
+    a, b = (box(engine_lib, n, **KINDS3[kind]) for _ in range(2))
+    engine_lib.set_ghost_fusion(b._sim, 0)
+    assert swept(engine_lib, a) and not swept(engine_lib, b)
+    for k in (1, 4):
+        a._advance(k)
+        b._advance(k)
+        t3.agree(a, b)
