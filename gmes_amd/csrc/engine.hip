@@ -1102,8 +1102,9 @@ void sweep_entry(const gmes_sim* s, const std::array<uint16_t, 3>& rec, StepEnt<
 constexpr int64_t kSweepSplitBytes = 5 << 20;
 constexpr int kSweepOuterPlanes = 6, kSweepInnerPlanes = 9;
 
-// Whole rows a block needs, so that the rim row, whose E it computes again, is
-// worth it: three; with UPML, or in complex sims CPML along x or y, whose
+// Whole rows that have to fit a block, so that the rim row, whose E it computes
+// again, is worth it (it may take fewer, three at least: 181 x 203 x 225 FP32 UPML
+// 168 us with three, 238 with four): three; with UPML, or in complex sims CPML along x or y, whose
 // bodies hold few waves, five of 8-byte words and four of 4-byte ones, unless
 // the launches bound the two-kernel step (us per step, that one against this:
 // complex FP32 CPML 120 x 30 x 200 46, 58; 160^3 163, 168; 144^3, five rows,
@@ -1131,7 +1132,8 @@ double sweep_shape(const gmes_sim* s, int nent, int absorber, int ni, int nj, gm
   const int nz = s->g.nz;
   double best = 0;
   part.absorber = absorber;
-  for (int rows = sweep_min_rows(s, absorber); rows <= nj + 1; ++rows) {
+  if (sweep_min_rows(s, absorber) * nz > step3_max_threads<T>(absorber)) return 0;
+  for (int rows = kSweepMinRows; rows <= nj + 1; ++rows) {
     const int threads = (rows * nz + 63) / 64 * 64, most = step3_max_threads<T>(absorber);
     if (threads > most) break;
     const int64_t lds = (int64_t)step3_lds<T>(threads, nent, rows, nz, absorber);
