@@ -565,13 +565,11 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
                   ry = CP && !LY ? dead_row<R, PML>() : lds_row<R, PML>(rows_y + tj * rs),
                  rz = lds_row<R, PML>(rows_z + k * rs);
       if constexpr (CP) {
-        T dead1, dead2;
         nex = cpml_value<true, X>(en.c[0], l.e0, vsub(l.hz, hzj), vsub(l.hy, hyk), d1, v1, d2, v2, ry, rz, s00, l.s[0],
                                   n[0][0], n[0][1], en.meta & 2u);
         ney = cpml_value<true, X>(en.c[1], l.e1, vsub(l.hx, hxk), vsub(l.hz, hzp), d2, v2, d0, v0, rz, rx, l.s[1], s11,
                                   n[1][0], n[1][1], en.meta & 4u);
-        if constexpr (!LX && !LY) nez = cpml_value<true, X>(en.c[2], l.e2, vsub(l.hy, hyp), vsub(l.hx, hxj), d0, v0, d1, v1,
-                                  dead_row<R, PML>(), dead_row<R, PML>(), T{}, T{}, dead1, dead2, en.meta & 8u);
+        if constexpr (!LX && !LY) nez = dead_value<true, X>(en.c[2], l.e2, vsub(l.hy, hyp), vsub(l.hx, hxj), d0, v0, d1, v1, en.meta & 8u);
         else nez = cpml_value<true, X>(en.c[2], l.e2, vsub(l.hy, hyp), vsub(l.hx, hxj), d0, v0, d1, v1, rx, ry, s20, s21,
                                   n[2][0], n[2][1], en.meta & 8u);
       } else {
@@ -680,13 +678,11 @@ __device__ __forceinline__ void step3d_tile(StepPtr<T> mp, unsigned blk, char* l
                     ry = CP && !LY ? dead_row<R, PML>() : lds_row<R, PML>(rows_yh + tj * rs),
                    rz = lds_row<R, PML>(rows_zh + k * rs);
         if constexpr (CP) {
-          T dead1, dead2;
           nhx = cpml_value<false, X>(eh.c[0], hx, vsub(ezj, ez), vsub(eyk, ey), d1, v1, d2, v2, ry, rz, g00, l.g[0],
                                      r[0][0], r[0][1], eh.meta & 2u);
           nhy = cpml_value<false, X>(eh.c[1], hy, vsub(exk, ex), vsub(ezi, ez), d2, v2, d0, v0, rz, rx, l.g[1], g11,
                                      r[1][0], r[1][1], eh.meta & 4u);
-          if constexpr (!LX && !LY) nhz = cpml_value<false, X>(eh.c[2], hz, vsub(eyi, ey), vsub(exj, ex), d0, v0, d1, v1,
-                                  dead_row<R, PML>(), dead_row<R, PML>(), T{}, T{}, dead1, dead2, eh.meta & 8u);
+          if constexpr (!LX && !LY) nhz = dead_value<false, X>(eh.c[2], hz, vsub(eyi, ey), vsub(exj, ex), d0, v0, d1, v1, eh.meta & 8u);
           else nhz = cpml_value<false, X>(eh.c[2], hz, vsub(eyi, ey), vsub(exj, ex), d0, v0, d1, v1, rx, ry, g20, g21,
                                      r[2][0], r[2][1], eh.meta & 8u);
         } else {

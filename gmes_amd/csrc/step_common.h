@@ -92,6 +92,31 @@ __device__ __forceinline__ T cpml_value(R c, T f, T D1, T D2, R d1, R i1, R d2, 
   }
 }
 
+// The same where both curl axes are dead: the words are +0, or NaN where the
+// difference is not finite.
+__device__ __forceinline__ float plus_zero(float a, float b) { return __builtin_fmaf(0.0f, a, b); }
+__device__ __forceinline__ double plus_zero(double a, double b) { return __builtin_fma(0.0, a, b); }
+template <class R>
+__device__ __forceinline__ cplx<R> plus_zero(cplx<R> a, cplx<R> b) {
+  return {plus_zero(a.re, b.re), plus_zero(a.im, b.im)};
+}
+template <bool E, bool X, class T, class R>
+__device__ __forceinline__ T dead_value(R c, T f, T D1, T D2, R d1, R i1, R d2, R i2, bool is) {
+  constexpr bool F = std::is_same<R, float>::value;
+  T a, b;
+  if constexpr (F) {
+    a = vscl(i1, D1);
+    b = vscl(i2, D2);
+  } else {
+    a = by_size<X>(D1, d1, i1);
+    b = by_size<X>(D2, d2, i2);
+  }
+  const T d = vsub(a, b), t = vadd(plus_zero(F ? b : D2, plus_zero(F ? a : D1, d)), T{});
+  const T u = vsel(is, E ? t : vneg(t), E ? d : vsub(b, a));
+  if constexpr (F) return fma_(c, u, f);
+  else return vadd(f, vscl(c, u));
+}
+
 // c: dt / eps; q: 1 / eps (FP32) or eps (FP64)
 template <bool E, bool X, class T, class R>
 __device__ __forceinline__ T upml_value(R q, T f, T D1, T D2, R d1, R i1, R d2, R i2, const Rows<R, 2>& r1,
