@@ -19,8 +19,12 @@
 // Neighbours come from LDS, not from overlapping global loads: with those
 // the L1 request rate bounds the kernel (256^3 FP32 without an absorber:
 // 228 us against 180 us, which is the rate of a copy of the same bytes).
-// Rows are whole so that every load starts on a line and the periodic wrap
-// along k stays inside the block.
+// Rows are whole so that the periodic wrap along k stays inside the block.
+//
+// A CPML cell and a Dielectric one beside it run the same instructions and differ
+// in the last operand, chosen by class (171 x 150 x 139 FP64 143 us without the
+// choice, 147 with it): where both words are dead the two values agree but where a
+// difference is not finite, and in zeros' signs.
 //
 // Blocks differ in the absorber words they hold: a body with none, with CPML
 // words along z (every row has those at both ends), along x and z, along y and
@@ -31,8 +35,8 @@
 //
 // Measured per step, two-kernel step first: FP32 256^3 CPML 344 -> 248 us (one
 // body for all blocks 293), 181 x 203 x 225 UPML 210 -> 168, 96^3 CPML 39 ->
-// 26, 64^3 UPML 24 -> 11; FP64 CPML 171 x 150 x 139 189 -> 143, 64^3 31 -> 19;
-// complex FP32 with z layers 192 x 192 x 128 190 -> 136, 112^3 72 -> 46.  What
+// 26, 64^3 UPML 24 -> 11; FP64 CPML 171 x 150 x 139 189 -> 147, 64^3 31 -> 17;
+// complex FP32 with z layers 192 x 192 x 128 190 -> 138, 112^3 72 -> 46.  What
 // bounds it: without an absorber the bytes (256^3 FP32 188 us, 4.3 TB/s); with
 // one the latency of a plane, 1 to 2 us, of which a CU has few in flight (24
 // waves in FP32, 12 to 16 with 8-byte words, by their registers: held to 128
