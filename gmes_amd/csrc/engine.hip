@@ -878,6 +878,7 @@ constexpr int64_t kSweepMaxTab = 24 * 1024;  // bytes of entries in LDS
 constexpr int kSweepMaxSrc = 16;
 constexpr int kSweepFloor = 20;        // waves whose plane takes as long as the latency of one
 constexpr int64_t kSweepLds = 160 * 1024;
+constexpr size_t kSweepAlign = 4096;
 
 // The two rows read along each axis by one field type agree; CPML: inside
 // the run without live state every row is (b, 0, 1).
@@ -1042,7 +1043,7 @@ std::vector<StepKey> sweep_keys(const std::vector<std::array<uint16_t, 3>>& ent)
   return tab;
 }
 
-int sweep_ids(gmes_sim* s) {
+int sweep_ids(gmes_sim* s, const std::vector<StepKey> (&tab)[2], char* d) {
   StepIdArgs a{};
   for (int c = 0; c < 6; ++c) {
     a.ids[c] = s->ids[c];
@@ -1056,23 +1057,16 @@ int sweep_ids(gmes_sim* s) {
   a.shift = s->step_eb;
   if (s->step_idw == 2) a.out16 = static_cast<uint16_t*>(s->d_step_ids);
   else a.out = static_cast<uint32_t*>(s->d_step_ids);
-  const std::vector<StepKey> tab[2] = {sweep_keys(s->step_e), sweep_keys(s->step_h)};
   const size_t b0 = tab[0].size() * sizeof(StepKey), b1 = tab[1].size() * sizeof(StepKey);
-  char* d = nullptr;
-  HIP_TRY(hipMalloc((void**)&d, b0 + b1));
-  hipError_t e = hipMemcpy(d, tab[0].data(), b0, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(d + b0, tab[1].data(), b1, hipMemcpyHostToDevice);
+  HIP_TRY(hipMemcpy(d, tab[0].data(), b0, hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(d + b0, tab[1].data(), b1, hipMemcpyHostToDevice));
   for (int h = 0; h < 2; ++h) {
     a.tab[h] = reinterpret_cast<const StepKey*>(d + (h ? b0 : 0));
     a.mask[h] = (uint32_t)tab[h].size() - 1;
   }
-  if (e == hipSuccess) {
-    launch_step_ids(a, s->stream);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-  (void)dev_release(d);
-  HIP_TRY(e);
+  launch_step_ids(a, s->stream);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipStreamSynchronize(s->stream));
   return GMES_OK;
 }
 
@@ -1259,22 +1253,40 @@ void fix_release(gmes_sim* s) {
   s->fix_bytes = 0;
 }
 
-void sweep_release(gmes_sim* s) {
-  void** bufs[] = {&s->f_alt[0], &s->f_alt[1], &s->f_alt[2], &s->f_alt[3], &s->f_alt[4], &s->f_alt[5],
-                   &s->pml_alt[0], &s->pml_alt[1], &s->pml_alt[2], &s->d_step_ids, &s->d_step_tab, (void**)&s->d_rare};
-  for (void** b : bufs)
-    if (*b) {
-      (void)dev_release(*b);
-      *b = nullptr;
+void sweep_swap(gmes_sim* s);
+
+// Gives back what one-sweep steps hold (the device is idle as far as s goes).
+// After an odd number of them the current buffers are the ones to be given back:
+// keep: their contents move to the sim's own.
+void sweep_release(gmes_sim* s, bool keep = true) {
+  if (s->sweep_mem && s->par != s->sweep_par0) {
+    auto move = [&](void* to, const void* from, size_t bytes) {
+      if (keep && to) (void)hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToDevice, s->stream);
+    };
+    for (int c = 0; c < 6; ++c) {
+      const size_t b = (size_t)s->dsize[c] * s->esize;
+      move(s->f_alt[c], s->f[c], b);
+      if (c >= 3) continue;
+      move(s->pml_alt[c], s->pml_state[c], (s->has_cls[c][GMES_CLS_CPML] ? 2 : 1) * b);
+      for (int k = 0; k < GMES_NCLS; ++k) {
+        const AdeList& L = s->ade[c][k];
+        move(s->ade_alt[c][k], L.state, (size_t)L.nstate * L.n * ade_word(s, k));
+      }
     }
-  for (int c = 0; c < 3; ++c) {
-    if (s->d_adeq[c]) (void)dev_release(s->d_adeq[c]);
-    s->d_adeq[c] = nullptr;
-    for (void*& p : s->ade_alt[c]) {
-      if (p) (void)dev_release(p);
-      p = nullptr;
-    }
+    if (keep) (void)hipStreamSynchronize(s->stream);
+    sweep_swap(s);
   }
+  s->clk_stale = true;  // Ctl::clk is by parity
+  if (s->sweep_mem) (void)dev_release(s->sweep_mem);
+  s->sweep_mem = nullptr;
+  for (void*& p : s->f_alt) p = nullptr;
+  for (int c = 0; c < 3; ++c) {
+    s->pml_alt[c] = nullptr;
+    s->d_adeq[c] = nullptr;
+    for (void*& p : s->ade_alt[c]) p = nullptr;
+  }
+  s->d_step_ids = s->d_step_tab = nullptr;
+  s->d_rare = nullptr;
   fix_release(s);
   s->sweep_fix = false;
   s->sweep_1d = s->sweep_2d = false;
@@ -1284,12 +1296,50 @@ void sweep_release(gmes_sim* s) {
   s->step_tab_cap = 0;
 }
 
+// What one-sweep steps hold, in one allocation (a dozen of them took 1 ms of
+// setting up a small sim): parts to be cleared, the others.
+struct SweepParts {
+  struct Part {
+    void** p;
+    size_t bytes;
+  };
+  std::vector<Part> cleared, other;
+  // E state of component c: its CPML or UPML words
+  void state(gmes_sim* s, int c) {
+    if (s->pml_state[c])
+      cleared.push_back({&s->pml_alt[c], (size_t)(s->has_cls[c][GMES_CLS_CPML] ? 2 : 1) * s->dsize[c] * s->esize});
+  }
+  // and that of its dispersive cells, with their places in the lists
+  void ade(gmes_sim* s, int c) {
+    bool any = false;
+    for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2; ++k) {
+      const AdeList& L = s->ade[c][k];
+      if (!L.n) continue;
+      any = true;
+      cleared.push_back({&s->ade_alt[c][k], (size_t)L.nstate * L.n * ade_word(s, k)});
+    }
+    if (any) other.push_back({(void**)&s->d_adeq[c], (size_t)s->dsize[c] * sizeof(int32_t)});
+  }
+};
+
 // (plain hipMalloc: a sim that finds no room does without)
-int sweep_alloc(gmes_sim* s, void** p, size_t bytes) {
-  if (bytes == 0) bytes = 16;
-  HIP_TRY(hipMalloc(p, bytes));
-  s->bytes += (int64_t)bytes;
-  s->sweep_bytes += (int64_t)bytes;
+int sweep_take(gmes_sim* s, const SweepParts& v) {
+  auto up = [](size_t b) { return (std::max<size_t>(b, 1) + kSweepAlign - 1) / kSweepAlign * kSweepAlign; };
+  size_t zero = 0, total = 0;
+  for (const auto& x : v.cleared) zero += up(x.bytes);
+  for (const auto& x : v.other) total += up(x.bytes);
+  total += zero;
+  HIP_TRY(hipMalloc(&s->sweep_mem, total));
+  s->bytes += (int64_t)total;
+  s->sweep_bytes += (int64_t)total;
+  s->sweep_par0 = s->par;
+  char* d = static_cast<char*>(s->sweep_mem);
+  for (const auto* list : {&v.cleared, &v.other})
+    for (const auto& x : *list) {
+      *x.p = d;
+      d += up(x.bytes);
+    }
+  if (zero) HIP_TRY(hipMemsetAsync(s->sweep_mem, 0, zero, s->stream));
   return GMES_OK;
 }
 
@@ -1411,25 +1461,11 @@ int sweep1_build(gmes_sim* s) {
   }
   std::unique_lock<std::mutex> room(g_room_mu);
   if (!sweep_room(s)) return GMES_OK;
-  int rc = GMES_OK;
-  for (const int c : comp) {
-    if (!rc) rc = sweep_alloc(s, &s->f_alt[c], (size_t)s->dsize[c] * s->esize);
-  }
-  if (!rc && s->pml_state[e]) {
-    const size_t b = (size_t)(cpml ? 2 : 1) * s->dsize[e] * s->esize;
-    rc = sweep_alloc(s, &s->pml_alt[e], b);
-    if (!rc) HIP_TRY(hipMemsetAsync(s->pml_alt[e], 0, b, s->stream));
-  }
-  bool any = false;
-  for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2 && !rc; ++k) {
-    const AdeList& L = s->ade[e][k];
-    if (!L.n) continue;
-    any = true;
-    const size_t b = std::max<size_t>(1, (size_t)L.nstate * L.n * ade_word(s, k));
-    rc = sweep_alloc(s, &s->ade_alt[e][k], b);
-    if (!rc) HIP_TRY(hipMemsetAsync(s->ade_alt[e][k], 0, b, s->stream));
-  }
-  if (any && !rc) rc = sweep_alloc(s, (void**)&s->d_adeq[e], (size_t)s->dsize[e] * sizeof(int32_t));
+  SweepParts parts;
+  for (const int c : comp) parts.other.push_back({&s->f_alt[c], (size_t)s->dsize[c] * s->esize});
+  parts.state(s, e);
+  parts.ade(s, e);
+  const int rc = sweep_take(s, parts);
   room.unlock();
   if (rc) {
     (void)hipGetLastError();
@@ -1562,9 +1598,14 @@ void sweep2_shape(gmes_sim* s) {
 }
 
 // Entries, their cells' details, the key table of the entry ids and the ids
-// themselves share one allocation, filled by one copy and one launch.
+// themselves are one part of a sim's second buffers, filled by one copy and one
+// launch: what is copied, and where its pieces begin.
+struct Sweep2Tables {
+  std::vector<char> host;
+  size_t cells_at, keys_at, ids_at, nkeys;
+};
 template <class R>
-int sweep2_tables(gmes_sim* s) {
+Sweep2Tables sweep2_host(const gmes_sim* s) {
   const size_t n = s->step_e.size();
   const std::vector<StepKey> keys = sweep_keys(s->step_e);
   const size_t cells_at = n * sizeof(Step2Ent<R>), keys_at = cells_at + 3 * n * sizeof(Step2Cell),
@@ -1585,12 +1626,15 @@ int sweep2_tables(gmes_sim* s) {
         tab[e].c[t] = r.cls == GMES_CLS_UPML ? (s->fp64 ? (R)r.eps_mu : (R)(1.0 / r.eps_mu)) : (R)(s->g.dt / r.eps_mu);
     }
   memcpy(host.data() + keys_at, keys.data(), keys.size() * sizeof(StepKey));
+  return {std::move(host), cells_at, keys_at, ids_at, keys.size()};
+}
+
+int sweep2_tables(gmes_sim* s, const Sweep2Tables& v) {
   const int64_t pi = s->pi[step2_comp(s, 0)];
-  if (int rc = sweep_alloc(s, &s->d_step_tab, ids_at + (size_t)(s->g.nx * pi) * sizeof(uint16_t))) return rc;
   char* d = static_cast<char*>(s->d_step_tab);
-  s->step2_cells = d + cells_at;
-  s->step2_ids = reinterpret_cast<uint16_t*>(d + ids_at);
-  HIP_TRY(hipMemcpy(d, host.data(), ids_at, hipMemcpyHostToDevice));
+  s->step2_cells = d + v.cells_at;
+  s->step2_ids = reinterpret_cast<uint16_t*>(d + v.ids_at);
+  HIP_TRY(hipMemcpy(d, v.host.data(), v.ids_at, hipMemcpyHostToDevice));
   StepIdArgs a{};
   for (int x = 0; x < 3; ++x) {
     const int c = step2_comp(s, x);
@@ -1598,8 +1642,8 @@ int sweep2_tables(gmes_sim* s) {
     a.first[x] = dev_index(s, c, step2_first(c, 0), step2_first(c, 1), s->shape[c][2] == 2 ? step2_first(c, 2) : 0);
     a.plane[x] = s->pi[c];
   }
-  a.tab[0] = reinterpret_cast<const StepKey*>(d + keys_at);
-  a.mask[0] = (uint32_t)keys.size() - 1;
+  a.tab[0] = reinterpret_cast<const StepKey*>(d + v.keys_at);
+  a.mask[0] = (uint32_t)v.nkeys - 1;
   a.n[0] = s->g.nx; a.n[1] = 1; a.n[2] = s->g.ny;
   a.pitch = (int)pi;
   a.types = 1;
@@ -1716,29 +1760,19 @@ int sweep2_build(gmes_sim* s) {
   std::unique_lock<std::mutex> room(g_room_mu);
   if (!sweep_room(s)) return GMES_OK;
   sweep2_shape(s);
-  int rc = GMES_OK;
-  for (int a = 0; a < 3 && !rc; ++a) {
+  const Sweep2Tables tables = s->fp64 ? sweep2_host<double>(s) : sweep2_host<float>(s);
+  SweepParts parts;
+  for (int a = 0; a < 3; ++a) {
     const int c = step2_comp(s, a);
-    rc = sweep_alloc(s, &s->f_alt[c], (size_t)s->dsize[c] * s->esize);
-    if (rc || c >= 3) continue;
-    if (s->pml_state[c]) {
-      const size_t b = (size_t)(cpml ? 2 : 1) * s->dsize[c] * s->esize;
-      rc = sweep_alloc(s, &s->pml_alt[c], b);
-      if (!rc) HIP_TRY(hipMemsetAsync(s->pml_alt[c], 0, b, s->stream));
-    }
-    bool any = false;
-    for (int k = GMES_CLS_DRUDE; k < GMES_CLS_DM2 && !rc; ++k) {
-      const AdeList& L = s->ade[c][k];
-      if (!L.n) continue;
-      any = true;
-      const size_t b = std::max<size_t>(1, (size_t)L.nstate * L.n * ade_word(s, k));
-      rc = sweep_alloc(s, &s->ade_alt[c][k], b);
-      if (!rc) HIP_TRY(hipMemsetAsync(s->ade_alt[c][k], 0, b, s->stream));
-    }
-    if (any && !rc) rc = sweep_alloc(s, (void**)&s->d_adeq[c], (size_t)s->dsize[c] * sizeof(int32_t));
+    parts.other.push_back({&s->f_alt[c], (size_t)s->dsize[c] * s->esize});
+    if (c >= 3) continue;
+    parts.state(s, c);
+    parts.ade(s, c);
   }
+  parts.other.push_back({&s->d_step_tab, tables.ids_at + (size_t)s->g.nx * s->pi[step2_comp(s, 0)] * sizeof(uint16_t)});
+  int rc = sweep_take(s, parts);
   room.unlock();
-  if (!rc) rc = s->fp64 ? sweep2_tables<double>(s) : sweep2_tables<float>(s);
+  if (!rc) rc = sweep2_tables(s, tables);
   if (rc) {  // no room for a second set of buffers
     (void)hipGetLastError();
     sweep_release(s);
@@ -2136,30 +2170,24 @@ int sweep_build(gmes_sim* s) {
   const int eb = bits(s->step_e.size() + kSweepMaxSrc), hb = bits(s->step_h.size() + kSweepMaxSrc);
   s->step_idw = eb + hb <= 16 ? 2 : 4;
   s->step_eb = eb + hb <= 16 ? eb : 16;
-  int rc = GMES_OK;
-  for (int c = 0; c < 6 && !rc; ++c) rc = sweep_alloc(s, &s->f_alt[c], (size_t)s->dsize[c] * s->esize);
-  for (int c = 0; c < 3 && !rc; ++c) {
-    if (!s->pml_state[c]) continue;
-    const size_t b = (size_t)(cpml ? 2 : 1) * s->dsize[c] * s->esize;
-    rc = sweep_alloc(s, &s->pml_alt[c], b);
-    if (!rc) HIP_TRY(hipMemset(s->pml_alt[c], 0, b));
-  }
-  if (!rc) rc = sweep_alloc(s, &s->d_step_ids, (size_t)s->g.nx * s->g.ny * s->pitch[0] * s->step_idw);
   s->step_tab_cap = (int64_t)(s->step_e.size() + s->step_h.size()) + 2 * kSweepMaxSrc;
-  if (!rc) rc = sweep_alloc(s, &s->d_step_tab, (size_t)s->step_tab_cap * ent);
-  if (!rc) rc = sweep_alloc(s, (void**)&s->d_rare, (size_t)s->step_tab_cap * 3 * sizeof(StepRare));
+  const std::vector<StepKey> keys[2] = {sweep_keys(s->step_e), sweep_keys(s->step_h)};
+  void* d_keys = nullptr;
+  SweepParts parts;
+  for (int c = 0; c < 6; ++c) parts.other.push_back({&s->f_alt[c], (size_t)s->dsize[c] * s->esize});
+  for (int c = 0; c < 3; ++c) parts.state(s, c);
+  parts.other.push_back({&s->d_step_ids, (size_t)s->g.nx * s->g.ny * s->pitch[0] * s->step_idw});
+  parts.other.push_back({&s->d_step_tab, (size_t)s->step_tab_cap * ent});
+  parts.other.push_back({(void**)&s->d_rare, (size_t)s->step_tab_cap * 3 * sizeof(StepRare)});
+  parts.other.push_back({&d_keys, (keys[0].size() + keys[1].size()) * sizeof(StepKey)});
+  int rc = sweep_take(s, parts);
   room.unlock();
   if (rc) {  // no room for a second set of buffers: the two-kernel step needs none
     (void)hipGetLastError();
     sweep_release(s);
     return GMES_OK;
   }
-  if ((rc = sweep_ids(s))) {
-    const bool room = rc != GMES_ENOMEM;
-    (void)hipGetLastError();
-    sweep_release(s);
-    return room ? rc : GMES_OK;
-  }
+  if ((rc = sweep_ids(s, keys, static_cast<char*>(d_keys)))) return rc;
   s->src_ids.clear();
   s->sweep_ok = true;
   return GMES_OK;
@@ -2874,6 +2902,7 @@ int gmes_sim_destroy(gmes_sim* s) {
     if (s->aux[i]) s->aux[i]->parent = nullptr;
   destroy_graph(s);
   collect_timing(s);
+  sweep_release(s, false);
   for (int c = 0; c < 6; ++c) {
     if (s->f[c]) (void)dev_release(s->f[c]);
     if (s->ids[c]) (void)dev_release(s->ids[c]);
@@ -2881,7 +2910,6 @@ int gmes_sim_destroy(gmes_sim* s) {
     if (s->pml_state[c]) (void)dev_release(s->pml_state[c]);
   }
   free_ade(s);
-  sweep_release(s);
   for (auto& d : s->dfts)
     if (d.acc) (void)dev_release(d.acc);
   void* bufs[] = {s->d_recs, s->d_coef, s->d_prof, s->d_prof_off, s->d_ops, s->d_groups, s->d_waves,

@@ -196,6 +196,8 @@ struct gmes_sim {
     int rect[9][6] = {};                      // i0, i1, j0, j1, planes per block, absorber
   };
   SweepPart sweep_part;
+  void* sweep_mem = nullptr;  // all of it, one allocation
+  int sweep_par0 = 0;         // parity at which f[] and its like are the sim's own buffers
   void* f_alt[6] = {};
   void* pml_alt[3] = {};
   int32_t sweep_run_e[3] = {}, sweep_run_h[3] = {};  // Step3Args::run_e, run_h

@@ -69,3 +69,49 @@ def test_sources_before_the_commit(engine_lib, case, precision, aux):
             x, y = np.array(a.field[c]), np.array(b.field[c])
             assert np.abs(y).max() > 0
             np.testing.assert_array_equal(x, y)
+
+
+KINDS = {"box": lambda lib, **k: box(lib, (22, 21, 24), bound=g.Cpml, **k),
+         "media": lambda lib, **k: media_box(lib, (22, 21, 24), wave=False, **k),
+         "plane": lambda lib, **k: plane(lib, "tez", (31, 33), bound=g.Upml, media=True, **k),
+         "line": lambda lib, **k: line(lib, "z", 300, bound=g.Cpml, media=True, **k)}
+
+
+@pytest.mark.parametrize("kind", sorted(KINDS))
+@pytest.mark.parametrize("what", ["commit", "aux"])
+@pytest.mark.parametrize("steps", [2, 3])
+def test_state_outlives_the_second_buffers(engine_lib, kind, what, steps):
+    """After an even or odd number of one-sweep steps the sim is committed
+    again, or (a plane or line) gets an auxiliary grid and takes two-kernel
+    steps; fields, absorber words, dispersive state and monitors go on."""
+    from gmes_amd.monitor import DftBox
+    lib = engine_lib
+    a, b = (KINDS[kind](lib, precision="fp64") for _ in range(2))
+    lib.set_ghost_fusion(b._sim, 0)
+    e, h = a._active[0], a._active[-1]
+    mons, pids, grids = [], [], []
+    for s in (a, b):
+        pids.append([lib.add_probe(s._sim, c.index, 2) for c in (e, h)])
+        mons.append(DftBox(s, h, (0, 0, 0), s._shape[h], [0.05, 0.1], 1))
+        s._advance(steps)
+        if what == "commit":
+            before = [np.array(s.field[c]) for c in s._active]
+            lib.commit(s._sim)
+            lib.sync(s._sim)
+            for c, x in zip(s._active, before):
+                s._dev_newer[c] = True
+                np.testing.assert_array_equal(np.array(s.field[c]), x)
+        else:
+            grids.append(line(lib, "z", 40, precision="fp64"))
+            lib.attach_aux(s._sim, grids[-1]._sim)
+            s._aux_fdtds.append(grids[-1])
+    for k in (1, 4, 2):
+        for s in (a, b):
+            s._advance(k)
+        for c in a._active:
+            np.testing.assert_array_equal(np.array(a.field[c]), np.array(b.field[c]))
+    np.testing.assert_array_equal(mons[0].values(), mons[1].values())
+    for p, q in zip(*pids):
+        x, y = lib.read_probe(a._sim, p), lib.read_probe(b._sim, q)
+        assert len(x) == steps + 7
+        np.testing.assert_array_equal(x, y)
