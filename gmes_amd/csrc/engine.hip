@@ -1726,7 +1726,13 @@ int sweep2_build(gmes_sim* s) {
     while (hi[1] < ny && !at(nx / 2, hi[1])) ++hi[1];
     bool free = hi[0] <= 0x7FFF && hi[1] <= 0x7FFF;
     for (int64_t i = lo[0]; free && i < hi[0]; ++i)
-      for (int64_t j = lo[1]; free && j < hi[1]; ++j) free = !at(i, j);
+      for (int a = 0; a < 3; ++a) {
+        const int64_t* n = s->shape[step2_comp(s, a)];
+        const uint16_t* r = ids[a] + i * n[1] * n[2];
+        char any = 0;
+        for (int64_t j = lo[1]; j < hi[1]; ++j) any |= is[r[j * n[2]]];
+        free = free && !any;
+      }
     for (int x = 0; x < 2; ++x) s->sweep_run2[0][x] = free ? (int32_t)(lo[x] | (hi[x] << 16)) : 0;
   }
   auto pow2 = [](double v) { int e; return std::frexp(v, &e) == 0.5; };
@@ -2988,12 +2994,18 @@ int gmes_sim_set_material_ids(gmes_sim* s, int32_t c, const uint16_t* ids, int64
   // in one contiguous transfer: a strided 2-D copy would wait for every
   // kernel running on the device, including other sims' batches
   std::vector<uint16_t> dev((size_t)s->dsize[c], 0);
-  const int64_t n1 = s->shape[c][1], n2 = s->shape[c][2], rows = s->shape[c][0] * n1;
-  for (int64_t r = 0; r < rows; ++r) {
-    uint16_t* d = dev.data() + dev_index(s, c, r / n1, r % n1, 0);
-    if (s->pk[c] == 1) memcpy(d, ids + r * n2, (size_t)n2 * sizeof(uint16_t));
-    else
-      for (int64_t k = 0; k < n2; ++k) d[k * s->pk[c]] = ids[r * n2 + k];
+  const int64_t n0 = s->shape[c][0], n1 = s->shape[c][1], n2 = s->shape[c][2];
+  for (int64_t i = 0; i < n0; ++i) {
+    const uint16_t* h = ids + i * n1 * n2;
+    if (s->pk[c] == 1) {
+      for (int64_t j = 0; j < n1; ++j)
+        memcpy(dev.data() + dev_index(s, c, i, j, 0), h + j * n2, (size_t)n2 * sizeof(uint16_t));
+    } else {  // collapsed z: rows along j, a plane for each k
+      for (int64_t k = 0; k < n2; ++k) {
+        uint16_t* d = dev.data() + dev_index(s, c, i, 0, k);
+        for (int64_t j = 0; j < n1; ++j) d[j] = h[j * n2 + k];
+      }
+    }
   }
   HIP_TRY(hipMemcpy(s->ids[c], dev.data(), dev.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
   s->committed = false;
