@@ -155,7 +155,8 @@ int gmes_sim_destroy(gmes_sim* sim);
 /* Shape of component comp (inactive -> 1,1,1). */
 int gmes_sim_shape(const gmes_sim* sim, int32_t comp, int64_t shape[3]);
 /* Bytes of device memory held by the sim (fields, state, tables; a sim that
- * takes one-sweep steps holds its fields and E state twice). */
+ * takes one-sweep steps holds its fields and E state twice, until another
+ * allocation of the engine finds no room: the second set is given back then). */
 int gmes_sim_footprint(const gmes_sim* sim, int64_t* bytes);
 
 /* ---- materials (replace PwMaterial attach/merge) ---------------------- */
